@@ -140,6 +140,23 @@ struct KParams
 };
 
 
+// Per macro-cell data of the element action (p2ElementAction), in a frame rotated
+// so that the shell map's normal n = grad lam is the third axis and scaled by |n|:
+// there lam(x) + lam0 = n . x is the third coordinate itself.  (Affine cells: the
+// computational frame.)  Rows of Dc: gradients of the barycentric coordinates
+// 1..3 of a micro-cell; xq: J (lam_1, lam_2, lam_3)_q; adet, cw: the factors of the
+// metric that are constant per micro-cell type (see p2ElementAction).
+template < class R >
+struct P2ActGeomT
+{
+   R   v0[3], hE[9];
+   R   Dc[6][9];
+   R   xq[6][11][3];
+   R   cw[6];
+   R   lam0, r0; // lam = z - lam0; radius / |dr| at the ray vertex
+   int kind;     // 0 affine, 1 shell
+};
+
 struct P2Operator : OperatorBase
 {
    Storage*               st = nullptr;
@@ -148,7 +165,8 @@ struct P2Operator : OperatorBase
    int                    nm                = 0; // number of sine modes of k (0: k = 1)
    DevBuf< CellGeom >     geom;
    std::map< int, DevBuf< P2CellGeom > >           tgeom;  // by P2 level
-   std::map< int, DevBuf< P2CellGeomT< float > > > tgeomF; // by P2 level, for the FP32 kernels
+   std::map< int, DevBuf< P2ActGeomT< double > > > ageom;  // by P2 level, of the element action
+   std::map< int, DevBuf< P2ActGeomT< float > > >  ageomF; // the same for the FP32 kernels
    DevBuf< KParams >      kpar;
    std::map< int, DevBuf< double > > invDiag; // by P2 level, lattice L+1 storage
    // k at the quadrature points (tile-major), by (level, value type of the table)
@@ -321,10 +339,24 @@ __device__ __forceinline__ double kAt( const P2CellGeom& g, const KParams& K, co
    return kEval( K, x );
 }
 
+// the coefficient of the element action at quadrature point q of a micro-cell of
+// type t: k(F(x)) times the factors of the blended metric that depend on the
+// point only, w_q |det J| |n|^2 |dr| / |x| with the sign of n . x (p2ElementAction)
+__device__ __forceinline__ double foldedCoefficient( const P2CellGeom& g, const KParams& K, int t, int q,
+                                                     const double x[3], double ls )
+{
+   const double c = cQW[q] * g.adet[t] * kAt( g, K, x, ls );
+   if ( !g.kind )
+      return c;
+   const double n2 = g.nl[0] * g.nl[0] + g.nl[1] * g.nl[1] + g.nl[2] * g.nl[2];
+   const double r2 = x[0] * x[0] + x[1] * x[1] + x[2] * x[2];
+   return copysign( c * n2 * fabs( g.dr ) / sqrt( r2 ), ls + g.lam0 );
+}
 
-// k(F(x_q)) for every quadrature point of every micro-cell, stored tile-major:
-// table[(tile * 11 + q) * 384 + thread] (zero for threads outside the macro-cell)
-// (computed in FP64 and rounded to the table's value type K)
+// the coefficient tables, tile-major: table[(tile * 11 + q) * 384 + thread] (zero
+// for threads outside the macro-cell).  FP64 tables hold foldedCoefficient, so
+// that the apply reads one value per point and forms no reciprocal square root;
+// FP32 and FP16 tables hold k itself, whose range those types can represent.
 template < class K >
 __global__ __launch_bounds__( kTileThreads ) void kP2TileCoefficients( const P2CellGeom* __restrict__ geom,
                                                                       const KParams* __restrict__ kp, int64_t mm,
@@ -340,7 +372,14 @@ __global__ __launch_bounds__( kTileThreads ) void kP2TileCoefficients( const P2C
    {
       const double* xq   = g.XQ[th.t][q];
       const double  x[3] = { th.p0[0] + xq[0], th.p0[1] + xq[1], th.p0[2] + xq[2] };
-      const double  v    = th.valid ? kAt( g, *kp, x, th.ls0 + xq[3] ) : 0.0;
+      double        v    = 0.0;
+      if constexpr ( std::is_same< K, double >::value )
+      {
+         if ( th.valid )
+            v = foldedCoefficient( g, *kp, th.t, q, x, th.ls0 + xq[3] );
+      }
+      else if ( th.valid )
+         v = kAt( g, *kp, x, th.ls0 + xq[3] );
       table[( lb * 11 + q ) * kTileThreads + threadIdx.x] = fromAcc< K >( typename Acc< K >::type( v ) );
    }
 }
@@ -647,9 +686,8 @@ static void surfacePointList( Context* ctx, Lattice& l )
    l.surfacePoints.upload( ctx, pts );
 }
 
-// y = A_e u for the micro-cell of th: the element action of
-// p2_div_k_grad_blending_q4 (11-point rule); kq(q) gives k at quadrature point q
-// of the micro-cell.
+// y = A_e u for a micro-cell: the element action of p2_div_k_grad_blending_q4
+// (11-point rule).
 //
 // With barycentric coordinates lam_0..3 (lam_0 = 1 - lam_1 - lam_2 - lam_3), the
 // P2 function u = sum_k u_k lam_k (2 lam_k - 1) + sum_(i<j) 4 u_ij lam_i lam_j has
@@ -665,17 +703,30 @@ static void surfacePointList( Context* ctx, Lattice& l )
 //   y_0 = 4 sum(T) - 3 sum(S),  y_k = 4 T_kk - S_k,
 //   y_0k = 4 (S_k - sum_j T_kj - sum_j T_jk),  y_kj = 4 (T_kj + T_jk).
 // Per quadrature point that leaves 9 FMA for g and 12 for the sums, besides
-// the blending.  The shell map F(x) = q(x) x has DF = q I + x w^T (w = grad q),
-// inverted in closed form (Sherman-Morrison); det DF = q^2 beta with
-// beta = q + w . x = s (n . x), s = sign(lam) dr / |x|, so the powers of q cancel.
-template < class R, class KQ >
-__device__ __forceinline__ void p2ElementAction( const P2CellGeomT< R >& g, const TileThread< R >& th, const R u[10],
-                                                 R y[10], KQ&& kq )
+// the blending.
+//
+// Blending.  The shell map F(x) = q(x) x, q = R / |x|, R = r0 + |lam| dr,
+// lam = n . x - lam0, has DF = q I + x w^T with w = s n - (q / |x|^2) x and
+// s = sign(lam) dr / |x|; with nu = n . x, beta = q + w . x = s nu, Sherman-Morrison
+// and det DF = q^2 beta give the metric
+//   |det DF| DF^-1 DF^-T = |s| sign(nu) { nu I - x n^T - n x^T
+//                                       + (|n|^2 + R^2 / (dr^2 |x|^2)) / nu  x x^T }.
+// In the frame of P2ActGeomT (third axis n, lengths times |n|) the braces are, with
+// z = nu, r2 = |x|^2 and rh = R / dr,  z I - x e_z^T - e_z x^T + (1 + rh^2/r2)/z x x^T,
+// and its product with v is, with p = (x . v) / (r2 z),
+//   (z v_x - gamma x, z v_y - gamma y, z p rh^2),  gamma = v_z - p (r2 + rh^2),
+// so that a point needs one reciprocal and no square root; the factor |s| sign(nu)
+// (and the scales of the frame) is part of the coefficient (foldedCoefficient).
+//
+// c0, c1, c2 and next: coefficients 0..2, and the one of point q + 3 (FOLDED: the
+// whole factor; otherwise k), so that three table loads are in flight.
+template < class R, bool FOLDED, bool STORED, class KQ >
+__device__ __forceinline__ void p2ElementAction( const P2ActGeomT< R >& g, int t, const R p0[3], const R u[10], R y[10],
+                                                 R c0, R c1, R c2, KQ&& next )
 {
-   using QC      = QuadConst< R >;
-   const R*  Dc  = g.Dc[th.t];
-   const R   adet = g.adet[th.t];
-   R         v0[3], V[3][3];
+   using QC     = QuadConst< R >;
+   const R* Dc  = g.Dc[t];
+   R        v0[3], V[3][3];
    {
       // d0 and B (symmetric) from the element values (edges 4..9 in the order
       // (0,1), (0,2), (0,3), (1,2), (1,3), (2,3))
@@ -702,51 +753,73 @@ __device__ __forceinline__ void p2ElementAction( const P2CellGeomT< R >& g, cons
       for ( int j = 0; j < 3; ++j )
          Tm[d][j] = R( 0 );
    }
+   // STORED is fully unrolled: the coefficient loads stay three points ahead without
+   // register moves that would wait for them, and the scalar loads of a point's
+   // constants are issued early
+   auto point = [&]( auto shell, int q, R cq ) {
+         const R* lq = QC::lam( q );
+         const R* xq = g.xq[t][q];
+         R        v[3], m[3];
+#pragma unroll
+         for ( int d = 0; d < 3; ++d )
+            v[d] = v0[d] + V[d][0] * lq[0] + V[d][1] * lq[1] + V[d][2] * lq[2];
+         if constexpr ( decltype( shell )::value )
+         {
+            const R x = p0[0] + xq[0], yy = p0[1] + xq[1], z = p0[2] + xq[2];
+            const R r2 = x * x + yy * yy + z * z;
+            const R rh = fabs( z - g.lam0 ) + g.r0;
+            const R r3 = rh * rh;
+            const R p  = ( x * v[0] + yy * v[1] + z * v[2] ) * fastRcp( r2 * z );
+            const R tt = p * r3;
+            const R ga = v[2] - ( p * r2 + tt );
+            if constexpr ( !FOLDED )
+               cq = cq * QC::w()[q] * g.cw[t] * copysign( fastRsqrt( r2 ), z );
+            const R cz = cq * z, cg = cq * ga;
+            m[0] = cz * v[0] - cg * x;
+            m[1] = cz * v[1] - cg * yy;
+            m[2] = cz * tt;
+         }
+         else
+         {
+            if constexpr ( !FOLDED )
+               cq = cq * QC::w()[q] * g.cw[t];
+#pragma unroll
+            for ( int d = 0; d < 3; ++d )
+               m[d] = cq * v[d];
+         }
+#pragma unroll
+         for ( int d = 0; d < 3; ++d )
+         {
+            Sm[d] += m[d];
+#pragma unroll
+            for ( int j = 0; j < 3; ++j )
+               Tm[d][j] += lq[j] * m[d];
+         }
+   };
+   auto points = [&]( auto shell ) {
+      if constexpr ( STORED )
+      {
+         R c[14] = { c0, c1, c2 };
+#pragma unroll
+         for ( int q = 0; q < 11; ++q )
+         {
+            if ( q + 3 < 11 )
+               c[q + 3] = next( q + 3 );
+            point( shell, q, c[q] );
+            __builtin_amdgcn_sched_barrier( 0 );
+         }
+      }
+      else
+      {
 #pragma unroll 1
-   for ( int q = 0; q < 11; ++q )
-   {
-      const R* lq = QC::lam( q );
-      R        v[3];
-#pragma unroll
-      for ( int d = 0; d < 3; ++d )
-         v[d] = v0[d] + V[d][0] * lq[0] + V[d][1] * lq[1] + V[d][2] * lq[2];
-      const R* xq = g.XQ[th.t][q];
-      R        cc = QC::w()[q] * adet * kq( q );
-      if ( g.kind )
-      {
-         const R x[3] = { th.p0[0] + xq[0], th.p0[1] + xq[1], th.p0[2] + xq[2] };
-         const R ls   = th.ls0 + xq[3];
-         const R r2   = x[0] * x[0] + x[1] * x[1] + x[2] * x[2];
-         const R irho = fastRsqrt( r2 );
-         const R qq   = ( g.r0 + fabs( ls ) * g.dr ) * irho;
-         const R s    = copysign( g.dr, ls ) * irho;
-         const R qr2  = qq * ( irho * irho );
-         R       w[3];
-#pragma unroll
-         for ( int d = 0; d < 3; ++d )
-            w[d] = s * g.nl[d] - qr2 * x[d];
-         const R beta = s * ( ls + g.lam0 );
-         const R ib   = fastRcp( beta );
-         const R t1   = ( x[0] * v[0] + x[1] * v[1] + x[2] * v[2] ) * ib;
-#pragma unroll
-         for ( int d = 0; d < 3; ++d )
-            v[d] -= w[d] * t1;
-         const R t2 = ( w[0] * v[0] + w[1] * v[1] + w[2] * v[2] ) * ib;
-#pragma unroll
-         for ( int d = 0; d < 3; ++d )
-            v[d] -= x[d] * t2;
-         cc *= fabs( beta );
+         for ( int q = 0; q < 11; ++q )
+            point( shell, q, next( q ) );
       }
-#pragma unroll
-      for ( int d = 0; d < 3; ++d )
-      {
-         const R m = cc * v[d];
-         Sm[d] += m;
-#pragma unroll
-         for ( int j = 0; j < 3; ++j )
-            Tm[d][j] += lq[j] * m;
-      }
-   }
+   };
+   if ( g.kind )
+      points( std::true_type{} );
+   else
+      points( std::false_type{} );
    R T[3][3], S[3];
 #pragma unroll
    for ( int k = 0; k < 3; ++k )
@@ -770,18 +843,41 @@ __device__ __forceinline__ void p2ElementAction( const P2CellGeomT< R >& g, cons
    y[9] = R( 4 ) * ( T[1][2] + T[2][1] );
 }
 
+// vertex 0 of the micro-cell of type t at anchor index a (ax + 4 ay + 16 az) of
+// tile tc in the frame of g, and whether the micro-cell lies in the macro-cell
+template < class R >
+__device__ __forceinline__ bool actVertex( const P2ActGeomT< R >& g, const TileCoord& tc, int64_t mm, int t, int a,
+                                           R p0[3] )
+{
+   const int32_t gx = int32_t( tc.x0 ) + ( a & 3 ), gy = int32_t( tc.y0 ) + ( ( a >> 2 ) & 3 ),
+                 gz = int32_t( tc.z0 ) + ( a >> 4 );
+   const R vx = R( gx + cVof[t][0][0] ), vy = R( gy + cVof[t][0][1] ), vz = R( gz + cVof[t][0][2] );
+#pragma unroll
+   for ( int d = 0; d < 3; ++d )
+      p0[d] = g.v0[d] + g.hE[3 * d] * vx + g.hE[3 * d + 1] * vy + g.hE[3 * d + 2] * vz;
+   return gx + gy + gz <= int32_t( mm ) - 1 - MicroCells::rowShift[t];
+}
+
+// k (FOLDED: the whole coefficient) of point q of the micro-cell (t, a), evaluated
+template < bool FOLDED >
+__device__ __forceinline__ double evaluatedCoefficient( const P2CellGeom& g, const KParams& K, const TileCoord& tc,
+                                                        int64_t mm, int t, int a, int q )
+{
+   const TileThread< double > th = tileThreadAt( g, tc, mm, t, a );
+   const double*              xq = g.XQ[t][q];
+   const double               x[3] = { th.p0[0] + xq[0], th.p0[1] + xq[1], th.p0[2] + xq[2] };
+   return FOLDED ? foldedCoefficient( g, K, t, q, x, th.ls0 + xq[3] ) : kAt( g, K, x, th.ls0 + xq[3] );
+}
+
 // y = A x on the cell lattices of level L+1 (halo positions included): the
-// element action of p2_div_k_grad_blending_q4 evaluated in barycentric form,
-//   gamma_k = sum_j u_j dphi_j/dlam_k,  g = sum_k gamma_k grad_c lam_k,
-//   y_i += sum_q w_q k_q |det DF J| dphi_i/dlam_k grad_c lam_k . (DF^-1 DF^-T g)
-// (grad_c: computational space), equal to the reference's element matrix times
-// the element vector.
+// element action of every micro-cell of a tile, equal to the reference's element
+// matrix times the element vector.
 // T: value type of src / dst; K: value type of the coefficient table; the
 // arithmetic runs in Acc<T> (FP64 for double, FP32 for float and half).
 // BATCH: 2^lv interleaved vectors (vector blockIdx.y, its coefficient table at
 // table + blockIdx.y * tstride); otherwise one vector.
 template < class T, class K, bool STORED, bool BATCH = false >
-__device__ __forceinline__ void p2TileApplyBody( const P2CellGeomT< typename Acc< T >::type >* __restrict__ geom,
+__device__ __forceinline__ void p2TileApplyBody( const P2ActGeomT< typename Acc< T >::type >* __restrict__ geom,
                                                  const P2CellGeom* __restrict__ geom64, const KParams* __restrict__ kp,
                                                  const K* __restrict__ table, int64_t mm, int64_t ntiles, int64_t sc1,
                                                  int64_t w1, const T* __restrict__ src, T* __restrict__ dst,
@@ -797,137 +893,109 @@ __device__ __forceinline__ void p2TileApplyBody( const P2CellGeomT< typename Acc
       src += blockIdx.y;
       dst += blockIdx.y;
    }
-   using R  = typename Acc< T >::type;
-   using QC = QuadConst< R >;
+   using R = typename Acc< T >::type;
    // Element results are summed with LDS atomics into a result box of their own
    // in FP64 (cleared while the loads are in flight, so a tile needs two
    // workgroup barriers), and in per-wavefront result boxes (waveBoxAccumulate)
    // in FP32, where the LDS atomics cost about half the kernel time (in FP64 the
-   // per-wavefront boxes are not faster).  LDS: the tile's source box and the
-   // staged coefficients (+ the FP64 result box; the FP32 result boxes reuse the
-   // staging space once every wavefront has integrated).
-   constexpr bool kAtomic = std::is_same< R, double >::value;
-   constexpr int  kStage  = kBox3 + ( STORED ? 11 * kTileThreads : 0 );
-   constexpr int  kLds    = kAtomic ? kStage + kBox3 : ( kStage > kWaveBoxes * kBox3 ? kStage : kWaveBoxes * kBox3 );
+   // per-wavefront boxes are not faster).
+   constexpr bool kFolded = std::is_same< R, double >::value;
+   constexpr int  kLds    = kFolded ? 2 * kBox3 : kWaveBoxes * kBox3;
    __shared__ R   lds[kLds];
    R* const       sb = lds;
-   R* const       sk = lds + kBox3;
-   R* const       sa = lds + kStage; // FP64: the result box, apart from the source box
+   R* const       sa = lds + kBox3; // FP64: the result box, apart from the source box
    const int64_t li = xcdBlock( ntiles );
    if ( li >= ntiles )
       return;
    int64_t         lb;
    const TileCoord tc   = tiles ? tileFromList( tiles, li, mm, lb ) : tileOfInterior( li, mm, lb );
    const int64_t   base = tc.c * sc1;
-   const int32_t   top  = int32_t( 2 * mm );
-   // the coefficient loads are issued first (their latency overlaps the box
-   // load) and parked in LDS, which keeps them out of the registers of the
-   // quadrature loop
-   // and the thread's (at most two) source-box values right behind them, so
-   // that the two load latencies overlap
-   static_assert( kBox3 <= 2 * kTileThreads, "two box points per thread" );
-   K kv[STORED ? 11 : 1];
+   const int       t = __builtin_amdgcn_readfirstlane( int( threadIdx.x ) >> 6 ), a = int( threadIdx.x ) & 63;
+   auto coefficient = [&]( int q ) -> R {
+      if constexpr ( STORED )
+         return R( toAcc( ( table + ( lb * 11 + q ) * kTileThreads )[threadIdx.x] ) );
+      else
+         return R( evaluatedCoefficient< kFolded >( geom64[tc.c], *kp, tc, mm, t, a, q ) );
+   };
+   // the first three coefficients and the thread's (at most two) source-box
+   // values are loaded back to back; the other coefficients follow three
+   // quadrature points ahead of their use
+   R c[3] = {};
    if constexpr ( STORED )
-   {
-#pragma unroll
-      for ( int q = 0; q < 11; ++q )
-         kv[q] = table[( lb * 11 + q ) * kTileThreads + threadIdx.x];
-   }
-   const T* srcC = src + ( base << lv );
-   T        bv[2];
-   bool     bin[2];
+      for ( int q = 0; q < 3; ++q )
+         c[q] = coefficient( q );
+   static_assert( kBox3 <= 2 * kTileThreads, "two box points per thread" );
+   const BoxOffsets bo( int32_t( w1 ), 2 * int32_t( tc.x0 ), 2 * int32_t( tc.y0 ), 2 * int32_t( tc.z0 ) );
+   const int32_t    room = int32_t( 2 * ( mm - tc.x0 - tc.y0 - tc.z0 ) ); // lx + ly + lz of the macro-cell's points
+   const T*         srcC = src + ( base << lv );
+   T*               dstC = dst + ( base << lv );
+   T                bv[2];
+   int32_t          off[2]; // lattice offset of the thread's box points, -1: outside
 #pragma unroll
    for ( int j = 0; j < 2; ++j )
    {
-      const int     p  = int( threadIdx.x ) + j * kTileThreads;
-      const int32_t lx = p % kBox, ly = ( p / kBox ) % kBox, lz = p / ( kBox * kBox );
-      const int32_t X = 2 * int32_t( tc.x0 ) + lx, Y = 2 * int32_t( tc.y0 ) + ly, Z = 2 * int32_t( tc.z0 ) + lz;
-      bin[j]          = p < kBox3 && X + Y + Z <= top;
-      bv[j]           = bin[j] ? srcC[int64_t( tetRowStart32( int32_t( w1 ), Y, Z ) + X ) << lv] : T( 0 );
+      const int32_t p = int32_t( threadIdx.x ) + j * kTileThreads;
+      int32_t       lx, ly, lz;
+      boxPoint( p, lx, ly, lz );
+      off[j] = ( j == 0 || p < kBox3 ) && lx + ly + lz <= room ? bo.at( lx, ly, lz ) : -1;
+      bv[j]  = off[j] >= 0 ? srcC[int64_t( off[j] ) << lv] : T( 0 );
    }
-   if constexpr ( kAtomic )
+   if constexpr ( kFolded )
    {
       // the result box is cleared while the loads are in flight
 #pragma unroll
       for ( int j = 0; j < 2; ++j )
-      {
-         const int p = int( threadIdx.x ) + j * kTileThreads;
-         if ( p < kBox3 )
-            sa[p] = R( 0 );
-      }
-   }
-   if constexpr ( STORED )
-   {
-#pragma unroll
-      for ( int q = 0; q < 11; ++q )
-         sk[q * kTileThreads + threadIdx.x] = R( toAcc( kv[q] ) );
+         if ( int( threadIdx.x ) + j * kTileThreads < kBox3 )
+            sa[int( threadIdx.x ) + j * kTileThreads] = R( 0 );
    }
 #pragma unroll
    for ( int j = 0; j < 2; ++j )
-   {
-      const int p = int( threadIdx.x ) + j * kTileThreads;
-      if ( p < kBox3 )
-         sb[p] = bin[j] ? R( toAcc( bv[j] ) ) : R( 0 );
-   }
+      if ( int( threadIdx.x ) + j * kTileThreads < kBox3 )
+         sb[int( threadIdx.x ) + j * kTileThreads] = R( toAcc( bv[j] ) );
    __syncthreads();
-   const P2CellGeomT< R >& g  = geom[tc.c];
-   const TileThread< R >   th = tileThread( g, tc, mm );
-   R                       u[10];
-   {
-      int pos[10];
-      elementBoxPositions( th, pos );
+   const P2ActGeomT< R >& g = geom[tc.c];
+   R                      p0[3];
+   const bool             valid = actVertex( g, tc, mm, t, a, p0 );
+   const int              at    = 2 * ( a & 3 ) + kBox * ( 2 * ( ( a >> 2 ) & 3 ) + kBox * 2 * ( a >> 4 ) );
+   R u[10], y[10];
+   forType( t, [&]( auto box ) {
 #pragma unroll
       for ( int i = 0; i < 10; ++i )
-         u[i] = th.valid ? sb[pos[i]] : R( 0 );
-   }
-   R y[10];
-   if ( th.valid )
+         u[i] = sb[at + box.at( i )];
+   } );
+   if ( valid )
+      p2ElementAction< R, kFolded, STORED >( g, t, p0, u, y, c[0], c[1], c[2], coefficient );
+   if constexpr ( kFolded )
    {
-      p2ElementAction( g, th, u, y, [&]( int q ) -> R {
-         if constexpr ( STORED )
-            return sk[q * kTileThreads + threadIdx.x];
-         else
-         {
-            // k from the FP64 geometry of the same point
-            const P2CellGeom&          g64  = geom64[tc.c];
-            const TileThread< double > t64  = tileThread( g64, tc, mm );
-            const double*              xq64 = g64.XQ[th.t][q];
-            const double x64[3] = { t64.p0[0] + xq64[0], t64.p0[1] + xq64[1], t64.p0[2] + xq64[2] };
-            return R( kAt( g64, *kp, x64, t64.ls0 + xq64[3] ) );
-         }
-      } );
-   }
-   {
-      int pos[10];
-      elementBoxPositions( th, pos );
-      if constexpr ( kAtomic )
-      {
-         if ( th.valid )
-         {
+      if ( valid )
+         forType( t, [&]( auto box ) {
 #pragma unroll
             for ( int i = 0; i < 10; ++i )
-               atomicAdd( &sa[pos[i]], y[i] );
-         }
-      }
-      else
-      {
-         __syncthreads(); // the source box and the coefficients are no longer read
-         waveBoxAccumulate( lds, th.valid, pos, y );
-      }
+               atomicAdd( &sa[at + box.at( i )], y[i] );
+         } );
+   }
+   else
+   {
+      int pos[10];
+      forType( t, [&]( auto box ) {
+#pragma unroll
+         for ( int i = 0; i < 10; ++i )
+            pos[i] = at + box.at( i );
+      } );
+      __syncthreads(); // the source box is no longer read
+      waveBoxAccumulate( lds, valid, pos, y );
    }
    __syncthreads();
    // every box point is added with an atomic that returns nothing: box-surface
    // points are shared with neighbouring tiles, and a read-modify-write of the
    // interior points would make the wave wait for its outstanding atomics too
    // (the vector-memory counter covers loads and atomics alike)
-   T* dstC = dst + ( base << lv );
-   for ( int p = threadIdx.x; p < kBox3; p += kTileThreads )
+#pragma unroll
+   for ( int j = 0; j < 2; ++j )
    {
-      const int32_t lx = p % kBox, ly = ( p / kBox ) % kBox, lz = p / ( kBox * kBox );
-      const int32_t X = 2 * int32_t( tc.x0 ) + lx, Y = 2 * int32_t( tc.y0 ) + ly, Z = 2 * int32_t( tc.z0 ) + lz;
-      if ( X + Y + Z <= top )
-         sharedAdd( dstC + ( int64_t( tetRowStart32( int32_t( w1 ), Y, Z ) + X ) << lv ),
-                    R( alpha ) * ( kAtomic ? sa[p] : waveBoxSum( lds, p ) ) );
+      const int p = int( threadIdx.x ) + j * kTileThreads;
+      if ( off[j] >= 0 )
+         sharedAdd( dstC + ( int64_t( off[j] ) << lv ), R( alpha ) * ( kFolded ? sa[p] : waveBoxSum( lds, p ) ) );
    }
 }
 
@@ -936,7 +1004,7 @@ __device__ __forceinline__ void p2TileApplyBody( const P2CellGeomT< typename Acc
 // same element action as the tile kernels, box staging, accumulation and
 // write-back over the 165 box points inside the macro-cell (cDiagBox).
 template < class T, class K, bool STORED >
-__global__ __launch_bounds__( 64 ) void kP2TileApplyDiag( const P2CellGeomT< typename Acc< T >::type >* __restrict__ geom,
+__global__ __launch_bounds__( 64 ) void kP2TileApplyDiag( const P2ActGeomT< typename Acc< T >::type >* __restrict__ geom,
                                                           const P2CellGeom* __restrict__ geom64,
                                                           const KParams* __restrict__ kp, const K* __restrict__ table,
                                                           int64_t mm, int64_t ndiag, int64_t sc1, int64_t w1,
@@ -945,6 +1013,7 @@ __global__ __launch_bounds__( 64 ) void kP2TileApplyDiag( const P2CellGeomT< typ
                                                           int64_t tstride = 0, const int32_t* __restrict__ on = nullptr )
 {
    using R = typename Acc< T >::type;
+   constexpr bool kFolded = std::is_same< R, double >::value;
    if ( on && !on[blockIdx.y] )
       return; // an inactive slot: its (zeroed) result stays zero
    // 2^lv interleaved vectors: vector blockIdx.y with its own coefficient table
@@ -959,56 +1028,63 @@ __global__ __launch_bounds__( 64 ) void kP2TileApplyDiag( const P2CellGeomT< typ
    const TileCoord tc   = tiles ? tileFromList( tiles, ld, mm, lb ) : tileOfDiagonal( ld, mm, lb );
    const int64_t   base = tc.c * sc1;
    const T*        srcC = src + ( base << lv );
+   const int32_t   pair = cDiagPairs[threadIdx.x];
+   const int       t = pair & 7, a = pair >> 3;
+   auto coefficient = [&]( int q ) -> R {
+      if constexpr ( STORED )
+         return R( toAcc( table[( lb * 11 + q ) * kTileThreads + t * 64 + a] ) );
+      else
+         return R( evaluatedCoefficient< kFolded >( geom64[tc.c], *kp, tc, mm, t, a, q ) );
+   };
+   R c[3] = {};
+   if constexpr ( STORED )
+      for ( int q = 0; q < 3; ++q )
+         c[q] = coefficient( q );
    // the lane's (at most three) of the 165 box points inside the macro-cell:
    // all loads issued before the first LDS write
-   constexpr int kPer = kDiagBoxP / 64;
-   int           bp[kPer];
-   T             bv[kPer];
+   constexpr int    kPer = kDiagBoxP / 64;
+   const BoxOffsets bo( int32_t( w1 ), 2 * int32_t( tc.x0 ), 2 * int32_t( tc.y0 ), 2 * int32_t( tc.z0 ) );
+   int              bp[kPer];
+   int32_t          off[kPer];
+   T                bv[kPer];
 #pragma unroll
    for ( int j = 0; j < kPer; ++j )
    {
-      bp[j]           = cDiagBox[int( threadIdx.x ) + 64 * j];
-      const int     p  = bp[j] < 0 ? 0 : bp[j];
-      const int32_t lx = p % kBox, ly = ( p / kBox ) % kBox, lz = p / ( kBox * kBox );
-      const int32_t X = 2 * int32_t( tc.x0 ) + lx, Y = 2 * int32_t( tc.y0 ) + ly, Z = 2 * int32_t( tc.z0 ) + lz;
-      bv[j]           = bp[j] >= 0 ? srcC[int64_t( tetRowStart32( int32_t( w1 ), Y, Z ) + X ) << lv] : T( 0 );
+      bp[j] = cDiagBox[int( threadIdx.x ) + 64 * j];
+      int32_t lx, ly, lz;
+      boxPoint( bp[j] < 0 ? 0 : bp[j], lx, ly, lz );
+      off[j] = bo.at( lx, ly, lz );
+      bv[j]  = bp[j] >= 0 ? srcC[int64_t( off[j] ) << lv] : T( 0 );
    }
 #pragma unroll
    for ( int j = 0; j < kPer; ++j )
       if ( bp[j] >= 0 )
          sb[bp[j]] = R( toAcc( bv[j] ) );
    __syncthreads();
-   const P2CellGeomT< R >& g    = geom[tc.c];
-   const int32_t           pair = cDiagPairs[threadIdx.x];
-   const int               t = pair & 7, a = pair >> 3;
-   const TileThread< R >   th = tileThreadAt( g, tc, mm, t, a );
-   int                     pos[10];
+   const P2ActGeomT< R >& g = geom[tc.c];
+   R                      p0[3];
+   const bool             valid = actVertex( g, tc, mm, t, a, p0 );
+   TileThread< R >        th;
+   th.t  = t;
+   th.ax = a & 3;
+   th.ay = ( a >> 2 ) & 3;
+   th.az = a >> 4;
+   int pos[10];
    elementBoxPositions( th, pos );
    R u[10];
 #pragma unroll
    for ( int i = 0; i < 10; ++i )
-      u[i] = th.valid ? sb[pos[i]] : R( 0 );
+      u[i] = sb[pos[i]];
    __syncthreads();
 #pragma unroll
    for ( int j = 0; j < kPer; ++j )
       if ( bp[j] >= 0 )
          sb[bp[j]] = R( 0 );
    __syncthreads();
-   if ( th.valid )
+   if ( valid )
    {
       R y[10];
-      p2ElementAction( g, th, u, y, [&]( int q ) -> R {
-         if constexpr ( STORED )
-            return R( toAcc( table[( lb * 11 + q ) * kTileThreads + t * 64 + a] ) );
-         else
-         {
-            const P2CellGeom&          g64  = geom64[tc.c];
-            const TileThread< double > t64  = tileThreadAt( g64, tc, mm, t, a );
-            const double*              xq64 = g64.XQ[t][q];
-            const double x64[3] = { t64.p0[0] + xq64[0], t64.p0[1] + xq64[1], t64.p0[2] + xq64[2] };
-            return R( kAt( g64, *kp, x64, t64.ls0 + xq64[3] ) );
-         }
-      } );
+      p2ElementAction< R, kFolded, STORED >( g, t, p0, u, y, c[0], c[1], c[2], coefficient );
 #pragma unroll
       for ( int i = 0; i < 10; ++i )
          atomicAdd( &sb[pos[i]], y[i] );
@@ -1017,22 +1093,14 @@ __global__ __launch_bounds__( 64 ) void kP2TileApplyDiag( const P2CellGeomT< typ
    T* dstC = dst + ( base << lv );
 #pragma unroll
    for ( int j = 0; j < kPer; ++j )
-   {
-      if ( bp[j] < 0 )
-         continue;
-      const int     p  = bp[j];
-      const int32_t lx = p % kBox, ly = ( p / kBox ) % kBox, lz = p / ( kBox * kBox );
-      const int32_t X = 2 * int32_t( tc.x0 ) + lx, Y = 2 * int32_t( tc.y0 ) + ly, Z = 2 * int32_t( tc.z0 ) + lz;
-      sharedAdd( dstC + ( int64_t( tetRowStart32( int32_t( w1 ), Y, Z ) + X ) << lv ), R( alpha ) * sb[p] );
-   }
+      if ( bp[j] >= 0 )
+         sharedAdd( dstC + ( int64_t( off[j] ) << lv ), R( alpha ) * sb[bp[j]] );
 }
 
-// stored coefficients, the compiler's own register budget: the FP64 kernel
-// holds 94 VGPRs (5 waves per SIMD) without spills; a budget of 80 (6 waves)
-// spills the micro-cell's vertex and shell coordinate inside the quadrature loop
+// stored coefficients: 5 waves per SIMD (a budget of 96 VGPRs), three workgroups a CU
 template < class T, class K >
-__global__ __launch_bounds__( kTileThreads ) void kP2TileApplyStored(
-    const P2CellGeomT< typename Acc< T >::type >* __restrict__ geom, const P2CellGeom* __restrict__ geom64,
+__global__ __launch_bounds__( kTileThreads ) __attribute__( ( amdgpu_waves_per_eu( 5 ) ) ) void kP2TileApplyStored(
+    const P2ActGeomT< typename Acc< T >::type >* __restrict__ geom, const P2CellGeom* __restrict__ geom64,
     const KParams* __restrict__ kp, const K* __restrict__ table, int64_t mm, int64_t ntiles, int64_t sc1, int64_t w1,
     const T* __restrict__ src, T* __restrict__ dst, double alpha, const uint64_t* __restrict__ tiles )
 {
@@ -1041,8 +1109,8 @@ __global__ __launch_bounds__( kTileThreads ) void kP2TileApplyStored(
 // the same over 2^lv interleaved vectors with one coefficient table each
 // (grid.y = vectors)
 template < class T, class K >
-__global__ __launch_bounds__( kTileThreads ) void kP2TileApplyStoredBatched(
-    const P2CellGeomT< typename Acc< T >::type >* __restrict__ geom, const K* __restrict__ table, int64_t tstride,
+__global__ __launch_bounds__( kTileThreads ) __attribute__( ( amdgpu_waves_per_eu( 5 ) ) ) void kP2TileApplyStoredBatched(
+    const P2ActGeomT< typename Acc< T >::type >* __restrict__ geom, const K* __restrict__ table, int64_t tstride,
     int64_t mm, int64_t ntiles, int64_t sc1, int64_t w1, const T* __restrict__ src, T* __restrict__ dst, double alpha,
     const uint64_t* __restrict__ tiles, int lv, const int32_t* __restrict__ on )
 {
@@ -1052,7 +1120,7 @@ __global__ __launch_bounds__( kTileThreads ) void kP2TileApplyStoredBatched(
 // coefficients evaluated in place (the compiler's own register budget)
 template < class T, class K >
 __global__ __launch_bounds__( kTileThreads ) void kP2TileApplyEval(
-    const P2CellGeomT< typename Acc< T >::type >* __restrict__ geom, const P2CellGeom* __restrict__ geom64,
+    const P2ActGeomT< typename Acc< T >::type >* __restrict__ geom, const P2CellGeom* __restrict__ geom64,
     const KParams* __restrict__ kp, const K* __restrict__ table, int64_t mm, int64_t ntiles, int64_t sc1, int64_t w1,
     const T* __restrict__ src, T* __restrict__ dst, double alpha, const uint64_t* __restrict__ tiles )
 {
@@ -1111,7 +1179,7 @@ static void p2CheckFunction( const P2Operator& op, const Function& f, int L )
 // table are the tile kernel's.
 constexpr int kSmallMaxMM = 2;
 template < class T, class K, bool STORED >
-__global__ __launch_bounds__( 64 ) void kP2SmallApply( const P2CellGeomT< typename Acc< T >::type >* __restrict__ geom,
+__global__ __launch_bounds__( 64 ) void kP2SmallApply( const P2ActGeomT< typename Acc< T >::type >* __restrict__ geom,
                                                        const P2CellGeom* __restrict__ geom64,
                                                        const KParams* __restrict__ kp, const K* __restrict__ table,
                                                        int64_t mm, int64_t nc, int64_t sc1, int64_t w1,
@@ -1120,6 +1188,7 @@ __global__ __launch_bounds__( 64 ) void kP2SmallApply( const P2CellGeomT< typena
                                                        const int32_t* __restrict__ on = nullptr )
 {
    using R = typename Acc< T >::type;
+   constexpr bool kFolded = std::is_same< R, double >::value;
    if ( on && !on[blockIdx.y] )
       return; // an inactive slot: its (zeroed) result stays zero
    // 2^lv interleaved vectors: vector blockIdx.y with its own coefficient table
@@ -1131,9 +1200,22 @@ __global__ __launch_bounds__( 64 ) void kP2SmallApply( const P2CellGeomT< typena
    if ( c >= nc )
       return;
    const TileCoord tc{ c, 0, 0, 0 };
-   const int32_t   w    = int32_t( w1 );
-   const int32_t   top  = w - 1;
-   const T*        srcC = src + ( ( c * sc1 ) << lv );
+   const int       l = int( threadIdx.x );
+   const int       t = l < 24 ? l >> 2 : 0;
+   const int       a = ( l & 3 ) == 0 ? 0 : 1 << ( 2 * ( ( l & 3 ) - 1 ) ); // 0, 1, 4, 16
+   auto coefficient = [&]( int q ) -> R {
+      if constexpr ( STORED )
+         return R( toAcc( table[( c * 11 + q ) * kTileThreads + 64 * t + a] ) );
+      else
+         return R( evaluatedCoefficient< kFolded >( geom64[c], *kp, tc, mm, t, a, q ) );
+   };
+   R cq[3] = {};
+   if constexpr ( STORED )
+      for ( int q = 0; q < 3; ++q )
+         cq[q] = coefficient( q );
+   const int32_t w    = int32_t( w1 );
+   const int32_t top  = w - 1;
+   const T*      srcC = src + ( ( c * sc1 ) << lv );
    for ( int p = threadIdx.x; p < w * w * w; p += 64 )
    {
       const int32_t X = p % w, Y = ( p / w ) % w, Z = p / ( w * w );
@@ -1141,18 +1223,20 @@ __global__ __launch_bounds__( 64 ) void kP2SmallApply( const P2CellGeomT< typena
          sb[X + kBox * ( Y + kBox * Z )] = R( toAcc( srcC[int64_t( tetRowStart32( w, Y, Z ) + X ) << lv] ) );
    }
    __syncthreads();
-   const int               l = int( threadIdx.x );
-   const int               t = l < 24 ? l >> 2 : 0;
-   const int               a = ( l & 3 ) == 0 ? 0 : 1 << ( 2 * ( ( l & 3 ) - 1 ) ); // 0, 1, 4, 16
-   const P2CellGeomT< R >& g  = geom[c];
-   TileThread< R >         th = tileThreadAt( g, tc, mm, t, a );
-   th.valid                   = th.valid && l < 24;
-   R u[10];
+   const P2ActGeomT< R >& g = geom[c];
+   R                      p0[3];
+   const bool             valid = actVertex( g, tc, mm, t, a, p0 ) && l < 24;
+   TileThread< R >        th;
+   th.t  = t;
+   th.ax = a & 3;
+   th.ay = ( a >> 2 ) & 3;
+   th.az = a >> 4;
+   R   u[10];
    int pos[10];
    elementBoxPositions( th, pos );
 #pragma unroll
    for ( int i = 0; i < 10; ++i )
-      u[i] = th.valid ? sb[pos[i]] : R( 0 );
+      u[i] = valid ? sb[pos[i]] : R( 0 );
    __syncthreads();
    for ( int p = threadIdx.x; p < w * w * w; p += 64 )
    {
@@ -1161,21 +1245,10 @@ __global__ __launch_bounds__( 64 ) void kP2SmallApply( const P2CellGeomT< typena
          sb[X + kBox * ( Y + kBox * Z )] = R( 0 );
    }
    __syncthreads();
-   if ( th.valid )
+   if ( valid )
    {
       R y[10];
-      p2ElementAction( g, th, u, y, [&]( int q ) -> R {
-         if constexpr ( STORED )
-            return R( toAcc( table[( c * 11 + q ) * kTileThreads + 64 * t + a] ) );
-         else
-         {
-            const P2CellGeom&          g64  = geom64[c];
-            const TileThread< double > t64  = tileThreadAt( g64, tc, mm, t, a );
-            const double*              xq64 = g64.XQ[t][q];
-            const double x64[3] = { t64.p0[0] + xq64[0], t64.p0[1] + xq64[1], t64.p0[2] + xq64[2] };
-            return R( kAt( g64, *kp, x64, t64.ls0 + xq64[3] ) );
-         }
-      } );
+      p2ElementAction< R, kFolded, STORED >( g, t, p0, u, y, cq[0], cq[1], cq[2], coefficient );
 #pragma unroll
       for ( int i = 0; i < 10; ++i )
          atomicAdd( &sb[pos[i]], y[i] );
@@ -1220,13 +1293,65 @@ static const K* p2Coefficients( Context* ctx, P2Operator& op, int L, int dtype )
    return (const K*) buf.p;
 }
 
+// the element action's geometry from the tile geometry of a level: lengths times
+// |n|, rotated by Q whose third row is n / |n| (affine cells: |n| = 1, Q = I)
+template < class R >
+static std::vector< P2ActGeomT< R > > actGeometry( const std::vector< P2CellGeom >& gs )
+{
+   std::vector< P2ActGeomT< R > > out( gs.size() );
+   for ( size_t c = 0; c < gs.size(); ++c )
+   {
+      const P2CellGeom& g = gs[c];
+      P2ActGeomT< R >&  o = out[c];
+      double            Q[3][3] = { { 1, 0, 0 }, { 0, 1, 0 }, { 0, 0, 1 } }, len = 1.0;
+      if ( g.kind )
+      {
+         len = std::sqrt( g.nl[0] * g.nl[0] + g.nl[1] * g.nl[1] + g.nl[2] * g.nl[2] );
+         for ( int d = 0; d < 3; ++d )
+            Q[2][d] = g.nl[d] / len;
+         // first row: the coordinate axis least aligned with n, made orthogonal to it
+         int k = 0;
+         for ( int d = 1; d < 3; ++d )
+            if ( std::fabs( Q[2][d] ) < std::fabs( Q[2][k] ) )
+               k = d;
+         const double s = 1.0 / std::sqrt( 1.0 - Q[2][k] * Q[2][k] );
+         for ( int d = 0; d < 3; ++d )
+            Q[0][d] = s * ( ( d == k ? 1.0 : 0.0 ) - Q[2][k] * Q[2][d] );
+         for ( int d = 0; d < 3; ++d )
+            Q[1][d] = Q[2][( d + 1 ) % 3] * Q[0][( d + 2 ) % 3] - Q[2][( d + 2 ) % 3] * Q[0][( d + 1 ) % 3];
+      }
+      auto turned = [&]( const double* v, int stride, int d ) {
+         return Q[d][0] * v[0] + Q[d][1] * v[stride] + Q[d][2] * v[2 * stride];
+      };
+      for ( int d = 0; d < 3; ++d )
+      {
+         o.v0[d] = R( len * turned( g.v0, 1, d ) );
+         for ( int k = 0; k < 3; ++k )
+            o.hE[3 * d + k] = R( len * turned( g.hE + k, 3, d ) );
+         for ( int t = 0; t < 6; ++t )
+         {
+            for ( int k = 0; k < 3; ++k )
+               o.Dc[t][3 * k + d] = R( turned( g.Dc[t] + 3 * k, 1, d ) / len );
+            for ( int q = 0; q < 11; ++q )
+               o.xq[t][q][d] = R( len * turned( g.XQ[t][q], 1, d ) );
+         }
+      }
+      for ( int t = 0; t < 6; ++t )
+         o.cw[t] = R( g.kind ? g.adet[t] * len * len * len * std::fabs( g.dr ) : g.adet[t] );
+      o.lam0 = R( g.lam0 );
+      o.r0   = R( g.kind ? g.r0 / g.dr : 0.0 );
+      o.kind = g.kind;
+   }
+   return out;
+}
+
 template < class T >
-static const P2CellGeomT< typename Acc< T >::type >* p2Geometry( P2Operator& op, int L )
+static const P2ActGeomT< typename Acc< T >::type >* p2Geometry( P2Operator& op, int L )
 {
    if constexpr ( std::is_same< typename Acc< T >::type, double >::value )
-      return op.tgeom.at( L ).p;
+      return op.ageom.at( L ).p;
    else
-      return op.tgeomF.at( L ).p;
+      return op.ageomF.at( L ).p;
 }
 
 // k at the blended centroids of the micro-cells of level L (tile-major, FP16),
@@ -1342,7 +1467,8 @@ static void p2ApplyBatched( Context* ctx, P2Operator& op, Lattice& lat, int L, F
    HG_CHECK_HIP( hipGetLastError() );
    const double*    table   = p2Coefficients< double >( ctx, op, L, 0 );
    const int64_t    tstride = op.tableStride.at( L );
-   const auto*      geom    = op.tgeom.at( L ).p;
+   const auto*      geom    = op.ageom.at( L ).p;
+   const auto*      geom64  = op.tgeom.at( L ).p;
    const int64_t    nint    = tet( tileEdges( mm ) - 1 ) * lat.nc;
    const int64_t    ndiag   = tri( tileEdges( mm ) ) * lat.nc;
    const uint64_t*  tint    = mm > kSmallMaxMM ? tileList( ctx, lat, mm, kTilesInterior ) : nullptr;
@@ -1350,7 +1476,7 @@ static void p2ApplyBatched( Context* ctx, P2Operator& op, Lattice& lat, int L, F
    ctx->beginTiming();
    if ( mm <= kSmallMaxMM )
       kP2SmallApply< double, double, true ><<< dim3( unsigned( lat.nc ), nv ), 64, 0, ctx->stream >>>(
-          geom, geom, nullptr, table, mm, lat.nc, lat.sc, lat.w, s, d, alpha, lv, tstride, op.slotOn.p );
+          geom, geom64, nullptr, table, mm, lat.nc, lat.sc, lat.w, s, d, alpha, lv, tstride, op.slotOn.p );
    else
    {
       if ( mm % kTile != 0 )
@@ -1360,7 +1486,7 @@ static void p2ApplyBatched( Context* ctx, P2Operator& op, Lattice& lat, int L, F
              geom, table, tstride, mm, nint, lat.sc, lat.w, s, d, alpha, tint, lv, op.slotOn.p );
       HG_CHECK_HIP( hipGetLastError() );
       kP2TileApplyDiag< double, double, true ><<< dim3( xcdGrid( ndiag ), nv ), 64, 0, ctx->stream >>>(
-          geom, geom, nullptr, table, mm, ndiag, lat.sc, lat.w, s, d, alpha, tlast, lv, tstride, op.slotOn.p );
+          geom, geom64, nullptr, table, mm, ndiag, lat.sc, lat.w, s, d, alpha, tlast, lv, tstride, op.slotOn.p );
    }
    HG_CHECK_HIP( hipGetLastError() );
    ctx->endTiming();
@@ -1787,7 +1913,9 @@ int hg_p2_divkgrad_create( hg_ctx* h, hg_handle s, int minLevel, int maxLevel, i
          std::vector< P2CellGeom > gl = tg;
          tileGeometryLevel( gl, int64_t( 1 ) << L, kQP, 11 );
          op->tgeom[L].upload( ctx, gl );
-         op->tgeomF[L].upload( ctx, toFloat( gl ) );
+         const std::vector< P2ActGeomT< double > > ga = actGeometry< double >( gl );
+         op->ageom[L].upload( ctx, ga );
+         op->ageomF[L].upload( ctx, actGeometry< float >( gl ) );
       }
       std::vector< KParams > kp( 1 );
       kp[0]    = KParams{};

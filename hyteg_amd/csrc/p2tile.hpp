@@ -230,6 +230,67 @@ inline std::vector< int32_t > diagonalBoxPoints()
    return out;
 }
 
+// Cell-local lattice offset of a tile's box point (lx, ly, lz): the tile's first
+// point (x0, y0, z0) of a lattice of width w lies at `first` (formed on the scalar
+// unit), the offset from it is a polynomial in the box coordinates whose
+// coefficients are uniform -- three 24-bit multiply-adds a point, where the row
+// start formula costs about 40 vector instructions with its 64-bit division.
+// Valid for w <= 1024 (every product below 2^24 in its factors and 2^31).
+struct BoxOffsets
+{
+   int32_t first, a, b, m;
+   __device__ __forceinline__ BoxOffsets( int32_t w, int32_t x0, int32_t y0, int32_t z0 )
+   {
+      m     = w - z0;
+      a     = m * ( m + 1 ) / 2 - y0;
+      b     = m - y0;
+      first = tetRowStart32( w, y0, z0 ) + x0;
+   }
+   __device__ __forceinline__ int32_t at( int32_t lx, int32_t ly, int32_t lz ) const
+   {
+      const int32_t c2 = __mul24( lz, lz - 1 ) >> 1;             // C(lz, 2)
+      const int32_t c3 = __mul24( c2, lz - 2 ) * 43691 >> 17;    // C(lz, 3) = c2 (lz - 2) / 3
+      const int32_t k  = lx + c3 - __mul24( ly, lz ) - ( __mul24( ly, ly - 1 ) >> 1 );
+      return first + __mul24( lz, a ) + __mul24( ly, b ) - __mul24( c2, m ) + k;
+   }
+};
+// box point number p (lx + 9 ly + 81 lz, p < 1024) -> its coordinates
+__device__ __forceinline__ void boxPoint( int32_t p, int32_t& lx, int32_t& ly, int32_t& lz )
+{
+   lz               = __mul24( p, 810 ) >> 16;
+   const int32_t r  = p - __mul24( lz, 81 );
+   ly               = __mul24( r, 57 ) >> 9;
+   lx               = r - __mul24( ly, 9 );
+}
+
+// box offsets of the 10 P2 DoFs of a micro-cell of type t relative to its anchor's
+// box point: compile-time constants, so that a wavefront of one type addresses
+// LDS with one register and immediate offsets
+template < int t >
+struct ElementBox
+{
+   static constexpr int vertex( int k )
+   {
+      return 2 * ( MicroCells::vof[t][k][0] + kBox * ( MicroCells::vof[t][k][1] + kBox * MicroCells::vof[t][k][2] ) );
+   }
+   static constexpr int edges[6][2] = { { 0, 1 }, { 0, 2 }, { 0, 3 }, { 1, 2 }, { 1, 3 }, { 2, 3 } };
+   static constexpr int at( int i ) { return i < 4 ? vertex( i ) : ( vertex( edges[i - 4][0] ) + vertex( edges[i - 4][1] ) ) / 2; }
+};
+// f(ElementBox< t >) for a wavefront-uniform type t
+template < class F >
+__device__ __forceinline__ void forType( int t, F&& f )
+{
+   switch ( t )
+   {
+   case 0: f( ElementBox< 0 >{} ); break;
+   case 1: f( ElementBox< 1 >{} ); break;
+   case 2: f( ElementBox< 2 >{} ); break;
+   case 3: f( ElementBox< 3 >{} ); break;
+   case 4: f( ElementBox< 4 >{} ); break;
+   default: f( ElementBox< 5 >{} ); break;
+   }
+}
+
 // 1/b and 1/sqrt(b) from the hardware estimates (relative error e below 2^-22)
 // refined by one third-order step each (error O(e^3), below the rounding of the
 // result): r (1 + e + e^2) with e = 1 - b r, and y (1 + e/2 + 3e^2/8) with
