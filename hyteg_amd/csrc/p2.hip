@@ -345,12 +345,14 @@ __device__ __forceinline__ double kAt( const P2CellGeom& g, const KParams& K, co
 __device__ __forceinline__ double foldedCoefficient( const P2CellGeom& g, const KParams& K, int t, int q,
                                                      const double x[3], double ls )
 {
-   const double c = cQW[q] * g.adet[t] * kAt( g, K, x, ls );
+   const double c = cQW[q] * g.adet[t];
    if ( !g.kind )
-      return c;
-   const double n2 = g.nl[0] * g.nl[0] + g.nl[1] * g.nl[1] + g.nl[2] * g.nl[2];
-   const double r2 = x[0] * x[0] + x[1] * x[1] + x[2] * x[2];
-   return copysign( c * n2 * fabs( g.dr ) / sqrt( r2 ), ls + g.lam0 );
+      return c * kEval( K, x );
+   const double n2   = g.nl[0] * g.nl[0] + g.nl[1] * g.nl[1] + g.nl[2] * g.nl[2];
+   const double irho = fastRsqrt( x[0] * x[0] + x[1] * x[1] + x[2] * x[2] );
+   const double qq   = ( g.r0 + fabs( ls ) * g.dr ) * irho;
+   const double F[3] = { qq * x[0], qq * x[1], qq * x[2] };
+   return copysign( c * kEval( K, F ) * n2 * fabs( g.dr ) * irho, ls + g.lam0 );
 }
 
 // the coefficient tables, tile-major: table[(tile * 11 + q) * 384 + thread] (zero
@@ -541,7 +543,7 @@ __global__ __launch_bounds__( kTileThreads ) void kP2TileReducedMetric( const P2
    if ( lb >= ntiles )
       return;
    int64_t         full;
-   const TileCoord tc = tiles ? tileFromList( tiles, lb, mm, full ) : tileOf( lb, mm );
+   const TileCoord tc = tileFromList( tiles, lb, mm, full );
    const float     ke = __half2float( kc[lb * kTileThreads + threadIdx.x] );
    stageBlendedVertices( geom[tc.c], tc, sv );
    __syncthreads();
@@ -570,7 +572,7 @@ __global__ __launch_bounds__( kTileThreads ) void kP2TileApplyReduced( const P2C
    if ( lb >= ntiles )
       return;
    int64_t         full;
-   const TileCoord tc   = tiles ? tileFromList( tiles, lb, mm, full ) : tileOf( lb, mm );
+   const TileCoord tc   = tileFromList( tiles, lb, mm, full );
    const int64_t   base = tc.c * sc1;
    const int32_t   top  = int32_t( 2 * mm );
    float           G[6];
@@ -718,14 +720,16 @@ static void surfacePointList( Context* ctx, Lattice& l )
 // so that a point needs one reciprocal and no square root; the factor |s| sign(nu)
 // (and the scales of the frame) is part of the coefficient (foldedCoefficient).
 //
+// Dc, XQ, cw: those of g for the micro-cell's type (in scalar registers where a
+// wavefront has one type, in LDS where its lanes differ).
 // c0, c1, c2 and next: coefficients 0..2, and the one of point q + 3 (FOLDED: the
 // whole factor; otherwise k), so that three table loads are in flight.
-template < class R, bool FOLDED, bool STORED, class KQ >
-__device__ __forceinline__ void p2ElementAction( const P2ActGeomT< R >& g, int t, const R p0[3], const R u[10], R y[10],
-                                                 R c0, R c1, R c2, KQ&& next )
+// BLEND: 0 affine cells, 1 shell cells, -1 by the cell's own kind.
+template < class R, bool FOLDED, bool STORED, int BLEND = -1, class KQ >
+__device__ __forceinline__ void p2ElementAction( const P2ActGeomT< R >& g, const R* Dc, const R ( *XQ )[3], R cw,
+                                                 const R p0[3], const R u[10], R y[10], R c0, R c1, R c2, KQ&& next )
 {
    using QC     = QuadConst< R >;
-   const R* Dc  = g.Dc[t];
    R        v0[3], V[3][3];
    {
       // d0 and B (symmetric) from the element values (edges 4..9 in the order
@@ -753,12 +757,21 @@ __device__ __forceinline__ void p2ElementAction( const P2ActGeomT< R >& g, int t
       for ( int j = 0; j < 3; ++j )
          Tm[d][j] = R( 0 );
    }
-   // STORED is fully unrolled: the coefficient loads stay three points ahead without
-   // register moves that would wait for them, and the scalar loads of a point's
-   // constants are issued early
-   auto point = [&]( auto shell, int q, R cq ) {
-         const R* lq = QC::lam( q );
-         const R* xq = g.xq[t][q];
+   // STORED is fully unrolled: the coefficient loads stay three points ahead and the
+   // scalar loads of a point's constants one, without register moves that would wait
+   // for them
+   struct Consts
+   {
+      R l[3], x[3];
+   };
+   auto constants = [&]( int q ) {
+      const R* lq = QC::lam( q );
+      const R* xq = XQ[q];
+      return Consts{ { lq[0], lq[1], lq[2] }, { xq[0], xq[1], xq[2] } };
+   };
+   auto point = [&]( auto shell, int q, R cq, const Consts& k ) {
+         const R* lq = k.l;
+         const R* xq = k.x;
          R        v[3], m[3];
 #pragma unroll
          for ( int d = 0; d < 3; ++d )
@@ -773,7 +786,7 @@ __device__ __forceinline__ void p2ElementAction( const P2ActGeomT< R >& g, int t
             const R tt = p * r3;
             const R ga = v[2] - ( p * r2 + tt );
             if constexpr ( !FOLDED )
-               cq = cq * QC::w()[q] * g.cw[t] * copysign( fastRsqrt( r2 ), z );
+               cq = cq * QC::w()[q] * cw * copysign( fastRsqrt( r2 ), z );
             const R cz = cq * z, cg = cq * ga;
             m[0] = cz * v[0] - cg * x;
             m[1] = cz * v[1] - cg * yy;
@@ -782,7 +795,7 @@ __device__ __forceinline__ void p2ElementAction( const P2ActGeomT< R >& g, int t
          else
          {
             if constexpr ( !FOLDED )
-               cq = cq * QC::w()[q] * g.cw[t];
+               cq = cq * QC::w()[q] * cw;
 #pragma unroll
             for ( int d = 0; d < 3; ++d )
                m[d] = cq * v[d];
@@ -799,13 +812,18 @@ __device__ __forceinline__ void p2ElementAction( const P2ActGeomT< R >& g, int t
    auto points = [&]( auto shell ) {
       if constexpr ( STORED )
       {
-         R c[14] = { c0, c1, c2 };
+         R      c[14] = { c0, c1, c2 };
+         Consts k[12];
+         k[0] = constants( 0 );
+         __builtin_amdgcn_sched_barrier( 0 );
 #pragma unroll
          for ( int q = 0; q < 11; ++q )
          {
             if ( q + 3 < 11 )
                c[q + 3] = next( q + 3 );
-            point( shell, q, c[q] );
+            if ( q + 1 < 11 )
+               k[q + 1] = constants( q + 1 );
+            point( shell, q, c[q], k[q] );
             __builtin_amdgcn_sched_barrier( 0 );
          }
       }
@@ -813,13 +831,21 @@ __device__ __forceinline__ void p2ElementAction( const P2ActGeomT< R >& g, int t
       {
 #pragma unroll 1
          for ( int q = 0; q < 11; ++q )
-            point( shell, q, next( q ) );
+            point( shell, q, next( q ), constants( q ) );
       }
    };
-   if ( g.kind )
-      points( std::true_type{} );
+   // (the branch is kept where the kind is known: it opens a block of its own, which
+   // the compiler does not move the points' loads out of)
+   if ( g.kind != 0 )
+   {
+      if constexpr ( BLEND != 0 )
+         points( std::true_type{} );
+   }
    else
-      points( std::false_type{} );
+   {
+      if constexpr ( BLEND != 1 )
+         points( std::false_type{} );
+   }
    R T[3][3], S[3];
 #pragma unroll
    for ( int k = 0; k < 3; ++k )
@@ -843,6 +869,34 @@ __device__ __forceinline__ void p2ElementAction( const P2ActGeomT< R >& g, int t
    y[9] = R( 4 ) * ( T[1][2] + T[2][1] );
 }
 
+// Dc and xq of a cell (all types) staged in LDS by one wavefront whose lanes take
+// different types: sg[9 t] = Dc[t], sg[54 + 33 t] = xq[t]
+constexpr int kActShared = 54 + 198;
+template < class R >
+struct ActShared
+{
+   R v[4];
+};
+template < class R >
+__device__ __forceinline__ ActShared< R > loadActShared( const P2ActGeomT< R >& g )
+{
+   static_assert( offsetof( P2ActGeomT< R >, xq ) == offsetof( P2ActGeomT< R >, Dc ) + 54 * sizeof( R ), "Dc, then xq" );
+   const R*       d = &g.Dc[0][0];
+   ActShared< R > s;
+#pragma unroll
+   for ( int j = 0; j < 4; ++j )
+      s.v[j] = d[min( int( threadIdx.x ) + 64 * j, kActShared - 1 )];
+   return s;
+}
+template < class R >
+__device__ __forceinline__ void storeActShared( const ActShared< R >& s, R* sg )
+{
+#pragma unroll
+   for ( int j = 0; j < 4; ++j )
+      if ( int( threadIdx.x ) + 64 * j < kActShared )
+         sg[int( threadIdx.x ) + 64 * j] = s.v[j];
+}
+
 // vertex 0 of the micro-cell of type t at anchor index a (ax + 4 ay + 16 az) of
 // tile tc in the frame of g, and whether the micro-cell lies in the macro-cell
 template < class R >
@@ -851,11 +905,12 @@ __device__ __forceinline__ bool actVertex( const P2ActGeomT< R >& g, const TileC
 {
    const int32_t gx = int32_t( tc.x0 ) + ( a & 3 ), gy = int32_t( tc.y0 ) + ( ( a >> 2 ) & 3 ),
                  gz = int32_t( tc.z0 ) + ( a >> 4 );
-   const R vx = R( gx + cVof[t][0][0] ), vy = R( gy + cVof[t][0][1] ), vz = R( gz + cVof[t][0][2] );
+   const R vx = R( gx + vertexOffset< 0 >( t, 0 ) ), vy = R( gy + vertexOffset< 1 >( t, 0 ) ), vz = R( gz + vertexOffset< 2 >( t, 0 ) );
 #pragma unroll
    for ( int d = 0; d < 3; ++d )
       p0[d] = g.v0[d] + g.hE[3 * d] * vx + g.hE[3 * d + 1] * vy + g.hE[3 * d + 2] * vz;
-   return gx + gy + gz <= int32_t( mm ) - 1 - MicroCells::rowShift[t];
+   // one micro-cell less fits along an edge for the types other than 0, two for type 3
+   return gx + gy + gz <= int32_t( mm ) - 1 - ( t == 0 ? 0 : ( t == 3 ? 2 : 1 ) );
 }
 
 // k (FOLDED: the whole coefficient) of point q of the micro-cell (t, a), evaluated
@@ -869,6 +924,18 @@ __device__ __forceinline__ double evaluatedCoefficient( const P2CellGeom& g, con
    return FOLDED ? foldedCoefficient( g, K, t, q, x, th.ls0 + xq[3] ) : kAt( g, K, x, th.ls0 + xq[3] );
 }
 
+// a coefficient of a table that is read once per apply: a non-temporal load, so that
+// the stream (8 times the bytes of the vectors) does not displace the box lines that
+// neighbouring tiles share in L2
+template < class K >
+__device__ __forceinline__ K streamed( const K* p )
+{
+   if constexpr ( std::is_same< K, __half >::value )
+      return *p;
+   else
+      return __builtin_nontemporal_load( p );
+}
+
 // y = A x on the cell lattices of level L+1 (halo positions included): the
 // element action of every micro-cell of a tile, equal to the reference's element
 // matrix times the element vector.
@@ -876,7 +943,7 @@ __device__ __forceinline__ double evaluatedCoefficient( const P2CellGeom& g, con
 // arithmetic runs in Acc<T> (FP64 for double, FP32 for float and half).
 // BATCH: 2^lv interleaved vectors (vector blockIdx.y, its coefficient table at
 // table + blockIdx.y * tstride); otherwise one vector.
-template < class T, class K, bool STORED, bool BATCH = false >
+template < class T, class K, bool STORED, int BLEND, bool BATCH = false >
 __device__ __forceinline__ void p2TileApplyBody( const P2ActGeomT< typename Acc< T >::type >* __restrict__ geom,
                                                  const P2CellGeom* __restrict__ geom64, const KParams* __restrict__ kp,
                                                  const K* __restrict__ table, int64_t mm, int64_t ntiles, int64_t sc1,
@@ -908,12 +975,12 @@ __device__ __forceinline__ void p2TileApplyBody( const P2ActGeomT< typename Acc<
    if ( li >= ntiles )
       return;
    int64_t         lb;
-   const TileCoord tc   = tiles ? tileFromList( tiles, li, mm, lb ) : tileOfInterior( li, mm, lb );
+   const TileCoord tc   = tileFromList( tiles, li, mm, lb );
    const int64_t   base = tc.c * sc1;
    const int       t = __builtin_amdgcn_readfirstlane( int( threadIdx.x ) >> 6 ), a = int( threadIdx.x ) & 63;
    auto coefficient = [&]( int q ) -> R {
       if constexpr ( STORED )
-         return R( toAcc( ( table + ( lb * 11 + q ) * kTileThreads )[threadIdx.x] ) );
+         return R( toAcc( streamed( table + ( lb * 11 + q ) * kTileThreads + threadIdx.x ) ) );
       else
          return R( evaluatedCoefficient< kFolded >( geom64[tc.c], *kp, tc, mm, t, a, q ) );
    };
@@ -964,7 +1031,7 @@ __device__ __forceinline__ void p2TileApplyBody( const P2ActGeomT< typename Acc<
          u[i] = sb[at + box.at( i )];
    } );
    if ( valid )
-      p2ElementAction< R, kFolded, STORED >( g, t, p0, u, y, c[0], c[1], c[2], coefficient );
+      p2ElementAction< R, kFolded, STORED, BLEND >( g, g.Dc[t], g.xq[t], g.cw[t], p0, u, y, c[0], c[1], c[2], coefficient );
    if constexpr ( kFolded )
    {
       if ( valid )
@@ -1021,11 +1088,12 @@ __global__ __launch_bounds__( 64 ) void kP2TileApplyDiag( const P2ActGeomT< type
    src += blockIdx.y;
    dst += blockIdx.y;
    __shared__ R  sb[kBox3];
+   __shared__ R  sg[kActShared];
    const int64_t ld = xcdBlock( ndiag );
    if ( ld >= ndiag )
       return;
    int64_t         lb;
-   const TileCoord tc   = tiles ? tileFromList( tiles, ld, mm, lb ) : tileOfDiagonal( ld, mm, lb );
+   const TileCoord tc   = tileFromList( tiles, ld, mm, lb );
    const int64_t   base = tc.c * sc1;
    const T*        srcC = src + ( base << lv );
    const int32_t   pair = cDiagPairs[threadIdx.x];
@@ -1040,8 +1108,10 @@ __global__ __launch_bounds__( 64 ) void kP2TileApplyDiag( const P2ActGeomT< type
    if constexpr ( STORED )
       for ( int q = 0; q < 3; ++q )
          c[q] = coefficient( q );
-   // the lane's (at most three) of the 165 box points inside the macro-cell:
-   // all loads issued before the first LDS write
+   // the lane's (at most three) of the 165 box points inside the macro-cell and its
+   // share of the cell's geometry: all loads issued before the first LDS write
+   const P2ActGeomT< R >& g  = geom[tc.c];
+   const ActShared< R >   gs = loadActShared( g );
    constexpr int    kPer = kDiagBoxP / 64;
    const BoxOffsets bo( int32_t( w1 ), 2 * int32_t( tc.x0 ), 2 * int32_t( tc.y0 ), 2 * int32_t( tc.z0 ) );
    int              bp[kPer];
@@ -1060,17 +1130,12 @@ __global__ __launch_bounds__( 64 ) void kP2TileApplyDiag( const P2ActGeomT< type
    for ( int j = 0; j < kPer; ++j )
       if ( bp[j] >= 0 )
          sb[bp[j]] = R( toAcc( bv[j] ) );
+   storeActShared( gs, sg );
    __syncthreads();
-   const P2ActGeomT< R >& g = geom[tc.c];
-   R                      p0[3];
-   const bool             valid = actVertex( g, tc, mm, t, a, p0 );
-   TileThread< R >        th;
-   th.t  = t;
-   th.ax = a & 3;
-   th.ay = ( a >> 2 ) & 3;
-   th.az = a >> 4;
+   R          p0[3];
+   const bool valid = actVertex( g, tc, mm, t, a, p0 );
    int pos[10];
-   elementBoxPositions( th, pos );
+   laneBoxPositions( t, a, pos );
    R u[10];
 #pragma unroll
    for ( int i = 0; i < 10; ++i )
@@ -1084,7 +1149,8 @@ __global__ __launch_bounds__( 64 ) void kP2TileApplyDiag( const P2ActGeomT< type
    if ( valid )
    {
       R y[10];
-      p2ElementAction< R, kFolded, STORED >( g, t, p0, u, y, c[0], c[1], c[2], coefficient );
+      p2ElementAction< R, kFolded, STORED >( g, sg + 9 * t, reinterpret_cast< const R( * )[3] >( sg + 54 + 33 * t ), g.cw[t], p0,
+                                             u, y, c[0], c[1], c[2], coefficient );
 #pragma unroll
       for ( int i = 0; i < 10; ++i )
          atomicAdd( &sb[pos[i]], y[i] );
@@ -1097,24 +1163,24 @@ __global__ __launch_bounds__( 64 ) void kP2TileApplyDiag( const P2ActGeomT< type
          sharedAdd( dstC + ( int64_t( off[j] ) << lv ), R( alpha ) * sb[bp[j]] );
 }
 
-// stored coefficients: 5 waves per SIMD (a budget of 96 VGPRs), three workgroups a CU
-template < class T, class K >
+// stored coefficients: 5 waves per SIMD (a budget of 96 VGPRs)
+template < class T, class K, bool SHELL >
 __global__ __launch_bounds__( kTileThreads ) __attribute__( ( amdgpu_waves_per_eu( 5 ) ) ) void kP2TileApplyStored(
-    const P2ActGeomT< typename Acc< T >::type >* __restrict__ geom, const P2CellGeom* __restrict__ geom64,
-    const KParams* __restrict__ kp, const K* __restrict__ table, int64_t mm, int64_t ntiles, int64_t sc1, int64_t w1,
-    const T* __restrict__ src, T* __restrict__ dst, double alpha, const uint64_t* __restrict__ tiles )
+    const P2ActGeomT< typename Acc< T >::type >* __restrict__ geom, const K* __restrict__ table, int64_t mm,
+    int64_t ntiles, int64_t sc1, int64_t w1, const T* __restrict__ src, T* __restrict__ dst, double alpha,
+    const uint64_t* __restrict__ tiles )
 {
-   p2TileApplyBody< T, K, true >( geom, geom64, kp, table, mm, ntiles, sc1, w1, src, dst, alpha, tiles );
+   p2TileApplyBody< T, K, true, SHELL >( geom, nullptr, nullptr, table, mm, ntiles, sc1, w1, src, dst, alpha, tiles );
 }
 // the same over 2^lv interleaved vectors with one coefficient table each
 // (grid.y = vectors)
-template < class T, class K >
+template < class T, class K, bool SHELL >
 __global__ __launch_bounds__( kTileThreads ) __attribute__( ( amdgpu_waves_per_eu( 5 ) ) ) void kP2TileApplyStoredBatched(
     const P2ActGeomT< typename Acc< T >::type >* __restrict__ geom, const K* __restrict__ table, int64_t tstride,
     int64_t mm, int64_t ntiles, int64_t sc1, int64_t w1, const T* __restrict__ src, T* __restrict__ dst, double alpha,
     const uint64_t* __restrict__ tiles, int lv, const int32_t* __restrict__ on )
 {
-   p2TileApplyBody< T, K, true, true >( geom, nullptr, nullptr, table, mm, ntiles, sc1, w1, src, dst, alpha, tiles, lv,
+   p2TileApplyBody< T, K, true, SHELL, true >( geom, nullptr, nullptr, table, mm, ntiles, sc1, w1, src, dst, alpha, tiles, lv,
                                         tstride, on );
 }
 // coefficients evaluated in place (the compiler's own register budget)
@@ -1124,7 +1190,7 @@ __global__ __launch_bounds__( kTileThreads ) void kP2TileApplyEval(
     const KParams* __restrict__ kp, const K* __restrict__ table, int64_t mm, int64_t ntiles, int64_t sc1, int64_t w1,
     const T* __restrict__ src, T* __restrict__ dst, double alpha, const uint64_t* __restrict__ tiles )
 {
-   p2TileApplyBody< T, K, false >( geom, geom64, kp, table, mm, ntiles, sc1, w1, src, dst, alpha, tiles );
+   p2TileApplyBody< T, K, false, -1 >( geom, geom64, kp, table, mm, ntiles, sc1, w1, src, dst, alpha, tiles );
 }
 
 __global__ void kP2ElementDiag( const CellGeom* __restrict__ geom, const KParams* __restrict__ kp, int64_t mm,
@@ -1196,9 +1262,12 @@ __global__ __launch_bounds__( 64 ) void kP2SmallApply( const P2ActGeomT< typenam
    src += blockIdx.y;
    dst += blockIdx.y;
    __shared__ R  sb[kBox3];
+   __shared__ R  sg[kActShared];
    const int64_t c = blockIdx.x;
    if ( c >= nc )
       return;
+   const P2ActGeomT< R >& g  = geom[c];
+   const ActShared< R >   gs = loadActShared( g );
    const TileCoord tc{ c, 0, 0, 0 };
    const int       l = int( threadIdx.x );
    const int       t = l < 24 ? l >> 2 : 0;
@@ -1222,18 +1291,13 @@ __global__ __launch_bounds__( 64 ) void kP2SmallApply( const P2ActGeomT< typenam
       if ( X + Y + Z <= top )
          sb[X + kBox * ( Y + kBox * Z )] = R( toAcc( srcC[int64_t( tetRowStart32( w, Y, Z ) + X ) << lv] ) );
    }
+   storeActShared( gs, sg );
    __syncthreads();
-   const P2ActGeomT< R >& g = geom[c];
-   R                      p0[3];
-   const bool             valid = actVertex( g, tc, mm, t, a, p0 ) && l < 24;
-   TileThread< R >        th;
-   th.t  = t;
-   th.ax = a & 3;
-   th.ay = ( a >> 2 ) & 3;
-   th.az = a >> 4;
+   R          p0[3];
+   const bool valid = actVertex( g, tc, mm, t, a, p0 ) && l < 24;
    R   u[10];
    int pos[10];
-   elementBoxPositions( th, pos );
+   laneBoxPositions( t, a, pos );
 #pragma unroll
    for ( int i = 0; i < 10; ++i )
       u[i] = valid ? sb[pos[i]] : R( 0 );
@@ -1248,7 +1312,8 @@ __global__ __launch_bounds__( 64 ) void kP2SmallApply( const P2ActGeomT< typenam
    if ( valid )
    {
       R y[10];
-      p2ElementAction< R, kFolded, STORED >( g, t, p0, u, y, cq[0], cq[1], cq[2], coefficient );
+      p2ElementAction< R, kFolded, STORED >( g, sg + 9 * t, reinterpret_cast< const R( * )[3] >( sg + 54 + 33 * t ), g.cw[t], p0,
+                                             u, y, cq[0], cq[1], cq[2], coefficient );
 #pragma unroll
       for ( int i = 0; i < 10; ++i )
          atomicAdd( &sb[pos[i]], y[i] );
@@ -1296,53 +1361,50 @@ static const K* p2Coefficients( Context* ctx, P2Operator& op, int L, int dtype )
 // the element action's geometry from the tile geometry of a level: lengths times
 // |n|, rotated by Q whose third row is n / |n| (affine cells: |n| = 1, Q = I)
 template < class R >
-static std::vector< P2ActGeomT< R > > actGeometry( const std::vector< P2CellGeom >& gs )
+__global__ void kP2ActGeometry( const P2CellGeom* __restrict__ geom, int64_t nc, P2ActGeomT< R >* __restrict__ out )
 {
-   std::vector< P2ActGeomT< R > > out( gs.size() );
-   for ( size_t c = 0; c < gs.size(); ++c )
+   const int64_t c = int64_t( blockIdx.x ) * blockDim.x + threadIdx.x;
+   if ( c >= nc )
+      return;
+   const P2CellGeom& g = geom[c];
+   P2ActGeomT< R >&  o = out[c];
+   double            Q[3][3] = { { 1, 0, 0 }, { 0, 1, 0 }, { 0, 0, 1 } }, len = 1.0;
+   if ( g.kind )
    {
-      const P2CellGeom& g = gs[c];
-      P2ActGeomT< R >&  o = out[c];
-      double            Q[3][3] = { { 1, 0, 0 }, { 0, 1, 0 }, { 0, 0, 1 } }, len = 1.0;
-      if ( g.kind )
-      {
-         len = std::sqrt( g.nl[0] * g.nl[0] + g.nl[1] * g.nl[1] + g.nl[2] * g.nl[2] );
-         for ( int d = 0; d < 3; ++d )
-            Q[2][d] = g.nl[d] / len;
-         // first row: the coordinate axis least aligned with n, made orthogonal to it
-         int k = 0;
-         for ( int d = 1; d < 3; ++d )
-            if ( std::fabs( Q[2][d] ) < std::fabs( Q[2][k] ) )
-               k = d;
-         const double s = 1.0 / std::sqrt( 1.0 - Q[2][k] * Q[2][k] );
-         for ( int d = 0; d < 3; ++d )
-            Q[0][d] = s * ( ( d == k ? 1.0 : 0.0 ) - Q[2][k] * Q[2][d] );
-         for ( int d = 0; d < 3; ++d )
-            Q[1][d] = Q[2][( d + 1 ) % 3] * Q[0][( d + 2 ) % 3] - Q[2][( d + 2 ) % 3] * Q[0][( d + 1 ) % 3];
-      }
-      auto turned = [&]( const double* v, int stride, int d ) {
-         return Q[d][0] * v[0] + Q[d][1] * v[stride] + Q[d][2] * v[2 * stride];
-      };
+      len = sqrt( g.nl[0] * g.nl[0] + g.nl[1] * g.nl[1] + g.nl[2] * g.nl[2] );
       for ( int d = 0; d < 3; ++d )
-      {
-         o.v0[d] = R( len * turned( g.v0, 1, d ) );
-         for ( int k = 0; k < 3; ++k )
-            o.hE[3 * d + k] = R( len * turned( g.hE + k, 3, d ) );
-         for ( int t = 0; t < 6; ++t )
-         {
-            for ( int k = 0; k < 3; ++k )
-               o.Dc[t][3 * k + d] = R( turned( g.Dc[t] + 3 * k, 1, d ) / len );
-            for ( int q = 0; q < 11; ++q )
-               o.xq[t][q][d] = R( len * turned( g.XQ[t][q], 1, d ) );
-         }
-      }
-      for ( int t = 0; t < 6; ++t )
-         o.cw[t] = R( g.kind ? g.adet[t] * len * len * len * std::fabs( g.dr ) : g.adet[t] );
-      o.lam0 = R( g.lam0 );
-      o.r0   = R( g.kind ? g.r0 / g.dr : 0.0 );
-      o.kind = g.kind;
+         Q[2][d] = g.nl[d] / len;
+      // first row: the coordinate axis least aligned with n, made orthogonal to it
+      const double f[3] = { fabs( Q[2][0] ), fabs( Q[2][1] ), fabs( Q[2][2] ) };
+      const int    k    = f[1] < f[0] ? ( f[2] < f[1] ? 2 : 1 ) : ( f[2] < f[0] ? 2 : 0 );
+      const double nk   = k == 0 ? Q[2][0] : ( k == 1 ? Q[2][1] : Q[2][2] );
+      const double s    = 1.0 / sqrt( 1.0 - nk * nk );
+      for ( int d = 0; d < 3; ++d )
+         Q[0][d] = s * ( ( d == k ? 1.0 : 0.0 ) - nk * Q[2][d] );
+      for ( int d = 0; d < 3; ++d )
+         Q[1][d] = Q[2][( d + 1 ) % 3] * Q[0][( d + 2 ) % 3] - Q[2][( d + 2 ) % 3] * Q[0][( d + 1 ) % 3];
    }
-   return out;
+   auto turned = [&]( const double* v, int stride, int d ) {
+      return Q[d][0] * v[0] + Q[d][1] * v[stride] + Q[d][2] * v[2 * stride];
+   };
+   for ( int d = 0; d < 3; ++d )
+   {
+      o.v0[d] = R( len * turned( g.v0, 1, d ) );
+      for ( int k = 0; k < 3; ++k )
+         o.hE[3 * d + k] = R( len * turned( g.hE + k, 3, d ) );
+      for ( int t = 0; t < 6; ++t )
+      {
+         for ( int k = 0; k < 3; ++k )
+            o.Dc[t][3 * k + d] = R( turned( g.Dc[t] + 3 * k, 1, d ) / len );
+         for ( int q = 0; q < 11; ++q )
+            o.xq[t][q][d] = R( len * turned( g.XQ[t][q], 1, d ) );
+      }
+   }
+   for ( int t = 0; t < 6; ++t )
+      o.cw[t] = R( g.kind ? g.adet[t] * len * len * len * fabs( g.dr ) : g.adet[t] );
+   o.lam0 = R( g.lam0 );
+   o.r0   = R( g.kind ? g.r0 / g.dr : 0.0 );
+   o.kind = g.kind;
 }
 
 template < class T >
@@ -1482,8 +1544,12 @@ static void p2ApplyBatched( Context* ctx, P2Operator& op, Lattice& lat, int L, F
       if ( mm % kTile != 0 )
          throw Error( HG_ERR_STATE, "P2 tile apply: micro-edge count not a multiple of the tile width" );
       if ( nint > 0 )
-         kP2TileApplyStoredBatched< double, double ><<< dim3( xcdGrid( nint ), nv ), kTileThreads, 0, ctx->stream >>>(
+      {
+         const auto run = st.topo.blend.empty() ? kP2TileApplyStoredBatched< double, double, false > :
+                                                  kP2TileApplyStoredBatched< double, double, true >;
+         run<<< dim3( xcdGrid( nint ), nv ), kTileThreads, 0, ctx->stream >>>(
              geom, table, tstride, mm, nint, lat.sc, lat.w, s, d, alpha, tint, lv, op.slotOn.p );
+      }
       HG_CHECK_HIP( hipGetLastError() );
       kP2TileApplyDiag< double, double, true ><<< dim3( xcdGrid( ndiag ), nv ), 64, 0, ctx->stream >>>(
           geom, geom64, nullptr, table, mm, ndiag, lat.sc, lat.w, s, d, alpha, tlast, lv, tstride, op.slotOn.p );
@@ -1556,9 +1622,11 @@ void p2Apply( Context* ctx, P2Operator& op, Function& src, Function& dst, int L,
          if ( mm % kTile != 0 )
             throw Error( HG_ERR_STATE, "P2 tile apply: micro-edge count not a multiple of the tile width" );
          if ( nint > 0 && table )
-            kP2TileApplyStored< T, K ><<< xcdGrid( nint ), kTileThreads, 0, ctx->stream >>>(
-                geom, op.tgeom.at( L ).p, op.kpar.p, table, mm, nint, lat.sc, lat.w, (const T*) s, (T*) d, alpha,
-                tint );
+         {
+            const auto run = st.topo.blend.empty() ? kP2TileApplyStored< T, K, false > : kP2TileApplyStored< T, K, true >;
+            run<<< xcdGrid( nint ), kTileThreads, 0, ctx->stream >>>( geom, table, mm, nint, lat.sc, lat.w, (const T*) s,
+                                                                      (T*) d, alpha, tint );
+         }
          else if ( nint > 0 )
             kP2TileApplyEval< T, K ><<< xcdGrid( nint ), kTileThreads, 0, ctx->stream >>>(
                 geom, op.tgeom.at( L ).p, op.kpar.p, nullptr, mm, nint, lat.sc, lat.w, (const T*) s, (T*) d, alpha,
@@ -1913,9 +1981,11 @@ int hg_p2_divkgrad_create( hg_ctx* h, hg_handle s, int minLevel, int maxLevel, i
          std::vector< P2CellGeom > gl = tg;
          tileGeometryLevel( gl, int64_t( 1 ) << L, kQP, 11 );
          op->tgeom[L].upload( ctx, gl );
-         const std::vector< P2ActGeomT< double > > ga = actGeometry< double >( gl );
-         op->ageom[L].upload( ctx, ga );
-         op->ageomF[L].upload( ctx, actGeometry< float >( gl ) );
+         op->ageom[L].alloc( ctx, size_t( t.nc ) );
+         op->ageomF[L].alloc( ctx, size_t( t.nc ) );
+         kP2ActGeometry< double ><<< gridFor( t.nc, 64 ), 64, 0, ctx->stream >>>( op->tgeom[L].p, t.nc, op->ageom[L].p );
+         kP2ActGeometry< float ><<< gridFor( t.nc, 64 ), 64, 0, ctx->stream >>>( op->tgeom[L].p, t.nc, op->ageomF[L].p );
+         HG_CHECK_HIP( hipGetLastError() );
       }
       std::vector< KParams > kp( 1 );
       kp[0]    = KParams{};

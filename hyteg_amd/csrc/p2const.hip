@@ -163,7 +163,7 @@ __global__ __launch_bounds__( kTileThreads ) void kP2ConstTileApply( const doubl
    if ( lb >= ntiles )
       return;
    int64_t         full;
-   const TileCoord tc   = tiles ? tileFromList( tiles, lb, mm, full ) : tileOf( lb, mm );
+   const TileCoord tc   = tileFromList( tiles, lb, mm, full );
    const int64_t   base = tc.c * sc1;
    const int32_t   top  = int32_t( 2 * mm );
    const double*   srcC = src + base;

@@ -100,47 +100,13 @@ __device__ __forceinline__ TileCoord tileOf( int64_t lb, int64_t mm )
 // inside the macro-cell up to a few micro-cells; they form the tile tetrahedron
 // of edge T - 1.  The last layer (ti + tj + tk = T - 1) holds 64 micro-cells per
 // tile (of 384 anchor/type pairs) and is handled by a one-wavefront kernel.
-// tileOfInterior decodes interior tile lb and returns its number `full` in the
-// numbering of all tiles (tileOf), which the coefficient tables use.
-__device__ __forceinline__ TileCoord tileOfInterior( int64_t lb, int64_t mm, int64_t& full )
-{
-   const int64_t T = tileEdges( mm );
-   TileCoord     tc;
-   const int64_t tpi = tet( T - 1 );
-   tc.c              = lb / tpi;
-   int64_t ti, tj, tk;
-   decodeMicro( T - 1, lb - tc.c * tpi, ti, tj, tk );
-   tc.x0 = kTile * ti;
-   tc.y0 = kTile * tj;
-   tc.z0 = kTile * tk;
-   full  = tc.c * tet( T ) + ( tet( T ) - tet( T - tk ) ) + triIndex( T - tk, ti, tj );
-   return tc;
-}
-// last-layer tile lb (of tri(T) per cell) and its number in the numbering of all tiles
-__device__ __forceinline__ TileCoord tileOfDiagonal( int64_t lb, int64_t mm, int64_t& full )
-{
-   const int64_t T = tileEdges( mm );
-   TileCoord     tc;
-   const int64_t per = tri( T );
-   tc.c              = lb / per;
-   int64_t ti, tj;
-   decodeTri( T, lb - tc.c * per, ti, tj );
-   const int64_t tk = T - 1 - ti - tj;
-   tc.x0            = kTile * ti;
-   tc.y0            = kTile * tj;
-   tc.z0            = kTile * tk;
-   full             = tc.c * tet( T ) + ( tet( T ) - tet( T - tk ) ) + triIndex( T - tk, ti, tj );
-   return tc;
-}
 // ---- tile lists -------------------------------------------------------------
 // Decoding a tile number by search costs a wavefront several hundred scalar
 // instructions (64-bit divisions) before its first load can issue.  The apply
 // kernels read their tile from a per-lattice list instead, one scalar load:
-// entry = c | m << 24 | ti << 40 | tj << 48 | tk << 56 (cell, number of the tile
-// in the cell in the numbering of all tiles, anchor / kTile).  List kTilesAll
-// follows tileOf, kTilesInterior tileOfInterior, kTilesLast tileOfDiagonal.
-// Lists exist while tet(T) < 2^16 and the cell count is below 2^24 (T: tile
-// edge count); otherwise the kernels decode.
+// entry = c | ti << 32 | tj << 40 | tk << 48 (cell, anchor / kTile).  List kTilesAll
+// follows tileOf; kTilesInterior holds the tiles with ti + tj + tk <= T - 2 (T: tile
+// edge count, at most 255: level 9), kTilesLast the last layer, both cell by cell.
 enum TileListKind
 {
    kTilesAll      = 0,
@@ -150,16 +116,14 @@ enum TileListKind
 inline const uint64_t* tileList( Context* ctx, Lattice& l, int64_t mm, int kind )
 {
    const int64_t T = tileEdges( mm );
-   if ( tet( T ) >= ( int64_t( 1 ) << 16 ) || l.nc >= ( int64_t( 1 ) << 24 ) || T > 255 )
-      return nullptr;
+   if ( T > 255 )
+      throw Error( -6, "P2 tile kernels support levels up to 9" );
    DevBuf< uint64_t >& buf = l.tileLists[kind];
    if ( !buf.p )
    {
       std::vector< uint64_t > e;
       auto put = [&]( int64_t c, int64_t ti, int64_t tj, int64_t tk ) {
-         const int64_t m = tet( T ) - tet( T - tk ) + triIndex( T - tk, ti, tj );
-         e.push_back( uint64_t( c ) | ( uint64_t( m ) << 24 ) | ( uint64_t( ti ) << 40 ) | ( uint64_t( tj ) << 48 ) |
-                      ( uint64_t( tk ) << 56 ) );
+         e.push_back( uint64_t( c ) | ( uint64_t( ti ) << 32 ) | ( uint64_t( tj ) << 40 ) | ( uint64_t( tk ) << 48 ) );
       };
       for ( int64_t c = 0; c < l.nc; ++c )
       {
@@ -188,12 +152,14 @@ __device__ __forceinline__ TileCoord tileFromList( const uint64_t* list, int64_t
 {
    using ConstU64   = const __attribute__( ( address_space( 4 ) ) ) uint64_t;
    const uint64_t e = ( (ConstU64*) list )[i];
+   const int32_t  ti = int32_t( e >> 32 ) & 255, tj = int32_t( e >> 40 ) & 255, tk = int32_t( e >> 48 ) & 255;
+   const int32_t  T  = int32_t( tileEdges( mm ) );
    TileCoord      tc;
-   tc.c  = int64_t( e & 0xFFFFFFu );
-   full  = tc.c * tilesPerCell( mm ) + int64_t( ( e >> 24 ) & 0xFFFFu );
-   tc.x0 = kTile * int64_t( ( e >> 40 ) & 255u );
-   tc.y0 = kTile * int64_t( ( e >> 48 ) & 255u );
-   tc.z0 = kTile * int64_t( e >> 56 );
+   tc.c  = int64_t( e & 0xFFFFFFFFu );
+   full  = tc.c * ( T * ( T + 1 ) * ( T + 2 ) / 6 ) + ( tetRowStart32( T, tj, tk ) + ti );
+   tc.x0 = kTile * ti;
+   tc.y0 = kTile * tj;
+   tc.z0 = kTile * tk;
    return tc;
 }
 
@@ -276,6 +242,35 @@ struct ElementBox
    static constexpr int edges[6][2] = { { 0, 1 }, { 0, 2 }, { 0, 3 }, { 1, 2 }, { 1, 3 }, { 2, 3 } };
    static constexpr int at( int i ) { return i < 4 ? vertex( i ) : ( vertex( edges[i - 4][0] ) + vertex( edges[i - 4][1] ) ) / 2; }
 };
+// coordinate d of vertex k of a micro-cell of type t (0 or 1) from a packed constant:
+// no table load where the type differs between lanes
+constexpr uint32_t vertexBits( int d )
+{
+   uint32_t b = 0;
+   for ( int t = 0; t < 6; ++t )
+      for ( int k = 0; k < 4; ++k )
+         b |= uint32_t( MicroCells::vof[t][k][d] ) << ( 4 * t + k );
+   return b;
+}
+template < int d >
+__device__ __forceinline__ int vertexOffset( int t, int k )
+{
+   constexpr uint32_t bits = vertexBits( d );
+   return int( ( bits >> ( 4 * t + k ) ) & 1u );
+}
+// box positions of the 10 P2 DoFs of the micro-cell (type t, anchor index a)
+__device__ __forceinline__ void laneBoxPositions( int t, int a, int pos[10] )
+{
+   constexpr int edges[6][2] = { { 0, 1 }, { 0, 2 }, { 0, 3 }, { 1, 2 }, { 1, 3 }, { 2, 3 } };
+#pragma unroll
+   for ( int k = 0; k < 4; ++k )
+      pos[k] = 2 * ( ( a & 3 ) + vertexOffset< 0 >( t, k ) ) +
+               kBox * ( 2 * ( ( ( a >> 2 ) & 3 ) + vertexOffset< 1 >( t, k ) ) +
+                        kBox * 2 * ( ( a >> 4 ) + vertexOffset< 2 >( t, k ) ) );
+#pragma unroll
+   for ( int e = 0; e < 6; ++e )
+      pos[4 + e] = ( pos[edges[e][0]] + pos[edges[e][1]] ) / 2;
+}
 // f(ElementBox< t >) for a wavefront-uniform type t
 template < class F >
 __device__ __forceinline__ void forType( int t, F&& f )

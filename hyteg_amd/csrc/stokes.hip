@@ -186,7 +186,7 @@ __global__ __launch_bounds__( kTileThreads ) void kStokesTileApply(
    if ( lb >= ntiles )
       return;
    int64_t         full;
-   const TileCoord tc    = tiles ? tileFromList( tiles, lb, mm, full ) : tileOf( lb, mm );
+   const TileCoord tc    = tileFromList( tiles, lb, mm, full );
    const int64_t   base1 = tc.c * sc1, base0 = tc.c * sc0;
    const int32_t   top1 = int32_t( 2 * mm ), top0 = int32_t( mm );
    const T*        uin[3] = { u0, u1, u2 };
