@@ -7,8 +7,8 @@
 // sub-stencils (vertex/edge to vertex/edge) are equivalent to the six 10x10
 // element matrices per macro-cell and level kept here.  The apply runs element
 // by element in the tile layout of the other P2 kernels (a 10x10 matrix-vector
-// product per micro-cell instead of a quadrature); the smoother gathers the
-// assembled row of a DoF from the element matrices of the micro-cells around it.
+// product per micro-cell instead of a quadrature); the smoother uses the assembled
+// rows, one per cell and parity class of a lattice point.
 //
 // Gauss-Seidel runs multicoloured: the owned macro vertex/edge/face DoFs first
 // (greedy colouring of their coupling graph, assembled rows), then the cell
@@ -38,8 +38,13 @@ namespace {
 constexpr int kMaxInc = 24;
 __constant__ int cIncN[8];
 __constant__ int cInc[8][kMaxInc][5];
-// lattice offsets of the 10 local DoFs of a type-t micro-cell from twice its anchor
-__constant__ int cLoc[6][10][3];
+// assembled row of a cell-interior point of parity class p: cRowN[p] entries at the
+// lattice offsets cRowOff[p] (dx + 2 | dy + 2 << 3 | dz + 2 << 6), the point itself among
+// them, padded to a multiple of kRowUnroll with its own offset (weight 0)
+constexpr int kRowMax    = 72; // a vertex couples with 65 points
+constexpr int kRowUnroll = 8;
+__constant__ int cRowN[8];
+__constant__ int cRowOff[8][kRowMax];
 
 struct IncTables
 {
@@ -97,6 +102,56 @@ const IncTables& incTables()
 {
    static const IncTables T = buildIncTables();
    return T;
+}
+
+// the assembled rows' offsets by parity class (cRowN, cRowOff) and the entry that
+// local DoF j of incident micro-cell k of the class adds to
+struct RowTables
+{
+   int n[8], off[8][kRowMax], self[8];
+   int slot[8][kMaxInc][10];
+};
+
+RowTables buildRowTables()
+{
+   const IncTables& T = incTables();
+   RowTables        R{};
+   for ( int cls = 0; cls < 8; ++cls )
+   {
+      const int        p[3] = { cls & 1, ( cls >> 1 ) & 1, ( cls >> 2 ) & 1 };
+      std::vector< int > offs;
+      auto             code = [&]( int k, int j ) {
+         int o[3];
+         for ( int d = 0; d < 3; ++d )
+            o[d] = 2 * T.e[cls][k][2 + d] + T.loc[T.e[cls][k][0]][j][d] - p[d] + 2;
+         return o[0] | ( o[1] << 3 ) | ( o[2] << 6 );
+      };
+      for ( int k = 0; k < T.n[cls]; ++k )
+         for ( int j = 0; j < 10; ++j )
+            offs.push_back( code( k, j ) );
+      // rows of the lattice one after the other (z, then y, then x)
+      std::sort( offs.begin(), offs.end() );
+      offs.erase( std::unique( offs.begin(), offs.end() ), offs.end() );
+      auto at = [&]( int o ) { return int( std::lower_bound( offs.begin(), offs.end(), o ) - offs.begin() ); };
+      for ( int k = 0; k < T.n[cls]; ++k )
+         for ( int j = 0; j < 10; ++j )
+            R.slot[cls][k][j] = at( code( k, j ) );
+      const int centre = 2 | ( 2 << 3 ) | ( 2 << 6 );
+      R.self[cls]      = at( centre );
+      while ( offs.size() % kRowUnroll != 0 )
+         offs.push_back( centre );
+      if ( offs.size() > size_t( kRowMax ) )
+         throw Error( HG_ERR_STATE, "P2 constant row longer than its table" );
+      R.n[cls] = int( offs.size() );
+      std::copy( offs.begin(), offs.end(), R.off[cls] );
+   }
+   return R;
+}
+
+const RowTables& rowTables()
+{
+   static const RowTables R = buildRowTables();
+   return R;
 }
 
 // exact P2 Laplace element matrix of the affine tetrahedron p[4]: the gradients
@@ -228,48 +283,76 @@ __global__ __launch_bounds__( kTileThreads ) void kP2ConstTileApply( const doubl
    }
 }
 
-// assembled row . x of the cell-interior point (X,Y,Z) of cell c, and its diagonal
-__device__ __forceinline__ double rowDot( const double* __restrict__ Ae, int64_t c, int32_t w1, int32_t X, int32_t Y,
-                                          int32_t Z, const double* __restrict__ xc, double& diag )
+// SOR on the cell-interior points of the rows (Y, Z) of one group (Y mod 3, Z mod 3),
+// in place: the three colours X mod 3 in turn (first 0, 1, 2, or backwards).  Rows of
+// a group are at least three apart in Y or Z and a point couples with points at most
+// two away, so rows are independent of each other, and within a row the next colour
+// follows after a workgroup-scope fence: a row's 2^gl lanes are in one wavefront.
+// A worker keeps its row's two assembled rows (even and odd X) in LDS, offsets
+// resolved to lattice positions, so a point costs its gathers and one multiply-add
+// each.  Bound by the latency of the gathers on small levels.  Cube level 5: 27
+// launches of 61 us a sweep with the row gathered from the 10x10 matrices of the
+// micro-cells around a point (a position formula and ten loads for each), 9 of 9 us
+// this way.
+__global__ __launch_bounds__( 256 ) void kP2ConstRowSOR( const int32_t* __restrict__ rows, int64_t nrows, int64_t nc,
+                                                        int64_t sc1, int32_t w, int gl, int backward, double relax,
+                                                        const double* __restrict__ W, const double* __restrict__ b,
+                                                        double* __restrict__ x )
 {
-   const int cls = ( X & 1 ) | ( ( Y & 1 ) << 1 ) | ( ( Z & 1 ) << 2 );
-   const int px = X & 1, py = Y & 1, pz = Z & 1;
-   double    acc = 0.0;
-   diag          = 0.0;
-   for ( int k = 0; k < cIncN[cls]; ++k )
-   {
-      const int*    e   = cInc[cls][k];
-      const int     t   = e[0], i = e[1];
-      const double* row = Ae + ( c * 6 + t ) * 100 + 10 * i;
-      const int32_t bx = X - px + 2 * e[2], by = Y - py + 2 * e[3], bz = Z - pz + 2 * e[4];
-#pragma unroll
-      for ( int j = 0; j < 10; ++j )
+   extern __shared__ double sRow[];
+   const int     workers = 256 >> gl, wk = int( threadIdx.x ) >> gl, lanes = 1 << gl, lane = int( threadIdx.x ) & ( lanes - 1 );
+   double*       sw = sRow + wk * 2 * kRowMax;
+   int32_t*      so = reinterpret_cast< int32_t* >( sRow + workers * 2 * kRowMax ) + wk * 2 * kRowMax;
+   const int64_t r  = xcdBlock( ( nrows * nc + workers - 1 ) / workers ) * workers + wk;
+   const bool    on = r < nrows * nc;
+   const int64_t c  = on ? r / nrows : 0;
+   const int32_t yz = on ? rows[r - c * nrows] : ( 1 | ( 1 << 16 ) );
+   const int32_t Y = yz & 0xFFFF, Z = yz >> 16;
+   const int     cls = ( ( Y & 1 ) << 1 ) | ( ( Z & 1 ) << 2 );
+   if ( on )
+      for ( int k = lane; k < 2 * kRowMax; k += lanes )
       {
-         const int32_t qx = bx + cLoc[t][j][0], qy = by + cLoc[t][j][1], qz = bz + cLoc[t][j][2];
-         acc += row[j] * xc[tetRowStart32( w1, qy, qz ) + qx];
+         const int px = k / kRowMax, j = k - px * kRowMax;
+         if ( j < cRowN[cls | px] )
+         {
+            const int o = cRowOff[cls | px][j];
+            so[k]       = tetRowStart32( w, Y + ( ( o >> 3 ) & 7 ) - 2, Z + ( o >> 6 ) - 2 ) + ( o & 7 ) - 2;
+            sw[k]       = W[( c * 8 + ( cls | px ) ) * ( kRowMax + 1 ) + j];
+         }
       }
-      diag += row[i];
+   __syncthreads();
+   if ( !on )
+      return;
+   const double*  inv  = W + ( c * 8 + cls ) * ( kRowMax + 1 ) + kRowMax; // 1 / diagonal, even and odd X
+   const double   inv0 = inv[0], inv1 = inv[kRowMax + 1];
+   const int      n0 = cRowN[cls], n1 = cRowN[cls | 1];
+   double*        xc   = x + c * sc1;
+   const int32_t  self = tetRowStart32( w, Y, Z ), last = w - 2 - Y - Z;
+   const double*  bc   = b + c * sc1 + self;
+   for ( int ph = 0; ph < 3; ++ph )
+   {
+      const int cx = backward ? 2 - ph : ph;
+      for ( int32_t X = ( cx == 0 ? 3 : cx ) + 3 * lane; X <= last; X += 3 * lanes )
+      {
+         const int      px = X & 1, n = px ? n1 : n0;
+         const double*  pw = sw + px * kRowMax;
+         const int32_t* po = so + px * kRowMax;
+         const double   rhs = bc[X];
+         double         acc = 0.0;
+         for ( int k = 0; k < n; k += kRowUnroll )
+         {
+            double v[kRowUnroll];
+#pragma unroll
+            for ( int u = 0; u < kRowUnroll; ++u )
+               v[u] = xc[po[k + u] + X];
+#pragma unroll
+            for ( int u = 0; u < kRowUnroll; ++u )
+               acc += pw[k + u] * v[u];
+         }
+         xc[self + X] += relax * ( rhs - acc ) * ( px ? inv1 : inv0 );
+      }
+      __threadfence_block();
    }
-   return acc;
-}
-
-// one colour (X,Y,Z mod 3 = cx,cy,cz) of SOR on the cell-interior points, in place
-__global__ void kP2ConstCellSOR( const double* __restrict__ Ae, int64_t mm, int64_t sc1, int64_t w1, int cx, int cy,
-                                 int cz, int32_t nb3, double relax, const double* __restrict__ b, double* __restrict__ x )
-{
-   const int64_t c   = blockIdx.y;
-   const int32_t tid = int32_t( blockIdx.x ) * blockDim.x + threadIdx.x;
-   if ( tid >= nb3 * nb3 * nb3 )
-      return;
-   const int32_t X = 3 * ( tid % nb3 ) + cx, Y = 3 * ( ( tid / nb3 ) % nb3 ) + cy, Z = 3 * ( tid / ( nb3 * nb3 ) ) + cz;
-   const int32_t top = int32_t( 2 * mm );
-   if ( X < 1 || Y < 1 || Z < 1 || X + Y + Z > top - 1 )
-      return;
-   double*       xc   = x + c * sc1;
-   const int64_t self = tetRowStart32( int32_t( w1 ), Y, Z ) + X;
-   double        diag;
-   const double  ax = rowDot( Ae, c, int32_t( w1 ), X, Y, Z, xc, diag );
-   xc[self] += relax * ( b[c * sc1 + self] - ax ) / diag;
 }
 
 // inverse diagonal of the cell-interior points (halo and boundary positions untouched)
@@ -292,25 +375,53 @@ __global__ void kP2ConstCellInvDiag( const double* __restrict__ Ae, int64_t mm, 
 }
 
 // SOR on the owned boundary DoFs of one colour through their assembled rows
-// (neighbour positions: owner slots of boundary DoFs, cell slots of interior ones)
-__global__ void kP2ConstBndSOR( int64_t n, const int32_t* __restrict__ list, int64_t ownerBase,
-                                const uint8_t* __restrict__ bndFlag, int flag, const int64_t* __restrict__ ptr,
-                                const int64_t* __restrict__ pos, const double* __restrict__ val,
-                                const double* __restrict__ invDiag, double relax, const double* __restrict__ b,
-                                double* __restrict__ x )
+// (neighbour positions: owner slots of boundary DoFs, cell slots of interior ones),
+// stored in colour order: rows [row0, row0 + n) of rowOf.  kBndLanes lanes take a
+// row's entries in turn and add their sums up, so that a row of up to some hundred
+// entries is two or three rounds of loads deep (one lane a row: 25 us a colour at
+// cube level 5, this way 5 us).
+constexpr int kBndLanes = 8, kBndUnroll = 4;
+__global__ __launch_bounds__( kBlock ) void kP2ConstBndSOR( int64_t row0, int64_t n, const int32_t* __restrict__ rowOf,
+                                                           int64_t ownerBase, const uint8_t* __restrict__ bndFlag,
+                                                           int flag, const int64_t* __restrict__ ptr,
+                                                           const int64_t* __restrict__ pos,
+                                                           const double* __restrict__ val,
+                                                           const double* __restrict__ invDiag, double relax,
+                                                           const double* __restrict__ b, double* __restrict__ x )
 {
-   const int64_t k = int64_t( blockIdx.x ) * blockDim.x + threadIdx.x;
+   const int64_t k    = ( int64_t( blockIdx.x ) * kBlock + threadIdx.x ) / kBndLanes;
+   const int     lane = int( threadIdx.x ) % kBndLanes;
    if ( k >= n )
       return;
-   const int32_t r = list[k];
+   const int32_t r = rowOf[row0 + k];
    if ( !( bndFlag[r] & flag ) )
       return;
-   double acc = 0.0;
-   for ( int64_t q = ptr[r]; q < ptr[r + 1]; ++q )
-      acc += val[q] * x[pos[q]];
-   const double d = 1.0 / invDiag[r];
-   const double o = x[ownerBase + r];
-   x[ownerBase + r] = o + relax * ( b[ownerBase + r] - acc - d * o ) * invDiag[r];
+   const int64_t e1 = ptr[row0 + k + 1];
+   const double  o = x[ownerBase + r], inv = invDiag[r], rhs = b[ownerBase + r];
+   double        acc = 0.0;
+   for ( int64_t q = ptr[row0 + k] + lane; q < e1; q += kBndLanes * kBndUnroll )
+   {
+      int64_t p[kBndUnroll];
+      double  w[kBndUnroll], v[kBndUnroll];
+#pragma unroll
+      for ( int u = 0; u < kBndUnroll; ++u )
+      {
+         const bool in = q + u * kBndLanes < e1;
+         p[u]          = in ? pos[q + u * kBndLanes] : ownerBase + r;
+         w[u]          = in ? val[q + u * kBndLanes] : 0.0;
+      }
+#pragma unroll
+      for ( int u = 0; u < kBndUnroll; ++u )
+         v[u] = x[p[u]];
+#pragma unroll
+      for ( int u = 0; u < kBndUnroll; ++u )
+         acc += w[u] * v[u];
+   }
+#pragma unroll
+   for ( int d = kBndLanes / 2; d > 0; d /= 2 )
+      acc += __shfl_xor( acc, d, kBndLanes );
+   if ( lane == 0 )
+      x[ownerBase + r] = o + relax * ( ( rhs - acc ) * inv - o );
 }
 
 // inverse diagonal of the owned boundary DoFs into their owner slots
@@ -327,10 +438,16 @@ struct P2ConstLevel
 {
    DevBuf< double >       Ae;      // nc * 6 * 100 element matrices
    DevBuf< double >       invDiag; // owned boundary DoFs of the level-(L+1) lattice
-   DevBuf< int64_t >      csrPtr, csrPos;
+   DevBuf< int64_t >      csrPtr, csrPos; // assembled boundary rows, in the order of colorRows
    DevBuf< double >       csrVal;
    std::vector< int64_t > colorStart;
    DevBuf< int32_t >      colorRows;
+   // assembled rows of the cell-interior points, per cell and parity class: kRowMax
+   // weights (cRowOff) and the inverse diagonal
+   DevBuf< double >       W;
+   // interior rows Y | Z << 16 of a cell grouped by (Y mod 3) + 3 (Z mod 3)
+   DevBuf< int32_t >      rows3;
+   int64_t                rowStart3[10] = {};
 };
 
 struct P2ConstOperator : OperatorBase
@@ -420,21 +537,9 @@ void buildLevel( Context* ctx, Storage& st, int L, P2ConstLevel& o )
                   }
                }
       }
-   std::vector< int64_t > ptr( lat.nb + 1, 0 ), pos;
-   std::vector< double >  val, inv( lat.nb );
+   std::vector< double > inv( lat.nb );
    for ( int64_t r = 0; r < lat.nb; ++r )
-   {
-      for ( const auto& e : row[r] )
-      {
-         pos.push_back( e.first );
-         val.push_back( e.second );
-      }
-      ptr[r + 1] = int64_t( pos.size() );
-      inv[r]     = 1.0 / diag[r];
-   }
-   o.csrPtr.upload( ctx, ptr );
-   o.csrPos.upload( ctx, pos.empty() ? std::vector< int64_t >( 1, 0 ) : pos );
-   o.csrVal.upload( ctx, val.empty() ? std::vector< double >( 1, 0.0 ) : val );
+      inv[r] = 1.0 / diag[r];
    o.invDiag.upload( ctx, inv.empty() ? std::vector< double >( 1, 0.0 ) : inv );
    // greedy colouring in canonical order
    std::vector< int >  color( lat.nb, -1 );
@@ -464,6 +569,44 @@ void buildLevel( Context* ctx, Storage& st, int L, P2ConstLevel& o )
    }
    o.colorStart[ncolor] = int64_t( rows.size() );
    o.colorRows.upload( ctx, rows.empty() ? std::vector< int32_t >( 1, 0 ) : rows );
+   std::vector< int64_t > ptr( 1, 0 ), pos;
+   std::vector< double >  val;
+   for ( int32_t r : rows )
+   {
+      for ( const auto& e : row[r] )
+      {
+         pos.push_back( e.first );
+         val.push_back( e.second );
+      }
+      ptr.push_back( int64_t( pos.size() ) );
+   }
+   o.csrPtr.upload( ctx, ptr );
+   o.csrPos.upload( ctx, pos.empty() ? std::vector< int64_t >( 1, 0 ) : pos );
+   o.csrVal.upload( ctx, val.empty() ? std::vector< double >( 1, 0.0 ) : val );
+   // assembled rows of the cell interiors
+   const RowTables&      R = rowTables();
+   std::vector< double > W( size_t( t.nc ) * 8 * ( kRowMax + 1 ), 0.0 );
+   for ( int c = 0; c < t.nc; ++c )
+      for ( int cls = 0; cls < 8; ++cls )
+      {
+         double* w = &W[( size_t( c ) * 8 + cls ) * ( kRowMax + 1 )];
+         for ( int k = 0; k < T.n[cls]; ++k )
+            for ( int j = 0; j < 10; ++j )
+               w[R.slot[cls][k][j]] += Ae[( size_t( c ) * 6 + T.e[cls][k][0] ) * 100 + 10 * T.e[cls][k][1] + j];
+         w[kRowMax] = 1.0 / w[R.self[cls]];
+      }
+   o.W.upload( ctx, W );
+   std::vector< int32_t > rows3;
+   for ( int g = 0; g < 9; ++g )
+   {
+      o.rowStart3[g] = int64_t( rows3.size() );
+      for ( int32_t z = 1; z <= 2 * mm - 2; ++z )
+         for ( int32_t y = 1; y + z <= 2 * mm - 2; ++y )
+            if ( y % 3 + 3 * ( z % 3 ) == g )
+               rows3.push_back( y | ( z << 16 ) );
+   }
+   o.rowStart3[9] = int64_t( rows3.size() );
+   o.rows3.upload( ctx, rows3.empty() ? std::vector< int32_t >( 1, 0 ) : rows3 );
 }
 
 void checkFn( const P2ConstOperator& op, const Function& f, int L )
@@ -474,7 +617,6 @@ void checkFn( const P2ConstOperator& op, const Function& f, int L )
       throw Error( HG_ERR_ARG, "level outside the operator's or function's level range" );
 }
 
-int32_t boxCount( int64_t w ) { return int32_t( ( w + 2 ) / 3 ); }
 } // namespace
 } // namespace hg
 
@@ -492,7 +634,9 @@ int hg_p2_const_create( hg_ctx* h, hg_handle s, int minLevel, int maxLevel, hg_h
          const IncTables& T = incTables();
          HG_CHECK_HIP( hipMemcpyToSymbol( HIP_SYMBOL( cIncN ), T.n, sizeof( T.n ) ) );
          HG_CHECK_HIP( hipMemcpyToSymbol( HIP_SYMBOL( cInc ), T.e, sizeof( T.e ) ) );
-         HG_CHECK_HIP( hipMemcpyToSymbol( HIP_SYMBOL( cLoc ), T.loc, sizeof( T.loc ) ) );
+         const RowTables& R = rowTables();
+         HG_CHECK_HIP( hipMemcpyToSymbol( HIP_SYMBOL( cRowN ), R.n, sizeof( R.n ) ) );
+         HG_CHECK_HIP( hipMemcpyToSymbol( HIP_SYMBOL( cRowOff ), R.off, sizeof( R.off ) ) );
       } );
       Storage& st = ctx->storage( s );
       auto     op = std::make_unique< P2ConstOperator >();
@@ -569,16 +713,24 @@ static void p2ConstSOR( Context* ctx, P2ConstOperator& op, Function& x, Function
       const int64_t n = o.colorStart[cc + 1] - o.colorStart[cc];
       if ( n == 0 )
          return;
-      kP2ConstBndSOR<<< gridFor( n ), kBlock, 0, ctx->stream >>>( n, o.colorRows.p + o.colorStart[cc], lat.nc * lat.sc,
-                                                                   lat.bndFlag.p, flag, o.csrPtr.p, o.csrPos.p,
-                                                                   o.csrVal.p, o.invDiag.p, relax, bp, xp );
+      kP2ConstBndSOR<<< gridFor( n * kBndLanes ), kBlock, 0, ctx->stream >>>(
+          o.colorStart[cc], n, o.colorRows.p, lat.nc * lat.sc, lat.bndFlag.p, flag, o.csrPtr.p, o.csrPos.p, o.csrVal.p,
+          o.invDiag.p, relax, bp, xp );
       HG_CHECK_HIP( hipGetLastError() );
    };
-   const int32_t nb3 = boxCount( lat.w );
-   const dim3    grid( unsigned( ( int64_t( nb3 ) * nb3 * nb3 + 255 ) / 256 ), unsigned( lat.nc ) );
-   auto interiorColour = [&]( int k ) {
-      kP2ConstCellSOR<<< grid, 256, 0, ctx->stream >>>( o.Ae.p, mm, lat.sc, lat.w, k % 3, ( k / 3 ) % 3, k / 9, nb3,
-                                                         relax, bp, xp );
+   // lanes of a row worker: enough for the points of one colour of the longest row
+   int gl = 4;
+   while ( gl < 6 && ( 1 << gl ) < ( lat.w - 3 ) / 3 )
+      ++gl;
+   const int    workers = 256 >> gl;
+   const size_t lds     = size_t( workers ) * 2 * kRowMax * ( sizeof( double ) + sizeof( int32_t ) );
+   // the three colours X mod 3 of the rows with (Y mod 3, Z mod 3) = (g % 3, g / 3)
+   auto interiorGroup = [&]( int g ) {
+      const int64_t n = o.rowStart3[g + 1] - o.rowStart3[g];
+      if ( n == 0 )
+         return;
+      kP2ConstRowSOR<<< xcdGrid( ( n * lat.nc + workers - 1 ) / workers ), 256, lds, ctx->stream >>>(
+          o.rows3.p + o.rowStart3[g], n, lat.nc, lat.sc, int32_t( lat.w ), gl, int( backward ), relax, o.W.p, bp, xp );
       HG_CHECK_HIP( hipGetLastError() );
    };
    if ( !backward )
@@ -588,14 +740,14 @@ static void p2ConstSOR( Context* ctx, P2ConstOperator& op, Function& x, Function
       // the cell interiors read the new boundary values through their halos
       pullHalos( ctx, st, lat, xp, 0 );
       if ( flag & kInner )
-         for ( int k = 0; k < 27; ++k )
-            interiorColour( k );
+         for ( int g = 0; g < 9; ++g )
+            interiorGroup( g );
    }
    else
    {
       if ( flag & kInner )
-         for ( int k = 26; k >= 0; --k )
-            interiorColour( k );
+         for ( int g = 8; g >= 0; --g )
+            interiorGroup( g );
       for ( size_t cc = nbc; cc-- > 0; )
          boundaryColour( cc );
       pullHalos( ctx, st, lat, xp, 0 );
