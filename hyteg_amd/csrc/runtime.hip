@@ -44,8 +44,46 @@ void Storage::init( Context* ctx )
          for ( int j = 0; j < 2; ++j )
             m[c].eperm[k][j] = localOf( t.ev[t.ce[c][k]][j] );
       }
+      auto codeOf = []( auto& list, const auto& perm ) {
+         for ( size_t i = 0; i < list.size(); ++i )
+            if ( list[i] == perm )
+               return int8_t( i );
+         list.push_back( perm );
+         return int8_t( list.size() - 1 );
+      };
+      for ( int k = 0; k < 4; ++k )
+         m[c].fcode[k] = codeOf( faceOrient, std::array< int8_t, 3 >{ m[c].fperm[k][0], m[c].fperm[k][1], m[c].fperm[k][2] } );
+      for ( int k = 0; k < 6; ++k )
+         m[c].ecode[k] = codeOf( edgeOrient, std::array< int8_t, 2 >{ m[c].eperm[k][0], m[c].eperm[k][1] } );
    }
    meta.upload( ctx, m );
+   std::vector< int32_t >                  fi( 4 * size_t( t.nf ), -1 ), ei;
+   std::vector< std::vector< int32_t > >   ec( t.ne );
+   std::vector< int >                      nfi( t.nf, 0 );
+   for ( int c = 0; c < t.nc; ++c )
+   {
+      for ( int k = 0; k < 4; ++k )
+      {
+         const int f = t.cf[c][k];
+         if ( nfi[f] > 1 )
+         {
+            facesShared2 = false; // the general halo kernels take any number
+            continue;
+         }
+         fi[4 * size_t( f ) + 2 * nfi[f]]     = c;
+         fi[4 * size_t( f ) + 2 * nfi[f] + 1] = m[c].fcode[k];
+         ++nfi[f];
+      }
+      for ( int k = 0; k < 6; ++k )
+      {
+         ec[t.ce[c][k]].push_back( c );
+         ec[t.ce[c][k]].push_back( m[c].ecode[k] );
+      }
+   }
+   for ( const auto& l : ec )
+      ei.insert( ei.end(), l.begin(), l.end() );
+   faceInc.upload( ctx, fi );
+   edgeInc.upload( ctx, ei );
 
    auto csr = [&]( int nprim, auto primOfLocal, int nlocal, DevBuf< int32_t >& ptr, DevBuf< int32_t >& ent ) {
       std::vector< std::vector< int32_t > > lists( nprim );
@@ -116,6 +154,33 @@ Lattice& Storage::lattice( Context* ctx, int L )
             }
    l.cellMask.upload( ctx, mask );
 
+   if ( l.sc < ( int64_t( 1 ) << 31 ) )
+   {
+      const int64_t fin = l.num.fin, ein = l.num.ein, mm = l.mm;
+      std::vector< int32_t > o;
+      o.reserve( faceOrient.size() * size_t( fin ) + edgeOrient.size() * size_t( ein ) + 1 );
+      for ( const auto& p : faceOrient )
+         for ( int64_t y = 1; y <= mm - 2; ++y )
+            for ( int64_t x = 1; x + y <= mm - 1; ++x )
+            {
+               int64_t t[4] = { 0, 0, 0, 0 };
+               t[p[0]]      = mm - x - y;
+               t[p[1]]      = x;
+               t[p[2]]      = y;
+               o.push_back( int32_t( tetIndex( l.w, t[1], t[2], t[3] ) ) );
+            }
+      for ( const auto& p : edgeOrient )
+         for ( int64_t s = 1; s <= mm - 1; ++s )
+         {
+            int64_t t[4] = { 0, 0, 0, 0 };
+            t[p[0]]      = mm - s;
+            t[p[1]]      = s;
+            o.push_back( int32_t( tetIndex( l.w, t[1], t[2], t[3] ) ) );
+         }
+      o.push_back( 0 ); // never empty
+      l.haloOffsets.upload( ctx, o );
+   }
+
    std::vector< int32_t > rows;
    for ( int g = 0; g < 4; ++g )
    {
@@ -145,96 +210,268 @@ Lattice& Storage::lattice( Context* ctx, int L )
    return l;
 }
 
-template < class T >
-__global__ void kPull( const CellMeta* __restrict__ meta, int64_t nc, int64_t sc, int64_t w, int64_t mm, int64_t fin,
-                       int64_t ein, int64_t eoff, int64_t foff, int lv, T* __restrict__ v )
+// ---- halo exchange ----------------------------------------------------------
+// A halo copy's place in its cell follows from the primitive's orientation alone:
+// the lattice keeps the cell-local offsets of the face and edge interiors for each
+// orientation that the mesh has (haloOffsets), so an exchange costs one table load,
+// one load and one store a value.  Bound by those loads' latency on small levels and
+// by the scattered lines on large ones.  (Formed in the kernel -- 64-bit divisions,
+// a square root for the row of a triangle, the tetrahedral index -- a pull took
+// 14 us and a push 19 us at shell level 3, P2, and 1.21 and 0.65 ms at level 6.)
+struct HaloGeom
 {
-   const int64_t per = 4 * fin + 6 * ein + 4;
-   const int64_t tid = int64_t( blockIdx.x ) * blockDim.x + threadIdx.x;
-   const int64_t gid = tid >> lv;
-   const int64_t vec = tid & ( ( int64_t( 1 ) << lv ) - 1 );
-   if ( gid >= per * nc )
-      return;
-   const int64_t   c = gid / per;
-   int64_t         j = gid - c * per;
-   const CellMeta& m = meta[c];
-   int64_t         t[4];
-   int64_t         src;
-   const int64_t   base = nc * sc;
-   if ( j < 4 * fin )
+   const CellMeta* meta;
+   const int32_t * off, *faceInc, *edgePtr, *edgeInc, *vertPtr, *vertInc;
+   int64_t         sc, base; // values of a cell lattice; first owned DoF
+   uint32_t        fin, ein, nf, ne, nv, nfo; // points of a face / edge interior; counts; face orientations
+   int64_t         eoff, foff;
+   int32_t         vo[4]; // cell-local offsets of the vertices
+   FastDiv         dfin, dein;
+};
+
+static HaloGeom haloGeom( const Storage& st, const Lattice& l )
+{
+   const int64_t fin = l.num.fin, ein = l.num.ein, mm = l.mm;
+   HaloGeom g;
+   g.meta    = st.meta.p;
+   g.off     = l.haloOffsets.p;
+   g.faceInc = st.faceInc.p;
+   g.edgePtr = st.edgeCellPtr.p;
+   g.edgeInc = st.edgeInc.p;
+   g.vertPtr = st.vertCellPtr.p;
+   g.vertInc = st.vertCells.p;
+   g.sc      = l.sc;
+   g.base    = l.nc * l.sc;
+   g.fin     = uint32_t( fin );
+   g.ein     = uint32_t( ein );
+   g.nf      = uint32_t( st.topo.nf );
+   g.ne      = uint32_t( st.topo.ne );
+   g.nv      = uint32_t( st.topo.nv );
+   g.nfo     = uint32_t( st.faceOrient.size() );
+   g.eoff    = l.num.eoff;
+   g.foff    = l.num.foff;
+   g.vo[0]   = 0;
+   g.vo[1]   = int32_t( tetIndex( l.w, mm, 0, 0 ) );
+   g.vo[2]   = int32_t( tetIndex( l.w, 0, mm, 0 ) );
+   g.vo[3]   = int32_t( tetIndex( l.w, 0, 0, mm ) );
+   g.dfin    = FastDiv( fin );
+   g.dein    = FastDiv( ein );
+   return g;
+}
+
+// whether a lattice's halo exchange runs on the offset tables: cell-local offsets in
+// 32 bits and block counts within a grid (beyond that the general kernels run)
+static bool haloTables( const Storage& st, const Lattice& l, int lv )
+{
+   const int64_t most = int64_t( 1 ) << 31, nf = st.topo.nf, ne = st.topo.ne, nv = st.topo.nv;
+   // threads of a launch over n primitives of `per` values: whole workgroups each, or packed
+   auto threads = []( int64_t per, int64_t n ) { return ( per / kBlock + 1 ) * kBlock * n; };
+   return st.facesShared2 && l.haloOffsets.p && threads( l.haloPerCell() << lv, l.nc ) / kBlock < most &&
+          ( l.haloPerCell() << lv ) < most && threads( l.num.fin << lv, nf ) / kBlock < most &&
+          ( ( l.haloPerCell() << lv ) >= kBlock / 2 || ( l.haloPerCell() << lv ) * l.nc < most ) &&
+          ( ( l.num.fin << lv ) >= kBlock / 2 || ( l.num.fin << lv ) * nf < most ) && ( l.num.ein << lv ) * ne < most &&
+          ( nv << lv ) < most;
+}
+
+// every halo copy from its owner.  blocks: workgroups of one cell (0: cells share
+// workgroups, for lattices whose halo is smaller than one)
+template < class T >
+__global__ __launch_bounds__( kBlock ) void kPull( HaloGeom g, uint32_t nc, uint32_t blocks, FastDiv per, int lv,
+                                                  T* __restrict__ v )
+{
+   uint32_t c, j;
+   if ( blocks )
    {
-      const int     k = int( j / fin );
-      const int64_t i = j - k * fin;
-      int64_t       a, b;
-      decodeTri( mm - 2, i, a, b );
-      faceToCell( m, k, mm, a + 1, b + 1, t );
-      src = base + foff + int64_t( m.face[k] ) * fin + i;
+      c = blockIdx.x / blocks;
+      j = ( blockIdx.x - c * blocks ) * kBlock + threadIdx.x;
    }
-   else if ( ( j -= 4 * fin ) < 6 * ein )
+   else
+      c = per.div( blockIdx.x * kBlock + threadIdx.x, j );
+   const uint32_t  vec = j & ( ( 1u << lv ) - 1u );
+   uint32_t        p   = j >> lv;
+   if ( c >= nc || j >= per.d )
+      return;
+   const CellMeta& m = g.meta[c];
+   int64_t         src;
+   int32_t         o;
+   if ( p < 4 * g.fin )
    {
-      const int     k = int( j / ein );
-      const int64_t s = j - k * ein + 1;
-      edgeToCell( m, k, mm, s, t );
-      src = base + eoff + int64_t( m.edge[k] ) * ein + ( s - 1 );
+      const uint32_t k = uint32_t( p >= g.fin ) + uint32_t( p >= 2 * g.fin ) + uint32_t( p >= 3 * g.fin );
+      p -= k * g.fin;
+      o   = g.off[uint32_t( m.fcode[k] ) * g.fin + p];
+      src = g.base + g.foff + int64_t( m.face[k] ) * g.fin + p;
+   }
+   else if ( ( p -= 4 * g.fin ) < 6 * g.ein )
+   {
+      uint32_t k = 0;
+#pragma unroll
+      for ( uint32_t i = 1; i < 6; ++i )
+         k += uint32_t( p >= i * g.ein );
+      p -= k * g.ein;
+      o   = g.off[g.nfo * g.fin + uint32_t( m.ecode[k] ) * g.ein + p];
+      src = g.base + g.eoff + int64_t( m.edge[k] ) * g.ein + p;
    }
    else
    {
-      const int k = int( j - 6 * ein );
-      t[0] = t[1] = t[2] = t[3] = 0;
-      t[k]                      = mm;
-      src                       = base + m.vert[k];
+      const uint32_t k = p - 6 * g.ein;
+      o                = k == 0 ? g.vo[0] : ( k == 1 ? g.vo[1] : ( k == 2 ? g.vo[2] : g.vo[3] ) );
+      src              = g.base + m.vert[k];
    }
-   v[( ( c * sc + tetIndex( w, t[1], t[2], t[3] ) ) << lv ) + vec] = v[( src << lv ) + vec];
+   v[( ( c * g.sc + o ) << lv ) + vec] = v[( src << lv ) + vec];
 }
 
+// the halo copies of every owned DoF summed into it, in the order of
+// forEachIncident, kPushUnroll loads in flight (a macro-vertex of the shell has up to
+// ~36 incident cells).  Workgroups [0, fb): faces (blocks of them a face, or sharing:
+// 0), [fb, fb + eb): edges, the rest: vertices.
+constexpr int kPushUnroll = 12;
 template < class T >
-__global__ void kPushAdditive( BndGeom g, const uint8_t* __restrict__ bndFlag, int64_t nb, int64_t nc,
-                               int excludeFlag, int zeroOut, int lv, T* __restrict__ v )
+__global__ __launch_bounds__( kBlock ) void kPushAdditive( HaloGeom g, uint32_t blocks, uint32_t fb, uint32_t eb,
+                                                          FastDiv perFace, FastDiv perEdge,
+                                                          const uint8_t* __restrict__ bndFlag, int excludeFlag,
+                                                          int zeroOut, int lv, T* __restrict__ v )
 {
-   using A           = typename Acc< T >::type;
-   const int64_t tid = int64_t( blockIdx.x ) * blockDim.x + threadIdx.x;
-   const int64_t b   = tid >> lv;
-   const int64_t vec = tid & ( ( int64_t( 1 ) << lv ) - 1 );
-   if ( b >= nb || ( bndFlag[b] & excludeFlag ) )
-      return;
-   const int64_t base = nc * g.sc;
-   A             s    = zeroOut ? A( 0 ) : toAcc( v[( ( base + b ) << lv ) + vec] );
-   // the halo copies in the order of forEachIncident, eight loads in flight (a
-   // macro-vertex of the shell has up to ~36 incident cells)
-   int32_t e0, e1;
-   incidentRange( g, b, e0, e1 );
-   for ( int32_t e = e0; e < e1; e += 8 )
+   using A            = typename Acc< T >::type;
+   const uint32_t msk = ( 1u << lv ) - 1u;
+   if ( blockIdx.x < fb )
    {
-      A buf[8];
-#pragma unroll
-      for ( int j = 0; j < 8; ++j )
+      uint32_t f, j;
+      if ( blocks )
       {
-         buf[j] = A( 0 );
-         if ( e + j < e1 )
-         {
-            int64_t       x, y, z;
-            const int64_t c = incidentAt( g, b, e + j, x, y, z );
-            buf[j]          = toAcc( v[( ( c * g.sc + tetIndex( g.w, x, y, z ) ) << lv ) + vec] );
-         }
+         f = blockIdx.x / blocks;
+         j = ( blockIdx.x - f * blocks ) * kBlock + threadIdx.x;
+      }
+      else
+         f = perFace.div( blockIdx.x * kBlock + threadIdx.x, j );
+      const uint32_t p = j >> lv, vec = j & msk;
+      if ( f >= g.nf || j >= perFace.d )
+         return;
+      const int64_t b = g.foff + int64_t( f ) * g.fin + p;
+      if ( bndFlag[b] & excludeFlag )
+         return;
+      const int32_t* inc = g.faceInc + 4 * size_t( f );
+      const int32_t  c0 = inc[0], c1 = inc[2];
+      const A        a0 = toAcc( v[( ( c0 * g.sc + g.off[uint32_t( inc[1] ) * g.fin + p] ) << lv ) + vec] );
+      const A  a1 = c1 >= 0 ? toAcc( v[( ( c1 * g.sc + g.off[uint32_t( inc[3] ) * g.fin + p] ) << lv ) + vec] ) : A( 0 );
+      T&       out = v[( ( g.base + b ) << lv ) + vec];
+      A        s   = zeroOut ? A( 0 ) : toAcc( out );
+      s += a0;
+      if ( c1 >= 0 )
+         s += a1;
+      out = fromAcc< T >( s );
+      return;
+   }
+   int64_t        b;
+   int32_t        e0, e1;
+   uint32_t       p, vec;
+   const int32_t *inc, *off;
+   const bool     edge = blockIdx.x < fb + eb;
+   if ( edge )
+   {
+      uint32_t       j;
+      const uint32_t e = perEdge.div( ( blockIdx.x - fb ) * kBlock + threadIdx.x, j );
+      if ( e >= g.ne )
+         return;
+      p   = j >> lv;
+      vec = j & msk;
+      b   = g.eoff + int64_t( e ) * g.ein + p;
+      e0  = g.edgePtr[e];
+      e1  = g.edgePtr[e + 1];
+      inc = g.edgeInc;
+      off = g.off + g.nfo * g.fin + p;
+   }
+   else
+   {
+      const uint32_t j = ( blockIdx.x - fb - eb ) * kBlock + threadIdx.x;
+      p                = j >> lv;
+      vec              = j & msk;
+      if ( p >= g.nv )
+         return;
+      b   = p;
+      e0  = g.vertPtr[p];
+      e1  = g.vertPtr[p + 1];
+      inc = g.vertInc;
+      off = nullptr;
+   }
+   if ( bndFlag[b] & excludeFlag )
+      return;
+   T& out = v[( ( g.base + b ) << lv ) + vec];
+   A  s   = zeroOut ? A( 0 ) : toAcc( out );
+   for ( int32_t e = e0; e < e1; e += kPushUnroll )
+   {
+      int64_t pos[kPushUnroll];
+      A       buf[kPushUnroll];
+#pragma unroll
+      for ( int j = 0; j < kPushUnroll; ++j )
+      {
+         const int32_t i = min( e + j, e1 - 1 );
+         const int32_t c = inc[2 * i], k = inc[2 * i + 1];
+         const int32_t o = edge ? off[uint32_t( k ) * g.ein] :
+                                  ( k == 0 ? g.vo[0] : ( k == 1 ? g.vo[1] : ( k == 2 ? g.vo[2] : g.vo[3] ) ) );
+         pos[j]          = ( ( c * g.sc + o ) << lv ) + vec;
       }
 #pragma unroll
-      for ( int j = 0; j < 8; ++j )
+      for ( int j = 0; j < kPushUnroll; ++j )
+         buf[j] = toAcc( v[pos[j]] );
+#pragma unroll
+      for ( int j = 0; j < kPushUnroll; ++j )
          if ( e + j < e1 )
             s += buf[j];
    }
-   v[( ( base + b ) << lv ) + vec] = fromAcc< T >( s );
+   out = fromAcc< T >( s );
+}
+
+// the same for lattices of 2^31 points a cell and more (haloTables)
+template < class T >
+__global__ void kPullGeneral( BndGeom g, int64_t nc, int64_t nb, int lv, T* __restrict__ v )
+{
+   const int64_t tid = int64_t( blockIdx.x ) * blockDim.x + threadIdx.x;
+   const int64_t b = tid >> lv, vec = tid & ( ( int64_t( 1 ) << lv ) - 1 );
+   if ( b >= nb )
+      return;
+   const T val = v[( ( nc * g.sc + b ) << lv ) + vec];
+   forEachIncident( g, b, [&]( int64_t c, int64_t x, int64_t y, int64_t z, int ) {
+      v[( ( c * g.sc + tetIndex( g.w, x, y, z ) ) << lv ) + vec] = val;
+   } );
+}
+template < class T >
+__global__ void kPushGeneral( BndGeom g, const uint8_t* __restrict__ bndFlag, int64_t nb, int64_t nc, int excludeFlag,
+                              int zeroOut, int lv, T* __restrict__ v )
+{
+   using A           = typename Acc< T >::type;
+   const int64_t tid = int64_t( blockIdx.x ) * blockDim.x + threadIdx.x;
+   const int64_t b = tid >> lv, vec = tid & ( ( int64_t( 1 ) << lv ) - 1 );
+   if ( b >= nb || ( bndFlag[b] & excludeFlag ) )
+      return;
+   T& out = v[( ( nc * g.sc + b ) << lv ) + vec];
+   A  s   = zeroOut ? A( 0 ) : toAcc( out );
+   forEachIncident( g, b, [&]( int64_t c, int64_t x, int64_t y, int64_t z, int ) {
+      s += toAcc( v[( ( c * g.sc + tetIndex( g.w, x, y, z ) ) << lv ) + vec] );
+   } );
+   out = fromAcc< T >( s );
 }
 
 void pullHalos( Context* ctx, Storage& st, Lattice& lat, void* data, int dtype, int lv )
 {
-   const int64_t n = lat.haloPerCell() * lat.nc;
-   if ( n == 0 )
+   const int64_t per = lat.haloPerCell() << lv;
+   if ( per * lat.nc == 0 )
       return;
+   if ( !haloTables( st, lat, lv ) )
+   {
+      dispatchType( dtype, [&]( auto tag ) {
+         using T = decltype( tag );
+         kPullGeneral< T ><<< gridFor( lat.nb << lv ), kBlock, 0, ctx->stream >>>( BndGeom::of( st, lat ), lat.nc, lat.nb,
+                                                                                  lv, (T*) data );
+      } );
+      HG_CHECK_HIP( hipGetLastError() );
+      return;
+   }
+   const HaloGeom g      = haloGeom( st, lat );
+   const uint32_t blocks = per >= kBlock / 2 ? uint32_t( ( per + kBlock - 1 ) / kBlock ) : 0;
+   const unsigned grid   = blocks ? unsigned( blocks * lat.nc ) : gridFor( per * lat.nc );
    dispatchType( dtype, [&]( auto tag ) {
       using T = decltype( tag );
-      kPull< T ><<< gridFor( n << lv ), kBlock, 0, ctx->stream >>>( st.meta.p, lat.nc, lat.sc, lat.w, lat.mm,
-                                                                   lat.num.fin, lat.num.ein, lat.num.eoff,
-                                                                   lat.num.foff, lv, (T*) data );
+      kPull< T ><<< grid, kBlock, 0, ctx->stream >>>( g, uint32_t( lat.nc ), blocks, FastDiv( per ), lv, (T*) data );
    } );
    HG_CHECK_HIP( hipGetLastError() );
 }
@@ -243,10 +480,27 @@ void pushAdditive( Context* ctx, Storage& st, Lattice& lat, void* data, int dtyp
 {
    if ( lat.nb == 0 )
       return;
+   if ( !haloTables( st, lat, lv ) )
+   {
+      dispatchType( dtype, [&]( auto tag ) {
+         using T = decltype( tag );
+         kPushGeneral< T ><<< gridFor( lat.nb << lv ), kBlock, 0, ctx->stream >>>(
+             BndGeom::of( st, lat ), lat.bndFlag.p, lat.nb, lat.nc, excludeFlag, zeroOut ? 1 : 0, lv, (T*) data );
+      } );
+      HG_CHECK_HIP( hipGetLastError() );
+      return;
+   }
+   const HaloGeom g    = haloGeom( st, lat );
+   const int64_t  perF = lat.num.fin << lv, perE = lat.num.ein << lv;
+   auto           blocksOf = []( int64_t n ) { return uint32_t( ( n + kBlock - 1 ) / kBlock ); };
+   const uint32_t blocks = perF >= kBlock / 2 ? blocksOf( perF ) : 0;
+   const uint32_t fb     = blocks ? uint32_t( blocks * g.nf ) : blocksOf( perF * g.nf );
+   const uint32_t eb = blocksOf( perE * g.ne ), vb = blocksOf( int64_t( g.nv ) << lv );
    dispatchType( dtype, [&]( auto tag ) {
       using T = decltype( tag );
-      kPushAdditive< T ><<< gridFor( lat.nb << lv ), kBlock, 0, ctx->stream >>>(
-          BndGeom::of( st, lat ), lat.bndFlag.p, lat.nb, lat.nc, excludeFlag, zeroOut ? 1 : 0, lv, (T*) data );
+      kPushAdditive< T ><<< fb + eb + vb, kBlock, 0, ctx->stream >>>( g, blocks, fb, eb, FastDiv( perF ), FastDiv( perE ),
+                                                                     lat.bndFlag.p, excludeFlag, zeroOut ? 1 : 0, lv,
+                                                                     (T*) data );
    } );
    HG_CHECK_HIP( hipGetLastError() );
 }

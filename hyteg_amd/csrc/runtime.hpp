@@ -5,6 +5,7 @@
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 
+#include <array>
 #include <cstdint>
 #include <map>
 #include <memory>
@@ -75,6 +76,8 @@ struct CellMeta
    int32_t edge[6];
    int8_t  eperm[6][2];
    int32_t vert[4];
+   // which of the storage's face / edge orientations (fperm, eperm) each has
+   int8_t fcode[4], ecode[6];
 };
 
 // One storage, one level: lattice layout and owners.  Storage of a function on
@@ -128,6 +131,11 @@ struct Lattice
    // bricks of the P1 cell-interior apply on this lattice (built on first use)
    DevBuf< uint64_t > p1Bricks;
 
+   // cell-local offsets of the halo points by orientation: the face interiors of
+   // every face orientation of the storage (num.fin each), then the edge interiors of
+   // every edge orientation (num.ein each); empty where they do not fit 32 bits.
+   DevBuf< int32_t > haloOffsets;
+
    int64_t cellPos( int c, int64_t x, int64_t y, int64_t z ) const { return c * sc + tetIndex( w, x, y, z ); }
    int64_t ownerPos( const Topology& t, int c, int64_t x, int64_t y, int64_t z ) const
    {
@@ -155,6 +163,12 @@ struct Storage
    DevBuf< double >                             clsInvN;
    // cells incident to each face / edge / vertex: CSR of (cell, local index)
    DevBuf< int32_t > faceCellPtr, faceCells, edgeCellPtr, edgeCells, vertCellPtr, vertCells;
+   // the same incidences as (cell, orientation): two entries a face (cell -1: none),
+   // the edges' in the order of edgeCellPtr
+   DevBuf< int32_t >                       faceInc, edgeInc;
+   bool                                    facesShared2 = true; // every face has at most two cells
+   std::vector< std::array< int8_t, 3 > > faceOrient; // CellMeta::fperm by fcode
+   std::vector< std::array< int8_t, 2 > > edgeOrient; // CellMeta::eperm by ecode
    Lattice&                                     lattice( Context* ctx, int L );
    void                                         init( Context* ctx );
 };
@@ -364,6 +378,35 @@ inline unsigned xcdGrid( int64_t n )
       throw Error( -1, "grid too large" );
    return unsigned( g );
 }
+
+// n / d for n < 2^31 by a multiplication: the high word of n times ceil(2^32 / d) is
+// the quotient or one more
+struct FastDiv
+{
+   uint32_t d = 1, m = 0;
+   FastDiv() = default;
+   explicit FastDiv( int64_t div )
+   : d( uint32_t( div < 1 ? 1 : div ) )
+   , m( uint32_t( ( ( uint64_t( 1 ) << 32 ) + d - 1 ) / d ) )
+   {}
+   __device__ __forceinline__ uint32_t div( uint32_t n, uint32_t& rem ) const
+   {
+      if ( d == 1 ) // its factor 2^32 does not fit
+      {
+         rem = 0;
+         return n;
+      }
+      uint32_t q = __umulhi( n, m );
+      int32_t  r = int32_t( n - q * d );
+      if ( r < 0 )
+      {
+         --q;
+         r += int32_t( d );
+      }
+      rem = uint32_t( r );
+      return q;
+   }
+};
 
 inline unsigned gridFor( int64_t n, int block = kBlock )
 {
