@@ -201,4 +201,99 @@ __device__ __forceinline__ int pointClass( int64_t mm, int64_t x, int64_t y, int
    return -1;
 }
 
+// ---- halo exchange ----------------------------------------------------------
+// A halo copy's place in its cell follows from the primitive's orientation alone:
+// the lattice keeps the cell-local offsets of the face and edge interiors for each
+// orientation that the mesh has (haloOffsets), so an exchange costs one table load,
+// one load and one store a value.  Bound by those loads' latency on small levels and
+// by the scattered lines on large ones.  (Formed in the kernel -- 64-bit divisions,
+// a square root for the row of a triangle, the tetrahedral index -- a pull took
+// 14 us and a push 19 us at shell level 3, P2, and 1.21 and 0.65 ms at level 6.)
+struct HaloGeom
+{
+   const CellMeta* meta;
+   const int32_t * off, *faceInc, *edgePtr, *edgeInc, *vertPtr, *vertInc;
+   int64_t         sc, base; // values of a cell lattice; first owned DoF
+   uint32_t        fin, ein, nf, ne, nv, nfo; // points of a face / edge interior; counts; face orientations
+   int64_t         eoff, foff;
+   int32_t         vo[4]; // cell-local offsets of the vertices
+   FastDiv         dfin, dein;
+};
+
+inline HaloGeom haloGeom( const Storage& st, const Lattice& l )
+{
+   const int64_t fin = l.num.fin, ein = l.num.ein, mm = l.mm;
+   HaloGeom g;
+   g.meta    = st.meta.p;
+   g.off     = l.haloOffsets.p;
+   g.faceInc = st.faceInc.p;
+   g.edgePtr = st.edgeCellPtr.p;
+   g.edgeInc = st.edgeInc.p;
+   g.vertPtr = st.vertCellPtr.p;
+   g.vertInc = st.vertCells.p;
+   g.sc      = l.sc;
+   g.base    = l.nc * l.sc;
+   g.fin     = uint32_t( fin );
+   g.ein     = uint32_t( ein );
+   g.nf      = uint32_t( st.topo.nf );
+   g.ne      = uint32_t( st.topo.ne );
+   g.nv      = uint32_t( st.topo.nv );
+   g.nfo     = uint32_t( st.faceOrient.size() );
+   g.eoff    = l.num.eoff;
+   g.foff    = l.num.foff;
+   g.vo[0]   = 0;
+   g.vo[1]   = int32_t( tetIndex( l.w, mm, 0, 0 ) );
+   g.vo[2]   = int32_t( tetIndex( l.w, 0, mm, 0 ) );
+   g.vo[3]   = int32_t( tetIndex( l.w, 0, 0, mm ) );
+   g.dfin    = FastDiv( fin );
+   g.dein    = FastDiv( ein );
+   return g;
+}
+
+// whether a lattice's halo exchange runs on the offset tables: cell-local offsets in
+// 32 bits and block counts within a grid (beyond that the general kernels run)
+inline bool haloTables( const Storage& st, const Lattice& l, int lv )
+{
+   const int64_t most = int64_t( 1 ) << 31, nf = st.topo.nf, ne = st.topo.ne, nv = st.topo.nv;
+   // threads of a launch over n primitives of `per` values: whole workgroups each, or packed
+   auto threads = []( int64_t per, int64_t n ) { return ( per / kBlock + 1 ) * kBlock * n; };
+   return st.facesShared2 && l.haloOffsets.p && threads( l.haloPerCell() << lv, l.nc ) / kBlock < most &&
+          ( l.haloPerCell() << lv ) < most && threads( l.num.fin << lv, nf ) / kBlock < most &&
+          ( ( l.haloPerCell() << lv ) >= kBlock / 2 || ( l.haloPerCell() << lv ) * l.nc < most ) &&
+          ( ( l.num.fin << lv ) >= kBlock / 2 || ( l.num.fin << lv ) * nf < most ) && ( l.num.ein << lv ) * ne < most &&
+          ( nv << lv ) < most;
+}
+
+// halo point p of cell c (4 fin face points, 6 ein edge points, 4 vertices): storage
+// positions of its owner and of the copy
+__device__ __forceinline__ void haloPoint( const HaloGeom& g, uint32_t c, uint32_t p, int64_t& src, int64_t& dst )
+{
+   const CellMeta& m = g.meta[c];
+   int32_t         o;
+   if ( p < 4 * g.fin )
+   {
+      const uint32_t k = uint32_t( p >= g.fin ) + uint32_t( p >= 2 * g.fin ) + uint32_t( p >= 3 * g.fin );
+      p -= k * g.fin;
+      o   = g.off[uint32_t( m.fcode[k] ) * g.fin + p];
+      src = g.base + g.foff + int64_t( m.face[k] ) * g.fin + p;
+   }
+   else if ( ( p -= 4 * g.fin ) < 6 * g.ein )
+   {
+      uint32_t k = 0;
+#pragma unroll
+      for ( uint32_t i = 1; i < 6; ++i )
+         k += uint32_t( p >= i * g.ein );
+      p -= k * g.ein;
+      o   = g.off[g.nfo * g.fin + uint32_t( m.ecode[k] ) * g.ein + p];
+      src = g.base + g.eoff + int64_t( m.edge[k] ) * g.ein + p;
+   }
+   else
+   {
+      const uint32_t k = p - 6 * g.ein;
+      o                = k == 0 ? g.vo[0] : ( k == 1 ? g.vo[1] : ( k == 2 ? g.vo[2] : g.vo[3] ) );
+      src              = g.base + m.vert[k];
+   }
+   dst = c * g.sc + o;
+}
+
 } // namespace hg

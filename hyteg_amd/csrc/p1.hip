@@ -14,6 +14,7 @@
 #include <array>
 #include <cmath>
 #include <map>
+#include <mutex>
 #include <thread>
 
 #include "abi_util.hpp"
@@ -105,7 +106,7 @@ static int slot15( int dx, int dy, int dz )
 // per macro-edge: which micro-cells of a cell contain a boundary point depends
 // on the point's class only.
 static constexpr int kVirt            = 8;
-static const int     kClassRep[14][3] = { { 2, 2, 0 }, { 2, 0, 2 }, { 0, 2, 2 }, { 2, 2, 4 }, { 4, 0, 0 },
+static constexpr int kClassRep[14][3] = { { 2, 2, 0 }, { 2, 0, 2 }, { 0, 2, 2 }, { 2, 2, 4 }, { 4, 0, 0 },
                                           { 0, 4, 0 }, { 4, 4, 0 }, { 0, 0, 4 }, { 4, 0, 4 }, { 0, 4, 4 },
                                           { 0, 0, 0 }, { 8, 0, 0 }, { 0, 8, 0 }, { 0, 0, 8 } };
 
@@ -140,6 +141,41 @@ static int hostPointClass( int64_t mm, int64_t x, int64_t y, int64_t z )
          return 10 + k;
    return -1;
 }
+
+// the class of the fine neighbour q (cOff15) of a coarse boundary point of class k:
+// the boundary class it lies in, -1 interior, -2 outside the cell
+struct RestrictClasses
+{
+   int8_t c[14][15];
+};
+static constexpr RestrictClasses restrictClasses()
+{
+   RestrictClasses t{};
+   constexpr int   mm = 2 * kVirt, pairs[6] = { 3, 5, 6, 9, 10, 12 };
+   for ( int k = 0; k < 14; ++k )
+      for ( int q = 0; q < 15; ++q )
+      {
+         const int x = 2 * kClassRep[k][0] + Stencil15::off[q][0], y = 2 * kClassRep[k][1] + Stencil15::off[q][1],
+                   z    = 2 * kClassRep[k][2] + Stencil15::off[q][2];
+         const int zero = ( x + y + z == mm ? 1 : 0 ) | ( x == 0 ? 2 : 0 ) | ( y == 0 ? 4 : 0 ) | ( z == 0 ? 8 : 0 );
+         int       cl   = zero == 0 ? -1 : -2;
+         for ( int i = 0; i < 4; ++i )
+         {
+            if ( zero == ( 1 << ( 3 - i ) ) )
+               cl = i;
+            if ( ( zero ^ 15 ) == ( 1 << i ) )
+               cl = 10 + i;
+         }
+         for ( int i = 0; i < 6; ++i )
+            if ( ( zero ^ 15 ) == pairs[i] )
+               cl = 4 + i;
+         if ( x < 0 || y < 0 || z < 0 || x + y + z > mm )
+            cl = -2;
+         t.c[k][q] = int8_t( cl );
+      }
+   return t;
+}
+__constant__ RestrictClasses cRestrictClasses = restrictClasses();
 
 // Sliced ELL rows: slot i (a row, or -1 for padding) lies in slice i / 64 at
 // lane i % 64; the slice's entries are column-major (entry j of the lane at
@@ -229,6 +265,7 @@ struct P1OpLevel
    bool                   csr = false;
    SellRows               applyRows, sorRows;
    std::vector< int64_t > sorColorStart;
+   DevBuf< int64_t >      sorColors; // sorColorStart on the device
    // inverse diagonal of every storage position (cell lattices, halo copies
    // included, then the owned DoFs), built on first use
    DevBuf< double > invDiagFull;
@@ -441,6 +478,7 @@ static void buildP1Level( Context* ctx, Storage& st, int L, P1OpLevel& o )
          sorOrder.resize( ( sorOrder.size() + kSellRows - 1 ) / kSellRows * kSellRows, -1 );
       }
       o.sorColorStart[size_t( ncolor )] = int64_t( sorOrder.size() );
+      o.sorColors.upload( ctx, o.sorColorStart );
       buildSell( ctx, o.applyRows, natural, row, inv, ownerBase, true );
       buildSell( ctx, o.sorRows, sorOrder, row, inv, ownerBase, false );
    }
@@ -734,6 +772,155 @@ __global__ __launch_bounds__( 64 * kCellWorkers ) void kCellSOR( const int32_t* 
    }
 }
 
+// The same two colours for single-vector functions: a lane takes the pair (2i, 2i + 1)
+// of its row, loads the seven rows' values for both points at once (15 loads for two
+// points where the kernel above issues 32, in two rounds) and passes the new values of
+// the first colour to the neighbouring lane in a register, so a row is read once and
+// nothing waits for a store.  A row of more pairs than lanes is swept in strides of
+// lanes - 1 pairs: the last lane's open point (the second colour's needs the next
+// pair) is the first of the next stride, its new value carried over.  Same sums in the
+// same order.  FULL: one row a wavefront (the cell, and with it the stencil, in scalar
+// registers).  Bound by HBM: a launch reads all of x, a quarter of b and writes a
+// quarter of x.  Cube level 8, a launch: 90 us above, 55 us here.
+template < class T >
+struct LoadPair
+{
+   T a, b;
+   __device__ __forceinline__ explicit LoadPair( const T* p )
+   : a( p[0] )
+   , b( p[1] )
+   {}
+};
+template <>
+struct LoadPair< double >
+{
+   double a, b;
+   __device__ __forceinline__ explicit LoadPair( const double* p )
+   {
+      typedef double Two __attribute__( ( ext_vector_type( 2 ), aligned( 8 ) ) ); // one load at 8-byte alignment
+      const Two v = *reinterpret_cast< const Two* >( p );
+      a           = v.x;
+      b           = v.y;
+   }
+};
+template < class T, bool FULL >
+__global__ __launch_bounds__( 64 * kCellWorkers ) void kCellSORPairs( const int32_t* __restrict__ rows, int64_t nrows,
+                                                                     int64_t nc, int64_t sc, int64_t w, int64_t mm,
+                                                                     const double* __restrict__ stencil, int oddFirst,
+                                                                     double relax, const T* __restrict__ b,
+                                                                     T* __restrict__ x, int rpbLog )
+{
+   using A        = typename Acc< T >::type;
+   RowWorker rw   = rowWorker( nrows * nc, FULL ? 0 : rpbLog );
+   const bool on  = rw.row < nrows * nc;
+   if ( FULL && !on )
+      return;
+   int64_t c = 0;
+   if ( on )
+      c = nrows * nc < ( int64_t( 1 ) << 32 ) ? int64_t( uint32_t( rw.row ) / uint32_t( nrows ) ) : rw.row / nrows;
+   int64_t r = on ? rw.row - c * nrows : 0;
+   if constexpr ( FULL )
+   {
+      c = __builtin_amdgcn_readfirstlane( int( c ) );
+      r = __builtin_amdgcn_readfirstlane( int( r ) );
+   }
+   const int32_t     y = rows[2 * r], z = rows[2 * r + 1];
+   const StencilRows sr( int32_t( w ), y, z );
+   const T*          bc = b + c * sc + sr.r00;
+   T*                xc = x + c * sc;
+   A                 st[15];
+#pragma unroll
+   for ( int q = 0; q < 15; ++q )
+      st[q] = A( stencil[15 * c + q] );
+   const A       invc = A( 1 ) / st[0];
+   const int32_t top = on ? int32_t( mm ) - y - z : 0, lane = rw.lane, lanes = rw.lanes;
+   auto          update = [&]( A rhs, const T val[15] ) -> T {
+      A v = rhs;
+#pragma unroll
+      for ( int q = 1; q < 15; ++q )
+         v -= st[q] * toAcc( val[q] );
+      return fromAcc< T >( ( A( 1 ) - A( relax ) ) * toAcc( val[0] ) + A( relax ) * invc * v );
+   };
+   auto pass = [&]( T v, int from ) -> T { return fromAcc< T >( __shfl( toAcc( v ), from, lanes ) ); };
+   T    carry = T( 0 );
+   // the strides of the longest row of the wavefront's rows
+   for ( int32_t base = 0; __any( 2 * base < top ); base += lanes - 1 )
+   {
+      const int32_t i = base + lane, xe = 2 * i;
+      T             m[3][3], p[3][3]; // rows z+1, y+1 z-1, y+1 at xe-1, xe, xe+1; rows y-1, y-1 z+1, z-1 at xe, xe+1, xe+2
+      T             e = T( 0 ), o = T( 0 ), before = T( 0 ), after = T( 0 );
+      A             be = A( 0 ), bo = A( 0 );
+      if ( xe < top )
+      {
+         const int32_t  mr[3] = { sr.r01, sr.r1m, sr.r10 }, pr[3] = { sr.rm0, sr.rm1, sr.r0m };
+         const int32_t  prev  = xe > 0 ? -1 : 0;
+#pragma unroll
+         for ( int k = 0; k < 3; ++k )
+         {
+            const LoadPair< T > vm( xc + mr[k] + xe ), vp( xc + pr[k] + xe );
+            m[k][0] = xc[mr[k] + xe + prev];
+            m[k][1] = vm.a;
+            m[k][2] = vm.b;
+            p[k][0] = vp.a;
+            p[k][1] = vp.b;
+            p[k][2] = xc[pr[k] + xe + 2];
+         }
+         const LoadPair< T > v( xc + sr.r00 + xe );
+         e      = v.a;
+         o      = v.b;
+         before = xc[sr.r00 + xe + prev];
+         after  = xc[sr.r00 + xe + 2];
+         be     = toAcc( bc[xe] );
+         bo     = toAcc( bc[xe + 1] );
+      }
+      else if ( xe == top )
+         e = xc[sr.r00 + xe]; // the halo value behind the row's last point
+      const bool mine = lane < lanes - 1;
+      if ( !oddFirst )
+      {
+         T ne = e;
+         if ( xe < top && xe > 0 && !( lane == 0 && base > 0 ) )
+         {
+            const T val[15] = { e,       before,  m[0][0], m[1][0], m[2][0], p[0][0], p[1][0], p[2][0],
+                                m[0][1], m[1][1], m[2][1], p[0][1], p[1][1], p[2][1], o };
+            ne              = update( be, val );
+            xc[sr.r00 + xe] = ne;
+         }
+         if ( lane == 0 && base > 0 )
+            ne = carry;
+         const T nx = pass( ne, lane + 1 );
+         carry      = pass( ne, lanes - 1 );
+         if ( xe + 1 < top && mine )
+         {
+            const T val[15] = { o,       ne,      m[0][1], m[1][1], m[2][1], p[0][1], p[1][1], p[2][1],
+                                m[0][2], m[1][2], m[2][2], p[0][2], p[1][2], p[2][2], nx };
+            xc[sr.r00 + xe + 1] = update( bo, val );
+         }
+      }
+      else
+      {
+         T no = o;
+         if ( xe + 1 < top && mine )
+         {
+            const T val[15] = { o,       e,       m[0][1], m[1][1], m[2][1], p[0][1], p[1][1], p[2][1],
+                                m[0][2], m[1][2], m[2][2], p[0][2], p[1][2], p[2][2], after };
+            no                  = update( bo, val );
+            xc[sr.r00 + xe + 1] = no;
+         }
+         T pv = pass( no, lane - 1 );
+         if ( lane == 0 )
+            pv = carry;
+         carry = pass( no, lanes - 2 );
+         if ( xe < top && xe > 0 && mine )
+         {
+            const T val[15] = { e,       pv,      m[0][0], m[1][0], m[2][0], p[0][0], p[1][0], p[2][0],
+                                m[0][1], m[1][1], m[2][1], p[0][1], p[1][1], p[2][1], no };
+            xc[sr.r00 + xe] = update( be, val );
+         }
+      }
+   }
+}
+
 // partial stencil sum of this DoF's share in cell c; skip = 1 leaves out the centre
 template < class T >
 __device__ __forceinline__ typename Acc< T >::type bndStencilSum( const BndGeom& g, const double* __restrict__ cls,
@@ -860,24 +1047,16 @@ __global__ void __launch_bounds__( kBlock ) kBndApplySell( int64_t nblk, int64_t
    dst[o] = fromAcc< T >( s );
 }
 
+// SOR on boundary slot i of the sliced rows (vector vec)
 template < class T >
-__global__ void __launch_bounds__( kBlock ) kBndSORSell( int64_t nblk, int64_t slot0, int64_t nslot,
-                                                        const int32_t* __restrict__ rowOf,
-                                                        const uint8_t* __restrict__ bndFlag, int flag,
-                                                        const int64_t* __restrict__ off, const int32_t* __restrict__ pos,
-                                                        const double* __restrict__ val, int64_t ownerBase,
-                                                        const double* __restrict__ invDiag, double relax,
-                                                        const T* __restrict__ rhs, T* __restrict__ x, int lv )
+__device__ __forceinline__ void bndSorSlot( int64_t i, int64_t vec, const int32_t* __restrict__ rowOf,
+                                            const uint8_t* __restrict__ bndFlag, int flag,
+                                            const int64_t* __restrict__ off, const int32_t* __restrict__ pos,
+                                            const double* __restrict__ val, int64_t ownerBase,
+                                            const double* __restrict__ invDiag, double relax, const T* __restrict__ rhs,
+                                            T* __restrict__ x, int lv )
 {
-   using A          = typename Acc< T >::type;
-   const int64_t lb = xcdBlock( nblk );
-   if ( lb >= nblk )
-      return;
-   const int64_t tid = lb * kBlock + threadIdx.x;
-   const int64_t li = tid >> lv, vec = tid & ( ( int64_t( 1 ) << lv ) - 1 );
-   if ( li >= nslot )
-      return;
-   const int64_t i = slot0 + li;
+   using A         = typename Acc< T >::type;
    const int32_t b = rowOf[i];
    if ( b < 0 || !( bndFlag[b] & flag ) )
       return;
@@ -903,6 +1082,215 @@ __global__ void __launch_bounds__( kBlock ) kBndSORSell( int64_t nblk, int64_t s
          s -= A( v[u] ) * xv[u];
    }
    x[o] = fromAcc< T >( ( A( 1 ) - A( relax ) ) * toAcc( x[o] ) + A( relax ) * A( invDiag[b] ) * s );
+}
+
+template < class T >
+__global__ void __launch_bounds__( kBlock ) kBndSORSell( int64_t nblk, int64_t slot0, int64_t nslot,
+                                                        const int32_t* __restrict__ rowOf,
+                                                        const uint8_t* __restrict__ bndFlag, int flag,
+                                                        const int64_t* __restrict__ off, const int32_t* __restrict__ pos,
+                                                        const double* __restrict__ val, int64_t ownerBase,
+                                                        const double* __restrict__ invDiag, double relax,
+                                                        const T* __restrict__ rhs, T* __restrict__ x, int lv )
+{
+   const int64_t lb = xcdBlock( nblk );
+   if ( lb >= nblk )
+      return;
+   const int64_t tid = lb * kBlock + threadIdx.x;
+   const int64_t li = tid >> lv, vec = tid & ( ( int64_t( 1 ) << lv ) - 1 );
+   if ( li < nslot )
+      bndSorSlot( slot0 + li, vec, rowOf, bndFlag, flag, off, pos, val, ownerBase, invDiag, relax, rhs, x, lv );
+}
+
+// A whole SOR sweep in one workgroup (per 2^lg vectors of an interleaved function), x in
+// LDS: on small lattices a sweep is a chain of about a dozen launches
+// of 3 us (one a boundary colour, one a halo pull, one a row group) that hold a few
+// thousand points, and a workgroup barrier costs a fraction of a launch.  The steps and
+// their order are those of the separate kernels (same results bit for bit).  Bound by
+// the chain of latencies: what a colour reads besides x (positions, right-hand side) is
+// loaded while the colour before it runs.  Cube levels 1 to 4: 16 us a sweep on average
+// where the launches took about 38 us.  (The boundary colours alone, where x is too large
+// for LDS: 37 us at cube level 5 against 20 us for the launches, so they stay launches.)
+constexpr int    kSweepThreads = 1024;
+constexpr int    kSweepRows    = 1024; // interior rows of a cell
+constexpr int    kSweepCells   = 128;
+constexpr size_t kSweepLds     = size_t( 128 ) << 10; // x in LDS
+struct SweepRows
+{
+   const int32_t *row, *pos, *rows; // slots, entries; interior rows by group
+   const int64_t *off, *colors;     // slices; slot ranges of the colours
+   const double * val, *invDiag, *stencil;
+   const uint8_t* bndFlag;
+   int64_t        ownerBase, nstore;
+   int32_t        group[5], ncolor, nc, w, mm;
+   uint32_t       halo; // halo points of a cell
+   FastDiv        dhalo, drow[4];
+};
+template < class T >
+struct SweepSlot
+{
+   using A = typename Acc< T >::type;
+   int32_t b = -1, w = 0; // row (-1: none), entries
+   int32_t p[kSellUnroll];
+   int64_t e0 = 0;
+   A       rhs, inv;
+   __device__ __forceinline__ void load( const SweepRows& r, int64_t i, int64_t end, int flag, const T* __restrict__ rhsAll,
+                                         int lv, int64_t vec )
+   {
+      b = i < end ? r.row[i] : -1;
+      if ( b < 0 )
+         return;
+      const int64_t sl = i / kSellRows, o0 = r.off[sl];
+      const uint8_t f  = r.bndFlag[b];
+      e0  = o0 + ( i % kSellRows );
+      w   = int32_t( ( r.off[sl + 1] - o0 ) / kSellRows );
+      rhs = toAcc( rhsAll[( ( r.ownerBase + b ) << lv ) + vec] );
+      inv = A( r.invDiag[b] );
+#pragma unroll
+      for ( int u = 0; u < kSellUnroll; ++u )
+         p[u] = r.pos[e0 + int64_t( u ) * kSellRows];
+      if ( !( f & flag ) )
+         b = -1;
+   }
+   // X(q): x at storage position q
+   template < class FX >
+   __device__ __forceinline__ void relaxed( const SweepRows& r, double relax, FX&& X )
+   {
+      if ( b < 0 )
+         return;
+      A s = rhs;
+      for ( int32_t j = 0; j < w; j += kSellUnroll )
+      {
+         int32_t pn[kSellUnroll];
+         double  v[kSellUnroll];
+         A       xv[kSellUnroll];
+         // the weights and the next positions are loaded together
+#pragma unroll
+         for ( int u = 0; u < kSellUnroll; ++u )
+         {
+            v[u]  = r.val[e0 + int64_t( j + u ) * kSellRows];
+            pn[u] = r.pos[e0 + int64_t( min( j + kSellUnroll, w - kSellUnroll ) + u ) * kSellRows];
+         }
+#pragma unroll
+         for ( int u = 0; u < kSellUnroll; ++u )
+            xv[u] = toAcc( X( p[u] ) );
+#pragma unroll
+         for ( int u = 0; u < kSellUnroll; ++u )
+            s -= A( v[u] ) * xv[u];
+#pragma unroll
+         for ( int u = 0; u < kSellUnroll; ++u )
+            p[u] = pn[u];
+      }
+      T& o = X( int32_t( r.ownerBase + b ) );
+      o    = fromAcc< T >( ( A( 1 ) - A( relax ) ) * toAcc( o ) + A( relax ) * inv * s );
+   }
+};
+template < class T >
+__global__ __launch_bounds__( kSweepThreads ) void kP1SweepSmall( SweepRows r, HaloGeom g, int backward, int flag,
+                                                                 double relax, const T* __restrict__ b,
+                                                                 T* __restrict__ x, int lv, int lg, int rowLanesLog )
+{
+   using A = typename Acc< T >::type;
+   extern __shared__ double sweepX[];
+   __shared__ int32_t       sRows[kSweepRows];
+   __shared__ double        sSt[15 * kSweepCells];
+   T* const      sx   = reinterpret_cast< T* >( sweepX );
+   const int     vl   = int( threadIdx.x & ( ( 1u << lg ) - 1u ) );
+   const int64_t v    = ( int64_t( blockIdx.x ) << lg ) + vl;
+   const int     item = int( threadIdx.x ) >> lg, items = kSweepThreads >> lg;
+   auto          X    = [&]( int32_t q ) -> T& { return sx[( q << lg ) + vl]; };
+   for ( int32_t i = item; i < int32_t( r.nstore ); i += items )
+      X( i ) = x[( int64_t( i ) << lv ) + v];
+   for ( int32_t i = int32_t( threadIdx.x ); i < r.group[4]; i += kSweepThreads )
+      sRows[i] = r.rows[2 * i] | ( r.rows[2 * i + 1] << 16 );
+   for ( int32_t i = int32_t( threadIdx.x ); i < 15 * r.nc; i += kSweepThreads )
+      sSt[i] = r.stencil[i];
+   auto boundary = [&]() {
+      SweepSlot< T > next;
+      auto           first = [&]( int k ) { return r.colors[backward ? r.ncolor - 1 - k : k]; };
+      int64_t        s0 = first( 0 ), s1 = r.colors[( backward ? r.ncolor - 1 : 0 ) + 1];
+      next.load( r, s0 + item, s1, flag, b, lv, v );
+      __syncthreads();
+      for ( int k = 0; k < r.ncolor; ++k )
+      {
+         SweepSlot< T > cur = next;
+         const int64_t  i0 = s0 + item + items, i1 = s1;
+         if ( k + 1 < r.ncolor )
+         {
+            s0 = first( k + 1 );
+            s1 = r.colors[( backward ? r.ncolor - 2 - k : k + 1 ) + 1];
+            next.load( r, s0 + item, s1, flag, b, lv, v );
+         }
+         cur.relaxed( r, relax, X );
+         for ( int64_t i = i0; i < i1; i += items )
+         {
+            SweepSlot< T > more;
+            more.load( r, i, i1, flag, b, lv, v );
+            more.relaxed( r, relax, X );
+         }
+         __syncthreads();
+      }
+   };
+   auto pull = [&]() {
+      for ( uint32_t i = item; i < uint32_t( r.nc ) * r.halo; i += items )
+      {
+         uint32_t       p;
+         const uint32_t c = r.dhalo.div( i, p );
+         int64_t        src, dst;
+         haloPoint( g, c, p, src, dst );
+         X( int32_t( dst ) ) = X( int32_t( src ) );
+      }
+      __syncthreads();
+   };
+   auto interior = [&]() {
+      const int lane = item & ( ( 1 << rowLanesLog ) - 1 ), worker = item >> rowLanesLog, workers = items >> rowLanesLog;
+      for ( int k = 0; k < 4; ++k )
+      {
+         const int     grp = backward ? 3 - k : k;
+         const int32_t n   = r.group[grp + 1] - r.group[grp];
+         for ( int ph = 0; ph < 2; ++ph )
+         {
+            const int32_t x0 = ( backward ? 1 - ph : ph ) ? 1 : 2; // forward: the even points first
+            for ( int32_t i = worker; i < n * r.nc; i += workers )
+            {
+               uint32_t          rr;
+               const int32_t     c  = int32_t( r.drow[grp].div( uint32_t( i ), rr ) );
+               const int32_t     yz = sRows[r.group[grp] + int32_t( rr )];
+               const int32_t     y = yz & 0xFFFF, z = yz >> 16, cell = c * int32_t( g.sc );
+               const StencilRows sr( r.w, y, z );
+               const double*     st = sSt + 15 * c;
+               for ( int32_t xx = x0 + 2 * lane; xx < r.mm - y - z; xx += 2 << rowLanesLog )
+               {
+                  const int32_t at = cell + sr.at( 0, xx );
+                  A             s  = toAcc( b[( int64_t( at ) << lv ) + v] );
+                  T             val[15];
+#pragma unroll
+                  for ( int q = 0; q < 15; ++q )
+                     val[q] = X( cell + sr.at( q, xx ) );
+#pragma unroll
+                  for ( int q = 1; q < 15; ++q )
+                     s -= A( st[q] ) * toAcc( val[q] );
+                  const A invc = A( 1 ) / A( st[0] );
+                  X( at )      = fromAcc< T >( ( A( 1 ) - A( relax ) ) * toAcc( val[0] ) + A( relax ) * invc * s );
+               }
+            }
+            __syncthreads();
+         }
+      }
+   };
+   __syncthreads();
+   if ( backward )
+   {
+      pull();
+      if ( flag & kInner )
+         interior();
+   }
+   boundary();
+   pull(); // backward: the boundary has changed after the interiors
+   if ( !backward && ( flag & kInner ) )
+      interior();
+   for ( int32_t i = item; i < int32_t( r.nstore ); i += items )
+      x[( int64_t( i ) << lv ) + v] = X( i );
 }
 
 // restriction to coarse cell-interior points (full weighting, R = P^T)
@@ -944,7 +1332,7 @@ __global__ void kRestrictCell( const int32_t* __restrict__ rows, int64_t nrows, 
 // primitive), i.e. restrict_3D_macrocell_P1_pull_additive + additive communication
 template < class T >
 __global__ void kRestrictBnd( BndGeom gc, int64_t nbc, int64_t nc, const uint8_t* __restrict__ bndFlag, int flag,
-                              const double* __restrict__ clsInvN, int64_t scf, int64_t wf, int64_t mmf,
+                              const double* __restrict__ clsInvN, int64_t scf, int64_t wf,
                               const T* __restrict__ fine, T* __restrict__ coarse, int lv )
 {
    using A           = typename Acc< T >::type;
@@ -953,16 +1341,28 @@ __global__ void kRestrictBnd( BndGeom gc, int64_t nbc, int64_t nc, const uint8_t
    if ( b >= nbc || !( bndFlag[b] & flag ) )
       return;
    A s = A( 0 );
-   forEachIncident( gc, b, [&]( int64_t c, int64_t x, int64_t y, int64_t z, int ) {
+   forEachIncident( gc, b, [&]( int64_t c, int64_t x, int64_t y, int64_t z, int k ) {
+      // offsets of the seven fine rows around the point from its own, and the class of
+      // each neighbour from the point's (cRestrictClasses): one after the other with their
+      // indices and classes formed in 64 bits, a launch took 23 us whatever its size
+      const int64_t m  = wf - 2 * z, fy = 2 * y;
+      const int64_t dz = m * ( m + 1 ) / 2 - fy, dy = m - fy;
+      const int64_t at = c * scf + tetRowStart( wf, fy, 2 * z ) + 2 * x;
+      const int64_t row[7] = { 0, dz, dy - dz - m, dy, -dy - 1, dz - dy, -dz - m - 1 }; // of StencilRows
+      constexpr int rowOf[15] = { 0, 0, 1, 2, 3, 4, 5, 6, 1, 2, 3, 4, 5, 6, 0 };
+      T             val[15];
+      A             wgt[15];
+#pragma unroll
       for ( int q = 0; q < 15; ++q )
       {
-         const int64_t fx = 2 * x + cOff15[q][0], fy = 2 * y + cOff15[q][1], fz = 2 * z + cOff15[q][2];
-         if ( fx < 0 || fy < 0 || fz < 0 || fx + fy + fz > mmf )
-            continue;
-         const int cl  = pointClass( mmf, fx, fy, fz );
-         const A   wgt = ( q == 0 ? A( 1 ) : A( 0.5 ) ) * ( cl < 0 ? A( 1 ) : A( clsInvN[14 * c + cl] ) );
-         s += wgt * toAcc( fine[( ( c * scf + tetIndex( wf, fx, fy, fz ) ) << lv ) + vec] );
+         const int cl = cRestrictClasses.c[k][q];
+         val[q]       = cl > -2 ? fine[( ( at + row[rowOf[q]] + cOff15[q][0] ) << lv ) + vec] : T( 0 );
+         wgt[q]       = ( q == 0 ? A( 1 ) : A( 0.5 ) ) * ( cl < 0 ? A( 1 ) : A( clsInvN[14 * c + cl] ) );
       }
+#pragma unroll
+      for ( int q = 0; q < 15; ++q )
+         if ( cRestrictClasses.c[k][q] > -2 )
+            s += wgt[q] * toAcc( val[q] );
    } );
    coarse[( ( nc * gc.sc + b ) << lv ) + vec] = fromAcc< T >( s );
 }
@@ -1171,6 +1571,63 @@ void p1Apply( Context* ctx, P1Operator& op, Function& src, Function& dst, int L,
    } );
 }
 
+// A sweep runs in one workgroup (per 2^lg vectors, lg = sweepVectorsLog) while x fits the
+// LDS budget, a boundary colour has at most about two points a thread and the interior
+// at most eight.
+static int    sweepVectorsLog( int lv ) { return std::min( lv, 2 ); }
+static size_t sweepLds( const Lattice& lat, size_t elem, int lv ) { return ( size_t( lat.nstore ) * elem ) << sweepVectorsLog( lv ); }
+static bool   sweepSmall( const Storage& st, const Lattice& lat, const P1OpLevel& o, size_t elem, int lv )
+{
+   if ( !o.csr || lat.nb == 0 || o.sorColorStart.size() < 2 || !haloTables( st, lat, lv ) )
+      return false;
+   const int     lg    = sweepVectorsLog( lv );
+   const int64_t nc    = int64_t( o.sorColorStart.size() ) - 1;
+   const int64_t inner = lat.nc * ( lat.mm >= 4 ? tet( lat.mm - 3 ) : 0 );
+   return ( o.sorColorStart.back() << lg ) <= 2 * kSweepThreads * nc && ( inner << lg ) <= 8 * kSweepThreads &&
+          sweepLds( lat, elem, lv ) <= kSweepLds && lat.nrows <= kSweepRows && lat.nc <= kSweepCells;
+}
+template < class T >
+static void p1SweepSmall( Context* ctx, Storage& st, Lattice& lat, P1OpLevel& o, bool backward, int flag, double relax,
+                          const T* b, T* x, int lv )
+{
+   const int lg = sweepVectorsLog( lv );
+   SweepRows r{};
+   r.row       = o.sorRows.row.p;
+   r.pos       = o.sorRows.pos.p;
+   r.rows      = lat.rows.p;
+   r.off       = o.sorRows.off.p;
+   r.colors    = o.sorColors.p;
+   r.val       = o.sorRows.val.p;
+   r.invDiag   = o.invDiag.p;
+   r.stencil   = o.stencil.p;
+   r.bndFlag   = lat.bndFlag.p;
+   r.ownerBase = lat.nc * lat.sc;
+   r.nstore    = lat.nstore;
+   for ( int k = 0; k < 5; ++k )
+      r.group[k] = int32_t( lat.rowGroup[k] );
+   r.ncolor = int32_t( o.sorColorStart.size() ) - 1;
+   r.nc     = int32_t( lat.nc );
+   r.w      = int32_t( lat.w );
+   r.mm     = int32_t( lat.mm );
+   r.halo   = uint32_t( lat.haloPerCell() );
+   r.dhalo  = FastDiv( lat.haloPerCell() );
+   for ( int k = 0; k < 4; ++k )
+      r.drow[k] = FastDiv( lat.rowGroup[k + 1] - lat.rowGroup[k] );
+   // lanes of a row: one colour of its longest row
+   int rl = 0;
+   while ( rl + lg < 6 && ( int64_t( 2 ) << rl ) < lat.mm - 2 )
+      ++rl;
+   const HaloGeom g = haloGeom( st, lat );
+   static std::once_flag once[64]; // per value type and device
+   std::call_once( once[ctx->device & 63], [] {
+      HG_CHECK_HIP( hipFuncSetAttribute( reinterpret_cast< const void* >( &kP1SweepSmall< T > ),
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, int( kSweepLds ) ) );
+   } );
+   kP1SweepSmall< T ><<< 1u << ( lv - lg ), kSweepThreads, sweepLds( lat, sizeof( T ), lv ), ctx->stream >>>(
+       r, g, int( backward ), flag, relax, b, x, lv, lg, rl );
+   HG_CHECK_HIP( hipGetLastError() );
+}
+
 // One SOR sweep in multicolour order.  Forward: the owned vertex/edge/face DoFs
 // colour by colour (greedy colours of their coupling graph), then the 8 parity
 // colours k = (x&1) + 2(y&1) + 4(z&1) of the cell interiors (every non-centre
@@ -1188,7 +1645,6 @@ void p1SOR( Context* ctx, P1Operator& op, Function& x, Function& b, double relax
    void*      xp  = x.ptr( L );
    const void* bp = b.ptr( L );
    ctx->beginTiming();
-   pullHalos( ctx, *op.st, lat, xp, x.dtype, lv );
    dispatchType( x.dtype, [&]( auto tag ) {
       using T = decltype( tag );
       const BndGeom g = BndGeom::of( *op.st, lat );
@@ -1220,6 +1676,17 @@ void p1SOR( Context* ctx, P1Operator& op, Function& x, Function& b, double relax
          const int64_t n = lat.rowGroup[grp + 1] - lat.rowGroup[grp];
          if ( n == 0 )
             return;
+         if ( lv == 0 )
+         {
+            // a lane more than the longest row has pairs, at least four
+            const int rpb = std::min( 4, rowsPerBlockLog( lat.mm / 2 + 1 ) );
+            const auto run = rpb == 0 ? kCellSORPairs< T, true > : kCellSORPairs< T, false >;
+            run<<< cellGrid( n * lat.nc, rpb ), 64 * kCellWorkers, 0, ctx->stream >>>(
+                lat.rows.p + 2 * lat.rowGroup[grp], n, lat.nc, lat.sc, lat.w, lat.mm, o.stencil.p, cxFirst, relax,
+                (const T*) bp, (T*) xp, rpb );
+            HG_CHECK_HIP( hipGetLastError() );
+            return;
+         }
          const int rpb = rowsPerBlockLog( ( ( lat.mm - 2 ) / 2 ) << lv );
          kCellSOR< T ><<< cellGrid( n * lat.nc, rpb ), 64 * kCellWorkers, 0, ctx->stream >>>(
              lat.rows.p + 2 * lat.rowGroup[grp], n, lat.nc, lat.sc, lat.w, lat.mm, o.stencil.p, cxFirst, relax,
@@ -1230,10 +1697,22 @@ void p1SOR( Context* ctx, P1Operator& op, Function& x, Function& b, double relax
       const bool   interior = ( flag & kInner ) && lat.nrows > 0;
       if ( interior )
          checkCellIndexing( lat, lv );
+      if ( sweepSmall( *op.st, lat, o, sizeof( T ), lv ) )
+      {
+         p1SweepSmall( ctx, *op.st, lat, o, backward, flag, relax, (const T*) bp, (T*) xp, lv );
+         return;
+      }
+      // the assembled boundary rows read the owners of boundary neighbours, not their
+      // halo copies: only the other boundary kernel and a leading interior need a pull
+      if ( backward || !o.csr || nbc == 0 )
+         pullHalos( ctx, *op.st, lat, xp, x.dtype, lv );
+      auto boundaryColours = [&]() {
+         for ( size_t cc = 0; cc < nbc; ++cc )
+            boundaryColour( backward ? nbc - 1 - cc : cc );
+      };
       if ( !backward )
       {
-         for ( size_t cc = 0; cc < nbc; ++cc )
-            boundaryColour( cc );
+         boundaryColours();
          // the CSR sweep updated the owners only: refresh the cell copies the
          // interior sweep reads
          if ( o.csr && nbc > 0 )
@@ -1247,8 +1726,7 @@ void p1SOR( Context* ctx, P1Operator& op, Function& x, Function& b, double relax
          if ( interior )
             for ( int grp = 3; grp >= 0; --grp )
                interiorGroup( grp, 1 );
-         for ( size_t cc = nbc; cc-- > 0; )
-            boundaryColour( cc );
+         boundaryColours();
          if ( o.csr && nbc > 0 )
             pullHalos( ctx, *op.st, lat, xp, x.dtype, lv );
       }
@@ -1278,7 +1756,7 @@ void p1Restrict( Context* ctx, Function& f, int fineL, int flag )
       if ( lc.nb > 0 )
       {
          kRestrictBnd< T ><<< gridFor( lc.nb << f.lv ), kBlock, 0, ctx->stream >>>(
-             BndGeom::of( st, lc ), lc.nb, lc.nc, lc.bndFlag.p, flag, st.clsInvN.p, lf.sc, lf.w, lf.mm, (const T*) fp,
+             BndGeom::of( st, lc ), lc.nb, lc.nc, lc.bndFlag.p, flag, st.clsInvN.p, lf.sc, lf.w, (const T*) fp,
              (T*) cp, f.lv );
          HG_CHECK_HIP( hipGetLastError() );
       }
