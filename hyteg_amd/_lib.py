@@ -113,6 +113,7 @@ SIGNATURES = {
     "hg_p2_prolongate": [_p, _i64, _i, _i, _i],
     "hg_p2_transfer_stencil": [_i, _i, _i, _p, _p, _p],
     "hg_p2_cg_solve": [_p, _i64, _i64, _i64, _i, _i, _d, _d, _i, _p],
+    "hg_p2_cg_assembled": [_p, _i64, _i64, _i64, _i, _i, _i, _d, _d, _i, _p, _p],
     "hg_p2_estimate_radius": [_p, _i64, _i64, _i, _i, _p],
     "hg_p2_chebyshev_smooth": [_p, _i64, _i64, _i64, _i, _i, _d, _i],
     "hg_p2_ir_solve": [_p, _i64, _i64, _i64, _i, _i, _i, _i, _i, _i, _d, _i, _i, _d, _i, _d, _p, _p],

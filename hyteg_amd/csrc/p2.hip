@@ -14,6 +14,7 @@
 // the element matrix of the reference applied to the element vector without
 // forming the 10x10 matrix.
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <mutex>
 #include <type_traits>
@@ -188,6 +189,9 @@ struct P2Operator : OperatorBase
    std::map< int, int64_t >               tableStride; // by P2 level
    std::map< int, DevBuf< double > >      invScratch;  // one slot's diagonal, by P2 level
    DevBuf< int32_t >                      slotOn;      // 1: the apply computes the slot, 0: its result is 0
+   // assembled form of small levels (p2AssembledCG): weights of the pattern's entries
+   std::map< int, DevBuf< double > >      assembled;
+   std::map< int, DevBuf< double > >      cgState; // scratch vectors and scalars of the solve
 };
 
 __device__ __forceinline__ double kEval( const KParams& K, const double x[3] )
@@ -1788,11 +1792,394 @@ __global__ void kChebyshevStep( int64_t ncell, int64_t nb, const uint8_t* __rest
    x[p] = fromAcc< T >( v );
 }
 
+// ---- conjugate gradients on an assembled small level ---------------------------
+// The coarse solve of the P2 V-cycles runs some ninety CG iterations on a few thousand
+// DoFs.  Iteration by iteration it is nine launches of latency-bound kernels and a read
+// back (70 us on the shell's level 0: halo pull, one wavefront a macro-cell, additive
+// push, two updates, three dot products); assembled, the matrix is about 1 MB, which one
+// workgroup reads from L2 in 8 us, and a whole solve is one launch.  The iteration, its
+// scalars and its stopping test are those of CGSolver.
+constexpr int     kCgThreads   = 1024;
+constexpr int     kCgMaxDofs   = 16384; // p in LDS; the matrix of a larger level costs more than the launches
+constexpr int     kCgMaxLevel  = 2;
+constexpr int     kCgPerLaunch = 1024;  // iterations a launch (bounds its time, at most about 50 ms)
+enum CgState
+{
+   kCgRz   = 0, // r . z
+   kCgR0   = 1, // sqrt(r . r) of the start
+   kCgIts  = 2, // iterations done
+   kCgDone = 3,
+   kCgVec  = 8, // then r, A p, p (n values each)
+};
+
+struct P2Pattern : OperatorBase
+{
+   int32_t           n = 0, nslice = 0;
+   int64_t           nent = 0;
+   DevBuf< int64_t > pos;     // storage position of each DoF
+   DevBuf< uint8_t > flag;    // its type
+   DevBuf< int64_t > off;     // slices of 64 rows: entry offsets, column-major
+   DevBuf< int32_t > rowOf;   // DoF of each row slot (-1: none), longest rows first
+   DevBuf< uint16_t > col;    // columns
+   DevBuf< int32_t > diag;    // entry of each DoF's diagonal
+   DevBuf< int32_t > elem;    // micro-cells: cell, type | anchor << 3
+   DevBuf< int32_t > entry;   // their 100 entries
+   int64_t           nelem = 0;
+};
+
+// null where the level is not solved in assembled form
+static const P2Pattern* p2Pattern( Context* ctx, Storage& st, int L )
+{
+   Lattice& lat = st.lattice( ctx, L + 1 );
+   if ( L > kCgMaxLevel || lat.num.n > kCgMaxDofs )
+      return nullptr;
+   auto it = st.p2Patterns.find( L );
+   if ( it != st.p2Patterns.end() )
+      return static_cast< const P2Pattern* >( it->second.get() );
+   auto            pat = std::make_unique< P2Pattern >();
+   const Topology& t   = st.topo;
+   const int64_t   mm  = int64_t( 1 ) << L;
+   const int32_t   n   = int32_t( lat.num.n );
+   std::vector< int64_t > pos( n );
+   std::vector< uint8_t > flag( n );
+   for ( int32_t i = 0; i < n; ++i )
+   {
+      pos[i]  = lat.nc * lat.sc + i; // owned; the cell interiors follow below
+      flag[i] = i < lat.nb ? lat.hBndFlag[i] : uint8_t( kInner );
+   }
+   std::vector< int32_t >                elem;
+   std::vector< std::array< int32_t, 10 > > ids;
+   const int edges[6][2] = { { 0, 1 }, { 0, 2 }, { 0, 3 }, { 1, 2 }, { 1, 3 }, { 2, 3 } };
+   for ( int c = 0; c < t.nc; ++c )
+      for ( int ty = 0; ty < 6; ++ty )
+         for ( int a = 0; a < 64; ++a )
+         {
+            const int64_t x = a & 3, y = ( a >> 2 ) & 3, z = a >> 4;
+            if ( x + y + z > mm - 1 - MicroCells::rowShift[ty] )
+               continue;
+            std::array< int32_t, 10 > id;
+            auto                      node = [&]( int j, int64_t X, int64_t Y, int64_t Z ) {
+               const int64_t d = lat.num.locate( t, c, X, Y, Z );
+               id[size_t( j )] = int32_t( d );
+               if ( d >= lat.nb )
+                  pos[size_t( d )] = lat.cellPos( c, X, Y, Z );
+            };
+            const int( *v )[3] = MicroCells::vof[ty];
+            for ( int k = 0; k < 4; ++k )
+               node( k, 2 * ( x + v[k][0] ), 2 * ( y + v[k][1] ), 2 * ( z + v[k][2] ) );
+            for ( int e = 0; e < 6; ++e )
+            {
+               const int *p = v[edges[e][0]], *q = v[edges[e][1]];
+               node( 4 + e, 2 * x + p[0] + q[0], 2 * y + p[1] + q[1], 2 * z + p[2] + q[2] );
+            }
+            elem.push_back( c );
+            elem.push_back( ty | ( a << 3 ) );
+            ids.push_back( id );
+         }
+   std::vector< std::vector< int32_t > > cols( n );
+   for ( const auto& id : ids )
+      for ( int i = 0; i < 10; ++i )
+         cols[id[size_t( i )]].insert( cols[id[size_t( i )]].end(), id.begin(), id.end() );
+   std::vector< int32_t > order( n );
+   for ( int32_t i = 0; i < n; ++i )
+   {
+      std::sort( cols[i].begin(), cols[i].end() );
+      cols[i].erase( std::unique( cols[i].begin(), cols[i].end() ), cols[i].end() );
+      order[i] = i;
+   }
+   std::stable_sort( order.begin(), order.end(),
+                     [&]( int32_t a, int32_t b ) { return cols[a].size() > cols[b].size(); } );
+   order.resize( size_t( n + 63 ) / 64 * 64, -1 );
+   const int32_t          nsl = int32_t( order.size() / 64 );
+   std::vector< int64_t > off( nsl + 1, 0 );
+   std::vector< int32_t > first( n ); // entry of a row's first column
+   for ( int32_t s = 0; s < nsl; ++s )
+   {
+      // the first row of a slice is its longest; widths in steps of 8
+      const size_t w = ( cols[order[64 * size_t( s )]].size() + 7 ) / 8 * 8;
+      off[s + 1]     = off[s] + int64_t( 64 * w );
+   }
+   std::vector< uint16_t > col( size_t( off[nsl] ), 0 );
+   std::vector< int32_t >  diag( n );
+   for ( size_t i = 0; i < order.size(); ++i )
+   {
+      if ( order[i] < 0 )
+         continue;
+      const auto&   cc = cols[order[i]];
+      const int64_t e0 = off[i / 64] + int64_t( i % 64 );
+      first[order[i]]  = int32_t( e0 );
+      for ( size_t j = 0; j < cc.size(); ++j )
+      {
+         col[size_t( e0 + 64 * int64_t( j ) )] = uint16_t( cc[j] );
+         if ( cc[j] == order[i] )
+            diag[order[i]] = int32_t( e0 + 64 * int64_t( j ) );
+      }
+   }
+   std::vector< int32_t > entry;
+   entry.reserve( 100 * ids.size() );
+   for ( const auto& id : ids )
+      for ( int i = 0; i < 10; ++i )
+         for ( int j = 0; j < 10; ++j )
+         {
+            const auto& cc = cols[id[size_t( i )]];
+            const auto  at = std::lower_bound( cc.begin(), cc.end(), id[size_t( j )] ) - cc.begin();
+            entry.push_back( first[id[size_t( i )]] + 64 * int32_t( at ) );
+         }
+   pat->n      = n;
+   pat->nslice = nsl;
+   pat->nent   = off[nsl];
+   pat->nelem  = int64_t( ids.size() );
+   pat->pos.upload( ctx, pos );
+   pat->flag.upload( ctx, flag );
+   pat->off.upload( ctx, off );
+   pat->rowOf.upload( ctx, order );
+   pat->col.upload( ctx, col );
+   pat->diag.upload( ctx, diag );
+   pat->elem.upload( ctx, elem );
+   pat->entry.upload( ctx, entry );
+   return static_cast< const P2Pattern* >( ( st.p2Patterns[L] = std::move( pat ) ).get() );
+}
+
+// element matrices into the pattern's entries: one thread a micro-cell and column
+__global__ void kP2Assemble( const P2ActGeomT< double >* __restrict__ geom, const P2CellGeom* __restrict__ geom64,
+                             const KParams* __restrict__ kp, int64_t mm, int64_t nelem, const int32_t* __restrict__ elem,
+                             const int32_t* __restrict__ entry, double* __restrict__ val )
+{
+   const int64_t i = int64_t( blockIdx.x ) * blockDim.x + threadIdx.x;
+   if ( i >= 10 * nelem )
+      return;
+   const int64_t e = i / 10;
+   const int     j = int( i - 10 * e );
+   const int32_t c = elem[2 * e], t = elem[2 * e + 1] & 7, a = elem[2 * e + 1] >> 3;
+   const TileCoord             tc{ c, 0, 0, 0 };
+   const P2ActGeomT< double >& g = geom[c];
+   double                      p0[3], u[10], y[10];
+   actVertex( g, tc, mm, t, a, p0 );
+#pragma unroll
+   for ( int k = 0; k < 10; ++k )
+      u[k] = k == j ? 1.0 : 0.0;
+   p2ElementAction< double, true, false >( g, g.Dc[t], g.xq[t], g.cw[t], p0, u, y, 0.0, 0.0, 0.0, [&]( int q ) {
+      return evaluatedCoefficient< true >( geom64[c], *kp, tc, mm, t, a, q );
+   } );
+#pragma unroll
+   for ( int k = 0; k < 10; ++k )
+      atomicAdd( &val[entry[100 * e + 10 * k + j]], y[k] );
+}
+
+// sums of up to two values over the workgroup, in every thread
+__device__ __forceinline__ void cgSum( double& a, double& b, double ( *red )[2] )
+{
+#pragma unroll
+   for ( int d = 32; d > 0; d /= 2 )
+   {
+      a += __shfl_xor( a, d );
+      b += __shfl_xor( b, d );
+   }
+   __syncthreads(); // the sums of the call before are read
+   if ( ( threadIdx.x & 63 ) == 0 )
+   {
+      red[threadIdx.x >> 6][0] = a;
+      red[threadIdx.x >> 6][1] = b;
+   }
+   __syncthreads();
+   a = b = 0.0;
+#pragma unroll
+   for ( int w = 0; w < kCgThreads / 64; ++w )
+   {
+      a += red[w][0];
+      b += red[w][1];
+   }
+}
+
+__global__ __launch_bounds__( kCgThreads ) void kP2AssembledCG( int32_t n, int32_t nslice, const int64_t* __restrict__ pos,
+                                                               const uint8_t* __restrict__ dofFlag, int flag,
+                                                               const int64_t* __restrict__ off,
+                                                               const int32_t* __restrict__ rowOf,
+                                                               const uint16_t* __restrict__ col,
+                                                               const int32_t* __restrict__ diag,
+                                                               const double* __restrict__ val, int jacobi, int start,
+                                                               int maxIter, int perLaunch, double relTol, double absTol,
+                                                               const double* __restrict__ b, double* __restrict__ x,
+                                                               double* __restrict__ state )
+{
+   extern __shared__ double sp[]; // p
+   __shared__ double        red[kCgThreads / 64][2];
+   double* const            r  = state + kCgVec;
+   double* const            ap = r + n;
+   double* const            ps = ap + n;
+   const int                wave = int( threadIdx.x ) >> 6, lane = int( threadIdx.x ) & 63;
+   // ap = A p on the rows; wavefronts take slices in turn
+   auto product = [&]() {
+      for ( int32_t s = wave; s < nslice; s += kCgThreads / 64 )
+      {
+         const int64_t e0 = off[s] + lane;
+         const int32_t w = int32_t( ( off[s + 1] - off[s] ) / 64 ), row = rowOf[64 * s + lane];
+         double        acc = 0.0;
+         for ( int32_t j = 0; j < w; j += 8 )
+         {
+            uint16_t cj[8];
+            double   vj[8];
+#pragma unroll
+            for ( int u = 0; u < 8; ++u )
+            {
+               cj[u] = col[e0 + 64 * int64_t( j + u )];
+               vj[u] = val[e0 + 64 * int64_t( j + u )];
+            }
+#pragma unroll
+            for ( int u = 0; u < 8; ++u )
+               acc += vj[u] * sp[cj[u]];
+         }
+         if ( row >= 0 )
+            ap[row] = acc;
+      }
+      __syncthreads();
+   };
+   auto isFree = [&]( int32_t i ) { return ( dofFlag[i] & flag ) != 0; };
+   auto inverse = [&]( int32_t i ) { return jacobi ? 1.0 / val[diag[i]] : 1.0; };
+   double rz, r0, its = 0.0;
+   if ( start )
+   {
+      for ( int32_t i = threadIdx.x; i < n; i += kCgThreads )
+         sp[i] = x[pos[i]];
+      __syncthreads();
+      product();
+      rz = r0 = 0.0;
+      for ( int32_t i = threadIdx.x; i < n; i += kCgThreads )
+      {
+         const bool   f  = isFree( i );
+         const double ri = f ? b[pos[i]] - ap[i] : 0.0, zi = f ? inverse( i ) * ri : 0.0;
+         r[i]  = ri;
+         sp[i] = zi;
+         rz += ri * zi;
+         r0 += ri * ri;
+      }
+      cgSum( rz, r0, red );
+      r0 = sqrt( r0 );
+      if ( threadIdx.x == 0 )
+      {
+         state[kCgR0]   = r0;
+         state[kCgIts]  = 0.0;
+         state[kCgDone] = r0 < absTol ? 1.0 : 0.0;
+      }
+      if ( r0 < absTol )
+         return;
+   }
+   else
+   {
+      rz  = state[kCgRz];
+      r0  = state[kCgR0];
+      its = state[kCgIts] + 1.0;
+      for ( int32_t i = threadIdx.x; i < n; i += kCgThreads )
+         sp[i] = ps[i];
+   }
+   __syncthreads();
+   for ( int k = 0; k < perLaunch; ++k )
+   {
+      product();
+      double pap = 0.0, rr = 0.0, rzn = 0.0, none = 0.0;
+      for ( int32_t i = threadIdx.x; i < n; i += kCgThreads )
+         if ( isFree( i ) )
+            pap += sp[i] * ap[i];
+      cgSum( pap, none, red );
+      const double alpha = rz / pap;
+      for ( int32_t i = threadIdx.x; i < n; i += kCgThreads )
+         if ( isFree( i ) )
+         {
+            x[pos[i]] += alpha * sp[i];
+            const double ri = r[i] - alpha * ap[i];
+            r[i]            = ri;
+            rr += ri * ri;
+            rzn += ri * ( inverse( i ) * ri );
+         }
+      cgSum( rr, rzn, red );
+      const double res  = sqrt( rr );
+      const bool   done = res / r0 < relTol || res < absTol || its + 1.0 >= double( maxIter );
+      if ( !done )
+      {
+         const double beta = rzn / rz;
+         for ( int32_t i = threadIdx.x; i < n; i += kCgThreads )
+            if ( isFree( i ) )
+               sp[i] = inverse( i ) * r[i] + beta * sp[i];
+         rz = rzn;
+      }
+      if ( threadIdx.x == 0 && ( done || k + 1 == perLaunch ) )
+      {
+         state[kCgRz]   = rz;
+         state[kCgIts]  = its;
+         state[kCgDone] = done ? 1.0 : 0.0;
+      }
+      if ( done )
+         return;
+      its += 1.0;
+      __syncthreads();
+   }
+   for ( int32_t i = threadIdx.x; i < n; i += kCgThreads )
+      ps[i] = sp[i];
+}
+
+// CGSolver::solve on a small level in assembled form; false where it does not apply
+static bool p2AssembledCG( Context* ctx, P2Operator& op, Function& x, Function& b, int L, int flag, int maxIter,
+                           double relTol, double absTol, int jacobi, int* iterations )
+{
+   if ( op.nslot != 1 || x.dtype != 0 || b.dtype != 0 || &x == &b || ctx->capturing || tlsCaptures > 0 )
+      return false;
+   p2CheckFunction( op, x, L );
+   p2CheckFunction( op, b, L );
+   const P2Pattern* pat = p2Pattern( ctx, *op.st, L );
+   if ( !pat || maxIter < 1 )
+      return false;
+   auto& val = op.assembled[L];
+   if ( !val.p )
+   {
+      val.alloc( ctx, size_t( pat->nent ) );
+      kP2Assemble<<< gridFor( 10 * pat->nelem, 64 ), 64, 0, ctx->stream >>>( op.ageom.at( L ).p, op.tgeom.at( L ).p,
+                                                                            op.kpar.p, int64_t( 1 ) << L, pat->nelem,
+                                                                            pat->elem.p, pat->entry.p, val.p );
+      HG_CHECK_HIP( hipGetLastError() );
+   }
+   auto& state = op.cgState[L];
+   if ( !state.p )
+      state.alloc( ctx, size_t( kCgVec ) + 3 * size_t( pat->n ) );
+   static std::once_flag once[64]; // per device
+   std::call_once( once[ctx->device & 63], [] {
+      HG_CHECK_HIP( hipFuncSetAttribute( reinterpret_cast< const void* >( &kP2AssembledCG ),
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, int( kCgMaxDofs * sizeof( double ) ) ) );
+   } );
+   double s[4] = { 0, 0, 0, 0 };
+   for ( int start = 1; s[kCgDone] == 0.0; start = 0 )
+   {
+      kP2AssembledCG<<< 1, kCgThreads, size_t( pat->n ) * sizeof( double ), ctx->stream >>>(
+          pat->n, pat->nslice, pat->pos.p, pat->flag.p, flag, pat->off.p, pat->rowOf.p, pat->col.p, pat->diag.p, val.p,
+          jacobi, start, maxIter, kCgPerLaunch, relTol, absTol, (const double*) b.ptr( L ), (double*) x.ptr( L ), state.p );
+      HG_CHECK_HIP( hipGetLastError() );
+      DeviceGateLock gate;
+      HG_CHECK_HIP( hipMemcpyAsync( ctx->hostResult, state.p, sizeof( s ), hipMemcpyDeviceToHost, ctx->stream ) );
+      HG_CHECK_HIP( hipStreamSynchronize( ctx->stream ) );
+      std::copy( ctx->hostResult, ctx->hostResult + 4, s );
+   }
+   if ( iterations )
+      *iterations = int( s[kCgIts] );
+   return true;
+}
+
 } // namespace hg
 
 using namespace hg;
 
 extern "C" {
+
+int hg_p2_cg_assembled( hg_ctx* h, hg_handle op, hg_handle x, hg_handle b, int level, int flag, int maxIter,
+                        double relTol, double absTol, int jacobi, int* iterations, int* applied )
+{
+   return hg_guard( h, [&]( Context* ctx ) {
+      if ( !applied )
+         throw Error( HG_ERR_ARG, "cg_assembled: null output" );
+      *applied = p2AssembledCG( ctx, ctx->op< P2Operator >( op ), ctx->function( x ), ctx->function( b ), level, flag,
+                                maxIter, relTol, absTol, jacobi, iterations ) ?
+                     1 :
+                     0;
+   } );
+}
 
 int hg_storage_shell( hg_ctx* h, int ntan, int nrad, double rmin, double rmax, hg_handle* out )
 {

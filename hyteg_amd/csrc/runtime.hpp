@@ -156,6 +156,8 @@ struct Storage
    Topology                                     topo;
    // grid-transfer data keyed by fine level (built on first use)
    std::map< int, std::unique_ptr< OperatorBase > > transfers;
+   // sparsity patterns of assembled P2 operators by level (built on first use)
+   std::map< int, std::unique_ptr< OperatorBase > > p2Patterns;
    std::map< int, std::unique_ptr< Lattice > >  lattices;
    DevBuf< CellMeta >                           meta;
    // 1 / (number of cells) of each cell's local faces (0..3), edges (4..9) and

@@ -404,6 +404,12 @@ int hg_ctx_last_kernel_ms( hg_ctx* ctx, double* ms );
  * inverse-diagonal multiplication, SubstitutePreconditioner.hpp:120-158) */
 int hg_p2_cg_solve( hg_ctx* ctx, hg_handle op, hg_handle x, hg_handle b, int level, int maxIter, double relTol,
                     double absTol, int jacobi, int* iterations );
+/* the same iteration on the DoFs of type `flag` with the operator assembled, in one
+ * launch, for small levels (no counterpart in the reference; CGSolver calls it on its
+ * own): *applied = 0, and nothing done, where the level is too large for it or a graph
+ * capture is open */
+int hg_p2_cg_assembled( hg_ctx* ctx, hg_handle op, hg_handle x, hg_handle b, int level, int flag, int maxIter,
+                        double relTol, double absTol, int jacobi, int* iterations, int* applied );
 /* `steps` ChebyshevSmoother::solve calls on `level` (solvers/ChebyshevSmoother.hpp:112-232)
  * after setupCoefficients(order, spectralRadius) with bounds 0.3/1.2 x radius */
 int hg_p2_chebyshev_smooth( hg_ctx* ctx, hg_handle op, hg_handle x, hg_handle b, int level, int order,

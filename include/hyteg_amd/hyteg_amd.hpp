@@ -794,6 +794,9 @@ class SORSmoother : public Solver< OperatorType >
    DoFType flag_ = Inner | NeumannBoundary | FreeslipBoundary;
 };
 
+template < class OperatorType >
+class InverseDiagonalPreconditioner;
+
 // CGSolver with the identity preconditioner (CGSolver.hpp:94-203, 340-358)
 template < class OperatorType >
 class CGSolver : public Solver< OperatorType >
@@ -900,6 +903,25 @@ class CGSolver : public Solver< OperatorType >
    // the iterates and the stopping step are those of the host-scalar loop.
    void solveDeviceScalars( const OperatorType& A, const FunctionType& x, const FunctionType& b, uint_t level )
    {
+      // the P2 diffusion operator solves its small levels in one launch
+      if constexpr ( std::is_same_v< OperatorType, P2ElementwiseBlendingDivKGradOperatorT< double > > )
+      {
+         const bool jacobi = dynamic_cast< InverseDiagonalPreconditioner< OperatorType >* >( prec_.get() ) != nullptr;
+         if ( !fixed_ && ( !prec_ || jacobi ) )
+         {
+            int its = 0, applied = 0;
+            check( ctx_,
+                   hg_p2_cg_assembled( ctx_, A.handle(), x.handle(), b.handle(), int( level ), int( flag_ ),
+                                       int( std::min< uint_t >( maxIter_, uint_t( std::numeric_limits< int >::max() ) ) ),
+                                       relTol_, absTol_, jacobi ? 1 : 0, &its, &applied ),
+                   "CGSolver" );
+            if ( applied )
+            {
+               iterations_ = uint_t( its );
+               return;
+            }
+         }
+      }
       const int rr = slot0_, pap = slot0_ + 1, rr0 = slot0_ + 4, done = slot0_ + 5;
       int       rz[2] = { slot0_ + 2, slot0_ + 3 }, cur = 0;
       copyBCs( x, p_ );
