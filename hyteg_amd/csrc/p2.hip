@@ -412,40 +412,43 @@ __global__ __launch_bounds__( kTileThreads ) void kP2TileCentroidK( const P2Cell
    table[lb * kTileThreads + threadIdx.x] = __float2half( th.valid ? float( kAt( g, *kp, x, ls ) ) : 0.0f );
 }
 
-// the 4-point degree-2 rule: one barycentric coordinate kB, the others kA
-constexpr float kQ2A = 0.1381966011250105f, kQ2B = 0.5854101966249685f;
-
-// y += A_e u of the reduced form: constant metric G (scaled by k |det| w) and
-// the 4 points of the degree-2 rule, in the barycentric form of p2ElementAction
+// y = A_e u of the reduced form: constant metric G (scaled by k |det| / 24, the weight
+// of the 4-point degree-2 rule's points).  With d = d0 + 4 B lam' (p2ElementAction) the
+// sums over the points need only those of 1, lam_j and lam_j lam_l, which the rule
+// integrates exactly -- 4, 1 and (1 + delta_jl) / 5 -- so that
+//   S = G 4 (d0 + B 1),  T_j = G (d0 + 4/5 (B 1 + B_j)):
+// four products with G instead of a gradient, a product and ten tests at each point.
 __device__ __forceinline__ void p2ReducedAction( const float G[6], const float u[10], float y[10] )
 {
+   const float d0[3] = { 4.0f * u[4] - 3.0f * u[0] - u[1], 4.0f * u[5] - 3.0f * u[0] - u[2],
+                         4.0f * u[6] - 3.0f * u[0] - u[3] };
+   const float b00 = u[1] + u[0] - 2.0f * u[4], b11 = u[2] + u[0] - 2.0f * u[5], b22 = u[3] + u[0] - 2.0f * u[6];
+   const float b01 = u[7] - u[5] - u[4] + u[0], b02 = u[8] - u[6] - u[4] + u[0], b12 = u[9] - u[6] - u[5] + u[0];
+   const float B[3][3] = { { b00, b01, b02 }, { b01, b11, b12 }, { b02, b12, b22 } };
+   const float b1[3]   = { b00 + b01 + b02, b01 + b11 + b12, b02 + b12 + b22 };
+   float       S[3], T[3][3]; // T[k][j]
+   auto        product = [&]( float v0, float v1, float v2, float& r0, float& r1, float& r2 ) {
+      r0 = G[0] * v0 + G[1] * v1 + G[2] * v2;
+      r1 = G[1] * v0 + G[3] * v1 + G[4] * v2;
+      r2 = G[2] * v0 + G[4] * v1 + G[5] * v2;
+   };
+   product( 4.0f * ( d0[0] + b1[0] ), 4.0f * ( d0[1] + b1[1] ), 4.0f * ( d0[2] + b1[2] ), S[0], S[1], S[2] );
 #pragma unroll
-   for ( int q = 0; q < 4; ++q )
+   for ( int j = 0; j < 3; ++j )
+      product( d0[0] + 0.8f * ( b1[0] + B[0][j] ), d0[1] + 0.8f * ( b1[1] + B[1][j] ), d0[2] + 0.8f * ( b1[2] + B[2][j] ),
+               T[0][j], T[1][j], T[2][j] );
+   const float rs[3] = { T[0][0] + T[0][1] + T[0][2], T[1][0] + T[1][1] + T[1][2], T[2][0] + T[2][1] + T[2][2] };
+   const float cs[3] = { T[0][0] + T[1][0] + T[2][0], T[0][1] + T[1][1] + T[2][1], T[0][2] + T[1][2] + T[2][2] };
+   y[0]              = 4.0f * ( rs[0] + rs[1] + rs[2] ) - 3.0f * ( S[0] + S[1] + S[2] );
+#pragma unroll
+   for ( int k = 0; k < 3; ++k )
    {
-      float l[4];
-#pragma unroll
-      for ( int k = 0; k < 4; ++k )
-         l[k] = k == q ? kQ2B : kQ2A;
-      const float g0 = ( 4.0f * l[0] - 1.0f ) * u[0] + 4.0f * ( l[1] * u[4] + l[2] * u[5] + l[3] * u[6] );
-      const float g1 = ( 4.0f * l[1] - 1.0f ) * u[1] + 4.0f * ( l[0] * u[4] + l[2] * u[7] + l[3] * u[8] );
-      const float g2 = ( 4.0f * l[2] - 1.0f ) * u[2] + 4.0f * ( l[0] * u[5] + l[1] * u[7] + l[3] * u[9] );
-      const float g3 = ( 4.0f * l[3] - 1.0f ) * u[3] + 4.0f * ( l[0] * u[6] + l[1] * u[8] + l[2] * u[9] );
-      const float d1 = g1 - g0, d2 = g2 - g0, d3 = g3 - g0;
-      const float e1 = G[0] * d1 + G[1] * d2 + G[2] * d3;
-      const float e2 = G[1] * d1 + G[3] * d2 + G[4] * d3;
-      const float e3 = G[2] * d1 + G[4] * d2 + G[5] * d3;
-      const float e0 = -( e1 + e2 + e3 );
-      y[0] += ( 4.0f * l[0] - 1.0f ) * e0;
-      y[1] += ( 4.0f * l[1] - 1.0f ) * e1;
-      y[2] += ( 4.0f * l[2] - 1.0f ) * e2;
-      y[3] += ( 4.0f * l[3] - 1.0f ) * e3;
-      y[4] += 4.0f * ( l[1] * e0 + l[0] * e1 );
-      y[5] += 4.0f * ( l[2] * e0 + l[0] * e2 );
-      y[6] += 4.0f * ( l[3] * e0 + l[0] * e3 );
-      y[7] += 4.0f * ( l[2] * e1 + l[1] * e2 );
-      y[8] += 4.0f * ( l[3] * e1 + l[1] * e3 );
-      y[9] += 4.0f * ( l[3] * e2 + l[2] * e3 );
+      y[1 + k] = 4.0f * T[k][k] - S[k];
+      y[4 + k] = 4.0f * ( S[k] - rs[k] - cs[k] );
    }
+   y[7] = 4.0f * ( T[0][1] + T[1][0] );
+   y[8] = 4.0f * ( T[0][2] + T[2][0] );
+   y[9] = 4.0f * ( T[1][2] + T[2][1] );
 }
 
 // Reduced-form apply, FP32 arithmetic on FP32 or FP16 values.  A tile's source
@@ -578,29 +581,38 @@ __global__ __launch_bounds__( kTileThreads ) void kP2TileApplyReduced( const P2C
    int64_t         full;
    const TileCoord tc   = tileFromList( tiles, lb, mm, full );
    const int64_t   base = tc.c * sc1;
-   const int32_t   top  = int32_t( 2 * mm );
    float           G[6];
    float           ke = 0.0f;
    if constexpr ( STORED_G )
    {
 #pragma unroll
       for ( int i = 0; i < 6; ++i )
-         G[i] = gm[( lb * 6 + i ) * kTileThreads + threadIdx.x];
+         G[i] = __builtin_nontemporal_load( gm + ( lb * 6 + i ) * kTileThreads + threadIdx.x ); // read once per apply
    }
    else
       ke = __half2float( kc[lb * kTileThreads + threadIdx.x] );
-   const T* srcC = src + base;
+   const T*         srcC = src + base;
+   const BoxOffsets bo( int32_t( w1 ), 2 * int32_t( tc.x0 ), 2 * int32_t( tc.y0 ), 2 * int32_t( tc.z0 ) );
+   const int32_t    room = int32_t( 2 * ( mm - tc.x0 - tc.y0 - tc.z0 ) );
+   // the thread's (at most two) box points: lattice offset (-1: none) and whether the
+   // point lies on the box surface
+   int32_t off[2];
+   bool    surface[2];
    {
-      // the thread's (at most two) box points, both loads in flight before the LDS writes
+      // both loads in flight before the LDS writes
       T bv[2];
 #pragma unroll
       for ( int j = 0; j < 2; ++j )
       {
-         const int     p  = int( threadIdx.x ) + j * kTileThreads;
-         const int32_t lx = p % kBox, ly = ( p / kBox ) % kBox, lz = p / ( kBox * kBox );
-         const int32_t X = 2 * int32_t( tc.x0 ) + lx, Y = 2 * int32_t( tc.y0 ) + ly, Z = 2 * int32_t( tc.z0 ) + lz;
-         bv[j]           = ( p < kBox3 && X + Y + Z <= top ) ? srcC[tetRowStart32( int32_t( w1 ), Y, Z ) + X] : T( 0 );
+         const int32_t p = int32_t( threadIdx.x ) + j * kTileThreads;
+         int32_t       lx, ly, lz;
+         boxPoint( p, lx, ly, lz );
+         off[j]     = ( j == 0 || p < kBox3 ) && lx + ly + lz <= room ? bo.at( lx, ly, lz ) : -1;
+         surface[j] = lx == 0 || ly == 0 || lz == 0 || lx == kBox - 1 || ly == kBox - 1 || lz == kBox - 1;
+         bv[j]      = off[j] >= 0 ? srcC[off[j]] : T( 0 );
       }
+      // the result boxes are cleared while the loads are in flight
+      waveBoxClear( sy );
 #pragma unroll
       for ( int j = 0; j < 2; ++j )
       {
@@ -616,48 +628,43 @@ __global__ __launch_bounds__( kTileThreads ) void kP2TileApplyReduced( const P2C
    const int a  = int( threadIdx.x ) & 63;
    const int ax = a & 3, ay = ( a >> 2 ) & 3, az = a >> 4;
    const bool valid = tc.x0 + ax + tc.y0 + ay + tc.z0 + az <= mm - 1 - MicroCells::rowShift[t];
-   float u[10];
-   int   pos[10];
-#pragma unroll
-   for ( int k = 0; k < 4; ++k )
-      pos[k] = 2 * ( ax + cVof[t][k][0] ) + kBox * ( 2 * ( ay + cVof[t][k][1] ) + kBox * 2 * ( az + cVof[t][k][2] ) );
-#pragma unroll
-   for ( int e = 0; e < 6; ++e )
-      pos[4 + e] = ( pos[cP2E[e][0]] + pos[cP2E[e][1]] ) / 2;
-#pragma unroll
-   for ( int i = 0; i < 10; ++i )
-      u[i] = valid ? sb[pos[i]] : 0.0f;
-   if constexpr ( !STORED_G )
-      reducedMetric( sv, t, ax, ay, az, ke, G );
-   {
-      float y[10];
+   const int  at    = 2 * ax + kBox * ( 2 * ay + kBox * 2 * az );
+   float      u[10];
+   forType( t, [&]( auto box ) {
 #pragma unroll
       for ( int i = 0; i < 10; ++i )
-         y[i] = 0.0f;
-      if ( valid )
-         p2ReducedAction( G, u, y );
-      waveBoxAccumulate( sy, valid, pos, y );
+         u[i] = sb[at + box.at( i )];
+   } );
+   if constexpr ( !STORED_G )
+      reducedMetric( sv, t, ax, ay, az, ke, G );
+   if ( valid )
+   {
+      float y[10];
+      p2ReducedAction( G, u, y );
+      // per-wavefront result boxes (waveBoxAccumulate)
+      forType( t, [&]( auto box ) {
+         using LdsR   = volatile __attribute__( ( address_space( 3 ) ) ) float;
+         LdsR* const b = (LdsR*) ( sy + kBox3 * t + at );
+#pragma unroll
+         for ( int i = 0; i < 10; ++i )
+            b[box.at( i )] = b[box.at( i )] + y[i];
+      } );
    }
    __syncthreads();
    T* dstC = dst + base;
-   for ( int p = threadIdx.x; p < kBox3; p += kTileThreads )
+#pragma unroll
+   for ( int j = 0; j < 2; ++j )
    {
-      const int32_t lx = p % kBox, ly = ( p / kBox ) % kBox, lz = p / ( kBox * kBox );
-      const int32_t X = 2 * int32_t( tc.x0 ) + lx, Y = 2 * int32_t( tc.y0 ) + ly, Z = 2 * int32_t( tc.z0 ) + lz;
-      if ( X + Y + Z > top )
+      if ( off[j] < 0 )
          continue;
-      const int64_t o = tetRowStart32( int32_t( w1 ), Y, Z ) + X;
-      const float   v = alpha * waveBoxSum( sy, p );
+      const int64_t o = off[j];
+      const float   v = alpha * waveBoxSum( sy, int( threadIdx.x ) + j * kTileThreads );
       if constexpr ( std::is_same< T, float >::value )
          atomicAdd( dstC + o, v );
+      else if ( surface[j] )
+         atomicAdd( accum + base + o, v );
       else
-      {
-         const bool surface = lx == 0 || ly == 0 || lz == 0 || lx == kBox - 1 || ly == kBox - 1 || lz == kBox - 1;
-         if ( surface )
-            atomicAdd( accum + base + o, v );
-         else
-            dstC[o] = __float2half( rmw ? __half2float( dstC[o] ) + v : v );
-      }
+         dstC[o] = __float2half( rmw ? __half2float( dstC[o] ) + v : v );
    }
 }
 
@@ -1797,7 +1804,7 @@ __global__ void kChebyshevStep( int64_t ncell, int64_t nb, const uint8_t* __rest
 // DoFs.  Iteration by iteration it is nine launches of latency-bound kernels and a read
 // back (70 us on the shell's level 0: halo pull, one wavefront a macro-cell, additive
 // push, two updates, three dot products); assembled, the matrix is about 1 MB, which one
-// workgroup reads from L2 in 8 us, and a whole solve is one launch.  The iteration, its
+// workgroup reads from L2 in about 10 us, and a whole solve is one launch.  The iteration, its
 // scalars and its stopping test are those of CGSolver.
 constexpr int     kCgThreads   = 1024;
 constexpr int     kCgMaxDofs   = 16384; // p in LDS; the matrix of a larger level costs more than the launches
@@ -1809,7 +1816,7 @@ enum CgState
    kCgR0   = 1, // sqrt(r . r) of the start
    kCgIts  = 2, // iterations done
    kCgDone = 3,
-   kCgVec  = 8, // then r, A p, p (n values each)
+   kCgVec  = 8, // then r, A p, p, x, the inverse diagonal (n values each)
 };
 
 struct P2Pattern : OperatorBase
@@ -2004,38 +2011,65 @@ __global__ __launch_bounds__( kCgThreads ) void kP2AssembledCG( int32_t n, int32
 {
    extern __shared__ double sp[]; // p
    __shared__ double        red[kCgThreads / 64][2];
-   double* const            r  = state + kCgVec;
-   double* const            ap = r + n;
-   double* const            ps = ap + n;
+   __shared__ int32_t       so[kCgMaxDofs / 64 + 1];
+   double* const            r   = state + kCgVec;
+   double* const            ap  = r + n;
+   double* const            ps  = ap + n;
+   double* const            xs  = ps + n;
+   double* const            inv = xs + n; // 1 / diagonal (1 without the preconditioner), 0 where x is fixed
    const int                wave = int( threadIdx.x ) >> 6, lane = int( threadIdx.x ) & 63;
-   // ap = A p on the rows; wavefronts take slices in turn
+   for ( int32_t s = threadIdx.x; s <= nslice; s += kCgThreads )
+      so[s] = int32_t( off[s] );
+   // ap = A p on the rows: wavefronts take slices in turn, a chunk of eight entries in
+   // flight while the one before it is summed
    auto product = [&]() {
-      for ( int32_t s = wave; s < nslice; s += kCgThreads / 64 )
+      struct Chunk
       {
-         const int64_t e0 = off[s] + lane;
-         const int32_t w = int32_t( ( off[s + 1] - off[s] ) / 64 ), row = rowOf[64 * s + lane];
-         double        acc = 0.0;
-         for ( int32_t j = 0; j < w; j += 8 )
+         uint16_t c[8];
+         double   v[8];
+      };
+      auto load = [&]( int32_t e ) {
+         Chunk k;
+#pragma unroll
+         for ( int u = 0; u < 8; ++u )
          {
-            uint16_t cj[8];
-            double   vj[8];
-#pragma unroll
-            for ( int u = 0; u < 8; ++u )
-            {
-               cj[u] = col[e0 + 64 * int64_t( j + u )];
-               vj[u] = val[e0 + 64 * int64_t( j + u )];
-            }
-#pragma unroll
-            for ( int u = 0; u < 8; ++u )
-               acc += vj[u] * sp[cj[u]];
+            k.c[u] = col[e + 64 * u];
+            k.v[u] = val[e + 64 * u];
          }
-         if ( row >= 0 )
-            ap[row] = acc;
+         return k;
+      };
+      int32_t s = wave;
+      if ( s < nslice )
+      {
+         int32_t e = so[s];
+         Chunk   next = load( e + lane );
+         int32_t row  = rowOf[64 * s + lane];
+         double  acc  = 0.0;
+         while ( s < nslice )
+         {
+            const Chunk cur  = next;
+            const int32_t rn = row;
+            const bool  last = e + 512 >= so[s + 1];
+            const int32_t sn = last ? s + kCgThreads / 64 : s;
+            const int32_t en = last ? so[min( sn, nslice - 1 )] : e + 512;
+            next = load( en + lane );
+            if ( last )
+               row = rowOf[64 * min( sn, nslice - 1 ) + lane];
+#pragma unroll
+            for ( int u = 0; u < 8; ++u )
+               acc += cur.v[u] * sp[cur.c[u]];
+            if ( last )
+            {
+               if ( rn >= 0 )
+                  ap[rn] = acc;
+               acc = 0.0;
+            }
+            s = sn;
+            e = en;
+         }
       }
       __syncthreads();
    };
-   auto isFree = [&]( int32_t i ) { return ( dofFlag[i] & flag ) != 0; };
-   auto inverse = [&]( int32_t i ) { return jacobi ? 1.0 / val[diag[i]] : 1.0; };
    double rz, r0, its = 0.0;
    if ( start )
    {
@@ -2046,10 +2080,12 @@ __global__ __launch_bounds__( kCgThreads ) void kP2AssembledCG( int32_t n, int32
       rz = r0 = 0.0;
       for ( int32_t i = threadIdx.x; i < n; i += kCgThreads )
       {
-         const bool   f  = isFree( i );
-         const double ri = f ? b[pos[i]] - ap[i] : 0.0, zi = f ? inverse( i ) * ri : 0.0;
-         r[i]  = ri;
-         sp[i] = zi;
+         const double d  = ( dofFlag[i] & flag ) ? ( jacobi ? 1.0 / val[diag[i]] : 1.0 ) : 0.0;
+         const double ri = d != 0.0 ? b[pos[i]] - ap[i] : 0.0, zi = d * ri;
+         inv[i] = d;
+         xs[i]  = sp[i];
+         r[i]   = ri;
+         sp[i]  = zi;
          rz += ri * zi;
          r0 += ri * ri;
       }
@@ -2073,48 +2109,54 @@ __global__ __launch_bounds__( kCgThreads ) void kP2AssembledCG( int32_t n, int32
          sp[i] = ps[i];
    }
    __syncthreads();
-   for ( int k = 0; k < perLaunch; ++k )
+   for ( int k = 0;; ++k )
    {
       product();
       double pap = 0.0, rr = 0.0, rzn = 0.0, none = 0.0;
       for ( int32_t i = threadIdx.x; i < n; i += kCgThreads )
-         if ( isFree( i ) )
-            pap += sp[i] * ap[i];
+         pap += inv[i] != 0.0 ? sp[i] * ap[i] : 0.0;
       cgSum( pap, none, red );
       const double alpha = rz / pap;
       for ( int32_t i = threadIdx.x; i < n; i += kCgThreads )
-         if ( isFree( i ) )
+      {
+         const double d = inv[i];
+         if ( d != 0.0 )
          {
-            x[pos[i]] += alpha * sp[i];
+            xs[i] += alpha * sp[i];
             const double ri = r[i] - alpha * ap[i];
             r[i]            = ri;
             rr += ri * ri;
-            rzn += ri * ( inverse( i ) * ri );
+            rzn += ri * ( d * ri );
          }
+      }
       cgSum( rr, rzn, red );
       const double res  = sqrt( rr );
       const bool   done = res / r0 < relTol || res < absTol || its + 1.0 >= double( maxIter );
+      const bool   stop = done || k + 1 == perLaunch;
+      const double beta = rzn / rz;
       if ( !done )
-      {
-         const double beta = rzn / rz;
          for ( int32_t i = threadIdx.x; i < n; i += kCgThreads )
-            if ( isFree( i ) )
-               sp[i] = inverse( i ) * r[i] + beta * sp[i];
-         rz = rzn;
-      }
-      if ( threadIdx.x == 0 && ( done || k + 1 == perLaunch ) )
+            sp[i] = inv[i] * r[i] + beta * sp[i]; // 0 where x is fixed
+      rz = rzn;
+      if ( stop )
       {
-         state[kCgRz]   = rz;
-         state[kCgIts]  = its;
-         state[kCgDone] = done ? 1.0 : 0.0;
-      }
-      if ( done )
+         for ( int32_t i = threadIdx.x; i < n; i += kCgThreads )
+         {
+            if ( inv[i] != 0.0 )
+               x[pos[i]] = xs[i];
+            ps[i] = sp[i];
+         }
+         if ( threadIdx.x == 0 )
+         {
+            state[kCgRz]   = rz;
+            state[kCgIts]  = its;
+            state[kCgDone] = done ? 1.0 : 0.0;
+         }
          return;
+      }
       its += 1.0;
       __syncthreads();
    }
-   for ( int32_t i = threadIdx.x; i < n; i += kCgThreads )
-      ps[i] = sp[i];
 }
 
 // CGSolver::solve on a small level in assembled form; false where it does not apply
@@ -2139,7 +2181,7 @@ static bool p2AssembledCG( Context* ctx, P2Operator& op, Function& x, Function& 
    }
    auto& state = op.cgState[L];
    if ( !state.p )
-      state.alloc( ctx, size_t( kCgVec ) + 3 * size_t( pat->n ) );
+      state.alloc( ctx, size_t( kCgVec ) + 5 * size_t( pat->n ) );
    static std::once_flag once[64]; // per device
    std::call_once( once[ctx->device & 63], [] {
       HG_CHECK_HIP( hipFuncSetAttribute( reinterpret_cast< const void* >( &kP2AssembledCG ),
@@ -2152,7 +2194,6 @@ static bool p2AssembledCG( Context* ctx, P2Operator& op, Function& x, Function& 
           pat->n, pat->nslice, pat->pos.p, pat->flag.p, flag, pat->off.p, pat->rowOf.p, pat->col.p, pat->diag.p, val.p,
           jacobi, start, maxIter, kCgPerLaunch, relTol, absTol, (const double*) b.ptr( L ), (double*) x.ptr( L ), state.p );
       HG_CHECK_HIP( hipGetLastError() );
-      DeviceGateLock gate;
       HG_CHECK_HIP( hipMemcpyAsync( ctx->hostResult, state.p, sizeof( s ), hipMemcpyDeviceToHost, ctx->stream ) );
       HG_CHECK_HIP( hipStreamSynchronize( ctx->stream ) );
       std::copy( ctx->hostResult, ctx->hostResult + 4, s );

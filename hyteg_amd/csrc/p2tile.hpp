@@ -387,14 +387,21 @@ __device__ __forceinline__ void elementBoxPositions( const TileThread< R >& th, 
 // on one shared box cost about twice the whole kernel time of this scheme.
 constexpr int kWaveBoxes = kTileThreads / 64;
 
+// the wavefront's copy set to zero
+template < class R >
+__device__ __forceinline__ void waveBoxClear( R* boxes )
+{
+   using LdsR = volatile __attribute__( ( address_space( 3 ) ) ) R;
+   LdsR* b    = (LdsR*) ( boxes + kBox3 * __builtin_amdgcn_readfirstlane( int( threadIdx.x ) >> 6 ) );
+   for ( int p = int( threadIdx.x ) & 63; p < kBox3; p += 64 )
+      b[p] = R( 0 );
+}
 template < class R >
 __device__ __forceinline__ void waveBoxAccumulate( R* boxes, bool valid, const int pos[10], const R y[10] )
 {
-   using LdsR     = volatile __attribute__( ( address_space( 3 ) ) ) R;
-   const int lane = int( threadIdx.x ) & 63;
-   LdsR*     b    = (LdsR*) ( boxes + kBox3 * __builtin_amdgcn_readfirstlane( int( threadIdx.x ) >> 6 ) );
-   for ( int p = lane; p < kBox3; p += 64 )
-      b[p] = R( 0 );
+   using LdsR = volatile __attribute__( ( address_space( 3 ) ) ) R;
+   LdsR* b    = (LdsR*) ( boxes + kBox3 * __builtin_amdgcn_readfirstlane( int( threadIdx.x ) >> 6 ) );
+   waveBoxClear( boxes );
    if ( valid )
    {
 #pragma unroll

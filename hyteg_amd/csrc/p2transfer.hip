@@ -625,49 +625,143 @@ static void classPointList( Context* ctx, Lattice& l )
    l.classPoints.upload( ctx, pts );
 }
 
-// one wavefront per owned boundary DoF: the lanes split the stencil entries of
-// each incident cell (a macro-vertex DoF of the shell sees up to ~36 cells with
-// 125 entries each) and the wave sums its lanes in a fixed butterfly order
-constexpr int kBndWaves = 4;
-template < class T >
-__global__ __launch_bounds__( 64 * kBndWaves ) void kP2RestrictBnd( BndGeom gc, int64_t nbc, int64_t nc,
-                                                                   const uint8_t* __restrict__ bndFlag, int flag,
-                                                                   const double* __restrict__ clsInvN, int64_t scf,
-                                                                   int64_t wf, int64_t mmf, const T* __restrict__ fine,
-                                                                   T* __restrict__ coarse, int lv )
+// zero pattern of a cell point's barycentric weights (Storage::maskInvN)
+__device__ __forceinline__ int zeroMask( int32_t mm, int32_t x, int32_t y, int32_t z )
 {
-   using A         = typename Acc< T >::type;
+   return ( x + y + z == mm ? 1 : 0 ) | ( x == 0 ? 2 : 0 ) | ( y == 0 ? 4 : 0 ) | ( z == 0 ? 8 : 0 );
+}
+
+// one workgroup per owned macro-vertex or -edge DoF (and vector): its (incident cell,
+// stencil entry) pairs -- a macro-vertex of the shell sees up to ~36 cells with 125
+// entries each -- go round the threads, one cell to half a workgroup, and the sums are
+// added in a fixed order.  Bound by the chain of loads of a cell: 68 us a launch on
+// small levels with a wavefront taking the cells in turn.
+constexpr int kBndThreads = 256;
+template < class T >
+__global__ __launch_bounds__( kBndThreads ) void kP2RestrictBnd( BndGeom gc, int64_t nbc, int64_t nc,
+                                                                const uint8_t* __restrict__ bndFlag, int flag,
+                                                                const double* __restrict__ maskInvN, int64_t scf,
+                                                                int32_t wf, const T* __restrict__ fine,
+                                                                T* __restrict__ coarse, int lv )
+{
+   using A = typename Acc< T >::type;
+   static_assert( kRMax <= 128, "a cell's entries in half a workgroup" );
+   __shared__ A  red[kBndThreads / 64];
    fine += blockIdx.y;
    coarse += blockIdx.y;
-   const int     l = int( threadIdx.x ) & 63;
-   const int64_t b = int64_t( blockIdx.x ) * kBndWaves + ( int( threadIdx.x ) >> 6 );
+   const int64_t b = blockIdx.x;
    if ( b >= nbc || !( bndFlag[b] & flag ) )
-      return; // uniform over the wave
-   A s = A( 0 );
-   forEachIncident( gc, b, [&]( int64_t c, int64_t x, int64_t y, int64_t z, int ) {
-      const int q = int( x & 1 ) + 2 * int( y & 1 ) + 4 * int( z & 1 );
-      for ( int e = l; e < cRN[q]; e += 64 )
+      return; // uniform over the workgroup
+   int32_t e0, e1;
+   incidentRange( gc, b, e0, e1 );
+   const int32_t mmf  = wf - 1, e = int32_t( threadIdx.x ) & 127;
+   const int     half = __builtin_amdgcn_readfirstlane( int( threadIdx.x ) >> 7 );
+   A             s    = A( 0 );
+#pragma unroll 2
+   for ( int32_t i = e0 + half; i < e1; i += kBndThreads / 128 )
+   {
+      int64_t       x, y, z;
+      const int64_t c = incidentAt( gc, b, i, x, y, z );
+      const int     q = int( x & 1 ) + 2 * int( y & 1 ) + 4 * int( z & 1 );
+      if ( e < cRN[q] )
       {
-         const int64_t fx = 2 * x + cROff[q][e][0], fy = 2 * y + cROff[q][e][1], fz = 2 * z + cROff[q][e][2];
-         if ( fx < 0 || fy < 0 || fz < 0 || fx + fy + fz > mmf )
-            continue;
-         const int cl = pointClass( mmf, fx, fy, fz );
-         const A   w  = A( cRW[q][e] ) * ( cl < 0 ? A( 1 ) : A( clsInvN[14 * c + cl] ) );
-         s += w * toAcc( fine[( c * scf + tetIndex( wf, fx, fy, fz ) ) << lv] );
+         const int32_t fx = 2 * int32_t( x ) + cROff[q][e][0], fy = 2 * int32_t( y ) + cROff[q][e][1],
+                       fz = 2 * int32_t( z ) + cROff[q][e][2];
+         if ( fx >= 0 && fy >= 0 && fz >= 0 && fx + fy + fz <= mmf )
+            s += A( cRW[q][e] ) * A( maskInvN[16 * c + zeroMask( mmf, fx, fy, fz )] ) *
+                 toAcc( fine[( c * scf + tetRowStart( wf, fy, fz ) + fx ) << lv] );
       }
-   } );
+   }
 #pragma unroll
    for ( int o = 32; o > 0; o >>= 1 )
       s += __shfl_xor( s, o, 64 );
-   if ( l == 0 )
-      coarse[( nc * gc.sc + b ) << lv] = fromAcc< T >( s );
+   if ( ( threadIdx.x & 63 ) == 0 )
+      red[threadIdx.x >> 6] = s;
+   __syncthreads();
+   if ( threadIdx.x == 0 )
+      coarse[( nc * gc.sc + b ) << lv] = fromAcc< T >( ( red[0] + red[1] ) + ( red[2] + red[3] ) );
 }
 
-// owned face DoFs (two incident cells each): one thread per DoF
+// owned face DoFs (two incident cells each): a wavefront takes 64 points of one face
+// with one parity class (facePoints), so that the cell, the orientation and the stencil
+// -- the row groups of the cell kernel -- are uniform over it; the entries of a row are
+// gathered before they are summed.  Bound by the gathers of the two cells' fine rows.
+// Shell level 5, FP64: 1.22 ms with a thread taking its DoF's entries one by one, 64-bit
+// indices and classes formed for each.
 template < class T >
-__global__ void kP2RestrictBndFace( BndGeom gc, int64_t nbc, int64_t nc, const uint8_t* __restrict__ bndFlag, int flag,
-                                    const double* __restrict__ clsInvN, int64_t scf, int64_t wf, int64_t mmf,
-                                    const T* __restrict__ fine, T* __restrict__ coarse, int lv )
+__global__ __launch_bounds__( 256 ) void kP2RestrictBndFace( BndGeom gc, const uint32_t* __restrict__ pts,
+                                                             uint32_t wavesPerFace, uint32_t nfaces, int64_t nc,
+                                                             const uint8_t* __restrict__ bndFlag, int flag,
+                                                             const double* __restrict__ maskInvN, int64_t scf, int32_t wf,
+                                                             const T* __restrict__ fine, T* __restrict__ coarse, int lv )
+{
+   using A = typename Acc< T >::type;
+   __shared__ int32_t sliceStart[kMaxSlices];
+   for ( int32_t z = threadIdx.x; z < wf; z += 256 )
+      sliceStart[z] = int32_t( tet( wf ) - tet( wf - z ) );
+   __syncthreads();
+   const uint32_t wv = uint32_t( __builtin_amdgcn_readfirstlane( int( blockIdx.x * 4 + ( threadIdx.x >> 6 ) ) ) );
+   const uint32_t f  = wv / wavesPerFace;
+   if ( f >= nfaces )
+      return;
+   const uint32_t p  = pts[( wv - f * wavesPerFace ) * 64 + ( threadIdx.x & 63 )];
+   const int32_t  pa = int32_t( p & 0xFFFFu ), pb = int32_t( p >> 16 ), mmc = int32_t( gc.mm );
+   if ( p == 0xFFFFFFFFu )
+      return;
+   const int64_t b = gc.foff + int64_t( f ) * gc.fin + triIndex( mmc - 2, pa - 1, pb - 1 );
+   if ( !( bndFlag[b] & flag ) )
+      return;
+   fine += blockIdx.y;
+   coarse += blockIdx.y;
+   const int32_t mmf = wf - 1;
+   A             s   = A( 0 );
+   for ( int32_t i = gc.fptr[f]; i < gc.fptr[f + 1]; ++i )
+   {
+      const int64_t   c  = gc.fcells[2 * i];
+      const CellMeta& m  = gc.meta[c];
+      const int8_t*   pm = m.fperm[gc.fcells[2 * i + 1]];
+      const int32_t   t0 = mmc - pa - pb;
+      auto weight = [&]( int v ) { return pm[0] == v ? t0 : ( pm[1] == v ? pa : ( pm[2] == v ? pb : 0 ) ); };
+      const int32_t x = weight( 1 ), y = weight( 2 ), z = weight( 3 );
+      const int     q = __builtin_amdgcn_readfirstlane( ( x & 1 ) + 2 * ( y & 1 ) + 4 * ( z & 1 ) );
+      const double* wi = maskInvN + 16 * c;
+      const T*      fc = fine + ( ( c * scf ) << lv );
+      for ( int g = 0; g < cRGN[q]; ++g )
+      {
+         const RowGroup rg = cRG[q][g];
+         const int32_t  fy = 2 * y + rg.oy, fz = 2 * z + rg.oz;
+         if ( fy < 0 || fz < 0 || fy + fz > mmf )
+            continue;
+         const int32_t rs  = sliceStart[fz] + fy * ( wf - fz ) - fy * ( fy - 1 ) / 2;
+         const int32_t lim = mmf - fy - fz, mk = ( fy == 0 ? 4 : 0 ) | ( fz == 0 ? 8 : 0 );
+         A             buf[7], wgt[7];
+#pragma unroll
+         for ( int j = 0; j < 7; ++j )
+         {
+            buf[j] = wgt[j] = A( 0 );
+            if ( j < rg.count )
+            {
+               const int32_t fx = 2 * x + cRGX[q][rg.first + j];
+               if ( fx >= 0 && fx <= lim )
+               {
+                  buf[j] = toAcc( fc[int64_t( rs + fx ) << lv] );
+                  wgt[j] = A( wi[mk | ( fx == 0 ? 2 : 0 ) | ( fx == lim ? 1 : 0 )] );
+               }
+            }
+         }
+#pragma unroll
+         for ( int j = 0; j < 7; ++j )
+            if ( j < rg.count )
+               s += A( cRGW[q][rg.first + j] ) * wgt[j] * buf[j];
+      }
+   }
+   coarse[( nc * gc.sc + b ) << lv] = fromAcc< T >( s );
+}
+// the same, a thread per DoF, for fine lattices wider than kMaxSlices
+template < class T >
+__global__ void kP2RestrictBndFaceGeneral( BndGeom gc, int64_t nbc, int64_t nc, const uint8_t* __restrict__ bndFlag,
+                                           int flag, const double* __restrict__ clsInvN, int64_t scf, int64_t wf,
+                                           int64_t mmf, const T* __restrict__ fine, T* __restrict__ coarse, int lv )
 {
    using A         = typename Acc< T >::type;
    fine += blockIdx.y;
@@ -691,6 +785,24 @@ __global__ void kP2RestrictBndFace( BndGeom gc, int64_t nbc, int64_t nc, const u
    coarse[( nc * gc.sc + b ) << lv] = fromAcc< T >( s );
 }
 
+// the face point list of a coarse lattice (built on first use)
+static void facePointList( Context* ctx, Lattice& l )
+{
+   if ( l.facePoints.p || l.num.fin == 0 || 2 * l.mm + 1 > kMaxSlices )
+      return;
+   std::vector< uint32_t > pts;
+   for ( int q = 0; q < 4; ++q )
+   {
+      for ( int64_t b = 1; b <= l.mm - 2; ++b )
+         for ( int64_t a = 1; a + b <= l.mm - 1; ++a )
+            if ( ( a & 1 ) + 2 * ( b & 1 ) == q )
+               pts.push_back( uint32_t( a ) | ( uint32_t( b ) << 16 ) );
+      while ( pts.size() % 64 )
+         pts.push_back( 0xFFFFFFFFu );
+   }
+   l.facePoints.upload( ctx, pts );
+}
+
 static constexpr int kRowBlockT = 64;
 
 void p2Restrict( Context* ctx, Function& f, int fineL, int flag )
@@ -702,6 +814,7 @@ void p2Restrict( Context* ctx, Function& f, int fineL, int flag )
    Lattice& lf = st.lattice( ctx, fineL + 1 );
    Lattice& lc = st.lattice( ctx, fineL );
    classPointList( ctx, lc );
+   facePointList( ctx, lc );
    void*    fp = f.ptr( fineL );
    void*    cp = f.ptr( fineL - 1 );
    const int      lv = f.lv;
@@ -736,10 +849,18 @@ void p2Restrict( Context* ctx, Function& f, int fineL, int flag )
          const BndGeom gc = BndGeom::of( st, lc );
          const int64_t nve = std::min( gc.foff, lc.nb );
          if ( nve > 0 )
-            kP2RestrictBnd< T ><<< dim3( gridFor( nve, kBndWaves ), nv ), 64 * kBndWaves, 0, ctx->stream >>>(
-                gc, nve, lc.nc, lc.bndFlag.p, flag, st.clsInvN.p, lf.sc, lf.w, lf.mm, (const T*) fp, (T*) cp, lv );
-         if ( lc.nb > nve )
-            kP2RestrictBndFace< T ><<< dim3( gridFor( lc.nb - nve ), nv ), kBlock, 0, ctx->stream >>>(
+            kP2RestrictBnd< T ><<< dim3( gridFor( nve, 1 ), nv ), kBndThreads, 0, ctx->stream >>>(
+                gc, nve, lc.nc, lc.bndFlag.p, flag, st.maskInvN.p, lf.sc, int32_t( lf.w ), (const T*) fp, (T*) cp, lv );
+         HG_CHECK_HIP( hipGetLastError() );
+         if ( lc.nb > nve && lc.facePoints.p )
+         {
+            const int64_t wpf = int64_t( lc.facePoints.n ) / 64;
+            kP2RestrictBndFace< T ><<< dim3( gridFor( wpf * st.topo.nf, 4 ), nv ), 256, 0, ctx->stream >>>(
+                gc, lc.facePoints.p, uint32_t( wpf ), uint32_t( st.topo.nf ), lc.nc, lc.bndFlag.p, flag, st.maskInvN.p,
+                lf.sc, int32_t( lf.w ), (const T*) fp, (T*) cp, lv );
+         }
+         else if ( lc.nb > nve )
+            kP2RestrictBndFaceGeneral< T ><<< dim3( gridFor( lc.nb - nve ), nv ), kBlock, 0, ctx->stream >>>(
                 gc, lc.nb, lc.nc, lc.bndFlag.p, flag, st.clsInvN.p, lf.sc, lf.w, lf.mm, (const T*) fp, (T*) cp, lv );
          HG_CHECK_HIP( hipGetLastError() );
       }

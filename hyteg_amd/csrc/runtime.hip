@@ -113,6 +113,19 @@ void Storage::init( Context* ctx )
          inv[14 * c + 10 + k] = 1.0 / t.vnc[t.cv[c][k]];
    }
    clsInvN.upload( ctx, inv );
+   std::vector< double > byMask( 16 * size_t( t.nc ), 1.0 );
+   for ( int c = 0; c < t.nc; ++c )
+   {
+      const int edgeKeep[6] = { 3, 5, 6, 9, 10, 12 };
+      for ( int k = 0; k < 4; ++k )
+      {
+         byMask[16 * size_t( c ) + ( size_t( 1 ) << ( 3 - k ) )]        = inv[14 * size_t( c ) + k];
+         byMask[16 * size_t( c ) + ( 15 ^ ( size_t( 1 ) << k ) )] = inv[14 * size_t( c ) + 10 + k];
+      }
+      for ( int k = 0; k < 6; ++k )
+         byMask[16 * size_t( c ) + size_t( 15 ^ edgeKeep[k] )] = inv[14 * size_t( c ) + 4 + k];
+   }
+   maskInvN.upload( ctx, byMask );
    csr( t.nf, [&]( int c, int k ) { return t.cf[c][k]; }, 4, faceCellPtr, faceCells );
    csr( t.ne, [&]( int c, int k ) { return t.ce[c][k]; }, 6, edgeCellPtr, edgeCells );
    csr( t.nv, [&]( int c, int k ) { return t.cv[c][k]; }, 4, vertCellPtr, vertCells );

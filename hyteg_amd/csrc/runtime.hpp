@@ -124,6 +124,10 @@ struct Lattice
    // (P2 prolongation into this lattice).
    DevBuf< uint32_t > prolongChunks;
 
+   // face-interior points (a | b << 16) grouped by (a mod 2, b mod 2), each group padded
+   // to whole wavefronts (0xFFFFFFFF).  Built on first use (P2 restriction).
+   DevBuf< uint32_t > facePoints;
+
    // tile lists of the P2 tile kernels on this lattice (all tiles, interior
    // tiles, last-layer tiles), built on first use
    DevBuf< uint64_t > tileLists[3];
@@ -163,6 +167,9 @@ struct Storage
    // 1 / (number of cells) of each cell's local faces (0..3), edges (4..9) and
    // vertices (10..13): nc*14
    DevBuf< double >                             clsInvN;
+   // the same by the zero pattern of a cell point's barycentric weights (bit 0:
+   // x + y + z = mm, 1: x = 0, 2: y = 0, 3: z = 0; no bit: 1): nc*16
+   DevBuf< double >                             maskInvN;
    // cells incident to each face / edge / vertex: CSR of (cell, local index)
    DevBuf< int32_t > faceCellPtr, faceCells, edgeCellPtr, edgeCells, vertCellPtr, vertCells;
    // the same incidences as (cell, orientation): two entries a face (cell -1: none),
