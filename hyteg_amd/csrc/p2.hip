@@ -189,7 +189,7 @@ struct P2Operator : OperatorBase
    std::map< int, int64_t >               tableStride; // by P2 level
    std::map< int, DevBuf< double > >      invScratch;  // one slot's diagonal, by P2 level
    DevBuf< int32_t >                      slotOn;      // 1: the apply computes the slot, 0: its result is 0
-   // assembled form of small levels (p2AssembledCG): weights of the pattern's entries
+   // element matrices of small levels (p2AssembledCG)
    std::map< int, DevBuf< double > >      assembled;
    std::map< int, DevBuf< double > >      cgState; // scratch vectors and scalars of the solve
 };
@@ -1803,38 +1803,35 @@ __global__ void kChebyshevStep( int64_t ncell, int64_t nb, const uint8_t* __rest
 // The coarse solve of the P2 V-cycles runs some ninety CG iterations on a few thousand
 // DoFs.  Iteration by iteration it is nine launches of latency-bound kernels and a read
 // back (70 us on the shell's level 0: halo pull, one wavefront a macro-cell, additive
-// push, two updates, three dot products); assembled, the matrix is about 1 MB, which one
-// workgroup reads from L2 in about 10 us, and a whole solve is one launch.  The iteration, its
-// scalars and its stopping test are those of CGSolver.
-constexpr int     kCgThreads   = 1024;
-constexpr int     kCgMaxDofs   = 16384; // p in LDS; the matrix of a larger level costs more than the launches
-constexpr int     kCgMaxLevel  = 2;
-constexpr int     kCgPerLaunch = 1024;  // iterations a launch (bounds its time, at most about 50 ms)
+// push, two updates, three dot products); with the element matrices kept (symmetric,
+// 55 values a micro-cell, 0.8 MB) one workgroup streams them from L2 and gathers and adds
+// in LDS, and a whole solve is one launch.  Bound by the matrix stream of one CU.  (With
+// assembled rows, 1 MB and one LDS gather an entry, an iteration took 24 us: the gathers'
+// bank conflicts.)  The iteration, its scalars and its stopping test are those of CGSolver.
+constexpr int kCgThreads   = 1024;
+constexpr int kCgMaxDofs   = 8192; // p and A p in LDS
+constexpr int kCgMaxLevel  = 2;
+constexpr int kCgPerLaunch = 1024; // iterations a launch (bounds its time)
+constexpr int kCgMatrix    = 55;   // upper triangle of a 10 x 10 matrix
 enum CgState
 {
    kCgRz   = 0, // r . z
    kCgR0   = 1, // sqrt(r . r) of the start
    kCgIts  = 2, // iterations done
    kCgDone = 3,
-   kCgVec  = 8, // then r, A p, p, x, the inverse diagonal (n values each)
+   kCgVec  = 8, // then r, p, x, the inverse diagonal (n values each)
 };
 
 struct P2Pattern : OperatorBase
 {
-   int32_t           n = 0, nslice = 0;
-   int64_t           nent = 0;
-   DevBuf< int64_t > pos;     // storage position of each DoF
-   DevBuf< uint8_t > flag;    // its type
-   DevBuf< int64_t > off;     // slices of 64 rows: entry offsets, column-major
-   DevBuf< int32_t > rowOf;   // DoF of each row slot (-1: none), longest rows first
-   DevBuf< uint16_t > col;    // columns
-   DevBuf< int32_t > diag;    // entry of each DoF's diagonal
-   DevBuf< int32_t > elem;    // micro-cells: cell, type | anchor << 3
-   DevBuf< int32_t > entry;   // their 100 entries
-   int64_t           nelem = 0;
+   int32_t            n = 0, nelem = 0, stride = 0; // DoFs, micro-cells, and those padded to wavefronts
+   DevBuf< int64_t >  pos;  // storage position of each DoF
+   DevBuf< uint8_t >  flag; // its type
+   DevBuf< int32_t >  elem; // micro-cells: cell, type | anchor << 3
+   DevBuf< uint16_t > id;   // their DoFs: id[i * stride + e], i < 10
 };
 
-// null where the level is not solved in assembled form
+// null where the level is not solved this way
 static const P2Pattern* p2Pattern( Context* ctx, Storage& st, int L )
 {
    Lattice& lat = st.lattice( ctx, L + 1 );
@@ -1854,7 +1851,7 @@ static const P2Pattern* p2Pattern( Context* ctx, Storage& st, int L )
       pos[i]  = lat.nc * lat.sc + i; // owned; the cell interiors follow below
       flag[i] = i < lat.nb ? lat.hBndFlag[i] : uint8_t( kInner );
    }
-   std::vector< int32_t >                elem;
+   std::vector< int32_t >                    elem;
    std::vector< std::array< int32_t, 10 > > ids;
    const int edges[6][2] = { { 0, 1 }, { 0, 2 }, { 0, 3 }, { 1, 2 }, { 1, 3 }, { 2, 3 } };
    for ( int c = 0; c < t.nc; ++c )
@@ -1883,80 +1880,30 @@ static const P2Pattern* p2Pattern( Context* ctx, Storage& st, int L )
             elem.push_back( ty | ( a << 3 ) );
             ids.push_back( id );
          }
-   std::vector< std::vector< int32_t > > cols( n );
-   for ( const auto& id : ids )
-      for ( int i = 0; i < 10; ++i )
-         cols[id[size_t( i )]].insert( cols[id[size_t( i )]].end(), id.begin(), id.end() );
-   std::vector< int32_t > order( n );
-   for ( int32_t i = 0; i < n; ++i )
-   {
-      std::sort( cols[i].begin(), cols[i].end() );
-      cols[i].erase( std::unique( cols[i].begin(), cols[i].end() ), cols[i].end() );
-      order[i] = i;
-   }
-   std::stable_sort( order.begin(), order.end(),
-                     [&]( int32_t a, int32_t b ) { return cols[a].size() > cols[b].size(); } );
-   order.resize( size_t( n + 63 ) / 64 * 64, -1 );
-   const int32_t          nsl = int32_t( order.size() / 64 );
-   std::vector< int64_t > off( nsl + 1, 0 );
-   std::vector< int32_t > first( n ); // entry of a row's first column
-   for ( int32_t s = 0; s < nsl; ++s )
-   {
-      // the first row of a slice is its longest; widths in steps of 8
-      const size_t w = ( cols[order[64 * size_t( s )]].size() + 7 ) / 8 * 8;
-      off[s + 1]     = off[s] + int64_t( 64 * w );
-   }
-   std::vector< uint16_t > col( size_t( off[nsl] ), 0 );
-   std::vector< int32_t >  diag( n );
-   for ( size_t i = 0; i < order.size(); ++i )
-   {
-      if ( order[i] < 0 )
-         continue;
-      const auto&   cc = cols[order[i]];
-      const int64_t e0 = off[i / 64] + int64_t( i % 64 );
-      first[order[i]]  = int32_t( e0 );
-      for ( size_t j = 0; j < cc.size(); ++j )
-      {
-         col[size_t( e0 + 64 * int64_t( j ) )] = uint16_t( cc[j] );
-         if ( cc[j] == order[i] )
-            diag[order[i]] = int32_t( e0 + 64 * int64_t( j ) );
-      }
-   }
-   std::vector< int32_t > entry;
-   entry.reserve( 100 * ids.size() );
-   for ( const auto& id : ids )
-      for ( int i = 0; i < 10; ++i )
-         for ( int j = 0; j < 10; ++j )
-         {
-            const auto& cc = cols[id[size_t( i )]];
-            const auto  at = std::lower_bound( cc.begin(), cc.end(), id[size_t( j )] ) - cc.begin();
-            entry.push_back( first[id[size_t( i )]] + 64 * int32_t( at ) );
-         }
    pat->n      = n;
-   pat->nslice = nsl;
-   pat->nent   = off[nsl];
-   pat->nelem  = int64_t( ids.size() );
+   pat->nelem  = int32_t( ids.size() );
+   pat->stride = ( pat->nelem + 63 ) / 64 * 64;
+   std::vector< uint16_t > id( 10 * size_t( pat->stride ), 0 );
+   for ( size_t e = 0; e < ids.size(); ++e )
+      for ( size_t i = 0; i < 10; ++i )
+         id[i * size_t( pat->stride ) + e] = uint16_t( ids[e][i] );
    pat->pos.upload( ctx, pos );
    pat->flag.upload( ctx, flag );
-   pat->off.upload( ctx, off );
-   pat->rowOf.upload( ctx, order );
-   pat->col.upload( ctx, col );
-   pat->diag.upload( ctx, diag );
    pat->elem.upload( ctx, elem );
-   pat->entry.upload( ctx, entry );
+   pat->id.upload( ctx, id );
    return static_cast< const P2Pattern* >( ( st.p2Patterns[L] = std::move( pat ) ).get() );
 }
 
-// element matrices into the pattern's entries: one thread a micro-cell and column
-__global__ void kP2Assemble( const P2ActGeomT< double >* __restrict__ geom, const P2CellGeom* __restrict__ geom64,
-                             const KParams* __restrict__ kp, int64_t mm, int64_t nelem, const int32_t* __restrict__ elem,
-                             const int32_t* __restrict__ entry, double* __restrict__ val )
+// element matrices mat[k * stride + e], k the upper triangle row by row: one thread a
+// micro-cell and column
+__global__ void kP2ElementMatrices( const P2ActGeomT< double >* __restrict__ geom, const P2CellGeom* __restrict__ geom64,
+                                    const KParams* __restrict__ kp, int64_t mm, int32_t nelem, int32_t stride,
+                                    const int32_t* __restrict__ elem, double* __restrict__ mat )
 {
-   const int64_t i = int64_t( blockIdx.x ) * blockDim.x + threadIdx.x;
-   if ( i >= 10 * nelem )
+   const int32_t i = int32_t( blockIdx.x * blockDim.x + threadIdx.x );
+   const int32_t j = i / stride, e = i - j * stride;
+   if ( j >= 10 || e >= nelem )
       return;
-   const int64_t e = i / 10;
-   const int     j = int( i - 10 * e );
    const int32_t c = elem[2 * e], t = elem[2 * e + 1] & 7, a = elem[2 * e + 1] >> 3;
    const TileCoord             tc{ c, 0, 0, 0 };
    const P2ActGeomT< double >& g = geom[c];
@@ -1970,10 +1917,11 @@ __global__ void kP2Assemble( const P2ActGeomT< double >* __restrict__ geom, cons
    } );
 #pragma unroll
    for ( int k = 0; k < 10; ++k )
-      atomicAdd( &val[entry[100 * e + 10 * k + j]], y[k] );
+      if ( k <= j )
+         mat[( k * 10 - k * ( k - 1 ) / 2 + ( j - k ) ) * stride + e] = y[k];
 }
 
-// sums of up to two values over the workgroup, in every thread
+// sums of two values over the workgroup, in every thread
 __device__ __forceinline__ void cgSum( double& a, double& b, double ( *red )[2] )
 {
 #pragma unroll
@@ -1998,94 +1946,86 @@ __device__ __forceinline__ void cgSum( double& a, double& b, double ( *red )[2] 
    }
 }
 
-__global__ __launch_bounds__( kCgThreads ) void kP2AssembledCG( int32_t n, int32_t nslice, const int64_t* __restrict__ pos,
+__global__ __launch_bounds__( kCgThreads ) void kP2AssembledCG( int32_t n, int32_t nelem, int32_t stride,
+                                                               const int64_t* __restrict__ pos,
                                                                const uint8_t* __restrict__ dofFlag, int flag,
-                                                               const int64_t* __restrict__ off,
-                                                               const int32_t* __restrict__ rowOf,
-                                                               const uint16_t* __restrict__ col,
-                                                               const int32_t* __restrict__ diag,
-                                                               const double* __restrict__ val, int jacobi, int start,
+                                                               const uint16_t* __restrict__ id,
+                                                               const double* __restrict__ mat, int jacobi, int start,
                                                                int maxIter, int perLaunch, double relTol, double absTol,
                                                                const double* __restrict__ b, double* __restrict__ x,
                                                                double* __restrict__ state )
 {
-   extern __shared__ double sp[]; // p
+   extern __shared__ double sp[]; // p, then A p
    __shared__ double        red[kCgThreads / 64][2];
-   __shared__ int32_t       so[kCgMaxDofs / 64 + 1];
+   double* const            sa  = sp + n;
    double* const            r   = state + kCgVec;
-   double* const            ap  = r + n;
-   double* const            ps  = ap + n;
+   double* const            ps  = r + n;
    double* const            xs  = ps + n;
    double* const            inv = xs + n; // 1 / diagonal (1 without the preconditioner), 0 where x is fixed
-   const int                wave = int( threadIdx.x ) >> 6, lane = int( threadIdx.x ) & 63;
-   for ( int32_t s = threadIdx.x; s <= nslice; s += kCgThreads )
-      so[s] = int32_t( off[s] );
-   // ap = A p on the rows: wavefronts take slices in turn, a chunk of eight entries in
-   // flight while the one before it is summed
+   auto clear = [&]() {
+      for ( int32_t i = threadIdx.x; i < n; i += kCgThreads )
+         sa[i] = 0.0;
+      __syncthreads();
+   };
+   // sa += A p (cleared before)
    auto product = [&]() {
-      struct Chunk
+      for ( int32_t e = threadIdx.x; e < nelem; e += kCgThreads )
       {
-         uint16_t c[8];
-         double   v[8];
-      };
-      auto load = [&]( int32_t e ) {
-         Chunk k;
+         int32_t d[10];
+         double  u[10], y[10];
 #pragma unroll
-         for ( int u = 0; u < 8; ++u )
+         for ( int i = 0; i < 10; ++i )
+            d[i] = id[i * stride + e];
+#pragma unroll
+         for ( int i = 0; i < 10; ++i )
          {
-            k.c[u] = col[e + 64 * u];
-            k.v[u] = val[e + 64 * u];
+            u[i] = sp[d[i]];
+            y[i] = 0.0;
          }
-         return k;
-      };
-      int32_t s = wave;
-      if ( s < nslice )
-      {
-         int32_t e = so[s];
-         Chunk   next = load( e + lane );
-         int32_t row  = rowOf[64 * s + lane];
-         double  acc  = 0.0;
-         while ( s < nslice )
-         {
-            const Chunk cur  = next;
-            const int32_t rn = row;
-            const bool  last = e + 512 >= so[s + 1];
-            const int32_t sn = last ? s + kCgThreads / 64 : s;
-            const int32_t en = last ? so[min( sn, nslice - 1 )] : e + 512;
-            next = load( en + lane );
-            if ( last )
-               row = rowOf[64 * min( sn, nslice - 1 ) + lane];
+         int k = 0;
 #pragma unroll
-            for ( int u = 0; u < 8; ++u )
-               acc += cur.v[u] * sp[cur.c[u]];
-            if ( last )
+         for ( int i = 0; i < 10; ++i )
+#pragma unroll
+            for ( int j = i; j < 10; ++j, ++k )
             {
-               if ( rn >= 0 )
-                  ap[rn] = acc;
-               acc = 0.0;
+               const double m = mat[k * stride + e];
+               y[i] += m * u[j];
+               if ( j > i )
+                  y[j] += m * u[i];
             }
-            s = sn;
-            e = en;
-         }
+#pragma unroll
+         for ( int i = 0; i < 10; ++i )
+            atomicAdd( &sa[d[i]], y[i] );
       }
       __syncthreads();
    };
    double rz, r0, its = 0.0;
    if ( start )
    {
+      // the diagonal into p's place, then x
       for ( int32_t i = threadIdx.x; i < n; i += kCgThreads )
-         sp[i] = x[pos[i]];
+         sp[i] = 0.0;
+      clear();
+      for ( int32_t e = threadIdx.x; e < nelem; e += kCgThreads )
+#pragma unroll
+         for ( int i = 0; i < 10; ++i )
+            atomicAdd( &sp[id[i * stride + e]], mat[( i * 10 - i * ( i - 1 ) / 2 ) * stride + e] );
+      __syncthreads();
+      for ( int32_t i = threadIdx.x; i < n; i += kCgThreads )
+      {
+         inv[i] = ( dofFlag[i] & flag ) ? ( jacobi ? 1.0 / sp[i] : 1.0 ) : 0.0;
+         sp[i]  = x[pos[i]];
+      }
       __syncthreads();
       product();
       rz = r0 = 0.0;
       for ( int32_t i = threadIdx.x; i < n; i += kCgThreads )
       {
-         const double d  = ( dofFlag[i] & flag ) ? ( jacobi ? 1.0 / val[diag[i]] : 1.0 ) : 0.0;
-         const double ri = d != 0.0 ? b[pos[i]] - ap[i] : 0.0, zi = d * ri;
-         inv[i] = d;
-         xs[i]  = sp[i];
-         r[i]   = ri;
-         sp[i]  = zi;
+         const double d  = inv[i];
+         const double ri = d != 0.0 ? b[pos[i]] - sa[i] : 0.0, zi = d * ri;
+         xs[i] = sp[i];
+         r[i]  = ri;
+         sp[i] = zi;
          rz += ri * zi;
          r0 += ri * ri;
       }
@@ -2111,10 +2051,11 @@ __global__ __launch_bounds__( kCgThreads ) void kP2AssembledCG( int32_t n, int32
    __syncthreads();
    for ( int k = 0;; ++k )
    {
+      clear();
       product();
       double pap = 0.0, rr = 0.0, rzn = 0.0, none = 0.0;
       for ( int32_t i = threadIdx.x; i < n; i += kCgThreads )
-         pap += inv[i] != 0.0 ? sp[i] * ap[i] : 0.0;
+         pap += inv[i] != 0.0 ? sp[i] * sa[i] : 0.0;
       cgSum( pap, none, red );
       const double alpha = rz / pap;
       for ( int32_t i = threadIdx.x; i < n; i += kCgThreads )
@@ -2123,7 +2064,7 @@ __global__ __launch_bounds__( kCgThreads ) void kP2AssembledCG( int32_t n, int32
          if ( d != 0.0 )
          {
             xs[i] += alpha * sp[i];
-            const double ri = r[i] - alpha * ap[i];
+            const double ri = r[i] - alpha * sa[i];
             r[i]            = ri;
             rr += ri * ri;
             rzn += ri * ( d * ri );
@@ -2155,7 +2096,6 @@ __global__ __launch_bounds__( kCgThreads ) void kP2AssembledCG( int32_t n, int32
          return;
       }
       its += 1.0;
-      __syncthreads();
    }
 }
 
@@ -2170,29 +2110,29 @@ static bool p2AssembledCG( Context* ctx, P2Operator& op, Function& x, Function& 
    const P2Pattern* pat = p2Pattern( ctx, *op.st, L );
    if ( !pat || maxIter < 1 )
       return false;
-   auto& val = op.assembled[L];
-   if ( !val.p )
+   auto& mat = op.assembled[L];
+   if ( !mat.p )
    {
-      val.alloc( ctx, size_t( pat->nent ) );
-      kP2Assemble<<< gridFor( 10 * pat->nelem, 64 ), 64, 0, ctx->stream >>>( op.ageom.at( L ).p, op.tgeom.at( L ).p,
-                                                                            op.kpar.p, int64_t( 1 ) << L, pat->nelem,
-                                                                            pat->elem.p, pat->entry.p, val.p );
+      mat.alloc( ctx, size_t( kCgMatrix ) * size_t( pat->stride ) );
+      kP2ElementMatrices<<< gridFor( 10 * int64_t( pat->stride ), 64 ), 64, 0, ctx->stream >>>(
+          op.ageom.at( L ).p, op.tgeom.at( L ).p, op.kpar.p, int64_t( 1 ) << L, pat->nelem, pat->stride, pat->elem.p, mat.p );
       HG_CHECK_HIP( hipGetLastError() );
    }
    auto& state = op.cgState[L];
    if ( !state.p )
-      state.alloc( ctx, size_t( kCgVec ) + 5 * size_t( pat->n ) );
+      state.alloc( ctx, size_t( kCgVec ) + 4 * size_t( pat->n ) );
    static std::once_flag once[64]; // per device
    std::call_once( once[ctx->device & 63], [] {
       HG_CHECK_HIP( hipFuncSetAttribute( reinterpret_cast< const void* >( &kP2AssembledCG ),
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, int( kCgMaxDofs * sizeof( double ) ) ) );
+                                         hipFuncAttributeMaxDynamicSharedMemorySize,
+                                         int( 2 * kCgMaxDofs * sizeof( double ) ) ) );
    } );
    double s[4] = { 0, 0, 0, 0 };
    for ( int start = 1; s[kCgDone] == 0.0; start = 0 )
    {
-      kP2AssembledCG<<< 1, kCgThreads, size_t( pat->n ) * sizeof( double ), ctx->stream >>>(
-          pat->n, pat->nslice, pat->pos.p, pat->flag.p, flag, pat->off.p, pat->rowOf.p, pat->col.p, pat->diag.p, val.p,
-          jacobi, start, maxIter, kCgPerLaunch, relTol, absTol, (const double*) b.ptr( L ), (double*) x.ptr( L ), state.p );
+      kP2AssembledCG<<< 1, kCgThreads, 2 * size_t( pat->n ) * sizeof( double ), ctx->stream >>>(
+          pat->n, pat->nelem, pat->stride, pat->pos.p, pat->flag.p, flag, pat->id.p, mat.p, jacobi, start, maxIter,
+          kCgPerLaunch, relTol, absTol, (const double*) b.ptr( L ), (double*) x.ptr( L ), state.p );
       HG_CHECK_HIP( hipGetLastError() );
       HG_CHECK_HIP( hipMemcpyAsync( ctx->hostResult, state.p, sizeof( s ), hipMemcpyDeviceToHost, ctx->stream ) );
       HG_CHECK_HIP( hipStreamSynchronize( ctx->stream ) );

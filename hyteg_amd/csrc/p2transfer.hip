@@ -533,6 +533,7 @@ struct ClassWaves
    int32_t w[9];
 };
 constexpr int kRestrictBlock = 256;
+constexpr int kRowsAhead     = 3;
 constexpr int kMaxSlices     = 1025;
 template < class T >
 __global__ __launch_bounds__( kRestrictBlock ) void kP2RestrictCellList( const uint32_t* __restrict__ pts, ClassWaves cw,
@@ -564,30 +565,41 @@ __global__ __launch_bounds__( kRestrictBlock ) void kP2RestrictCellList( const u
    const int32_t mmf = wf - 1;
    const T*      f   = fine + blockIdx.y + ( ( c * scf ) << lv );
    A             v   = A( 0 );
-   for ( int g = 0; g < cRGN[q]; ++g )
+   // kRowsAhead fine rows' entries in flight together
+   const int ng = cRGN[q];
+   for ( int g0 = 0; g0 < ng; g0 += kRowsAhead )
    {
-      const RowGroup rg = cRG[q][g];
-      const int32_t  fy = 2 * y + rg.oy, fz = 2 * z + rg.oz;
-      if ( fy < 0 || fz < 0 || fy + fz > mmf )
-         continue;
-      const int32_t rs  = sliceStart[fz] + fy * ( wf - fz ) - fy * ( fy - 1 ) / 2;
-      const int32_t lim = mmf - fy - fz;
-      A             buf[7];
+      A buf[kRowsAhead][7];
 #pragma unroll
-      for ( int j = 0; j < 7; ++j )
+      for ( int i = 0; i < kRowsAhead; ++i )
       {
-         buf[j] = A( 0 );
-         if ( j < rg.count )
+         const RowGroup rg = cRG[q][min( g0 + i, ng - 1 )];
+         const int32_t  fy = 2 * y + rg.oy, fz = 2 * z + rg.oz;
+         const bool     in = g0 + i < ng && fy >= 0 && fz >= 0 && fy + fz <= mmf;
+         const int32_t  rs = in ? sliceStart[fz] + fy * ( wf - fz ) - fy * ( fy - 1 ) / 2 : 0;
+         const int32_t  lim = in ? mmf - fy - fz : -1;
+#pragma unroll
+         for ( int j = 0; j < 7; ++j )
          {
-            const int32_t fx = 2 * x + cRGX[q][rg.first + j];
-            if ( fx >= 0 && fx <= lim )
-               buf[j] = toAcc( f[int64_t( rs + fx ) << lv] );
+            buf[i][j] = A( 0 );
+            if ( j < rg.count )
+            {
+               const int32_t fx = 2 * x + cRGX[q][rg.first + j];
+               if ( fx >= 0 && fx <= lim )
+                  buf[i][j] = toAcc( f[int64_t( rs + fx ) << lv] );
+            }
          }
       }
 #pragma unroll
-      for ( int j = 0; j < 7; ++j )
-         if ( j < rg.count )
-            v += A( cRGW[q][rg.first + j] ) * buf[j];
+      for ( int i = 0; i < kRowsAhead; ++i )
+         if ( g0 + i < ng )
+         {
+            const RowGroup rg = cRG[q][g0 + i];
+#pragma unroll
+            for ( int j = 0; j < 7; ++j )
+               if ( j < rg.count )
+                  v += A( cRGW[q][rg.first + j] ) * buf[i][j];
+         }
    }
    coarse[blockIdx.y + ( ( c * scc + tetRowStart( wc, y, z ) + x ) << lv )] = fromAcc< T >( v );
 }
@@ -726,33 +738,46 @@ __global__ __launch_bounds__( 256 ) void kP2RestrictBndFace( BndGeom gc, const u
       const int     q = __builtin_amdgcn_readfirstlane( ( x & 1 ) + 2 * ( y & 1 ) + 4 * ( z & 1 ) );
       const double* wi = maskInvN + 16 * c;
       const T*      fc = fine + ( ( c * scf ) << lv );
-      for ( int g = 0; g < cRGN[q]; ++g )
+      const int     ng = cRGN[q];
+      for ( int g0 = 0; g0 < ng; g0 += kRowsAhead )
       {
-         const RowGroup rg = cRG[q][g];
-         const int32_t  fy = 2 * y + rg.oy, fz = 2 * z + rg.oz;
-         if ( fy < 0 || fz < 0 || fy + fz > mmf )
-            continue;
-         const int32_t rs  = sliceStart[fz] + fy * ( wf - fz ) - fy * ( fy - 1 ) / 2;
-         const int32_t lim = mmf - fy - fz, mk = ( fy == 0 ? 4 : 0 ) | ( fz == 0 ? 8 : 0 );
-         A             buf[7], wgt[7];
+         A buf[kRowsAhead][7], wgt[kRowsAhead][7];
 #pragma unroll
-         for ( int j = 0; j < 7; ++j )
+         for ( int r = 0; r < kRowsAhead; ++r )
          {
-            buf[j] = wgt[j] = A( 0 );
-            if ( j < rg.count )
+            const RowGroup rg = cRG[q][min( g0 + r, ng - 1 )];
+            const int32_t  fy = 2 * y + rg.oy, fz = 2 * z + rg.oz;
+            const bool     in = g0 + r < ng && fy >= 0 && fz >= 0 && fy + fz <= mmf;
+            const int32_t  rs = in ? sliceStart[fz] + fy * ( wf - fz ) - fy * ( fy - 1 ) / 2 : 0;
+            const int32_t  lim = in ? mmf - fy - fz : -1, mk = ( fy == 0 ? 4 : 0 ) | ( fz == 0 ? 8 : 0 );
+#pragma unroll
+            for ( int j = 0; j < 7; ++j )
             {
-               const int32_t fx = 2 * x + cRGX[q][rg.first + j];
-               if ( fx >= 0 && fx <= lim )
+               buf[r][j] = A( 0 );
+               wgt[r][j] = A( 1 );
+               if ( j < rg.count )
                {
-                  buf[j] = toAcc( fc[int64_t( rs + fx ) << lv] );
-                  wgt[j] = A( wi[mk | ( fx == 0 ? 2 : 0 ) | ( fx == lim ? 1 : 0 )] );
+                  const int32_t fx = 2 * x + cRGX[q][rg.first + j];
+                  if ( fx >= 0 && fx <= lim )
+                  {
+                     const int mask = mk | ( fx == 0 ? 2 : 0 ) | ( fx == lim ? 1 : 0 );
+                     buf[r][j]      = toAcc( fc[int64_t( rs + fx ) << lv] );
+                     if ( mask )
+                        wgt[r][j] = A( wi[mask] );
+                  }
                }
             }
          }
 #pragma unroll
-         for ( int j = 0; j < 7; ++j )
-            if ( j < rg.count )
-               s += A( cRGW[q][rg.first + j] ) * wgt[j] * buf[j];
+         for ( int r = 0; r < kRowsAhead; ++r )
+            if ( g0 + r < ng )
+            {
+               const RowGroup rg = cRG[q][g0 + r];
+#pragma unroll
+               for ( int j = 0; j < 7; ++j )
+                  if ( j < rg.count )
+                     s += A( cRGW[q][rg.first + j] ) * wgt[r][j] * buf[r][j];
+            }
       }
    }
    coarse[( nc * gc.sc + b ) << lv] = fromAcc< T >( s );

@@ -160,7 +160,7 @@ struct Storage
    Topology                                     topo;
    // grid-transfer data keyed by fine level (built on first use)
    std::map< int, std::unique_ptr< OperatorBase > > transfers;
-   // sparsity patterns of assembled P2 operators by level (built on first use)
+   // DoF numbers of the micro-cells of small P2 levels, by level (built on first use)
    std::map< int, std::unique_ptr< OperatorBase > > p2Patterns;
    std::map< int, std::unique_ptr< Lattice > >  lattices;
    DevBuf< CellMeta >                           meta;
