@@ -1803,23 +1803,23 @@ __global__ void kChebyshevStep( int64_t ncell, int64_t nb, const uint8_t* __rest
 // The coarse solve of the P2 V-cycles runs some ninety CG iterations on a few thousand
 // DoFs.  Iteration by iteration it is nine launches of latency-bound kernels and a read
 // back (70 us on the shell's level 0: halo pull, one wavefront a macro-cell, additive
-// push, two updates, three dot products); with the element matrices kept (symmetric,
-// 55 values a micro-cell, 0.8 MB) one workgroup streams them from L2 and gathers and adds
+// push, two updates, three dot products); with the element matrices kept (symmetric with
+// vanishing row sums: 45 values a micro-cell, 0.7 MB) one workgroup streams them from L2 and gathers and adds
 // in LDS, and a whole solve is one launch.  Bound by the matrix stream of one CU.  (With
 // assembled rows, 1 MB and one LDS gather an entry, an iteration took 24 us: the gathers'
 // bank conflicts.)  The iteration, its scalars and its stopping test are those of CGSolver.
 constexpr int kCgThreads   = 1024;
-constexpr int kCgMaxDofs   = 8192; // p and A p in LDS
+constexpr int kCgMaxDofs   = 4992; // p, A p, r and the inverse diagonal in LDS
 constexpr int kCgMaxLevel  = 2;
 constexpr int kCgPerLaunch = 1024; // iterations a launch (bounds its time)
-constexpr int kCgMatrix    = 55;   // upper triangle of a 10 x 10 matrix
+constexpr int kCgMatrix    = 45;   // strict upper triangle of a 10 x 10 matrix
 enum CgState
 {
    kCgRz   = 0, // r . z
    kCgR0   = 1, // sqrt(r . r) of the start
    kCgIts  = 2, // iterations done
    kCgDone = 3,
-   kCgVec  = 8, // then r, p, x, the inverse diagonal (n values each)
+   kCgVec  = 8, // then x and, between launches, p, r and the inverse diagonal (n values each)
 };
 
 struct P2Pattern : OperatorBase
@@ -1894,8 +1894,8 @@ static const P2Pattern* p2Pattern( Context* ctx, Storage& st, int L )
    return static_cast< const P2Pattern* >( ( st.p2Patterns[L] = std::move( pat ) ).get() );
 }
 
-// element matrices mat[k * stride + e], k the upper triangle row by row: one thread a
-// micro-cell and column
+// element matrices mat[k * stride + e], k the strict upper triangle row by row: one thread
+// a micro-cell and column
 __global__ void kP2ElementMatrices( const P2ActGeomT< double >* __restrict__ geom, const P2CellGeom* __restrict__ geom64,
                                     const KParams* __restrict__ kp, int64_t mm, int32_t nelem, int32_t stride,
                                     const int32_t* __restrict__ elem, double* __restrict__ mat )
@@ -1917,11 +1917,12 @@ __global__ void kP2ElementMatrices( const P2ActGeomT< double >* __restrict__ geo
    } );
 #pragma unroll
    for ( int k = 0; k < 10; ++k )
-      if ( k <= j )
-         mat[( k * 10 - k * ( k - 1 ) / 2 + ( j - k ) ) * stride + e] = y[k];
+      if ( k < j )
+         mat[( k * 9 - k * ( k - 1 ) / 2 + ( j - k - 1 ) ) * stride + e] = y[k];
 }
 
-// sums of two values over the workgroup, in every thread
+// sums of two values over the workgroup, in every thread; calls with the same red are
+// at least one other barrier apart
 __device__ __forceinline__ void cgSum( double& a, double& b, double ( *red )[2] )
 {
 #pragma unroll
@@ -1930,7 +1931,6 @@ __device__ __forceinline__ void cgSum( double& a, double& b, double ( *red )[2] 
       a += __shfl_xor( a, d );
       b += __shfl_xor( b, d );
    }
-   __syncthreads(); // the sums of the call before are read
    if ( ( threadIdx.x & 63 ) == 0 )
    {
       red[threadIdx.x >> 6][0] = a;
@@ -1955,19 +1955,13 @@ __global__ __launch_bounds__( kCgThreads ) void kP2AssembledCG( int32_t n, int32
                                                                const double* __restrict__ b, double* __restrict__ x,
                                                                double* __restrict__ state )
 {
-   extern __shared__ double sp[]; // p, then A p
-   __shared__ double        red[kCgThreads / 64][2];
+   extern __shared__ double sp[]; // p, A p, r and the inverse diagonal (n values each)
+   __shared__ double        red[2][kCgThreads / 64][2];
    double* const            sa  = sp + n;
-   double* const            r   = state + kCgVec;
-   double* const            ps  = r + n;
-   double* const            xs  = ps + n;
-   double* const            inv = xs + n; // 1 / diagonal (1 without the preconditioner), 0 where x is fixed
-   auto clear = [&]() {
-      for ( int32_t i = threadIdx.x; i < n; i += kCgThreads )
-         sa[i] = 0.0;
-      __syncthreads();
-   };
-   // sa += A p (cleared before)
+   double* const            r   = sa + n;
+   double* const            inv = r + n; // 1 / diagonal (1 without the preconditioner), 0 where x is fixed
+   double* const            xs  = state + kCgVec;
+   // sa += A p
    auto product = [&]() {
       for ( int32_t e = threadIdx.x; e < nelem; e += kCgThreads )
       {
@@ -1985,14 +1979,17 @@ __global__ __launch_bounds__( kCgThreads ) void kP2AssembledCG( int32_t n, int32
          int k = 0;
 #pragma unroll
          for ( int i = 0; i < 10; ++i )
+         {
 #pragma unroll
-            for ( int j = i; j < 10; ++j, ++k )
+            for ( int j = i + 1; j < 10; ++j, ++k )
             {
-               const double m = mat[k * stride + e];
-               y[i] += m * u[j];
-               if ( j > i )
-                  y[j] += m * u[i];
+               const double f = mat[k * stride + e] * ( u[j] - u[i] );
+               y[i] += f;
+               y[j] -= f;
             }
+            if ( i == 2 )
+               __builtin_amdgcn_sched_barrier( 0 ); // 24 values in flight: all 45 spill
+         }
 #pragma unroll
          for ( int i = 0; i < 10; ++i )
             atomicAdd( &sa[d[i]], y[i] );
@@ -2002,34 +1999,49 @@ __global__ __launch_bounds__( kCgThreads ) void kP2AssembledCG( int32_t n, int32
    double rz, r0, its = 0.0;
    if ( start )
    {
-      // the diagonal into p's place, then x
-      for ( int32_t i = threadIdx.x; i < n; i += kCgThreads )
-         sp[i] = 0.0;
-      clear();
-      for ( int32_t e = threadIdx.x; e < nelem; e += kCgThreads )
-#pragma unroll
-         for ( int i = 0; i < 10; ++i )
-            atomicAdd( &sp[id[i * stride + e]], mat[( i * 10 - i * ( i - 1 ) / 2 ) * stride + e] );
-      __syncthreads();
+      // the diagonal into inv, then x into p's place
       for ( int32_t i = threadIdx.x; i < n; i += kCgThreads )
       {
-         inv[i] = ( dofFlag[i] & flag ) ? ( jacobi ? 1.0 / sp[i] : 1.0 ) : 0.0;
-         sp[i]  = x[pos[i]];
+         sa[i] = inv[i] = 0.0;
+         sp[i] = x[pos[i]];
       }
       __syncthreads();
+      for ( int32_t e = threadIdx.x; e < nelem; e += kCgThreads )
+      {
+         double d[10] = {};
+         int    k     = 0;
+#pragma unroll
+         for ( int i = 0; i < 10; ++i )
+         {
+#pragma unroll
+            for ( int j = i + 1; j < 10; ++j, ++k )
+            {
+               const double m = mat[k * stride + e];
+               d[i] -= m;
+               d[j] -= m;
+            }
+            if ( i == 2 )
+               __builtin_amdgcn_sched_barrier( 0 );
+         }
+#pragma unroll
+         for ( int i = 0; i < 10; ++i )
+            atomicAdd( &inv[id[i * stride + e]], d[i] );
+      }
       product();
       rz = r0 = 0.0;
       for ( int32_t i = threadIdx.x; i < n; i += kCgThreads )
       {
-         const double d  = inv[i];
+         const double d  = ( dofFlag[i] & flag ) ? ( jacobi ? 1.0 / inv[i] : 1.0 ) : 0.0;
          const double ri = d != 0.0 ? b[pos[i]] - sa[i] : 0.0, zi = d * ri;
-         xs[i] = sp[i];
-         r[i]  = ri;
-         sp[i] = zi;
+         xs[i]  = sp[i];
+         inv[i] = d;
+         r[i]   = ri;
+         sp[i]  = zi;
+         sa[i]  = 0.0;
          rz += ri * zi;
          r0 += ri * ri;
       }
-      cgSum( rz, r0, red );
+      cgSum( rz, r0, red[1] );
       r0 = sqrt( r0 );
       if ( threadIdx.x == 0 )
       {
@@ -2046,46 +2058,55 @@ __global__ __launch_bounds__( kCgThreads ) void kP2AssembledCG( int32_t n, int32
       r0  = state[kCgR0];
       its = state[kCgIts] + 1.0;
       for ( int32_t i = threadIdx.x; i < n; i += kCgThreads )
-         sp[i] = ps[i];
+      {
+         sp[i]  = xs[n + i];
+         r[i]   = xs[2 * n + i];
+         inv[i] = xs[3 * n + i];
+         sa[i]  = 0.0;
+      }
+      __syncthreads();
    }
-   __syncthreads();
+   // every thread keeps the same entries of the vectors through all passes; p and A p are
+   // exchanged in product()
    for ( int k = 0;; ++k )
    {
-      clear();
       product();
       double pap = 0.0, rr = 0.0, rzn = 0.0, none = 0.0;
       for ( int32_t i = threadIdx.x; i < n; i += kCgThreads )
          pap += inv[i] != 0.0 ? sp[i] * sa[i] : 0.0;
-      cgSum( pap, none, red );
+      cgSum( pap, none, red[0] );
       const double alpha = rz / pap;
       for ( int32_t i = threadIdx.x; i < n; i += kCgThreads )
       {
-         const double d = inv[i];
+         const double d = inv[i], ap = sa[i];
+         sa[i] = 0.0;
          if ( d != 0.0 )
          {
             xs[i] += alpha * sp[i];
-            const double ri = r[i] - alpha * sa[i];
+            const double ri = r[i] - alpha * ap;
             r[i]            = ri;
             rr += ri * ri;
             rzn += ri * ( d * ri );
          }
       }
-      cgSum( rr, rzn, red );
+      cgSum( rr, rzn, red[1] );
       const double res  = sqrt( rr );
       const bool   done = res / r0 < relTol || res < absTol || its + 1.0 >= double( maxIter );
       const bool   stop = done || k + 1 == perLaunch;
       const double beta = rzn / rz;
+      rz                = rzn;
       if ( !done )
          for ( int32_t i = threadIdx.x; i < n; i += kCgThreads )
             sp[i] = inv[i] * r[i] + beta * sp[i]; // 0 where x is fixed
-      rz = rzn;
       if ( stop )
       {
          for ( int32_t i = threadIdx.x; i < n; i += kCgThreads )
          {
             if ( inv[i] != 0.0 )
                x[pos[i]] = xs[i];
-            ps[i] = sp[i];
+            xs[n + i]     = sp[i];
+            xs[2 * n + i] = r[i];
+            xs[3 * n + i] = inv[i];
          }
          if ( threadIdx.x == 0 )
          {
@@ -2096,6 +2117,7 @@ __global__ __launch_bounds__( kCgThreads ) void kP2AssembledCG( int32_t n, int32
          return;
       }
       its += 1.0;
+      __syncthreads();
    }
 }
 
@@ -2125,12 +2147,12 @@ static bool p2AssembledCG( Context* ctx, P2Operator& op, Function& x, Function& 
    std::call_once( once[ctx->device & 63], [] {
       HG_CHECK_HIP( hipFuncSetAttribute( reinterpret_cast< const void* >( &kP2AssembledCG ),
                                          hipFuncAttributeMaxDynamicSharedMemorySize,
-                                         int( 2 * kCgMaxDofs * sizeof( double ) ) ) );
+                                         int( 4 * kCgMaxDofs * sizeof( double ) ) ) );
    } );
    double s[4] = { 0, 0, 0, 0 };
    for ( int start = 1; s[kCgDone] == 0.0; start = 0 )
    {
-      kP2AssembledCG<<< 1, kCgThreads, 2 * size_t( pat->n ) * sizeof( double ), ctx->stream >>>(
+      kP2AssembledCG<<< 1, kCgThreads, 4 * size_t( pat->n ) * sizeof( double ), ctx->stream >>>(
           pat->n, pat->nelem, pat->stride, pat->pos.p, pat->flag.p, flag, pat->id.p, mat.p, jacobi, start, maxIter,
           kCgPerLaunch, relTol, absTol, (const double*) b.ptr( L ), (double*) x.ptr( L ), state.p );
       HG_CHECK_HIP( hipGetLastError() );
