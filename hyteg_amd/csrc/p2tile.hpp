@@ -242,6 +242,19 @@ struct ElementBox
    static constexpr int edges[6][2] = { { 0, 1 }, { 0, 2 }, { 0, 3 }, { 1, 2 }, { 1, 3 }, { 2, 3 } };
    static constexpr int at( int i ) { return i < 4 ? vertex( i ) : ( vertex( edges[i - 4][0] ) + vertex( edges[i - 4][1] ) ) / 2; }
 };
+// Spread box layout: the box points split by the parity of lx, rows and planes padded, so
+// that the 64 anchors of a wavefront address every LDS bank equally often for any local
+// DoF (2 ax + 18 ay + 162 az of the plain layout meet 16 of the 32 8-byte banks, up to
+// eight lanes on one)
+constexpr int kSpreadOdd = 504, kSpreadRow = 6, kSpreadPlane = 56, kSpreadBox = 2 * kSpreadOdd;
+__host__ __device__ constexpr int spreadPos( int lx, int ly, int lz )
+{
+   return ( lx & 1 ) * kSpreadOdd + ( lx >> 1 ) + kSpreadRow * ly + kSpreadPlane * lz;
+}
+static_assert( spreadPos( kBox - 1, kBox - 1, kBox - 1 ) < kSpreadOdd, "spread box layout" );
+// of a plain box position
+__host__ __device__ constexpr int spreadOf( int p ) { return spreadPos( p % kBox, p / kBox % kBox, p / ( kBox * kBox ) ); }
+
 // coordinate d of vertex k of a micro-cell of type t (0 or 1) from a packed constant:
 // no table load where the type differs between lanes
 constexpr uint32_t vertexBits( int d )

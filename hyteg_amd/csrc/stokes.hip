@@ -96,23 +96,10 @@ __device__ __forceinline__ void baryGrad( const R* a4, const R* b4, const R u[10
    g[3] = b4[3] * u[3] + a4[0] * u[6] + a4[1] * u[8] + a4[2] * u[9];
 }
 
-// computational-space gradient sum_k (g_k - g_0) grad lam_k
+// y_j += grad phi_j . tau for the 10 P2 functions; e_k = grad lam_k . tau, k = 1..3
 template < class R >
-__device__ __forceinline__ void compGrad( const R* Dc, const R g[4], R v[3] )
+__device__ __forceinline__ void testGrad( const R* a4, const R* b4, R e1, R e2, R e3, R y[10] )
 {
-   const R d1 = g[1] - g[0], d2 = g[2] - g[0], d3 = g[3] - g[0];
-#pragma unroll
-   for ( int d = 0; d < 3; ++d )
-      v[d] = d1 * Dc[d] + d2 * Dc[3 + d] + d3 * Dc[6 + d];
-}
-
-// y_j += grad phi_j . tau for the 10 P2 functions (tau in computational space)
-template < class R >
-__device__ __forceinline__ void testGrad( const R* a4, const R* b4, const R* Dc, const R tau[3], R y[10] )
-{
-   const R e1 = Dc[0] * tau[0] + Dc[1] * tau[1] + Dc[2] * tau[2];
-   const R e2 = Dc[3] * tau[0] + Dc[4] * tau[1] + Dc[5] * tau[2];
-   const R e3 = Dc[6] * tau[0] + Dc[7] * tau[1] + Dc[8] * tau[2];
    const R e0 = -( e1 + e2 + e3 );
    y[0] += b4[0] * e0;
    y[1] += b4[1] * e1;
@@ -124,6 +111,22 @@ __device__ __forceinline__ void testGrad( const R* a4, const R* b4, const R* Dc,
    y[7] += a4[2] * e1 + a4[1] * e2;
    y[8] += a4[3] * e1 + a4[1] * e3;
    y[9] += a4[3] * e2 + a4[2] * e3;
+}
+
+// With T = q DF^-T the gradient of component c is G_c = T D^T (g_k - g_0); M = T D^T
+// (3 x 3, M[d][k - 1] = d-th component of T grad lam_k) serves all three components and,
+// transposed, their test functions: T = I - w x^T / beta, a rank-one correction of D^T.
+template < class R >
+__device__ __forceinline__ void mapGradients( const R* Dc, const R x[3], const R w[3], R ib, R M[3][3] )
+{
+#pragma unroll
+   for ( int k = 0; k < 3; ++k )
+   {
+      const R z = ib * ( x[0] * Dc[3 * k] + x[1] * Dc[3 * k + 1] + x[2] * Dc[3 * k + 2] );
+#pragma unroll
+      for ( int d = 0; d < 3; ++d )
+         M[d][k] = Dc[3 * k + d] - w[d] * z;
+   }
 }
 
 // quadrature point q of the thread's micro-cell: computational point x, the
@@ -164,8 +167,17 @@ __device__ __forceinline__ QPoint< R > qpoint( const P2CellGeomT< R >& g, const 
 // of the block-factorisation preconditioner), 4-point degree-2 rule.
 // T is the value type of the functions (double; float or half for the
 // reduced-precision velocity block), the arithmetic runs in Acc<T>.
-template < int MASK, class T >
-__global__ __launch_bounds__( kTileThreads ) void kStokesTileApply(
+//
+// LAST = false: one tile a workgroup, one micro-cell type a wavefront.  LAST = true: a
+// last-layer tile (tileList) by one wavefront, its 64 micro-cells with the type varying
+// over the lanes -- a workgroup of the other form would run six wavefronts for them.
+// Results go through copies of the result box, one a wavefront, one component after the
+// other, with plain LDS reads and writes (waveBoxAccumulate); LDS atomics on one box
+// bounded the kernel (14.5 ms, shell level 5, full operator).
+constexpr int kPBox3P = 128; // a pressure box, padded
+constexpr int kStokesTiles = 2;
+template < int MASK, class T, bool LAST >
+__global__ __launch_bounds__( LAST ? 64 : kStokesTiles * kTileThreads, LAST ? 2 : 3 ) void kStokesTileApply(
     const P2CellGeomT< typename Acc< T >::type >* __restrict__ geom, typename Acc< T >::type c0,
     typename Acc< T >::type c1, int64_t mm, int64_t ntiles, int64_t sc1, int64_t w1, int64_t sc0, int64_t w0,
     const T* __restrict__ u0, const T* __restrict__ u1, const T* __restrict__ u2, const T* __restrict__ pin,
@@ -174,260 +186,365 @@ __global__ __launch_bounds__( kTileThreads ) void kStokesTileApply(
    using R  = typename Acc< T >::type;
    using QC = SQ< R >;
    constexpr bool DO_A = MASK & 1, DO_BT = MASK & 2, DO_B = MASK & 4, DO_M = MASK & 8;
+   constexpr int HELD = LAST || sizeof( R ) == 4 ? 3 : 1;
    constexpr bool NEED_U = DO_A || DO_B, OUT_U = DO_A || DO_BT, NEED_P = DO_BT || DO_M, OUT_P = DO_B || DO_M;
-   // LDS boxes of the tile's input values and, apart from them, the result
-   // boxes (cleared while the input loads are in flight: two workgroup barriers
-   // per tile)
-   __shared__ R su[3][kBox3];
-   __shared__ R sp[kPBox3];
-   __shared__ R au[OUT_U ? 3 : 1][OUT_U ? kBox3 : 1];
-   __shared__ R ap[OUT_P ? kPBox3 : 1];
-   const int64_t lb = xcdBlock( ntiles );
-   if ( lb >= ntiles )
+   constexpr int  kThreads = LAST ? 64 : kTileThreads, kWaves = kThreads / 64;
+   constexpr int  kPoints  = LAST ? kDiagBoxP / 64 : 2; // velocity box points a thread
+   constexpr int  kPPoints = LAST ? 2 : 1;              // and pressure box points
+   static_assert( LAST || kBox3 <= 2 * kTileThreads, "box points per thread" );
+   // the tile's velocity values and, when they have been used, the wavefronts' result boxes
+   constexpr int kULds = ( OUT_U && kWaves > 3 ? kWaves : 3 ) * kSpreadBox;
+   constexpr int kTiles = LAST ? 1 : kStokesTiles;
+   __shared__ R  suAll[kTiles][NEED_U || OUT_U ? kULds : 1];
+   __shared__ R  spAll[kTiles][NEED_P ? kPBox3P : 1];
+   __shared__ R  apAll[kTiles][OUT_P ? kWaves * kPBox3P : 1];
+   const int64_t lw = xcdBlock( ( ntiles + kTiles - 1 ) / kTiles );
+   if ( lw * kTiles >= ntiles )
       return;
+   const int     lane = int( threadIdx.x ) & 63, wgWave = LAST ? 0 : __builtin_amdgcn_readfirstlane( int( threadIdx.x ) >> 6 );
+   const int     sub = LAST ? 0 : wgWave / kWaves, wave = wgWave - sub * kWaves; // tile of the workgroup
+   R* const      su  = suAll[sub];
+   R* const      sp  = spAll[sub];
+   R* const      ap  = apAll[sub];
+   const int     tid0 = wave * 64 + lane; // thread number in the tile
+   const bool    live = lw * kTiles + sub < ntiles;
+   const int64_t lb   = live ? lw * kTiles + sub : ntiles - 1;
    int64_t         full;
    const TileCoord tc    = tileFromList( tiles, lb, mm, full );
    const int64_t   base1 = tc.c * sc1, base0 = tc.c * sc0;
-   const int32_t   top1 = int32_t( 2 * mm ), top0 = int32_t( mm );
    const T*        uin[3] = { u0, u1, u2 };
-   // the thread's (at most two) velocity box points and one pressure box point:
+   const int       pair = LAST ? cDiagPairs[lane] : 0;
+   const int       t = LAST ? pair & 7 : wave, a = LAST ? pair >> 3 : lane;
    // all loads issued before the first LDS write, so their latencies overlap
-   static_assert( kBox3 <= 2 * kTileThreads && kPBox3 <= kTileThreads, "box points per thread" );
-   T    uv[2][3], pvl = T( 0 );
-   bool uok[2] = { false, false }, pok = false;
+   const BoxOffsets box1( int32_t( w1 ), 2 * int32_t( tc.x0 ), 2 * int32_t( tc.y0 ), 2 * int32_t( tc.z0 ) );
+   const BoxOffsets box0( int32_t( w0 ), int32_t( tc.x0 ), int32_t( tc.y0 ), int32_t( tc.z0 ) );
+   const int32_t    rest0 = live ? int32_t( mm ) - int32_t( tc.x0 + tc.y0 + tc.z0 ) : -1, rest1 = 2 * rest0; // -1: no points
+   // the thread's j-th box points: their LDS positions and lattice offsets (-1: none)
+   auto velocityPoint = [&]( int tid, int j, int32_t& bp, int32_t& off ) {
+      const int p   = tid + j * kThreads;
+      const int box = LAST ? cDiagBox[p] : ( p < kBox3 ? p : -1 );
+      int32_t   lx, ly, lz;
+      boxPoint( box, lx, ly, lz );
+      bp  = box >= 0 ? spreadPos( lx, ly, lz ) : -1;
+      off = box >= 0 && lx + ly + lz <= rest1 ? box1.at( lx, ly, lz ) : -1;
+   };
+   auto pressurePoint = [&]( int tid, int j ) {
+      const int p = tid + j * kThreads, lx = p % kPBox, ly = ( p / kPBox ) % kPBox, lz = p / ( kPBox * kPBox );
+      return p < kPBox3 && lx + ly + lz <= rest0 ? box0.at( lx, ly, lz ) : -1;
+   };
+   int32_t bp[kPoints], off[kPoints], poff[kPPoints];
+   T       uv[kPoints][3], pvl[kPPoints];
    if constexpr ( NEED_U )
-   {
 #pragma unroll
-      for ( int j = 0; j < 2; ++j )
+      for ( int j = 0; j < kPoints; ++j )
       {
-         const int     p  = int( threadIdx.x ) + j * kTileThreads;
-         const int32_t lx = p % kBox, ly = ( p / kBox ) % kBox, lz = p / ( kBox * kBox );
-         const int32_t X = 2 * int32_t( tc.x0 ) + lx, Y = 2 * int32_t( tc.y0 ) + ly, Z = 2 * int32_t( tc.z0 ) + lz;
-         uok[j]          = p < kBox3 && X + Y + Z <= top1;
-         const int64_t idx = base1 + tetRowStart32( int32_t( w1 ), Y, Z ) + X;
+         velocityPoint( tid0, j, bp[j], off[j] );
 #pragma unroll
          for ( int c = 0; c < 3; ++c )
-            uv[j][c] = uok[j] ? uin[c][idx] : T( 0 );
+            uv[j][c] = off[j] >= 0 ? ( uin[c] + base1 )[uint32_t( off[j] )] : T( 0 );
       }
-   }
    if constexpr ( NEED_P )
-   {
-      const int     p  = int( threadIdx.x );
-      const int32_t lx = p % kPBox, ly = ( p / kPBox ) % kPBox, lz = p / ( kPBox * kPBox );
-      const int32_t X = int32_t( tc.x0 ) + lx, Y = int32_t( tc.y0 ) + ly, Z = int32_t( tc.z0 ) + lz;
-      pok             = p < kPBox3 && X + Y + Z <= top0;
-      pvl             = pok ? pin[base0 + tetRowStart32( int32_t( w0 ), Y, Z ) + X] : T( 0 );
-   }
-   if constexpr ( OUT_U )
-   {
 #pragma unroll
-      for ( int j = 0; j < 2; ++j )
+      for ( int j = 0; j < kPPoints; ++j )
       {
-         const int p = int( threadIdx.x ) + j * kTileThreads;
-         if ( p < kBox3 )
-            au[0][p] = au[1][p] = au[2][p] = R( 0 );
+         poff[j] = pressurePoint( tid0, j );
+         pvl[j]  = poff[j] >= 0 ? ( pin + base0 )[uint32_t( poff[j] )] : T( 0 );
       }
-   }
-   if constexpr ( OUT_P )
-   {
-      if ( int( threadIdx.x ) < kPBox3 )
-         ap[threadIdx.x] = R( 0 );
-   }
    if constexpr ( NEED_U )
    {
 #pragma unroll
-      for ( int j = 0; j < 2; ++j )
-      {
-         const int p = int( threadIdx.x ) + j * kTileThreads;
-         if ( p < kBox3 )
-         {
+      for ( int j = 0; j < kPoints; ++j )
+         if ( bp[j] >= 0 )
 #pragma unroll
             for ( int c = 0; c < 3; ++c )
-               su[c][p] = uok[j] ? R( toAcc( uv[j][c] ) ) : R( 0 );
-         }
-      }
+               su[c * kSpreadBox + bp[j]] = toAcc( uv[j][c] );
    }
    if constexpr ( NEED_P )
    {
-      if ( int( threadIdx.x ) < kPBox3 )
-         sp[threadIdx.x] = pok ? R( toAcc( pvl ) ) : R( 0 );
+#pragma unroll
+      for ( int j = 0; j < kPPoints; ++j )
+         if ( tid0 + j * kThreads < kPBox3P )
+            sp[tid0 + j * kThreads] = toAcc( pvl[j] );
    }
    __syncthreads();
    const P2CellGeomT< R >& g  = geom[tc.c];
-   const TileThread< R >   th = tileThread( g, tc, mm );
-   int                     pos[10], ppos[4];
-   elementBoxPositions( th, pos );
-#pragma unroll
-   for ( int k = 0; k < 4; ++k )
-      ppos[k] = ( th.ax + cVof[th.t][k][0] ) + kPBox * ( ( th.ay + cVof[th.t][k][1] ) + kPBox * ( th.az + cVof[th.t][k][2] ) );
-   R u[3][10], pv[4];
-   if constexpr ( NEED_U )
+   TileThread< R >         th; // (32-bit tile coordinates: 64-bit ones held two registers each)
    {
+      th.t  = t;
+      th.ax = a & 3;
+      th.ay = ( a >> 2 ) & 3;
+      th.az = a >> 4;
+      const R vx = R( int32_t( tc.x0 ) + th.ax + vertexOffset< 0 >( t, 0 ) ), vy = R( int32_t( tc.y0 ) + th.ay + vertexOffset< 1 >( t, 0 ) ),
+              vz = R( int32_t( tc.z0 ) + th.az + vertexOffset< 2 >( t, 0 ) );
 #pragma unroll
-      for ( int c = 0; c < 3; ++c )
+      for ( int d = 0; d < 3; ++d )
+         th.p0[d] = g.v0[d] + g.hE[3 * d] * vx + g.hE[3 * d + 1] * vy + g.hE[3 * d + 2] * vz;
+      th.ls0   = g.nl[0] * th.p0[0] + g.nl[1] * th.p0[1] + g.nl[2] * th.p0[2] - g.lam0;
+      th.valid = LAST || th.ax + th.ay + th.az < rest0 - MicroCells::rowShift[t];
+   }
+   int                     lanePos[LAST ? 10 : 1];
+   const int               b1 = LAST ? 0 : spreadPos( 2 * th.ax, 2 * th.ay, 2 * th.az );
+   if constexpr ( LAST )
+   {
+      laneBoxPositions( t, a, lanePos );
+#pragma unroll
+      for ( int i = 0; i < 10; ++i )
+      {
+         int32_t lx, ly, lz;
+         boxPoint( lanePos[i], lx, ly, lz );
+         lanePos[i] = spreadPos( lx, ly, lz );
+      }
+   }
+   // f( at ): at( i ) = box position of local DoF i, from b1
+   auto withPositions = [&]( auto&& f ) {
+      if constexpr ( LAST )
+         f( [&]( int i ) { return lanePos[i]; } );
+      else
+         forType( t, [&]( auto box ) { f( [&]( int i ) { return spreadOf( box.at( i ) ); } ); } );
+   };
+   auto ppos = [&]( int k ) {
+      return ( th.ax + vertexOffset< 0 >( t, k ) ) +
+             kPBox * ( ( th.ay + vertexOffset< 1 >( t, k ) ) + kPBox * ( th.az + vertexOffset< 2 >( t, k ) ) );
+   };
+   // LDS accesses of a wavefront to its own copies: volatile, they complete in order
+   using LdsR = volatile __attribute__( ( address_space( 3 ) ) ) R;
+   LdsR* const apw = (LdsR*) ( ap + ( OUT_P ? wave * kPBox3P : 0 ) );
+   auto pressureResults = [&]( const R yq[4] ) {
+      apw[lane]      = R( 0 );
+      apw[lane + 64] = R( 0 );
+      if ( th.valid )
+      {
+         if constexpr ( LAST )
+#pragma unroll
+            for ( int k = 0; k < 4; ++k )
+               atomicAdd( &ap[ppos( k )], yq[k] );
+         else
+#pragma unroll
+            for ( int k = 0; k < 4; ++k )
+               apw[ppos( k )] = apw[ppos( k )] + yq[k];
+      }
+   };
+   const R* Dc   = g.Dc[t];
+   const R  adet = g.adet[t];
+   R        u[3][10], y[3][10];
+   // (one opaque base address: the loops would keep the address of every value otherwise)
+   using LdsIn = const __attribute__( ( address_space( 3 ) ) ) R;
+   auto component = [&]( int c ) {
+      LdsIn* base = (LdsIn*) su + c * kSpreadBox + b1;
+      asm volatile( "" : "+v"( base ) );
+      withPositions( [&]( auto at ) {
 #pragma unroll
          for ( int i = 0; i < 10; ++i )
-            u[c][i] = th.valid ? su[c][pos[i]] : R( 0 );
+            u[c][i] = base[at( i )];
+      } );
+   };
+   if constexpr ( NEED_U )
+#pragma unroll
+      for ( int c = 0; c < 3; ++c )
+         component( c );
+   if constexpr ( DO_B )
+   {
+      R yq[4] = { R( 0 ), R( 0 ), R( 0 ), R( 0 ) };
+#pragma unroll 1
+      for ( int q = 5; q < 9; ++q )
+      {
+         const R*          a4  = QC::a4( q );
+         const R*          b4  = QC::b4( q );
+         const R*          lam = QC::lam( q );
+         const QPoint< R > P   = qpoint( g, th, q );
+         const R           cc  = QC::w( q ) * adet * fabs( P.beta ) * P.qq;
+         R                 M[3][3];
+         mapGradients( Dc, P.x, P.w, P.ib, M );
+         // q div u = trace of q grad u
+         R dq = R( 0 );
+#pragma unroll
+         for ( int c = 0; c < 3; ++c )
+         {
+            R gm[4];
+            baryGrad( a4, b4, u[c], gm );
+            dq += ( gm[1] - gm[0] ) * M[c][0] + ( gm[2] - gm[0] ) * M[c][1] + ( gm[3] - gm[0] ) * M[c][2];
+         }
+         const R s = -cc * dq;
+#pragma unroll
+         for ( int k = 0; k < 4; ++k )
+            yq[k] += lam[k] * s;
+      }
+      pressureResults( yq );
+   }
+#pragma unroll
+   for ( int c = 0; c < 3; ++c )
+#pragma unroll
+      for ( int i = 0; i < 10; ++i )
+         y[c][i] = R( 0 );
+   if constexpr ( DO_A )
+   {
+#pragma unroll 1
+      for ( int q = 0; q < 5; ++q )
+      {
+         const R* a4 = QC::a4( q );
+         const R* b4 = QC::b4( q );
+         R        M[3][3], cc;
+         {
+            const QPoint< R > P = qpoint( g, th, q );
+            cc                  = QC::w( q ) * adet * fabs( P.beta ) * rexp( c0 + c1 * P.r );
+            mapGradients( Dc, P.x, P.w, P.ib, M );
+         }
+         // S = G + G^T, G[c][d]: q times the d-th derivative of component c
+         R S[3][3];
+#pragma unroll
+         for ( int c = 0; c < 3; ++c )
+         {
+            R gm[4];
+            if ( c >= HELD )
+            {
+               __builtin_amdgcn_sched_barrier( 0 );
+               component( c );
+            }
+            baryGrad( a4, b4, u[c], gm );
+            const R d1 = gm[1] - gm[0], d2 = gm[2] - gm[0], d3 = gm[3] - gm[0];
+#pragma unroll
+            for ( int d = 0; d < 3; ++d )
+            {
+               const R G = d1 * M[d][0] + d2 * M[d][1] + d3 * M[d][2];
+               if ( d < c )
+                  S[d][c] += G;
+               else
+                  S[c][d] = G; // the upper triangle
+            }
+         }
+         // stress times the weight and the coefficient
+         const R tr = ( R( 2 ) / R( 3 ) ) * ( S[0][0] + S[1][1] + S[2][2] );
+#pragma unroll
+         for ( int c = 0; c < 3; ++c )
+         {
+            S[c][c] = cc * ( R( 2 ) * S[c][c] - tr );
+#pragma unroll
+            for ( int d = c + 1; d < 3; ++d )
+               S[d][c] = S[c][d] = cc * S[c][d];
+         }
+#pragma unroll
+         for ( int c = 0; c < 3; ++c )
+            testGrad( a4, b4, M[0][0] * S[c][0] + M[1][0] * S[c][1] + M[2][0] * S[c][2],
+                      M[0][1] * S[c][0] + M[1][1] * S[c][1] + M[2][1] * S[c][2],
+                      M[0][2] * S[c][0] + M[1][2] * S[c][1] + M[2][2] * S[c][2], y[c] );
+      }
    }
    if constexpr ( NEED_P )
    {
+      R pv[4], yq[4] = { R( 0 ), R( 0 ), R( 0 ), R( 0 ) };
 #pragma unroll
       for ( int k = 0; k < 4; ++k )
-         pv[k] = th.valid ? sp[ppos[k]] : R( 0 );
-   }
-   if ( th.valid )
-   {
-      const R* Dc   = g.Dc[th.t];
-      const R  adet = g.adet[th.t];
-      R        y[3][10], yq[4];
-#pragma unroll
-      for ( int c = 0; c < 3; ++c )
-#pragma unroll
-         for ( int i = 0; i < 10; ++i )
-            y[c][i] = R( 0 );
-#pragma unroll
-      for ( int k = 0; k < 4; ++k )
-         yq[k] = R( 0 );
-      if constexpr ( DO_A )
-      {
+         pv[k] = sp[ppos( k )];
 #pragma unroll 1
-         for ( int q = 0; q < 5; ++q )
-         {
-            const R*          a4 = QC::a4( q );
-            const R*          b4 = QC::b4( q );
-            const QPoint< R > P  = qpoint( g, th, q );
-            // q DF^-T (computational gradient) of each component: rows of q grad u
-            R G[3][3];
-#pragma unroll
-            for ( int c = 0; c < 3; ++c )
-            {
-               R gm[4];
-               baryGrad( a4, b4, u[c], gm );
-               compGrad( Dc, gm, G[c] );
-               const R t = ( P.x[0] * G[c][0] + P.x[1] * G[c][1] + P.x[2] * G[c][2] ) * P.ib;
-#pragma unroll
-               for ( int d = 0; d < 3; ++d )
-                  G[c][d] -= P.w[d] * t;
-            }
-            const R eta = rexp( c0 + c1 * P.r );
-            const R tr  = ( R( 2 ) / R( 3 ) ) * eta * ( G[0][0] + G[1][1] + G[2][2] );
-            const R cc  = QC::w( q ) * adet * fabs( P.beta );
-#pragma unroll
-            for ( int c = 0; c < 3; ++c )
-            {
-               // row c of the stress (times q), then q DF^-1 of it
-               R s[3];
-#pragma unroll
-               for ( int d = 0; d < 3; ++d )
-                  s[d] = eta * ( G[c][d] + G[d][c] ) - ( c == d ? tr : R( 0 ) );
-               const R t = ( P.w[0] * s[0] + P.w[1] * s[1] + P.w[2] * s[2] ) * P.ib;
-#pragma unroll
-               for ( int d = 0; d < 3; ++d )
-                  s[d] = cc * ( s[d] - P.x[d] * t );
-               testGrad( a4, b4, Dc, s, y[c] );
-            }
-         }
-      }
-      if constexpr ( DO_M )
+      for ( int q = 5; q < 9; ++q )
       {
-#pragma unroll 1
-         for ( int q = 5; q < 9; ++q )
+         const R*          lam = QC::lam( q );
+         const QPoint< R > P   = qpoint( g, th, q );
+         const R           pq  = lam[0] * pv[0] + lam[1] * pv[1] + lam[2] * pv[2] + lam[3] * pv[3];
+         const R           cc  = QC::w( q ) * adet * fabs( P.beta ) * P.qq;
+         if constexpr ( DO_M )
          {
-            const R*          lam = QC::lam( q );
-            const QPoint< R > P   = qpoint( g, th, q );
             // |det D(F J)| = q^2 |beta| adet; k = 1/eta at the blended point
-            const R cc = QC::w( q ) * adet * fabs( P.beta ) * P.qq * P.qq * rexp( -( c0 + c1 * P.r ) );
-            const R s  = cc * ( lam[0] * pv[0] + lam[1] * pv[1] + lam[2] * pv[2] + lam[3] * pv[3] );
+            const R s = cc * P.qq * rexp( -( c0 + c1 * P.r ) ) * pq;
 #pragma unroll
             for ( int k = 0; k < 4; ++k )
                yq[k] += lam[k] * s;
          }
-      }
-      if constexpr ( DO_B || DO_BT )
-      {
-#pragma unroll 1
-         for ( int q = 5; q < 9; ++q )
+         else
          {
-            const R*          a4  = QC::a4( q );
-            const R*          b4  = QC::b4( q );
-            const R*          lam = QC::lam( q );
-            const QPoint< R > P   = qpoint( g, th, q );
-            const R           cc  = QC::w( q ) * adet * fabs( P.beta ) * P.qq;
-            if constexpr ( DO_B )
-            {
-               // q div u = trace of q grad u
-               R dq = R( 0 );
+            const R* a4 = QC::a4( q );
+            const R* b4 = QC::b4( q );
+            const R  s  = -cc * pq;
+            R        M[3][3];
+            mapGradients( Dc, P.x, P.w, P.ib, M );
 #pragma unroll
-               for ( int c = 0; c < 3; ++c )
-               {
-                  R gm[4], v[3];
-                  baryGrad( a4, b4, u[c], gm );
-                  compGrad( Dc, gm, v );
-                  dq += v[c] - P.w[c] * ( P.x[0] * v[0] + P.x[1] * v[1] + P.x[2] * v[2] ) * P.ib;
-               }
-               const R s = -cc * dq;
-#pragma unroll
-               for ( int k = 0; k < 4; ++k )
-                  yq[k] += lam[k] * s;
-            }
-            if constexpr ( DO_BT )
-            {
-               const R s = -cc * ( lam[0] * pv[0] + lam[1] * pv[1] + lam[2] * pv[2] + lam[3] * pv[3] );
-#pragma unroll
-               for ( int c = 0; c < 3; ++c )
-               {
-                  // q DF^-1 e_c, scaled
-                  R tau[3];
-#pragma unroll
-                  for ( int d = 0; d < 3; ++d )
-                     tau[d] = s * ( ( c == d ? R( 1 ) : R( 0 ) ) - P.x[d] * P.w[c] * P.ib );
-                  testGrad( a4, b4, Dc, tau, y[c] );
-               }
-            }
+            for ( int c = 0; c < 3; ++c )
+               testGrad( a4, b4, s * M[c][0], s * M[c][1], s * M[c][2], y[c] );
          }
       }
-      if constexpr ( OUT_U )
+      if constexpr ( DO_M )
+         pressureResults( yq );
+   }
+   __syncthreads(); // the velocity values are read
+   // lane, anchor and box points again, rather than kept through the quadrature loops
+   int ones = -1;
+   asm volatile( "" : "+s"( ones ) );
+   const int  laneEnd = int( __builtin_amdgcn_mbcnt_hi( uint32_t( ones ), __builtin_amdgcn_mbcnt_lo( uint32_t( ones ), 0 ) ) );
+   const int  tid = wave * 64 + laneEnd, axEnd = laneEnd & 3, ayEnd = ( laneEnd >> 2 ) & 3, azEnd = laneEnd >> 4;
+   if constexpr ( OUT_P )
+   {
+#pragma unroll
+      for ( int j = 0; j < kPPoints; ++j )
       {
+         const int32_t o = pressurePoint( tid, j );
+         if ( o >= 0 )
+         {
+            R v = ap[tid + j * kThreads];
+#pragma unroll
+            for ( int w = 1; w < kWaves; ++w )
+               v += ap[w * kPBox3P + tid];
+            sharedAdd( yp + base0 + uint32_t( o ), v );
+         }
+      }
+   }
+   if constexpr ( OUT_U )
+   {
+      // atomics for every point: a read-modify-write of the box interior would wait for
+      // the outstanding atomics of the box surface
+      T* yout[3] = { y0, y1, y2 };
+#pragma unroll
+      for ( int j = 0; j < kPoints; ++j )
+         velocityPoint( tid, j, bp[j], off[j] );
+      if constexpr ( LAST )
+      {
+         for ( int p = tid; p < 3 * kSpreadBox; p += 64 )
+            su[p] = R( 0 );
+         __syncthreads();
 #pragma unroll
          for ( int c = 0; c < 3; ++c )
 #pragma unroll
             for ( int i = 0; i < 10; ++i )
-               atomicAdd( &au[c][pos[i]], y[c][i] );
-      }
-      if constexpr ( OUT_P )
-      {
+               atomicAdd( &su[c * kSpreadBox + lanePos[i]], y[c][i] ); // every pair is a micro-cell
+         __syncthreads();
 #pragma unroll
-         for ( int k = 0; k < 4; ++k )
-            atomicAdd( &ap[ppos[k]], yq[k] );
+         for ( int j = 0; j < kPoints; ++j )
+            if ( off[j] >= 0 )
+#pragma unroll
+               for ( int c = 0; c < 3; ++c )
+                  sharedAdd( yout[c] + base1 + uint32_t( off[j] ), su[c * kSpreadBox + bp[j]] );
       }
-   }
-   __syncthreads();
-   if constexpr ( OUT_U )
-   {
-      T* yout[3] = { y0, y1, y2 };
-      for ( int p = threadIdx.x; p < kBox3; p += kTileThreads )
+      else
       {
-         const int32_t lx = p % kBox, ly = ( p / kBox ) % kBox, lz = p / ( kBox * kBox );
-         const int32_t X = 2 * int32_t( tc.x0 ) + lx, Y = 2 * int32_t( tc.y0 ) + ly, Z = 2 * int32_t( tc.z0 ) + lz;
-         if ( X + Y + Z > top1 )
-            continue;
-         // atomics for every point: a read-modify-write of the box interior would
-         // wait for the outstanding atomics of the box surface
-         const int64_t idx = base1 + tetRowStart32( int32_t( w1 ), Y, Z ) + X;
+         LdsR* const own = (LdsR*) ( su + wave * kSpreadBox );
+         const int   b1e = spreadPos( 2 * axEnd, 2 * ayEnd, 2 * azEnd );
 #pragma unroll
          for ( int c = 0; c < 3; ++c )
-            sharedAdd( yout[c] + idx, au[c][p] );
+         {
+            if ( c > 0 )
+               __syncthreads(); // the component before is summed
+#pragma unroll
+            for ( int p = 0; p < kSpreadBox; p += 64 )
+               if ( p + 64 <= kSpreadBox || laneEnd < kSpreadBox - p )
+                  own[p + laneEnd] = R( 0 );
+            if ( axEnd + ayEnd + azEnd < rest0 - MicroCells::rowShift[t] )
+               withPositions( [&]( auto at ) {
+#pragma unroll
+                  for ( int i = 0; i < 10; ++i )
+                     own[b1e + at( i )] = own[b1e + at( i )] + y[c][i];
+               } );
+            __syncthreads();
+#pragma unroll
+            for ( int j = 0; j < kPoints; ++j )
+               if ( off[j] >= 0 )
+               {
+                  const R* b = su + bp[j];
+                  sharedAdd( yout[c] + base1 + uint32_t( off[j] ),
+                             ( ( b[0] + b[kSpreadBox] ) + ( b[2 * kSpreadBox] + b[3 * kSpreadBox] ) ) +
+                                 ( b[4 * kSpreadBox] + b[5 * kSpreadBox] ) );
+               }
+         }
       }
    }
-   if constexpr ( OUT_P )
-      for ( int p = threadIdx.x; p < kPBox3; p += kTileThreads )
-      {
-         const int32_t lx = p % kPBox, ly = ( p / kPBox ) % kPBox, lz = p / ( kPBox * kPBox );
-         const int32_t X = int32_t( tc.x0 ) + lx, Y = int32_t( tc.y0 ) + ly, Z = int32_t( tc.z0 ) + lz;
-         if ( X + Y + Z > top0 )
-            continue;
-         sharedAdd( yp + base0 + tetRowStart32( int32_t( w0 ), Y, Z ) + X, ap[p] );
-      }
 }
 
 // diagonal of the three diagonal blocks of A:
@@ -636,15 +753,30 @@ void zeroTarget( Context* ctx, Storage& st, Lattice& lat, T* d, bool replaceAll 
    HG_CHECK_HIP( hipGetLastError() );
 }
 
-template < int MASK >
-void launchStokes( Context* ctx, StokesOperator& op, int L, int64_t ntiles, Lattice& l1, Lattice& l0, double* const u[3],
-                   const double* p, double* const y[3], double* yp )
+// Levels of at least 4 micro-edges (a multiple of kTile): the interior tiles a workgroup
+// each and the last layer a wavefront each; smaller levels, one partial tile a cell, in
+// the general form.
+template < int MASK, class T >
+void launchStokes( Context* ctx, StokesOperator& op, const P2CellGeomT< typename Acc< T >::type >* geom, int L, Lattice& l1,
+                   Lattice& l0, T* const u[3], const T* p, T* const y[3], T* yp )
 {
-   const uint64_t* tiles = tileList( ctx, l1, int64_t( 1 ) << L, kTilesAll );
-   kStokesTileApply< MASK, double ><<< xcdGrid( ntiles ), kTileThreads, 0, ctx->stream >>>(
-       op.tgeom.at( L ).p, op.c0, op.c1, int64_t( 1 ) << L, ntiles, l1.sc, l1.w, l0.sc, l0.w, u[0], u[1], u[2], p, y[0],
-       y[1], y[2], yp, tiles );
-   HG_CHECK_HIP( hipGetLastError() );
+   using R          = typename Acc< T >::type;
+   const int64_t mm = int64_t( 1 ) << L, T0 = tileEdges( mm );
+   auto launch = [&]( auto last, int kind, int64_t ntiles ) {
+      constexpr bool LAST = decltype( last )::value;
+      if ( ntiles < 1 )
+         return;
+      constexpr int kTiles = LAST ? 1 : kStokesTiles;
+      kStokesTileApply< MASK, T, LAST >
+          <<< xcdGrid( ( ntiles + kTiles - 1 ) / kTiles ), LAST ? 64 : kTiles * kTileThreads, 0, ctx->stream >>>(
+          geom, R( op.c0 ), R( op.c1 ), mm, ntiles, l1.sc, l1.w, l0.sc, l0.w, u[0], u[1], u[2], p, y[0], y[1], y[2], yp,
+          tileList( ctx, l1, mm, kind ) );
+      HG_CHECK_HIP( hipGetLastError() );
+   };
+   if ( mm < kTile )
+      return launch( std::false_type{}, kTilesAll, tilesPerCell( mm ) * l1.nc );
+   launch( std::false_type{}, kTilesInterior, tet( T0 - 1 ) * l1.nc );
+   launch( std::true_type{}, kTilesLast, T0 * ( T0 + 1 ) / 2 * l1.nc );
 }
 
 // the velocity block alone on FP32 or FP16 velocity functions (FP32 arithmetic)
@@ -682,12 +814,8 @@ void stokesViscousLowPrecision( Context* ctx, StokesOperator& op, Function* cons
             y[c] = (T*) dst[c]->ptr( L );
             zeroTarget( ctx, st, l1, y[c], update == HG_REPLACE && ( flag & kInner ) );
          }
-         const uint64_t* tiles = tileList( ctx, l1, mm, kTilesAll );
          ctx->beginTiming();
-         kStokesTileApply< 1, T ><<< xcdGrid( ntiles ), kTileThreads, 0, ctx->stream >>>(
-             op.tgeom32.at( L ).p, float( op.c0 ), float( op.c1 ), mm, ntiles, l1.sc, l1.w, l0.sc, l0.w, u[0], u[1], u[2],
-             nullptr, y[0], y[1], y[2], nullptr, tiles );
-         HG_CHECK_HIP( hipGetLastError() );
+         launchStokes< 1, T >( ctx, op, op.tgeom32.at( L ).p, L, l1, l0, u, nullptr, y, nullptr );
          ctx->endTiming();
          for ( int c = 0; c < 3; ++c )
             pushAdditive( ctx, st, l1, y[c], dtype, kAll ^ flag, update == HG_REPLACE );
@@ -764,14 +892,14 @@ void stokesApply( Context* ctx, StokesOperator& op, Function* const src[4], Func
    ctx->beginTiming();
    switch ( mask )
    {
-   case 1: launchStokes< 1 >( ctx, op, L, ntiles, l1, l0, u, p, y, yp ); break;
-   case 2: launchStokes< 2 >( ctx, op, L, ntiles, l1, l0, u, p, y, yp ); break;
-   case 3: launchStokes< 3 >( ctx, op, L, ntiles, l1, l0, u, p, y, yp ); break;
-   case 4: launchStokes< 4 >( ctx, op, L, ntiles, l1, l0, u, p, y, yp ); break;
-   case 5: launchStokes< 5 >( ctx, op, L, ntiles, l1, l0, u, p, y, yp ); break;
-   case 6: launchStokes< 6 >( ctx, op, L, ntiles, l1, l0, u, p, y, yp ); break;
-   case 7: launchStokes< 7 >( ctx, op, L, ntiles, l1, l0, u, p, y, yp ); break;
-   default: launchStokes< 8 >( ctx, op, L, ntiles, l1, l0, u, p, y, yp ); break;
+   case 1: launchStokes< 1, double >( ctx, op, op.tgeom.at( L ).p, L, l1, l0, u, p, y, yp ); break;
+   case 2: launchStokes< 2, double >( ctx, op, op.tgeom.at( L ).p, L, l1, l0, u, p, y, yp ); break;
+   case 3: launchStokes< 3, double >( ctx, op, op.tgeom.at( L ).p, L, l1, l0, u, p, y, yp ); break;
+   case 4: launchStokes< 4, double >( ctx, op, op.tgeom.at( L ).p, L, l1, l0, u, p, y, yp ); break;
+   case 5: launchStokes< 5, double >( ctx, op, op.tgeom.at( L ).p, L, l1, l0, u, p, y, yp ); break;
+   case 6: launchStokes< 6, double >( ctx, op, op.tgeom.at( L ).p, L, l1, l0, u, p, y, yp ); break;
+   case 7: launchStokes< 7, double >( ctx, op, op.tgeom.at( L ).p, L, l1, l0, u, p, y, yp ); break;
+   default: launchStokes< 8, double >( ctx, op, op.tgeom.at( L ).p, L, l1, l0, u, p, y, yp ); break;
    }
    ctx->endTiming();
    if ( outU )
@@ -917,6 +1045,9 @@ int hg_stokes_create( hg_ctx* h, hg_handle s, int minLevel, int maxLevel, double
          HG_CHECK_HIP( hipMemcpyToSymbol( HIP_SYMBOL( cSQ4mf ), f4m, sizeof( f4m ) ) );
          HG_CHECK_HIP( hipMemcpyToSymbol( HIP_SYMBOL( cSQLf ), fl, sizeof( fl ) ) );
          HG_CHECK_HIP( hipMemcpyToSymbol( HIP_SYMBOL( cSQWf ), fw, sizeof( fw ) ) );
+         const std::vector< int32_t > pairs = diagonalPairs(), boxp = diagonalBoxPoints();
+         HG_CHECK_HIP( hipMemcpyToSymbol( HIP_SYMBOL( cDiagPairs ), pairs.data(), sizeof( int32_t ) * 64 ) );
+         HG_CHECK_HIP( hipMemcpyToSymbol( HIP_SYMBOL( cDiagBox ), boxp.data(), sizeof( int32_t ) * kDiagBoxP ) );
       } );
       Storage& st = ctx->storage( s );
       auto     op = std::make_unique< StokesOperator >();
