@@ -168,16 +168,24 @@ __device__ __forceinline__ QPoint< R > qpoint( const P2CellGeomT< R >& g, const 
 // T is the value type of the functions (double; float or half for the
 // reduced-precision velocity block), the arithmetic runs in Acc<T>.
 //
-// LAST = false: one tile a workgroup, one micro-cell type a wavefront.  LAST = true: a
-// last-layer tile (tileList) by one wavefront, its 64 micro-cells with the type varying
-// over the lanes -- a workgroup of the other form would run six wavefronts for them.
+// LAST = false: stokesTiles tiles a workgroup, one micro-cell type a wavefront.  LAST =
+// true: a last-layer tile (tileList) by one wavefront, its 64 micro-cells with the type
+// varying over the lanes -- a workgroup of the other form would run six wavefronts for them.
 // Results go through copies of the result box, one a wavefront, one component after the
-// other, with plain LDS reads and writes (waveBoxAccumulate); LDS atomics on one box
-// bounded the kernel (14.5 ms, shell level 5, full operator).
+// other, with plain LDS reads and writes in the spread layout; LDS atomics on one box took
+// about 2 ms of 14.5 (shell level 5, full operator).
+// Bound by FP64 issue and its latencies at three wavefronts a SIMD (11.1 ms for 117 GFLOP,
+// the vector unit about half busy).  168 registers a lane without spills: two of the three
+// velocity components are read from LDS again at each point of the viscous block (HELD
+// in registers), box points and anchors are formed again for the write-back.
 constexpr int kPBox3P = 128; // a pressure box, padded
-constexpr int kStokesTiles = 2;
+// Tiles a workgroup: two, for three wavefronts on each SIMD; of a workgroup of six two of
+// the four SIMDs hold two (full operator 11.5 against 10.3 ms, mask 6 11.1 against 9.2 ms,
+// shell level 5).  B^T alone has registers for two workgroups of one tile a CU, which
+// overlap one's memory phases with the other's arithmetic (5.2 against 6.2 ms).
+constexpr int stokesTiles( int mask, bool last ) { return last || mask == 2 ? 1 : 2; }
 template < int MASK, class T, bool LAST >
-__global__ __launch_bounds__( LAST ? 64 : kStokesTiles * kTileThreads, LAST ? 2 : 3 ) void kStokesTileApply(
+__global__ __launch_bounds__( LAST ? 64 : stokesTiles( MASK, LAST ) * kTileThreads, LAST ? 2 : 3 ) void kStokesTileApply(
     const P2CellGeomT< typename Acc< T >::type >* __restrict__ geom, typename Acc< T >::type c0,
     typename Acc< T >::type c1, int64_t mm, int64_t ntiles, int64_t sc1, int64_t w1, int64_t sc0, int64_t w0,
     const T* __restrict__ u0, const T* __restrict__ u1, const T* __restrict__ u2, const T* __restrict__ pin,
@@ -194,7 +202,7 @@ __global__ __launch_bounds__( LAST ? 64 : kStokesTiles * kTileThreads, LAST ? 2 
    static_assert( LAST || kBox3 <= 2 * kTileThreads, "box points per thread" );
    // the tile's velocity values and, when they have been used, the wavefronts' result boxes
    constexpr int kULds = ( OUT_U && kWaves > 3 ? kWaves : 3 ) * kSpreadBox;
-   constexpr int kTiles = LAST ? 1 : kStokesTiles;
+   constexpr int kTiles = stokesTiles( MASK, LAST );
    __shared__ R  suAll[kTiles][NEED_U || OUT_U ? kULds : 1];
    __shared__ R  spAll[kTiles][NEED_P ? kPBox3P : 1];
    __shared__ R  apAll[kTiles][OUT_P ? kWaves * kPBox3P : 1];
@@ -766,7 +774,7 @@ void launchStokes( Context* ctx, StokesOperator& op, const P2CellGeomT< typename
       constexpr bool LAST = decltype( last )::value;
       if ( ntiles < 1 )
          return;
-      constexpr int kTiles = LAST ? 1 : kStokesTiles;
+      constexpr int kTiles = stokesTiles( MASK, LAST );
       kStokesTileApply< MASK, T, LAST >
           <<< xcdGrid( ( ntiles + kTiles - 1 ) / kTiles ), LAST ? 64 : kTiles * kTileThreads, 0, ctx->stream >>>(
           geom, R( op.c0 ), R( op.c1 ), mm, ntiles, l1.sc, l1.w, l0.sc, l0.w, u[0], u[1], u[2], p, y[0], y[1], y[2], yp,

@@ -1,0 +1,185 @@
+"""Kernel variants at the sizes where their rules change, against the general path or
+the oracle:
+
+* P1 Gauss-Seidel of single vectors (small sweeps in one workgroup, point pairs in
+  registers) against the interleaved form, which runs neither;
+* P2 constant Gauss-Seidel (assembled rows) against a sweep colour by colour with the
+  apply kernel;
+* the P2 coarse conjugate gradients on element matrices (levels 0 to 2) and the
+  launch-by-launch iteration above, against the same iteration in numpy, over more
+  iterations than one launch runs;
+* P2 restriction into levels whose face points fill several wavefronts;
+* the Stokes blocks over an odd number of interior tiles.
+"""
+import numpy as np
+import pytest
+
+import hyteg_amd as hg
+from hyteg_amd import problems
+from meshes import octahedron, relmax
+from oracle import pyoracle as po
+from test_stokes_gpu import _apply_parity
+
+pytestmark = pytest.mark.gpu
+
+EPS = {hg.F64: 2.0**-53, hg.F32: 2.0**-24, hg.F16: 2.0**-11}
+
+
+def _storage(ctx, name):
+    return hg.PrimitiveStorage.cuboid(ctx) if name == "cube" else hg.PrimitiveStorage.from_cells(ctx, *octahedron())
+
+
+@pytest.mark.parametrize("dtype", [hg.F64, hg.F32, hg.F16])
+@pytest.mark.parametrize("name,levels", [("cube", range(1, 9)), ("octa", range(1, 7))])
+def test_p1_sweep_variants_equal_the_interleaved_sweep(ctx, name, levels, dtype):
+    st = _storage(ctx, name)
+    for L in levels:
+        A = hg.P1ConstantLaplaceOperator(st, L, L)
+        n = st.ndofs(L)
+        rng = np.random.default_rng(L)
+        x0, b = rng.uniform(-1, 1, (n, 2)), rng.uniform(-1, 1, (n, 2))
+        xb, bb = (hg.P1Function("f", st, L, L, dtype, nvec=2) for _ in range(2))
+        xs, bs = (hg.P1Function("g", st, L, L, dtype) for _ in range(2))
+        bb.upload(L, b)
+        for flag, relax, sweep in ((hg.GMG_FLAG, 1.0, "smooth_sor"), (hg.ALL, 1.3, "smooth_sor_backwards")):
+            print(f"P1 {sweep} {name} L{L} dtype {dtype}", flush=True)
+            xb.upload(L, x0)
+            getattr(A, sweep)(xb, bb, relax, L, flag)
+            ref = xb.download(L)
+            for k in range(2):
+                xs.upload(L, x0[:, k])
+                bs.upload(L, b[:, k])
+                getattr(A, sweep)(xs, bs, relax, L, flag)
+                # rows of at most 30 entries (a boundary row adds one partial sum a cell)
+                # in another order; errors of earlier colours enter with row sums below 2
+                assert relmax(xs.download(L), ref[:, k]) <= 64 * EPS[dtype], (L, sweep, k)
+        for f in (xb, bb, xs, bs):
+            f.destroy()
+
+
+@pytest.mark.parametrize("name,L", [("cube", 4), ("cube", 5), ("cube", 6), ("octa", 4)])
+def test_p2_constant_sweep_equals_the_sweep_by_colours(ctx, name, L):
+    st = _storage(ctx, name)
+    A = hg.P2ConstantLaplaceOperator(st, L, L)
+    colour, _ = A.sor_colours(L)
+    free = (st.flags(L + 1) & hg.GMG_FLAG) != 0
+    n = len(colour)
+    rng = np.random.default_rng(L)
+    x0, b = rng.uniform(-1, 1, n), rng.uniform(-1, 1, n)
+    x, fb, y = (hg.P2Function("f", st, L, L) for _ in range(3))
+    A.inverse_diagonal(L, y)
+    inv = y.download(L)
+    fb.upload(L, b)
+    for backward in (False, True):
+        print(f"P2 constant sweep {name} L{L} backward {backward}", flush=True)
+        ref = x0.copy()
+        for c in sorted(set(colour[free]), reverse=backward):
+            x.upload(L, ref)
+            A.apply(x, y, L, hg.ALL)
+            rows = free & (colour == c)
+            ref[rows] += 1.2 * inv[rows] * (b - y.download(L))[rows]
+        x.upload(L, x0)
+        (A.smooth_sor_backwards if backward else A.smooth_sor)(x, fb, L, hg.GMG_FLAG, 1.2)
+        assert relmax(x.download(L), ref) < 1e-12
+    for f in (x, fb, y):
+        f.destroy()
+    A.destroy()
+
+
+@pytest.mark.parametrize("jacobi", [True, False])
+@pytest.mark.parametrize("name,L", [("cube", 1), ("cube", 2), ("cube", 3), ("shell", 0), ("shell", 1)])
+def test_p2_cg_iterates(ctx, name, L, jacobi):
+    st = hg.PrimitiveStorage.cuboid(ctx) if name == "cube" else hg.PrimitiveStorage.shell(ctx, 2, 2, 0.55, 1.0)
+    A = hg.P2DivKGradOperator(st, L, L, *problems.shell_coefficient(3))
+    n = st.p2_ndofs(L)
+    free = (st.flags(L + 1) & hg.GMG_FLAG) != 0
+    rng = np.random.default_rng(L)
+    b, x0 = rng.uniform(-1, 1, n), rng.uniform(-1, 1, n)
+    x, fb, y = (hg.P2Function("f", st, L, L) for _ in range(3))
+    fb.upload(L, b)
+
+    def mul(v):
+        x.upload(L, v)
+        A.apply(x, y, L, hg.ALL)
+        return np.where(free, y.download(L), 0.0)
+
+    d = np.where(free, 1.0, 0.0)
+    if jacobi:
+        A.inverse_diagonal(L, y)
+        d = np.where(free, y.download(L), 0.0)
+    for iterations in (1, 2, 7):
+        print(f"P2 CG {name} L{L} jacobi {jacobi}: {iterations} iterations", flush=True)
+        ref = x0.copy()
+        r = np.where(free, b, 0.0) - mul(ref)
+        p = d * r
+        rz = r @ p
+        for _ in range(iterations):
+            ap = mul(p)
+            alpha = rz / (p @ ap)
+            ref += alpha * p
+            r -= alpha * ap
+            rz, old = r @ (d * r), rz
+            p = d * r + (rz / old) * p
+        x.upload(L, x0)
+        hg.p2_cg_solve(A, x, fb, L, iterations, 0.0, 0.0, jacobi)
+        got = x.download(L)
+        assert np.array_equal(got[~free], x0[~free])
+        assert relmax(got, ref) < 1e-11, (iterations, relmax(got, ref))
+    for f in (x, fb, y):
+        f.destroy()
+    A.destroy()
+
+
+def test_p2_cg_runs_on_over_several_launches(ctx):
+    """1100 iterations (a launch runs 1024) of a system scaled so that r.z does not
+    underflow: the residual stays at its rounding limit"""
+    st = hg.PrimitiveStorage.cuboid(ctx)
+    L = 2
+    A = hg.P2DivKGradOperator(st, L, L, *problems.shell_coefficient(3))
+    free = (st.flags(L + 1) & hg.GMG_FLAG) != 0
+    b = np.where(free, 1e120 * np.random.default_rng(0).uniform(-1, 1, len(free)), 0.0)
+    x, fb, y = (hg.P2Function("f", st, L, L) for _ in range(3))
+    fb.upload(L, b)
+    x.upload(L, 0.0 * b)
+    print("P2 CG over two launches", flush=True)
+    assert hg.p2_cg_solve(A, x, fb, L, 1100, 0.0, 0.0) == 1099
+    A.apply(x, y, L, hg.ALL)
+    r = np.where(free, b - y.download(L), 0.0)
+    assert np.abs(r).max() < 1e-11 * np.abs(b).max()
+    for f in (x, fb, y):
+        f.destroy()
+    A.destroy()
+
+
+@pytest.mark.parametrize("dtype", [hg.F64, hg.F32, hg.F16])
+@pytest.mark.parametrize("name,L", [("cube", 5), ("octa", 4)])
+def test_p2_restriction_into_large_levels(ctx, name, L, dtype):
+    st = _storage(ctx, name)
+    om = po.Mesh.cuboid() if name == "cube" else po.Mesh.from_arrays(*octahedron())
+    f = hg.P2Function("f", st, L - 1, L, dtype)
+    rng = np.random.default_rng(L)
+    c0, fine = rng.uniform(-1, 1, om.ndofs(L)), rng.uniform(-1, 1, om.ndofs(L + 1))
+    f.upload(L, fine)
+    fine = f.download(L)  # rounded to the storage type
+    for flag in (hg.ALL, hg.GMG_FLAG):
+        print(f"P2 restriction {name} {L}->{L - 1} dtype {dtype} flag {flag}", flush=True)
+        f.upload(L - 1, c0)
+        ref = f.download(L - 1)
+        hg.restrict(f, L, flag)
+        om.p2_restrict(L, fine, ref, flag)
+        # a sum of at most 125 a cell products with weights of sum 8, then one rounding
+        assert relmax(f.download(L - 1), ref) < (1e-12 if dtype == hg.F64 else 256 * EPS[hg.F32] if dtype == hg.F32
+                                                 else 2 * EPS[hg.F16]), flag
+    f.destroy()
+
+
+@pytest.mark.parametrize("cells", [1, 3])
+@pytest.mark.parametrize("L", [2, 3, 4])
+def test_stokes_blocks_over_odd_tile_counts(ctx, cells, L):
+    X, c = octahedron()
+    c = np.ascontiguousarray(c[:cells])
+    used = np.unique(c)
+    lut = np.zeros(len(X), dtype=c.dtype)
+    lut[used] = np.arange(len(used))
+    X, c = np.ascontiguousarray(X[used]), lut[c]
+    _apply_parity(hg.PrimitiveStorage.from_cells(ctx, X, c), po.Mesh.from_arrays(X, c), L, (0.3, 0.5))
