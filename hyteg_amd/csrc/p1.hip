@@ -781,7 +781,7 @@ __global__ __launch_bounds__( 64 * kCellWorkers ) void kCellSOR( const int32_t* 
 // pair) is the first of the next stride, its new value carried over.  Same sums in the
 // same order.  FULL: one row a wavefront (the cell, and with it the stencil, in scalar
 // registers).  Bound by HBM: a launch reads all of x, a quarter of b and writes a
-// quarter of x.  Cube level 8, a launch: 90 us above, 55 us here.
+// quarter of x.  Cube level 8, a launch: 90 us above, 51 us here.
 template < class T >
 struct LoadPair
 {

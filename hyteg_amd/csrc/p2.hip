@@ -417,7 +417,8 @@ __global__ __launch_bounds__( kTileThreads ) void kP2TileCentroidK( const P2Cell
 // sums over the points need only those of 1, lam_j and lam_j lam_l, which the rule
 // integrates exactly -- 4, 1 and (1 + delta_jl) / 5 -- so that
 //   S = G 4 (d0 + B 1),  T_j = G (d0 + 4/5 (B 1 + B_j)):
-// four products with G instead of a gradient, a product and ten tests at each point.
+// four products with G instead of a gradient, a product and ten tests at each point
+// (kernel with FP16 vectors, shell level 5: 1.46 -> 1.19 ms, box offsets included).
 __device__ __forceinline__ void p2ReducedAction( const float G[6], const float u[10], float y[10] )
 {
    const float d0[3] = { 4.0f * u[4] - 3.0f * u[0] - u[1], 4.0f * u[5] - 3.0f * u[0] - u[2],
@@ -1804,10 +1805,11 @@ __global__ void kChebyshevStep( int64_t ncell, int64_t nb, const uint8_t* __rest
 // DoFs.  Iteration by iteration it is nine launches of latency-bound kernels and a read
 // back (70 us on the shell's level 0: halo pull, one wavefront a macro-cell, additive
 // push, two updates, three dot products); with the element matrices kept (symmetric with
-// vanishing row sums: 45 values a micro-cell, 0.7 MB) one workgroup streams them from L2 and gathers and adds
-// in LDS, and a whole solve is one launch.  Bound by the matrix stream of one CU.  (With
-// assembled rows, 1 MB and one LDS gather an entry, an iteration took 24 us: the gathers'
-// bank conflicts.)  The iteration, its scalars and its stopping test are those of CGSolver.
+// vanishing row sums: 45 values a micro-cell, 0.7 MB) one workgroup streams them from L2,
+// gathers and adds in LDS, and a whole solve is one launch: 15.2 us an iteration there, 4
+// of them the two reductions, the rest one CU's loads.  (Assembled rows, 1 MB and an LDS
+// gather an entry, took 24 us; 55 values, vectors in memory and seven barriers 22.)  The
+// iteration, its scalars and its stopping test are those of CGSolver.
 constexpr int kCgThreads   = 1024;
 constexpr int kCgMaxDofs   = 4992; // p, A p, r and the inverse diagonal in LDS
 constexpr int kCgMaxLevel  = 2;

@@ -292,7 +292,7 @@ __global__ __launch_bounds__( kTileThreads ) void kP2ConstTileApply( const doubl
 // resolved to lattice positions, so a point costs its gathers and one multiply-add
 // each.  Bound by the latency of the gathers on small levels.  Cube level 5: 27
 // launches of 61 us a sweep with the row gathered from the 10x10 matrices of the
-// micro-cells around a point (a position formula and ten loads for each), 9 of 9 us
+// micro-cells around a point (a position formula and ten loads for each), 9 of 12 us
 // this way.
 __global__ __launch_bounds__( 256 ) void kP2ConstRowSOR( const int32_t* __restrict__ rows, int64_t nrows, int64_t nc,
                                                         int64_t sc1, int32_t w, int gl, int backward, double relax,
