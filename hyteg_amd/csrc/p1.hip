@@ -714,6 +714,27 @@ static const uint64_t* p1BrickList( Context* ctx, Lattice& l )
    return l.p1Bricks.p;
 }
 
+// V neighbouring vectors' values of a DoF of an interleaved function, loaded and stored
+// together (the buffers are allocations of their own, offsets multiples of V)
+template < class T, int V >
+struct alignas( sizeof( T ) * V ) ValuePack
+{
+   T v[V];
+};
+// values a lane of the interleaved sweeps takes: 8 or 16 bytes, at most all vectors
+template < class T >
+constexpr int kPackLog = sizeof( T ) == 2 ? 2 : 1;
+template < class T, class F >
+static void forPack( int lv, F&& f )
+{
+   if ( lv >= kPackLog< T > )
+      f( std::integral_constant< int, kPackLog< T > >{} );
+   else if ( lv == 1 )
+      f( std::integral_constant< int, 1 >{} );
+   else
+      f( std::integral_constant< int, 0 >{} );
+}
+
 // SOR on the cell-interior points of the two parity colours (cx, cy, cz) and
 // (1 - cx, cy, cz) of one row group, in place: colour cxFirst first, then the
 // other.  The only stencil neighbours of a point that lie in rows of the same
@@ -721,7 +742,10 @@ static const uint64_t* p1BrickList( Context* ctx, Lattice& l )
 // first through the row alone; a row's lanes are in one wavefront, and a
 // workgroup-scope fence between the two passes makes the first pass's stores
 // visible to the second (the result is that of two colour sweeps in turn).
-template < class T >
+// Interleaved functions; a lane takes 2^lgV vectors.  Bound by the rounds of loads of a
+// row: 64 FP16 vectors, cube level 6, a launch: 19.8 us with a lane a vector, 15.0 us with four
+// (31 rounds of 16 two-byte loads a row, now 8 of eight-byte loads).
+template < class T, int lgV >
 __global__ __launch_bounds__( 64 * kCellWorkers ) void kCellSOR( const int32_t* __restrict__ rows, int64_t nrows,
                                                                  int64_t nc, int64_t sc, int64_t w, int64_t mm,
                                                                  const double* __restrict__ stencil, int cxFirst,
@@ -729,6 +753,8 @@ __global__ __launch_bounds__( 64 * kCellWorkers ) void kCellSOR( const int32_t* 
                                                                  T* __restrict__ x, int lv, int rpbLog )
 {
    using A              = typename Acc< T >::type;
+   constexpr int   V    = 1 << lgV;
+   using P              = ValuePack< T, V >;
    const int64_t   nrc  = nrows * nc;
    const RowWorker rw   = rowWorker( nrc, rpbLog );
    if ( rw.row >= nrc )
@@ -744,28 +770,35 @@ __global__ __launch_bounds__( 64 * kCellWorkers ) void kCellSOR( const int32_t* 
    for ( int q = 0; q < 15; ++q )
       st[q] = A( stencil[15 * c + q] );
    const A       invc = A( 1 ) / st[0];
-   const int32_t msk = ( 1 << lv ) - 1, top = int32_t( mm ) - y - z;
+   const int32_t lvp = lv - lgV, msk = ( 1 << lvp ) - 1, top = int32_t( mm ) - y - z;
    for ( int ph = 0; ph < 2; ++ph )
    {
       const int32_t x0 = ( ph ? 1 - cxFirst : cxFirst ) ? 1 : 2;
       for ( int32_t t = rw.lane;; t += rw.lanes )
       {
-         const int32_t xx = x0 + 2 * ( t >> lv ), k = t & msk;
+         const int32_t xx = x0 + 2 * ( t >> lvp ), k = ( t & msk ) << lgV;
          if ( xx >= top )
             break;
          const int32_t o = ( sr.at( 0, xx ) << lv ) + k;
          // all loads in flight before the sum (same order of the sum)
-         T val[15];
+         P val[15];
 #pragma unroll
          for ( int q = 0; q < 15; ++q )
-            val[q] = xc[( sr.at( q, xx ) << lv ) + k];
-         A v = toAcc( bc[o] );
+            val[q] = *reinterpret_cast< const P* >( xc + ( ( sr.at( q, xx ) << lv ) + k ) );
+         const P rhs = *reinterpret_cast< const P* >( bc + o );
          __builtin_amdgcn_sched_barrier( 0 ); // keeps the scheduler from moving the loads down to their uses
+         P out;
 #pragma unroll
-         for ( int q = 1; q < 15; ++q )
-            v -= st[q] * toAcc( val[q] );
-         const A xo = toAcc( val[0] );
-         xc[o]      = fromAcc< T >( ( A( 1 ) - A( relax ) ) * xo + A( relax ) * invc * v );
+         for ( int l = 0; l < V; ++l )
+         {
+            A v = toAcc( rhs.v[l] );
+#pragma unroll
+            for ( int q = 1; q < 15; ++q )
+               v -= st[q] * toAcc( val[q].v[l] );
+            const A xo = toAcc( val[0].v[l] );
+            out.v[l]   = fromAcc< T >( ( A( 1 ) - A( relax ) ) * xo + A( relax ) * invc * v );
+         }
+         *reinterpret_cast< P* >( xc + o ) = out;
       }
       if ( ph == 0 )
          __threadfence_block();
@@ -1047,44 +1080,9 @@ __global__ void __launch_bounds__( kBlock ) kBndApplySell( int64_t nblk, int64_t
    dst[o] = fromAcc< T >( s );
 }
 
-// SOR on boundary slot i of the sliced rows (vector vec)
-template < class T >
-__device__ __forceinline__ void bndSorSlot( int64_t i, int64_t vec, const int32_t* __restrict__ rowOf,
-                                            const uint8_t* __restrict__ bndFlag, int flag,
-                                            const int64_t* __restrict__ off, const int32_t* __restrict__ pos,
-                                            const double* __restrict__ val, int64_t ownerBase,
-                                            const double* __restrict__ invDiag, double relax, const T* __restrict__ rhs,
-                                            T* __restrict__ x, int lv )
-{
-   using A         = typename Acc< T >::type;
-   const int32_t b = rowOf[i];
-   if ( b < 0 || !( bndFlag[b] & flag ) )
-      return;
-   const int64_t sl = i / kSellRows, e0 = off[sl] + ( i % kSellRows ), w = ( off[sl + 1] - off[sl] ) / kSellRows;
-   const int64_t o  = ( ( ownerBase + b ) << lv ) + vec;
-   A             s  = toAcc( rhs[o] );
-   for ( int64_t j = 0; j < w; j += kSellUnroll )
-   {
-      int32_t p[kSellUnroll];
-      double  v[kSellUnroll];
-      A       xv[kSellUnroll];
-#pragma unroll
-      for ( int u = 0; u < kSellUnroll; ++u )
-      {
-         p[u] = pos[e0 + ( j + u ) * kSellRows];
-         v[u] = val[e0 + ( j + u ) * kSellRows];
-      }
-#pragma unroll
-      for ( int u = 0; u < kSellUnroll; ++u )
-         xv[u] = toAcc( x[( int64_t( p[u] ) << lv ) + vec] );
-#pragma unroll
-      for ( int u = 0; u < kSellUnroll; ++u )
-         s -= A( v[u] ) * xv[u];
-   }
-   x[o] = fromAcc< T >( ( A( 1 ) - A( relax ) ) * toAcc( x[o] ) + A( relax ) * A( invDiag[b] ) * s );
-}
-
-template < class T >
+// SOR on the boundary rows of one colour (slots of the sliced rows), 2^lgV vectors a lane
+// (64 FP16 vectors, cube level 6, a launch: 5.3 us one vector a lane, 4.5 us four)
+template < class T, int lgV >
 __global__ void __launch_bounds__( kBlock ) kBndSORSell( int64_t nblk, int64_t slot0, int64_t nslot,
                                                         const int32_t* __restrict__ rowOf,
                                                         const uint8_t* __restrict__ bndFlag, int flag,
@@ -1093,13 +1091,53 @@ __global__ void __launch_bounds__( kBlock ) kBndSORSell( int64_t nblk, int64_t s
                                                         const double* __restrict__ invDiag, double relax,
                                                         const T* __restrict__ rhs, T* __restrict__ x, int lv )
 {
+   using A         = typename Acc< T >::type;
+   constexpr int V = 1 << lgV;
+   using P         = ValuePack< T, V >;
    const int64_t lb = xcdBlock( nblk );
    if ( lb >= nblk )
       return;
    const int64_t tid = lb * kBlock + threadIdx.x;
-   const int64_t li = tid >> lv, vec = tid & ( ( int64_t( 1 ) << lv ) - 1 );
-   if ( li < nslot )
-      bndSorSlot( slot0 + li, vec, rowOf, bndFlag, flag, off, pos, val, ownerBase, invDiag, relax, rhs, x, lv );
+   const int64_t li = tid >> ( lv - lgV ), vec = ( tid & ( ( int64_t( 1 ) << ( lv - lgV ) ) - 1 ) ) << lgV;
+   if ( li >= nslot )
+      return;
+   const int64_t i = slot0 + li;
+   const int32_t b = rowOf[i];
+   if ( b < 0 || !( bndFlag[b] & flag ) )
+      return;
+   const int64_t sl = i / kSellRows, e0 = off[sl] + ( i % kSellRows ), w = ( off[sl + 1] - off[sl] ) / kSellRows;
+   const int64_t o  = ( ( ownerBase + b ) << lv ) + vec;
+   const P       f  = *reinterpret_cast< const P* >( rhs + o );
+   A             s[V];
+#pragma unroll
+   for ( int l = 0; l < V; ++l )
+      s[l] = toAcc( f.v[l] );
+   for ( int64_t j = 0; j < w; j += kSellUnroll )
+   {
+      int32_t p[kSellUnroll];
+      double  v[kSellUnroll];
+      P       xv[kSellUnroll];
+#pragma unroll
+      for ( int u = 0; u < kSellUnroll; ++u )
+      {
+         p[u] = pos[e0 + ( j + u ) * kSellRows];
+         v[u] = val[e0 + ( j + u ) * kSellRows];
+      }
+#pragma unroll
+      for ( int u = 0; u < kSellUnroll; ++u )
+         xv[u] = *reinterpret_cast< const P* >( x + ( ( int64_t( p[u] ) << lv ) + vec ) );
+#pragma unroll
+      for ( int u = 0; u < kSellUnroll; ++u )
+#pragma unroll
+         for ( int l = 0; l < V; ++l )
+            s[l] -= A( v[u] ) * toAcc( xv[u].v[l] );
+   }
+   const P xo = *reinterpret_cast< const P* >( x + o );
+   P       out;
+#pragma unroll
+   for ( int l = 0; l < V; ++l )
+      out.v[l] = fromAcc< T >( ( A( 1 ) - A( relax ) ) * toAcc( xo.v[l] ) + A( relax ) * A( invDiag[b] ) * s[l] );
+   *reinterpret_cast< P* >( x + o ) = out;
 }
 
 // A whole SOR sweep in one workgroup (per 2^lg vectors of an interleaved function), x in
@@ -1658,10 +1696,13 @@ void p1SOR( Context* ctx, P1Operator& op, Function& x, Function& b, double relax
          {
             const SellRows& sr    = o.sorRows;
             const int64_t   slot0 = o.sorColorStart[cc], ns = o.sorColorStart[cc + 1] - slot0;
-            const int64_t   nblk  = ( ( ns << lv ) + kBlock - 1 ) / kBlock;
-            kBndSORSell< T ><<< xcdGrid( nblk ), kBlock, 0, ctx->stream >>>(
-                nblk, slot0, ns, sr.row.p, lat.bndFlag.p, flag, sr.off.p, sr.pos.p, sr.val.p, lat.nc * lat.sc,
-                o.invDiag.p, relax, (const T*) bp, (T*) xp, lv );
+            forPack< T >( lv, [&]( auto lg ) {
+               constexpr int lgV  = decltype( lg )::value;
+               const int64_t nblk = ( ( ns << ( lv - lgV ) ) + kBlock - 1 ) / kBlock;
+               kBndSORSell< T, lgV ><<< xcdGrid( nblk ), kBlock, 0, ctx->stream >>>(
+                   nblk, slot0, ns, sr.row.p, lat.bndFlag.p, flag, sr.off.p, sr.pos.p, sr.val.p, lat.nc * lat.sc,
+                   o.invDiag.p, relax, (const T*) bp, (T*) xp, lv );
+            } );
          }
          else
             kBndSOR< T ><<< gridFor( n << lv ), kBlock, 0, ctx->stream >>>( g, n, o.colorRows.p + o.colorStart[cc],
@@ -1687,10 +1728,16 @@ void p1SOR( Context* ctx, P1Operator& op, Function& x, Function& b, double relax
             HG_CHECK_HIP( hipGetLastError() );
             return;
          }
-         const int rpb = rowsPerBlockLog( ( ( lat.mm - 2 ) / 2 ) << lv );
-         kCellSOR< T ><<< cellGrid( n * lat.nc, rpb ), 64 * kCellWorkers, 0, ctx->stream >>>(
-             lat.rows.p + 2 * lat.rowGroup[grp], n, lat.nc, lat.sc, lat.w, lat.mm, o.stencil.p, cxFirst, relax,
-             (const T*) bp, (T*) xp, lv, rpb );
+         forPack< T >( lv, [&]( auto lg ) {
+            constexpr int lgV = decltype( lg )::value;
+            if constexpr ( lgV > 0 ) // single vectors: above
+            {
+               const int rpb = rowsPerBlockLog( ( ( lat.mm - 2 ) / 2 ) << ( lv - lgV ) );
+               kCellSOR< T, lgV ><<< cellGrid( n * lat.nc, rpb ), 64 * kCellWorkers, 0, ctx->stream >>>(
+                   lat.rows.p + 2 * lat.rowGroup[grp], n, lat.nc, lat.sc, lat.w, lat.mm, o.stencil.p, cxFirst, relax,
+                   (const T*) bp, (T*) xp, lv, rpb );
+            }
+         } );
          HG_CHECK_HIP( hipGetLastError() );
       };
       const size_t nbc      = o.colorStart.empty() ? 0 : o.colorStart.size() - 1;

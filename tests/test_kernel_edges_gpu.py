@@ -57,6 +57,33 @@ def test_p1_sweep_variants_equal_the_interleaved_sweep(ctx, name, levels, dtype)
             f.destroy()
 
 
+@pytest.mark.parametrize("dtype", [hg.F64, hg.F32, hg.F16])
+@pytest.mark.parametrize("nvec", [2, 4, 8, 64])
+def test_p1_interleaved_sweep_by_vectors_a_lane(ctx, nvec, dtype):
+    """every width of the interleaved sweep's packs (1, 2 or 4 vectors a lane) on levels
+    with more and with fewer points a row than a wavefront takes: each vector as alone"""
+    st = hg.PrimitiveStorage.cuboid(ctx)
+    for L in (3, 5):
+        A = hg.P1ConstantLaplaceOperator(st, L, L)
+        n = st.ndofs(L)
+        rng = np.random.default_rng(nvec + L)
+        x0, b = rng.uniform(-1, 1, (n, nvec)), rng.uniform(-1, 1, (n, nvec))
+        xb, bb = (hg.P1Function("f", st, L, L, dtype, nvec=nvec) for _ in range(2))
+        xs, bs = (hg.P1Function("g", st, L, L, dtype) for _ in range(2))
+        xb.upload(L, x0)
+        bb.upload(L, b)
+        print(f"P1 interleaved sweep L{L} nvec {nvec} dtype {dtype}", flush=True)
+        A.smooth_sor(xb, bb, 1.1, L, hg.GMG_FLAG)
+        got = xb.download(L)
+        for k in {0, 1, nvec // 2, nvec - 1}:
+            xs.upload(L, x0[:, k])
+            bs.upload(L, b[:, k])
+            A.smooth_sor(xs, bs, 1.1, L, hg.GMG_FLAG)
+            assert relmax(got[:, k], xs.download(L)) <= 64 * EPS[dtype], (L, k)
+        for f in (xb, bb, xs, bs):
+            f.destroy()
+
+
 @pytest.mark.parametrize("name,L", [("cube", 4), ("cube", 5), ("cube", 6), ("octa", 4)])
 def test_p2_constant_sweep_equals_the_sweep_by_colours(ctx, name, L):
     st = _storage(ctx, name)
