@@ -38,10 +38,9 @@ sys.path.insert(0, ROOT)
 HBM_PEAK_GBS = 8000.0
 FP64_PEAK_TFLOPS = 78.6
 # FP64 operations of one micro-cell action in kP2TileApplyStored<double>, counted
-# from its instruction stream (FMA = 2): 11 quadrature points x (43 FMA + 21 MUL +
-# 5 ADD + 2 reciprocal / reciprocal-sqrt seeds) + about 230 for the gradient set-up
-# and the result = 1484
-P2_FLOPS_PER_ELEMENT = 11 * (2 * 43 + 21 + 5 + 2) + 230
+# from its instruction stream (FMA = 2; 11 quadrature points, gradient set-up and
+# result together): 386 FMA + 164 MUL + 128 ADD + 11 reciprocal seeds = 1075
+P2_FLOPS_PER_ELEMENT = 2 * 386 + 164 + 128 + 11
 METRIC = "DoF/s per apply; time-to-1e-8 residual mixed vs FP64; solves/s + p99 latency"
 
 
@@ -102,7 +101,7 @@ def p2_shell(hg, ctx, L, steps, warmup):
     roof = {"bound": "hbm", "achieved": alg / (kms * 1e-3) / 1e9, "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "algorithmic_bytes_per_launch": alg,
             "note": "algorithmic bytes = 24 per P2 DoF (src, dst, one k value, FP64); the exact "
-                    "p2_div_k_grad_blending_q4 element integration issues ~1.5 kflop FP64 per micro-cell, so "
+                    "p2_div_k_grad_blending_q4 element integration issues ~1.1 kflop FP64 per micro-cell, so "
                     "the kernel is bound by FP64 VALU issue and latency, not by HBM (compute_fp64 below)",
             "compute_fp64": {"achieved_tflops": P2_FLOPS_PER_ELEMENT * nelem / (kms * 1e-3) / 1e12,
                              "peak_tflops": FP64_PEAK_TFLOPS,
