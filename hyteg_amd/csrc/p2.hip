@@ -2077,7 +2077,7 @@ __global__ __launch_bounds__( kCgThreads ) void kP2AssembledCG( int32_t n, int32
       for ( int32_t i = threadIdx.x; i < n; i += kCgThreads )
          pap += inv[i] != 0.0 ? sp[i] * sa[i] : 0.0;
       cgSum( pap, none, red[0] );
-      const double alpha = rz / pap;
+      const double alpha = pap == 0.0 ? 0.0 : rz / pap; // 0 / 0 once r = 0: no step (slotCoef)
       for ( int32_t i = threadIdx.x; i < n; i += kCgThreads )
       {
          const double d = inv[i], ap = sa[i];
@@ -2095,7 +2095,7 @@ __global__ __launch_bounds__( kCgThreads ) void kP2AssembledCG( int32_t n, int32
       const double res  = sqrt( rr );
       const bool   done = res / r0 < relTol || res < absTol || its + 1.0 >= double( maxIter );
       const bool   stop = done || k + 1 == perLaunch;
-      const double beta = rzn / rz;
+      const double beta = rz == 0.0 ? 0.0 : rzn / rz;
       rz                = rzn;
       if ( !done )
          for ( int32_t i = threadIdx.x; i < n; i += kCgThreads )

@@ -178,6 +178,31 @@ def test_p2_cg_runs_on_over_several_launches(ctx):
     A.destroy()
 
 
+@pytest.mark.parametrize("jacobi", [True, False])
+def test_p2_cg_stands_still_at_a_zero_residual(ctx, jacobi):
+    """iterations after the residual is exactly zero (one free DoF, or b = 0), zero
+    tolerances: the ratios 0 / 0 count as 0 and x keeps the solution"""
+    st = hg.PrimitiveStorage.cuboid(ctx)
+    A = hg.P2DivKGradOperator(st, 0, 0, *problems.shell_coefficient(3))
+    free = (st.flags(1) & hg.GMG_FLAG) != 0
+    assert free.sum() == 1
+    x, fb, y = (hg.P2Function("f", st, 0, 0) for _ in range(3))
+    A.inverse_diagonal(0, y)
+    inv = y.download(0)[free]
+    for b in (0.0, 0.7):
+        fb.upload(0, np.where(free, b, 0.0))
+        x.upload(0, np.zeros(len(free)))
+        print(f"P2 CG from a zero residual, b {b}, jacobi {jacobi}", flush=True)
+        assert hg.p2_cg_solve(A, x, fb, 0, 25, 0.0, 0.0, jacobi) == 24
+        got = x.download(0)
+        assert np.all(got[~free] == 0.0)
+        # the diagonal: a sum of at most 24 micro-cells times 11 points, in another order
+        assert abs(got[free] - b * inv) <= 512 * EPS[hg.F64] * abs(b * inv)
+    for f in (x, fb, y):
+        f.destroy()
+    A.destroy()
+
+
 @pytest.mark.parametrize("dtype", [hg.F64, hg.F32, hg.F16])
 @pytest.mark.parametrize("name,L", [("cube", 5), ("octa", 4)])
 def test_p2_restriction_into_large_levels(ctx, name, L, dtype):
