@@ -907,7 +907,8 @@ class CGSolver : public Solver< OperatorType >
       if constexpr ( std::is_same_v< OperatorType, P2ElementwiseBlendingDivKGradOperatorT< double > > )
       {
          const bool jacobi = dynamic_cast< InverseDiagonalPreconditioner< OperatorType >* >( prec_.get() ) != nullptr;
-         if ( !fixed_ && ( !prec_ || jacobi ) )
+         // its DoF types are the mesh's: not for an x that counts every DoF as Inner
+         if ( !fixed_ && !x.isAllInner() && ( !prec_ || jacobi ) )
          {
             int its = 0, applied = 0;
             check( ctx_,
