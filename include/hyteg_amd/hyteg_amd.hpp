@@ -26,6 +26,7 @@
 #include <stdexcept>
 #include <string>
 #include <type_traits>
+#include <typeinfo>
 #include <utility>
 #include <vector>
 
@@ -906,9 +907,11 @@ class CGSolver : public Solver< OperatorType >
       // the P2 diffusion operator solves its small levels in one launch
       if constexpr ( std::is_same_v< OperatorType, P2ElementwiseBlendingDivKGradOperatorT< double > > )
       {
-         const bool jacobi = dynamic_cast< InverseDiagonalPreconditioner< OperatorType >* >( prec_.get() ) != nullptr;
-         // its DoF types are the mesh's: not for an x that counts every DoF as Inner
-         if ( !fixed_ && !x.isAllInner() && ( !prec_ || jacobi ) )
+         // its DoF types are the mesh's: not for an x that counts every DoF as Inner; its
+         // operator and preconditioner are these classes themselves, not derived ones
+         const Solver< OperatorType >* prec = prec_.get();
+         const bool jacobi = prec && typeid( *prec ) == typeid( InverseDiagonalPreconditioner< OperatorType > );
+         if ( !fixed_ && !x.isAllInner() && typeid( A ) == typeid( OperatorType ) && ( !prec || jacobi ) )
          {
             int its = 0, applied = 0;
             check( ctx_,

@@ -135,6 +135,9 @@ def _run(program, what):
     ("fixed", (0, 1, 0, 0)),
     # x with every DoF counted as Inner: the call's DoF types are the mesh's
     ("all_inner", (0, 1, 1, 0)),
+    # classes derived from the operator and from the preconditioner override its steps
+    ("operator", (0, 1, 0, 0)),
+    ("preconditioner", (0, 1, 1, 0)),
 ])
 def test_cg_uses_the_one_launch_solve_only_where_it_is_its_own(program, what, expected):
     assert _run(program, what) == expected
