@@ -817,10 +817,13 @@ class CGSolver : public Solver< OperatorType >
    , z_( "z", storage, minLevel, maxLevel )
    , ap_( "ap", storage, minLevel, maxLevel )
    , r_( "r", storage, minLevel, maxLevel )
+   , minLevel_( minLevel )
+   , maxLevel_( maxLevel )
    {
       if constexpr ( kDeviceScalars )
       {
-         ctx_ = storage->ctx();
+         ctx_     = storage->ctx();
+         storage_ = storage->handle();
          check( ctx_, hg_slots_alloc( ctx_, kSlotCount, &slot0_ ), "CGSolver slots" );
       }
    }
@@ -911,7 +914,8 @@ class CGSolver : public Solver< OperatorType >
          // operator and preconditioner are these classes themselves, not derived ones
          const Solver< OperatorType >* prec = prec_.get();
          const bool jacobi = prec && typeid( *prec ) == typeid( InverseDiagonalPreconditioner< OperatorType > );
-         if ( !fixed_ && !x.isAllInner() && typeid( A ) == typeid( OperatorType ) && ( !prec || jacobi ) )
+         if ( !fixed_ && !x.isAllInner() && typeid( A ) == typeid( OperatorType ) && ( !prec || jacobi ) &&
+              workspaceFits( x, level ) )
          {
             int its = 0, applied = 0;
             check( ctx_,
@@ -988,6 +992,15 @@ class CGSolver : public Solver< OperatorType >
       }
    }
 
+   // whether p, z, ap and r hold the level and live on x's storage (the loop fails
+   // where they do not)
+   bool workspaceFits( const FunctionType& x, uint_t level ) const
+   {
+      hg_handle s = 0;
+      check( ctx_, hg_function_storage( ctx_, x.handle(), &s ), "CGSolver" );
+      return s == storage_ && level >= minLevel_ && level <= maxLevel_;
+   }
+
    // z = M^-1 r (identity when no preconditioner is given)
    void precondition( const OperatorType& A, uint_t level )
    {
@@ -1000,9 +1013,11 @@ class CGSolver : public Solver< OperatorType >
    ValueType                                 relTol_, absTol_;
    std::shared_ptr< Solver< OperatorType > > prec_;
    FunctionType                              p_, z_, ap_, r_;
+   uint_t                                    minLevel_, maxLevel_;
    DoFType                                   flag_       = Inner | NeumannBoundary | FreeslipBoundary;
    uint_t                                    iterations_ = 0;
    hg_ctx*                                   ctx_        = nullptr;
+   hg_handle                                 storage_    = 0;
    int                                       slot0_      = -1;
    bool                                      fixed_      = false;
 };

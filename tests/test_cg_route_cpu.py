@@ -138,6 +138,9 @@ def _run(program, what):
     # classes derived from the operator and from the preconditioner override its steps
     ("operator", (0, 1, 0, 0)),
     ("preconditioner", (0, 1, 1, 0)),
+    # a level or a storage that the solver was not made for
+    ("level", (0, 0, 0, 1)),
+    ("storage", (0, 1, 0, 1)),
 ])
 def test_cg_uses_the_one_launch_solve_only_where_it_is_its_own(program, what, expected):
     assert _run(program, what) == expected
