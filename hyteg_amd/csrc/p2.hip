@@ -2134,6 +2134,12 @@ static bool p2AssembledCG( Context* ctx, P2Operator& op, Function& x, Function& 
    const P2Pattern* pat = p2Pattern( ctx, *op.st, L );
    if ( !pat || maxIter < 1 )
       return false;
+   // the tables of the level's applies, as the launch-by-launch iteration leaves them: an
+   // apply captured after the solve cannot allocate them
+   p2Coefficients< double >( ctx, op, L, 0 );
+   if ( ( int64_t( 1 ) << L ) > kSmallMaxMM )
+      for ( int kind : { kTilesInterior, kTilesLast } )
+         tileList( ctx, op.st->lattice( ctx, L + 1 ), int64_t( 1 ) << L, kind );
    auto& mat = op.assembled[L];
    if ( !mat.p )
    {

@@ -925,6 +925,9 @@ class CGSolver : public Solver< OperatorType >
                    "CGSolver" );
             if ( applied )
             {
+               // left behind as by the loop: a solve captured later cannot allocate it
+               if ( jacobi )
+                  A.getInverseDiagonalValues();
                iterations_ = uint_t( its );
                return;
             }

@@ -11,11 +11,14 @@ the oracle:
 * P2 restriction into levels whose face points fill several wavefronts;
 * the Stokes blocks over an odd number of interior tiles.
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
 import hyteg_amd as hg
 from hyteg_amd import problems
+from hyteg_amd._lib import lib
 from meshes import octahedron, relmax
 from oracle import pyoracle as po
 from test_stokes_gpu import _apply_parity
@@ -199,6 +202,36 @@ def test_p2_cg_stands_still_at_a_zero_residual(ctx, jacobi):
         # the diagonal: a sum of at most 24 micro-cells times 11 points, in another order
         assert abs(got[free] - b * inv) <= 512 * EPS[hg.F64] * abs(b * inv)
     for f in (x, fb, y):
+        f.destroy()
+    A.destroy()
+
+
+@pytest.mark.parametrize("L", [0, 1, 2])
+def test_an_apply_can_be_captured_after_a_cg_solve(ctx, L):
+    """a solve builds what the applies of its level need (coefficient table, tile lists):
+    a capture, which cannot allocate, finds them"""
+    st = hg.PrimitiveStorage.cuboid(ctx)
+    A = hg.P2DivKGradOperator(st, L, L, *problems.shell_coefficient(3))
+    x, b, y = (hg.P2Function("f", st, L, L) for _ in range(3))
+    rng = np.random.default_rng(L)
+    b.upload(L, np.where(st.flags(L + 1) == hg.INNER, rng.uniform(-1, 1, st.p2_ndofs(L)), 0.0))
+    print(f"P2 apply captured after a CG solve, L{L}", flush=True)
+    hg.p2_cg_solve(A, x, b, L, 20)
+    graph = C.c_int64()
+    ctx.check(lib().hg_graph_begin_capture(ctx.h), "begin capture")
+    try:
+        A.apply(x, y, L, hg.ALL)
+    finally:
+        ctx.check(lib().hg_graph_end_capture(ctx.h, C.byref(graph)), "end capture")
+    A.apply(x, b, L, hg.ALL)
+    ref = b.download(L)
+    for _ in range(3):
+        y.interpolate(0.0, L)
+        ctx.check(lib().hg_graph_launch(ctx.h, graph), "graph launch")
+        # sums of the micro-cells around a DoF by atomics, in any order
+        assert relmax(y.download(L), ref) <= 64 * EPS[hg.F64]
+    ctx.check(lib().hg_graph_destroy(ctx.h, graph), "graph destroy")
+    for f in (x, b, y):
         f.destroy()
     A.destroy()
 
