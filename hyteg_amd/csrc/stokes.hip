@@ -168,24 +168,74 @@ __device__ __forceinline__ QPoint< R > qpoint( const P2CellGeomT< R >& g, const 
 // T is the value type of the functions (double; float or half for the
 // reduced-precision velocity block), the arithmetic runs in Acc<T>.
 //
-// LAST = false: stokesTiles tiles a workgroup, one micro-cell type a wavefront.  LAST =
-// true: a last-layer tile (tileList) by one wavefront, its 64 micro-cells with the type
-// varying over the lanes -- a workgroup of the other form would run six wavefronts for them.
-// Results go through copies of the result box, one a wavefront, one component after the
-// other, with plain LDS reads and writes in the spread layout; LDS atomics on one box took
-// about 2 ms of 14.5 (shell level 5, full operator).
-// Bound by FP64 issue and its latencies at three wavefronts a SIMD (11.1 ms for 117 GFLOP,
-// the vector unit about half busy).  168 registers a lane without spills: two of the three
-// velocity components are read from LDS again at each point of the viscous block (HELD
-// in registers), box points and anchors are formed again for the write-back.
+// Three forms, chosen by stokesForm:
+// kStokesWide: stokesTiles tiles a workgroup, one micro-cell type a wavefront.  Results go
+//   through copies of the result box, one a wavefront, one component after the other, with
+//   plain LDS reads and writes in the spread layout.  Bound by FP64 issue and its latencies
+//   at three wavefronts a SIMD (11.1 ms for 117 GFLOP, the vector unit about half busy).
+//   168 registers a lane (masks 3 and 7 spill three and four, 16 and 20 bytes of scratch):
+//   two of the three velocity components are read from LDS again at each point of the
+//   viscous block (HELD in registers), box points and anchors are formed again for the
+//   write-back.
+// kStokesShared: one tile a workgroup, one result box filled with LDS atomics, the three
+//   components in registers.  Two barriers where the wide form has seven: the shortest
+//   chain, for launches that are bound by one workgroup's latency.
+// kStokesLast: a last-layer tile (tileList) by one wavefront, its 64 micro-cells with the
+//   type varying over the lanes -- a workgroup of the other forms would run six wavefronts
+//   for them.
 constexpr int kPBox3P = 128; // a pressure box, padded
-// Tiles a workgroup: two, for three wavefronts on each SIMD; of a workgroup of six two of
-// the four SIMDs hold two (full operator 11.5 against 10.3 ms, mask 6 11.1 against 9.2 ms,
-// shell level 5).  B^T alone has registers for two workgroups of one tile a CU, which
-// overlap one's memory phases with the other's arithmetic (5.2 against 6.2 ms).
-constexpr int stokesTiles( int mask, bool last ) { return last || mask == 2 ? 1 : 2; }
-template < int MASK, class T, bool LAST >
-__global__ __launch_bounds__( LAST ? 64 : stokesTiles( MASK, LAST ) * kTileThreads, LAST ? 2 : 3 ) void kStokesTileApply(
+enum StokesForm
+{
+   kStokesWide   = 0,
+   kStokesShared = 1,
+   kStokesLast   = 2
+};
+// Tiles a workgroup of the wide form: two, for three wavefronts on each SIMD; of a workgroup
+// of six two of the four SIMDs hold two (full operator 11.5 against 10.3 ms, mask 6 11.1
+// against 9.2 ms, shell level 5).  B^T alone has registers for two workgroups of one tile a
+// CU, which overlap one's memory phases with the other's arithmetic (5.2 against 6.2 ms).
+constexpr int stokesTiles( int mask, int form ) { return form != kStokesWide || mask == 2 ? 1 : 2; }
+// wavefronts a SIMD that the registers leave room for (the shared form's merged divergence
+// loop needs 192 registers)
+constexpr int stokesWaves( int mask, int form )
+{
+   return form == kStokesLast || ( form == kStokesShared && ( ( mask & 1 ) || mask == 6 ) ) ? 2 : 3;
+}
+// The form of a launch over n tiles of lattices with mm micro-edges; kStokesLast: the
+// interior tiles in the wide form and the last layer behind them.  Kernel times in us of
+// shared / wide / wide and last, n tiles, on 256 CUs:
+//   mask 7: 19 / 29 / 44 (cube level 4, 120), 35 / 33 / 48 (480), 50 / 57 / 49 (720),
+//           428 / 439 / 365 (7200); level 1: 17 / 28 (36), 118 / 109 (1920)
+//   mask 2: 9.5 / 11 / 19 (24), 21 / 23 / 26 (720), 274 / 306 / 306 (14400),
+//           737 / 864 / 717 (38400); level 3: 144 / 173 / 111 (7680)
+//   mask 4: 9.2 / 9.9 / 17 (24), 25 / 25 / 26 (1200), 44 / 39 / 35 (2400)
+//   mask 6: 12 / 18 / 29 (24), 51 / 58 / 57 (1200), 93 / 94 / 86 (2400)
+//   mask 8: 7.4 / 7.7 / 12 (24), 13 / 14 / 16 (1200), 23 / 20 / 19 (2400)
+//   FP32 velocities: 22 / 16 / 28 (24), 141 / 70 / 73 (2400), 258 / 136 / 115 (4800);
+//           level 1: 11 / 15 (36)
+// Up to a tile a CU the chain of one workgroup counts (shared; FP32 has cheap wavefront
+// boxes and expensive atomics), up to two a CU the wide form still is one round; beyond,
+// the last layer by wavefronts saves more than its launch costs, later for the masks with
+// less arithmetic.  On levels 0 and 1 a tile holds few micro-cells.
+inline int stokesForm( int mask, bool fp32, int64_t mm, int64_t n )
+{
+   const bool viscous = mask & 1;
+   if ( mm < kTile )
+      return n <= 512 || mask == 2 || fp32 ? kStokesShared : kStokesWide;
+   if ( mm == kTile ) // every tile is in the last layer
+      return n <= 256 && ( fp32 || !( viscous || mask == 8 ) ) ? kStokesShared : kStokesLast;
+   if ( fp32 )
+      return n <= 3072 ? kStokesWide : kStokesLast;
+   if ( mask == 2 )
+      return n <= ( mm == 2 * kTile ? 512 : 16384 ) ? kStokesShared : kStokesLast;
+   if ( n <= ( mask == 8 ? 2048 : 512 ) )
+      return n <= 256 ? kStokesShared : kStokesWide;
+   // (of eight micro-edges three tiles in four are in the last layer)
+   return viscous || mask == 8 || n > 1440 || mm == 2 * kTile ? kStokesLast : kStokesShared;
+}
+template < int MASK, class T, int FORM >
+__global__ __launch_bounds__( FORM == kStokesLast ? 64 : stokesTiles( MASK, FORM ) * kTileThreads,
+                              stokesWaves( MASK, FORM ) ) void kStokesTileApply(
     const P2CellGeomT< typename Acc< T >::type >* __restrict__ geom, typename Acc< T >::type c0,
     typename Acc< T >::type c1, int64_t mm, int64_t ntiles, int64_t sc1, int64_t w1, int64_t sc0, int64_t w0,
     const T* __restrict__ u0, const T* __restrict__ u1, const T* __restrict__ u2, const T* __restrict__ pin,
@@ -194,18 +244,21 @@ __global__ __launch_bounds__( LAST ? 64 : stokesTiles( MASK, LAST ) * kTileThrea
    using R  = typename Acc< T >::type;
    using QC = SQ< R >;
    constexpr bool DO_A = MASK & 1, DO_BT = MASK & 2, DO_B = MASK & 4, DO_M = MASK & 8;
-   constexpr int HELD = LAST || sizeof( R ) == 4 ? 3 : 1;
+   constexpr bool LAST = FORM == kStokesLast, SHARED = FORM == kStokesShared;
+   constexpr int HELD = LAST || SHARED || sizeof( R ) == 4 ? 3 : 1;
+   constexpr bool MERGED = SHARED && DO_B && DO_BT; // one loop over the divergence points
    constexpr bool NEED_U = DO_A || DO_B, OUT_U = DO_A || DO_BT, NEED_P = DO_BT || DO_M, OUT_P = DO_B || DO_M;
    constexpr int  kThreads = LAST ? 64 : kTileThreads, kWaves = kThreads / 64;
    constexpr int  kPoints  = LAST ? kDiagBoxP / 64 : 2; // velocity box points a thread
    constexpr int  kPPoints = LAST ? 2 : 1;              // and pressure box points
    static_assert( LAST || kBox3 <= 2 * kTileThreads, "box points per thread" );
    // the tile's velocity values and, when they have been used, the wavefronts' result boxes
-   constexpr int kULds = ( OUT_U && kWaves > 3 ? kWaves : 3 ) * kSpreadBox;
-   constexpr int kTiles = stokesTiles( MASK, LAST );
+   // (SHARED: the one result box behind them)
+   constexpr int kULds = ( SHARED ? ( NEED_U ? 3 : 0 ) + ( OUT_U ? 3 : 0 ) : OUT_U && kWaves > 3 ? kWaves : 3 ) * kSpreadBox;
+   constexpr int kTiles = stokesTiles( MASK, FORM ), kPCopies = SHARED ? 1 : kWaves;
    __shared__ R  suAll[kTiles][NEED_U || OUT_U ? kULds : 1];
    __shared__ R  spAll[kTiles][NEED_P ? kPBox3P : 1];
-   __shared__ R  apAll[kTiles][OUT_P ? kWaves * kPBox3P : 1];
+   __shared__ R  apAll[kTiles][OUT_P ? kPCopies * kPBox3P : 1];
    const int64_t lw = xcdBlock( ( ntiles + kTiles - 1 ) / kTiles );
    if ( lw * kTiles >= ntiles )
       return;
@@ -214,6 +267,7 @@ __global__ __launch_bounds__( LAST ? 64 : stokesTiles( MASK, LAST ) * kTileThrea
    R* const      su  = suAll[sub];
    R* const      sp  = spAll[sub];
    R* const      ap  = apAll[sub];
+   R* const      au  = su + ( SHARED && NEED_U ? 3 * kSpreadBox : 0 ); // result boxes
    const int     tid0 = wave * 64 + lane; // thread number in the tile
    const bool    live = lw * kTiles + sub < ntiles;
    const int64_t lb   = live ? lw * kTiles + sub : ntiles - 1;
@@ -258,6 +312,16 @@ __global__ __launch_bounds__( LAST ? 64 : stokesTiles( MASK, LAST ) * kTileThrea
          poff[j] = pressurePoint( tid0, j );
          pvl[j]  = poff[j] >= 0 ? ( pin + base0 )[uint32_t( poff[j] )] : T( 0 );
       }
+   if constexpr ( SHARED )
+   {
+      // cleared while the loads are in flight
+      if constexpr ( OUT_U )
+         for ( int p = tid0; p < 3 * kSpreadBox; p += kThreads )
+            au[p] = R( 0 );
+      if constexpr ( OUT_P )
+         if ( tid0 < kPBox3P )
+            ap[tid0] = R( 0 );
+   }
    if constexpr ( NEED_U )
    {
 #pragma unroll
@@ -316,13 +380,16 @@ __global__ __launch_bounds__( LAST ? 64 : stokesTiles( MASK, LAST ) * kTileThrea
    };
    // LDS accesses of a wavefront to its own copies: volatile, they complete in order
    using LdsR = volatile __attribute__( ( address_space( 3 ) ) ) R;
-   LdsR* const apw = (LdsR*) ( ap + ( OUT_P ? wave * kPBox3P : 0 ) );
+   LdsR* const apw = (LdsR*) ( ap + ( OUT_P && !SHARED ? wave * kPBox3P : 0 ) );
    auto pressureResults = [&]( const R yq[4] ) {
-      apw[lane]      = R( 0 );
-      apw[lane + 64] = R( 0 );
+      if constexpr ( !SHARED )
+      {
+         apw[lane]      = R( 0 );
+         apw[lane + 64] = R( 0 );
+      }
       if ( th.valid )
       {
-         if constexpr ( LAST )
+         if constexpr ( LAST || SHARED )
 #pragma unroll
             for ( int k = 0; k < 4; ++k )
                atomicAdd( &ap[ppos( k )], yq[k] );
@@ -346,15 +413,38 @@ __global__ __launch_bounds__( LAST ? 64 : stokesTiles( MASK, LAST ) * kTileThrea
             u[c][i] = base[at( i )];
       } );
    };
+   auto clear = [&]() {
+#pragma unroll
+      for ( int c = 0; c < 3; ++c )
+#pragma unroll
+         for ( int i = 0; i < 10; ++i )
+            y[c][i] = R( 0 );
+   };
+   // y += s (q div of the test functions)
+   auto gradientTests = [&]( const R* a4, const R* b4, R s, const R M[3][3] ) {
+#pragma unroll
+      for ( int c = 0; c < 3; ++c )
+         testGrad( a4, b4, s * M[c][0], s * M[c][1], s * M[c][2], y[c] );
+   };
    if constexpr ( NEED_U )
 #pragma unroll
       for ( int c = 0; c < 3; ++c )
          component( c );
+   // a wavefront without micro-cells in the macro-cell (lattices of one or two micro-edges)
+   // has no quadrature points
+   const bool work = __any( th.valid );
+   const int  qA = work ? 5 : 0, qB = work ? 9 : 0;
+   if constexpr ( MERGED )
+      clear();
    if constexpr ( DO_B )
    {
-      R yq[4] = { R( 0 ), R( 0 ), R( 0 ), R( 0 ) };
+      R pv[4], yq[4] = { R( 0 ), R( 0 ), R( 0 ), R( 0 ) };
+      if constexpr ( MERGED )
+#pragma unroll
+         for ( int k = 0; k < 4; ++k )
+            pv[k] = sp[ppos( k )];
 #pragma unroll 1
-      for ( int q = 5; q < 9; ++q )
+      for ( int q = 5; q < qB; ++q )
       {
          const R*          a4  = QC::a4( q );
          const R*          b4  = QC::b4( q );
@@ -376,18 +466,17 @@ __global__ __launch_bounds__( LAST ? 64 : stokesTiles( MASK, LAST ) * kTileThrea
 #pragma unroll
          for ( int k = 0; k < 4; ++k )
             yq[k] += lam[k] * s;
+         if constexpr ( MERGED )
+            gradientTests( a4, b4, -cc * ( lam[0] * pv[0] + lam[1] * pv[1] + lam[2] * pv[2] + lam[3] * pv[3] ), M );
       }
       pressureResults( yq );
    }
-#pragma unroll
-   for ( int c = 0; c < 3; ++c )
-#pragma unroll
-      for ( int i = 0; i < 10; ++i )
-         y[c][i] = R( 0 );
+   if constexpr ( !MERGED )
+      clear();
    if constexpr ( DO_A )
    {
 #pragma unroll 1
-      for ( int q = 0; q < 5; ++q )
+      for ( int q = 0; q < qA; ++q )
       {
          const R* a4 = QC::a4( q );
          const R* b4 = QC::b4( q );
@@ -437,14 +526,14 @@ __global__ __launch_bounds__( LAST ? 64 : stokesTiles( MASK, LAST ) * kTileThrea
                       M[0][2] * S[c][0] + M[1][2] * S[c][1] + M[2][2] * S[c][2], y[c] );
       }
    }
-   if constexpr ( NEED_P )
+   if constexpr ( NEED_P && !MERGED )
    {
       R pv[4], yq[4] = { R( 0 ), R( 0 ), R( 0 ), R( 0 ) };
 #pragma unroll
       for ( int k = 0; k < 4; ++k )
          pv[k] = sp[ppos( k )];
 #pragma unroll 1
-      for ( int q = 5; q < 9; ++q )
+      for ( int q = 5; q < qB; ++q )
       {
          const R*          lam = QC::lam( q );
          const QPoint< R > P   = qpoint( g, th, q );
@@ -462,18 +551,24 @@ __global__ __launch_bounds__( LAST ? 64 : stokesTiles( MASK, LAST ) * kTileThrea
          {
             const R* a4 = QC::a4( q );
             const R* b4 = QC::b4( q );
-            const R  s  = -cc * pq;
             R        M[3][3];
             mapGradients( Dc, P.x, P.w, P.ib, M );
-#pragma unroll
-            for ( int c = 0; c < 3; ++c )
-               testGrad( a4, b4, s * M[c][0], s * M[c][1], s * M[c][2], y[c] );
+            gradientTests( a4, b4, -cc * pq, M );
          }
       }
       if constexpr ( DO_M )
          pressureResults( yq );
    }
-   __syncthreads(); // the velocity values are read
+   if constexpr ( SHARED && OUT_U )
+      if ( th.valid )
+         withPositions( [&]( auto at ) {
+#pragma unroll
+            for ( int c = 0; c < 3; ++c )
+#pragma unroll
+               for ( int i = 0; i < 10; ++i )
+                  atomicAdd( &au[c * kSpreadBox + b1 + at( i )], y[c][i] );
+         } );
+   __syncthreads(); // the velocity values are read (SHARED: the results added)
    // lane, anchor and box points again, rather than kept through the quadrature loops
    int ones = -1;
    asm volatile( "" : "+s"( ones ) );
@@ -489,7 +584,7 @@ __global__ __launch_bounds__( LAST ? 64 : stokesTiles( MASK, LAST ) * kTileThrea
          {
             R v = ap[tid + j * kThreads];
 #pragma unroll
-            for ( int w = 1; w < kWaves; ++w )
+            for ( int w = 1; w < kPCopies; ++w )
                v += ap[w * kPBox3P + tid];
             sharedAdd( yp + base0 + uint32_t( o ), v );
          }
@@ -503,7 +598,17 @@ __global__ __launch_bounds__( LAST ? 64 : stokesTiles( MASK, LAST ) * kTileThrea
 #pragma unroll
       for ( int j = 0; j < kPoints; ++j )
          velocityPoint( tid, j, bp[j], off[j] );
-      if constexpr ( LAST )
+      auto writeBoxes = [&]( const R* box ) {
+#pragma unroll
+         for ( int j = 0; j < kPoints; ++j )
+            if ( off[j] >= 0 )
+#pragma unroll
+               for ( int c = 0; c < 3; ++c )
+                  sharedAdd( yout[c] + base1 + uint32_t( off[j] ), box[c * kSpreadBox + bp[j]] );
+      };
+      if constexpr ( SHARED )
+         writeBoxes( au );
+      else if constexpr ( LAST )
       {
          for ( int p = tid; p < 3 * kSpreadBox; p += 64 )
             su[p] = R( 0 );
@@ -514,12 +619,7 @@ __global__ __launch_bounds__( LAST ? 64 : stokesTiles( MASK, LAST ) * kTileThrea
             for ( int i = 0; i < 10; ++i )
                atomicAdd( &su[c * kSpreadBox + lanePos[i]], y[c][i] ); // every pair is a micro-cell
          __syncthreads();
-#pragma unroll
-         for ( int j = 0; j < kPoints; ++j )
-            if ( off[j] >= 0 )
-#pragma unroll
-               for ( int c = 0; c < 3; ++c )
-                  sharedAdd( yout[c] + base1 + uint32_t( off[j] ), su[c * kSpreadBox + bp[j]] );
+         writeBoxes( su );
       }
       else
       {
@@ -761,30 +861,34 @@ void zeroTarget( Context* ctx, Storage& st, Lattice& lat, T* d, bool replaceAll 
    HG_CHECK_HIP( hipGetLastError() );
 }
 
-// Levels of at least 4 micro-edges (a multiple of kTile): the interior tiles a workgroup
-// each and the last layer a wavefront each; smaller levels, one partial tile a cell, in
-// the general form.
 template < int MASK, class T >
 void launchStokes( Context* ctx, StokesOperator& op, const P2CellGeomT< typename Acc< T >::type >* geom, int L, Lattice& l1,
                    Lattice& l0, T* const u[3], const T* p, T* const y[3], T* yp )
 {
    using R          = typename Acc< T >::type;
    const int64_t mm = int64_t( 1 ) << L, T0 = tileEdges( mm );
-   auto launch = [&]( auto last, int kind, int64_t ntiles ) {
-      constexpr bool LAST = decltype( last )::value;
+   auto launch = [&]( auto which, int kind, int64_t ntiles ) {
+      constexpr int FORM = decltype( which )::value, kTiles = stokesTiles( MASK, FORM );
       if ( ntiles < 1 )
          return;
-      constexpr int kTiles = stokesTiles( MASK, LAST );
-      kStokesTileApply< MASK, T, LAST >
-          <<< xcdGrid( ( ntiles + kTiles - 1 ) / kTiles ), LAST ? 64 : kTiles * kTileThreads, 0, ctx->stream >>>(
+      kStokesTileApply< MASK, T, FORM >
+          <<< xcdGrid( ( ntiles + kTiles - 1 ) / kTiles ), FORM == kStokesLast ? 64 : kTiles * kTileThreads, 0, ctx->stream >>>(
           geom, R( op.c0 ), R( op.c1 ), mm, ntiles, l1.sc, l1.w, l0.sc, l0.w, u[0], u[1], u[2], p, y[0], y[1], y[2], yp,
           tileList( ctx, l1, mm, kind ) );
       HG_CHECK_HIP( hipGetLastError() );
    };
-   if ( mm < kTile )
-      return launch( std::false_type{}, kTilesAll, tilesPerCell( mm ) * l1.nc );
-   launch( std::false_type{}, kTilesInterior, tet( T0 - 1 ) * l1.nc );
-   launch( std::true_type{}, kTilesLast, T0 * ( T0 + 1 ) / 2 * l1.nc );
+   using Wide   = std::integral_constant< int, kStokesWide >;
+   using Shared = std::integral_constant< int, kStokesShared >;
+   using Last   = std::integral_constant< int, kStokesLast >;
+   const int64_t n = tilesPerCell( mm ) * l1.nc;
+   switch ( stokesForm( MASK, std::is_same< R, float >::value, mm, n ) )
+   {
+   case kStokesShared: launch( Shared{}, kTilesAll, n ); break;
+   case kStokesWide: launch( Wide{}, kTilesAll, n ); break;
+   default:
+      launch( Wide{}, kTilesInterior, tet( T0 - 1 ) * l1.nc );
+      launch( Last{}, kTilesLast, T0 * ( T0 + 1 ) / 2 * l1.nc );
+   }
 }
 
 // the velocity block alone on FP32 or FP16 velocity functions (FP32 arithmetic)

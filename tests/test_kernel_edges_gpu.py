@@ -9,7 +9,7 @@ the oracle:
   launch-by-launch iteration above, against the same iteration in numpy, over more
   iterations than one launch runs;
 * P2 restriction into levels whose face points fill several wavefronts;
-* the Stokes blocks over an odd number of interior tiles.
+* the Stokes blocks over an odd number of interior tiles, and by each of the apply's forms.
 """
 import ctypes as C
 
@@ -268,3 +268,55 @@ def test_stokes_blocks_over_odd_tile_counts(ctx, cells, L):
     lut[used] = np.arange(len(used))
     X, c = np.ascontiguousarray(X[used]), lut[c]
     _apply_parity(hg.PrimitiveStorage.from_cells(ctx, X, c), po.Mesh.from_arrays(X, c), L, (0.3, 0.5))
+
+
+# (mesh, level): launches of 24 tiles (one result box a tile), 480 (result boxes a wavefront),
+# 720 and 1200 (the last layer apart for the viscous masks only), 960 (three tiles in four
+# in the last layer) and 1920 of one micro-cell; level 2 has last-layer tiles only
+@pytest.mark.parametrize("mesh,L", [("cube", 3), ("cube", 2), ((2, 3), 3), ((3, 2), 3), ((3, 2), 2), ("cube32", 4),
+                                    ((2, 2), 4), ((5, 3), 0)])
+def test_stokes_masks_agree_over_the_forms(ctx, mesh, L):
+    """the blocks one by one, in pairs and all together, whose launches take different
+    forms, and the velocity block on FP32 and FP16 functions"""
+    st = (hg.PrimitiveStorage.shell(ctx, *mesh, 0.55, 1.0) if isinstance(mesh, tuple) else
+          hg.PrimitiveStorage.cuboid(ctx, n=(3, 2, 1) if mesh == "cube32" else (1, 1, 1)))
+    # (a viscosity whose results stay in the FP16 range, also at the cube's corner r = 0)
+    A = hg.P2P1StokesOperator(st, L, L, 0.3, 0.5)
+    src, dst = (hg.P2P1TaylorHoodFunction("f", st, L, L) for _ in range(2))
+    for k, f in enumerate([*src.uvw, src.p]):
+        f.interpolate_random(7 + k, -1.0, 1.0, L)
+
+    def apply(mask):
+        for f in (*dst.uvw, dst.p):
+            f.interpolate(0.0, L)
+        print(f"Stokes forms {mesh} L{L} mask {mask}", flush=True)
+        A.apply(src, dst, L, hg.ALL, hg.REPLACE, mask)
+        return dst.download(L)
+
+    u1, u2, p4 = apply(1)[0], apply(2)[0], apply(4)[1]
+    scale, pscale = np.abs(u1).max(), np.abs(p4).max()
+    # every result: sums over the micro-cells around a DoF (at most some hundred terms) in
+    # another order, of terms within a small factor of the largest result
+    tol = 1024 * EPS[hg.F64]
+    for mask in (3, 5, 6, 7):
+        u, p = apply(mask)
+        ref = (u1 if mask & 1 else 0.0) + (u2 if mask & 2 else 0.0)
+        assert np.abs(u - ref).max() <= tol * (scale if mask & 1 else np.abs(u2).max()), mask
+        if mask & 4:
+            assert np.abs(p - p4).max() <= tol * pscale, mask
+    for dtype in (hg.F32, hg.F16):
+        low, out = ([hg.P2Function("f", st, L, L, dtype) for _ in range(3)] for _ in range(2))
+        for a, f in zip(src.uvw, low):
+            f.copy_from(a, L)
+            a.copy_from(f, L)  # rounded to the storage type
+        ref = apply(1)[0]
+        hs, hd = (np.array([*(f.h for f in fs), 0], dtype=np.int64) for fs in (low, out))
+        print(f"Stokes forms {mesh} L{L} dtype {dtype}", flush=True)
+        ctx.check(lib().hg_stokes_apply(ctx.h, A.h, hs.ctypes.data_as(C.c_void_p), hd.ctypes.data_as(C.c_void_p), L, hg.ALL,
+                                        1, hg.REPLACE), "Stokes apply")
+        got = np.concatenate([f.download(L) for f in out])
+        # FP32 arithmetic throughout; FP16 results are rounded once a tile that adds to them
+        assert np.abs(got - ref).max() <= (1024 * EPS[hg.F32] if dtype == hg.F32 else 32 * EPS[hg.F16]) * np.abs(ref).max()
+        for f in (*low, *out):
+            f.destroy()
+    A.destroy()
