@@ -861,6 +861,19 @@ void zeroTarget( Context* ctx, Storage& st, Lattice& lat, T* d, bool replaceAll 
    HG_CHECK_HIP( hipGetLastError() );
 }
 
+// the lists that the launches on a lattice read, built ahead of a timed region, whatever
+// the mask: a launch captured after one of another mask cannot allocate its list
+void stokesTileLists( Context* ctx, Lattice& l1, int64_t mm )
+{
+   const int64_t n = tilesPerCell( mm ) * l1.nc;
+   for ( int mask = 0; mask <= 8; ++mask ) // 0: the velocity block in FP32
+      if ( stokesForm( mask ? mask : 1, mask == 0, mm, n ) != kStokesLast )
+         tileList( ctx, l1, mm, kTilesAll );
+      else
+         for ( int kind : { kTilesInterior, kTilesLast } )
+            tileList( ctx, l1, mm, kind );
+}
+
 template < int MASK, class T >
 void launchStokes( Context* ctx, StokesOperator& op, const P2CellGeomT< typename Acc< T >::type >* geom, int L, Lattice& l1,
                    Lattice& l0, T* const u[3], const T* p, T* const y[3], T* yp )
@@ -910,7 +923,7 @@ void stokesViscousLowPrecision( Context* ctx, StokesOperator& op, Function* cons
    const int64_t mm = int64_t( 1 ) << L;
    if ( l1.w > 1024 )
       throw Error( HG_ERR_UNSUPPORT, "Stokes apply supports levels up to 9 (32-bit lattice offsets)" );
-   const int64_t ntiles = tilesPerCell( mm ) * l1.nc;
+   stokesTileLists( ctx, l1, mm );
    dispatchType( dtype, [&]( auto tag ) {
       using T = decltype( tag );
       if constexpr ( std::is_same< T, double >::value )
@@ -999,8 +1012,7 @@ void stokesApply( Context* ctx, StokesOperator& op, Function* const src[4], Func
       yp = (double*) dst[3]->ptr( L );
       zeroTarget( ctx, st, l0, yp, update == HG_REPLACE && ( pflag & kInner ) );
    }
-   const int64_t ntiles = tilesPerCell( mm ) * l1.nc;
-   tileList( ctx, l1, mm, kTilesAll ); // built before the timed region on first use
+   stokesTileLists( ctx, l1, mm );
    ctx->beginTiming();
    switch ( mask )
    {

@@ -320,3 +320,61 @@ def test_stokes_masks_agree_over_the_forms(ctx, mesh, L):
         for f in (*low, *out):
             f.destroy()
     A.destroy()
+
+
+@pytest.mark.parametrize("dtype", [hg.F64, hg.F32])
+def test_stokes_kernel_time_of_a_first_apply_is_the_kernels(ctx, dtype):
+    """the first apply on a storage builds its tile lists ahead of the timed kernels"""
+    L, first, later = 4, [], []
+    ctx.event_timing(True)
+    try:
+        for k in range(6):
+            st = hg.PrimitiveStorage.cuboid(ctx, n=(3, 2, 1))
+            A = hg.P2P1StokesOperator(st, L, L, 0.3, 0.5)
+            fs = [hg.P2Function("f", st, L, L, dtype) for _ in range(6)]
+            hs, hd = (np.array([*(f.h for f in x), 0], dtype=np.int64) for x in (fs[:3], fs[3:]))
+            for f in fs[:3]:
+                f.interpolate_random(k, -1.0, 1.0, L)
+            for j in range(4):
+                print(f"Stokes kernel time, dtype {dtype}, storage {k}, apply {j}", flush=True)
+                ctx.check(lib().hg_stokes_apply(ctx.h, A.h, hs.ctypes.data_as(C.c_void_p), hd.ctypes.data_as(C.c_void_p), L,
+                                                hg.GMG_FLAG, 1, hg.REPLACE), "Stokes apply")
+                ctx.synchronize()
+                (later if j else first).append(ctx.last_ms())
+            for f in fs:
+                f.destroy()
+            A.destroy()
+    finally:
+        ctx.event_timing(False)
+    # (the first storage's launch loads the kernel's code)
+    assert min(first[1:]) < 2 * np.median(later), (first, np.median(later))
+
+
+def test_stokes_masks_can_be_captured_after_one_of_them(ctx):
+    """720 tiles, where the viscous masks and B^T read different tile lists: a capture,
+    which cannot allocate, finds the lists of every mask after an apply of one"""
+    L = 4
+    for eager, captured in ((1, 2), (2, 7)):
+        st = hg.PrimitiveStorage.cuboid(ctx, n=(3, 2, 1))
+        A = hg.P2P1StokesOperator(st, L, L, 0.3, 0.5)
+        src, dst = (hg.P2P1TaylorHoodFunction("f", st, L, L) for _ in range(2))
+        for k, f in enumerate([*src.uvw, src.p]):
+            f.interpolate_random(7 + k, -1.0, 1.0, L)
+        print(f"Stokes mask {captured} captured after mask {eager}", flush=True)
+        A.apply(src, dst, L, hg.ALL, hg.REPLACE, eager)
+        graph = C.c_int64()
+        ctx.check(lib().hg_graph_begin_capture(ctx.h), "begin capture")
+        try:
+            A.apply(src, dst, L, hg.ALL, hg.REPLACE, captured)
+        finally:
+            ctx.check(lib().hg_graph_end_capture(ctx.h, C.byref(graph)), "end capture")
+        A.apply(src, dst, L, hg.ALL, hg.REPLACE, captured)
+        ref = dst.download(L)[0]
+        for _ in range(3):
+            dst.interpolate(0.0, L)
+            ctx.check(lib().hg_graph_launch(ctx.h, graph), "graph launch")
+            assert relmax(dst.download(L)[0], ref) <= 64 * EPS[hg.F64]  # atomics, in any order
+        ctx.check(lib().hg_graph_destroy(ctx.h, graph), "graph destroy")
+        src.destroy()
+        dst.destroy()
+        A.destroy()
