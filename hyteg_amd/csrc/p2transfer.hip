@@ -695,16 +695,25 @@ __global__ __launch_bounds__( kBndThreads ) void kP2RestrictBnd( BndGeom gc, int
       coarse[( nc * gc.sc + b ) << lv] = fromAcc< T >( ( red[0] + red[1] ) + ( red[2] + red[3] ) );
 }
 
-// owned face DoFs (two incident cells each): a wavefront takes 64 points of one face
-// with one parity class (facePoints), so that the cell, the orientation and the stencil
-// -- the row groups of the cell kernel -- are uniform over it; the entries of a row are
-// gathered before they are summed.  Bound by the gathers of the two cells' fine rows.
+// the first point of each class in a face point list, and the first of the wavefronts of a
+// face that take it
+struct FaceWaves
+{
+   uint32_t point[5], wave[5];
+};
+
+// owned face DoFs (two incident cells each): a wavefront takes points of one face with one
+// parity class (facePoints), so that the cell, the orientation and the stencil -- the row
+// groups of the cell kernel -- are uniform over it, 64 of them, or of an interleaved
+// function 64 / 2^lv with all their vectors, whose values lie side by side; the entries of a
+// row are gathered before they are summed.  Bound by the gathers of the two cells' fine rows.
 // Shell level 5, FP64: 1.22 ms with a thread taking its DoF's entries one by one, 64-bit
 // indices and classes formed for each; 0.76 ms in this form, 0.65 ms with kRowsAhead rows
-// loaded before the first is summed.
+// loaded before the first is summed.  Eight FP64 vectors, shell levels 2 and 3, a launch:
+// 81 and 721 us a thread a DoF, 443 and 1185 us a wavefront a class and vector, 75 and 172 so.
 template < class T >
-__global__ __launch_bounds__( 256 ) void kP2RestrictBndFace( BndGeom gc, const uint32_t* __restrict__ pts,
-                                                             uint32_t wavesPerFace, uint32_t nfaces, int64_t nc,
+__global__ __launch_bounds__( 256 ) void kP2RestrictBndFace( BndGeom gc, const uint32_t* __restrict__ pts, FaceWaves fw,
+                                                             uint32_t nfaces, int64_t nc,
                                                              const uint8_t* __restrict__ bndFlag, int flag,
                                                              const double* __restrict__ maskInvN, int64_t scf, int32_t wf,
                                                              const T* __restrict__ fine, T* __restrict__ coarse, int lv )
@@ -715,18 +724,21 @@ __global__ __launch_bounds__( 256 ) void kP2RestrictBndFace( BndGeom gc, const u
       sliceStart[z] = int32_t( tet( wf ) - tet( wf - z ) );
    __syncthreads();
    const uint32_t wv = uint32_t( __builtin_amdgcn_readfirstlane( int( blockIdx.x * 4 + ( threadIdx.x >> 6 ) ) ) );
-   const uint32_t f  = wv / wavesPerFace;
+   const uint32_t f  = wv / fw.wave[4], w = wv - f * fw.wave[4];
    if ( f >= nfaces )
       return;
-   const uint32_t p  = pts[( wv - f * wavesPerFace ) * 64 + ( threadIdx.x & 63 )];
-   const int32_t  pa = int32_t( p & 0xFFFFu ), pb = int32_t( p >> 16 ), mmc = int32_t( gc.mm );
-   if ( p == 0xFFFFFFFFu )
+   const uint32_t cl = uint32_t( w >= fw.wave[1] ) + uint32_t( w >= fw.wave[2] ) + uint32_t( w >= fw.wave[3] );
+   const uint32_t at = fw.point[cl] + ( ( ( w - fw.wave[cl] ) * 64 + ( threadIdx.x & 63 ) ) >> lv );
+   if ( at >= fw.point[cl + 1] )
       return;
-   const int64_t b = gc.foff + int64_t( f ) * gc.fin + triIndex( mmc - 2, pa - 1, pb - 1 );
+   const uint32_t p  = pts[at];
+   const int32_t  pa = int32_t( p & 0xFFFFu ), pb = int32_t( p >> 16 ), mmc = int32_t( gc.mm );
+   const int64_t  b  = gc.foff + int64_t( f ) * gc.fin + triIndex( mmc - 2, pa - 1, pb - 1 );
+   const int      vec = int( threadIdx.x ) & ( ( 1 << lv ) - 1 );
    if ( !( bndFlag[b] & flag ) )
       return;
-   fine += blockIdx.y;
-   coarse += blockIdx.y;
+   fine += vec;
+   coarse += vec;
    const int32_t mmf = wf - 1;
    A             s   = A( 0 );
    for ( int32_t i = gc.fptr[f]; i < gc.fptr[f + 1]; ++i )
@@ -820,13 +832,13 @@ static void facePointList( Context* ctx, Lattice& l )
    std::vector< uint32_t > pts;
    for ( int q = 0; q < 4; ++q )
    {
+      l.faceClass[q] = uint32_t( pts.size() );
       for ( int64_t b = 1; b <= l.mm - 2; ++b )
          for ( int64_t a = 1; a + b <= l.mm - 1; ++a )
             if ( ( a & 1 ) + 2 * ( b & 1 ) == q )
                pts.push_back( uint32_t( a ) | ( uint32_t( b ) << 16 ) );
-      while ( pts.size() % 64 )
-         pts.push_back( 0xFFFFFFFFu );
    }
+   l.faceClass[4] = uint32_t( pts.size() );
    l.facePoints.upload( ctx, pts );
 }
 
@@ -881,10 +893,14 @@ void p2Restrict( Context* ctx, Function& f, int fineL, int flag )
          HG_CHECK_HIP( hipGetLastError() );
          if ( lc.nb > nve && lc.facePoints.p )
          {
-            const int64_t wpf = int64_t( lc.facePoints.n ) / 64;
-            kP2RestrictBndFace< T ><<< dim3( gridFor( wpf * st.topo.nf, 4 ), nv ), 256, 0, ctx->stream >>>(
-                gc, lc.facePoints.p, uint32_t( wpf ), uint32_t( st.topo.nf ), lc.nc, lc.bndFlag.p, flag, st.maskInvN.p,
-                lf.sc, int32_t( lf.w ), (const T*) fp, (T*) cp, lv );
+            FaceWaves fw{};
+            for ( int q = 0; q < 5; ++q )
+               fw.point[q] = lc.faceClass[q];
+            for ( int q = 0; q < 4; ++q )
+               fw.wave[q + 1] = fw.wave[q] + ( ( ( fw.point[q + 1] - fw.point[q] ) << lv ) + 63 ) / 64;
+            kP2RestrictBndFace< T ><<< gridFor( int64_t( fw.wave[4] ) * st.topo.nf, 4 ), 256, 0, ctx->stream >>>(
+                gc, lc.facePoints.p, fw, uint32_t( st.topo.nf ), lc.nc, lc.bndFlag.p, flag, st.maskInvN.p, lf.sc,
+                int32_t( lf.w ), (const T*) fp, (T*) cp, lv );
          }
          else if ( lc.nb > nve )
             kP2RestrictBndFaceGeneral< T ><<< dim3( gridFor( lc.nb - nve ), nv ), kBlock, 0, ctx->stream >>>(

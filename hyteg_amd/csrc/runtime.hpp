@@ -124,9 +124,10 @@ struct Lattice
    // (P2 prolongation into this lattice).
    DevBuf< uint32_t > prolongChunks;
 
-   // face-interior points (a | b << 16) grouped by (a mod 2, b mod 2), each group padded
-   // to whole wavefronts (0xFFFFFFFF).  Built on first use (P2 restriction).
+   // face-interior points (a | b << 16) grouped by (a mod 2, b mod 2), first point of each
+   // group.  Built on first use (P2 restriction).
    DevBuf< uint32_t > facePoints;
+   uint32_t           faceClass[5] = {};
 
    // tile lists of the P2 tile kernels on this lattice (all tiles, interior
    // tiles, last-layer tiles), built on first use

@@ -258,6 +258,32 @@ def test_p2_restriction_into_large_levels(ctx, name, L, dtype):
     f.destroy()
 
 
+@pytest.mark.parametrize("dtype", [hg.F64, hg.F32, hg.F16])
+@pytest.mark.parametrize("nvec", [2, 8, 64])
+@pytest.mark.parametrize("name,levels", [("octa", (1, 2, 3, 4)), ("shell", (1, 2))])
+def test_p2_restriction_of_interleaved_vectors(ctx, name, levels, nvec, dtype):
+    """each vector as alone, whether its face points fill a wavefront or share it with
+    other vectors"""
+    st = _storage(ctx, name) if name == "octa" else hg.PrimitiveStorage.shell(ctx, 2, 2, 0.55, 1.0)
+    for L in levels:
+        f, g = hg.P2Function("f", st, L - 1, L, dtype, nvec=nvec), hg.P2Function("g", st, L - 1, L, dtype)
+        rng = np.random.default_rng(nvec + L)
+        # values that every type holds exactly
+        fine = rng.uniform(-1, 1, (st.p2_ndofs(L), nvec)).astype(np.float16).astype(np.float64)
+        print(f"P2 restriction {name} {L}->{L - 1} nvec {nvec} dtype {dtype}", flush=True)
+        f.upload(L, fine)
+        f.upload(L - 1, np.zeros((st.p2_ndofs(L - 1), nvec)))
+        hg.restrict(f, L, hg.ALL)
+        got = f.download(L - 1)
+        for k in {0, 1, nvec // 2, nvec - 1}:
+            g.upload(L, fine[:, k])
+            g.upload(L - 1, np.zeros(st.p2_ndofs(L - 1)))
+            hg.restrict(g, L, hg.ALL)
+            assert np.array_equal(got[:, k], g.download(L - 1)), (L, k)  # the same sums in the same order
+        f.destroy()
+        g.destroy()
+
+
 @pytest.mark.parametrize("cells", [1, 3])
 @pytest.mark.parametrize("L", [2, 3, 4])
 def test_stokes_blocks_over_odd_tile_counts(ctx, cells, L):
