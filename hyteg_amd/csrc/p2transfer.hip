@@ -562,10 +562,12 @@ __global__ __launch_bounds__( kRestrictBlock ) void kP2RestrictCellList( const u
    const int32_t x = int32_t( p & 1023u ), y = int32_t( ( p >> 10 ) & 1023u ), z = int32_t( p >> 20 );
    // the wavefront's parity class (uniform over its points), from its first active lane
    const int q = __builtin_amdgcn_readfirstlane( int( x & 1 ) + 2 * int( y & 1 ) + 4 * int( z & 1 ) );
-   const int32_t mmf = wf - 1;
-   const T*      f   = fine + blockIdx.y + ( ( c * scf ) << lv );
-   A             v   = A( 0 );
-   // kRowsAhead fine rows' entries in flight together (shell level 5: 0.79 -> 0.75 ms)
+   const T* f = fine + blockIdx.y + ( ( c * scf ) << lv );
+   A        v = A( 0 );
+   // kRowsAhead fine rows' entries in flight together (shell level 5: 0.79 -> 0.75 ms).  An
+   // interior coarse point's basis function vanishes on the boundary, so that all its entries
+   // lie in the cell and no bounds are tested (one cell, FP32, a launch: 27.4 -> 22.1 us;
+   // eight FP64 vectors, shell level 3: 686 -> 571).
    const int ng = cRGN[q];
    for ( int g0 = 0; g0 < ng; g0 += kRowsAhead )
    {
@@ -575,20 +577,10 @@ __global__ __launch_bounds__( kRestrictBlock ) void kP2RestrictCellList( const u
       {
          const RowGroup rg = cRG[q][min( g0 + i, ng - 1 )];
          const int32_t  fy = 2 * y + rg.oy, fz = 2 * z + rg.oz;
-         const bool     in = g0 + i < ng && fy >= 0 && fz >= 0 && fy + fz <= mmf;
-         const int32_t  rs = in ? sliceStart[fz] + fy * ( wf - fz ) - fy * ( fy - 1 ) / 2 : 0;
-         const int32_t  lim = in ? mmf - fy - fz : -1;
+         const int32_t  rs = sliceStart[fz] + fy * ( wf - fz ) - fy * ( fy - 1 ) / 2 + 2 * x;
 #pragma unroll
          for ( int j = 0; j < 7; ++j )
-         {
-            buf[i][j] = A( 0 );
-            if ( j < rg.count )
-            {
-               const int32_t fx = 2 * x + cRGX[q][rg.first + j];
-               if ( fx >= 0 && fx <= lim )
-                  buf[i][j] = toAcc( f[int64_t( rs + fx ) << lv] );
-            }
-         }
+            buf[i][j] = j < rg.count ? toAcc( f[int64_t( rs + cRGX[q][rg.first + j] ) << lv] ) : A( 0 );
       }
 #pragma unroll
       for ( int i = 0; i < kRowsAhead; ++i )

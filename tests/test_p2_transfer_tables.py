@@ -36,6 +36,17 @@ def test_restriction_weights_match_reference_test(cls, expected):
     assert abs(w.sum() - expected) < 1e-13
 
 
+@pytest.mark.parametrize("mm", [4, 8])
+def test_restriction_of_an_interior_point_stays_in_the_cell(mm):
+    """the cell-interior restriction tests no bounds: every entry of an interior coarse
+    point of the smallest lattices (even micro-edge counts) is a point of the fine cell"""
+    stencils = [hg.p2_transfer_stencil(1, q)[0] for q in range(8)]
+    for x, y, z in itertools.product(range(1, mm), repeat=3):
+        if x + y + z < mm:
+            f = 2 * np.array([x, y, z]) + stencils[(x & 1) + 2 * (y & 1) + 4 * (z & 1)]
+            assert (f >= 0).all() and (f.sum(axis=1) <= 2 * mm).all()
+
+
 def test_restriction_is_transpose_of_pull():
     """every (fine, coarse, weight) triple of the pull tables on a patch appears in the
     restriction tables and vice versa"""
