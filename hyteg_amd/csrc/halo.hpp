@@ -251,13 +251,14 @@ inline HaloGeom haloGeom( const Storage& st, const Lattice& l )
 }
 
 // whether a lattice's halo exchange runs on the offset tables: cell-local offsets in
-// 32 bits and block counts within a grid (beyond that the general kernels run)
+// 32 bits and block counts within a grid (beyond that the general kernels run; the sums
+// of a mesh with a face of three or more cells too, Storage::facesShared2)
 inline bool haloTables( const Storage& st, const Lattice& l, int lv )
 {
    const int64_t most = int64_t( 1 ) << 31, nf = st.topo.nf, ne = st.topo.ne, nv = st.topo.nv;
    // threads of a launch over n primitives of `per` values: whole workgroups each, or packed
    auto threads = []( int64_t per, int64_t n ) { return ( per / kBlock + 1 ) * kBlock * n; };
-   return st.facesShared2 && l.haloOffsets.p && threads( l.haloPerCell() << lv, l.nc ) / kBlock < most &&
+   return l.haloOffsets.p && threads( l.haloPerCell() << lv, l.nc ) / kBlock < most &&
           ( l.haloPerCell() << lv ) < most && threads( l.num.fin << lv, nf ) / kBlock < most &&
           ( ( l.haloPerCell() << lv ) >= kBlock / 2 || ( l.haloPerCell() << lv ) * l.nc < most ) &&
           ( ( l.num.fin << lv ) >= kBlock / 2 || ( l.num.fin << lv ) * nf < most ) && ( l.num.ein << lv ) * ne < most &&

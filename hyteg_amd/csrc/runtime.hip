@@ -67,7 +67,7 @@ void Storage::init( Context* ctx )
          const int f = t.cf[c][k];
          if ( nfi[f] > 1 )
          {
-            facesShared2 = false; // the general halo kernels take any number
+            facesShared2 = false; // the general sum takes any number
             continue;
          }
          fi[4 * size_t( f ) + 2 * nfi[f]]     = c;
@@ -347,18 +347,45 @@ __global__ __launch_bounds__( kBlock ) void kPushAdditive( HaloGeom g, uint32_t 
    out = fromAcc< T >( s );
 }
 
-// the same for lattices of 2^31 points a cell and more (haloTables)
+// the same without tables (haloTables): offsets formed in 64 bits
 template < class T >
-__global__ void kPullGeneral( BndGeom g, int64_t nc, int64_t nb, int lv, T* __restrict__ v )
+__global__ void kPullGeneral( const CellMeta* __restrict__ meta, int64_t nc, int64_t sc, int64_t w, int64_t mm,
+                              int64_t fin, int64_t ein, int64_t eoff, int64_t foff, int lv, T* __restrict__ v )
 {
+   const int64_t per = 4 * fin + 6 * ein + 4;
    const int64_t tid = int64_t( blockIdx.x ) * blockDim.x + threadIdx.x;
-   const int64_t b = tid >> lv, vec = tid & ( ( int64_t( 1 ) << lv ) - 1 );
-   if ( b >= nb )
+   const int64_t gid = tid >> lv, vec = tid & ( ( int64_t( 1 ) << lv ) - 1 );
+   if ( gid >= per * nc )
       return;
-   const T val = v[( ( nc * g.sc + b ) << lv ) + vec];
-   forEachIncident( g, b, [&]( int64_t c, int64_t x, int64_t y, int64_t z, int ) {
-      v[( ( c * g.sc + tetIndex( g.w, x, y, z ) ) << lv ) + vec] = val;
-   } );
+   const int64_t   c = gid / per;
+   int64_t         j = gid - c * per;
+   const CellMeta& m = meta[c];
+   int64_t         t[4], src;
+   const int64_t   base = nc * sc;
+   if ( j < 4 * fin )
+   {
+      const int     k = int( j / fin );
+      const int64_t i = j - k * fin;
+      int64_t       a, b;
+      decodeTri( mm - 2, i, a, b );
+      faceToCell( m, k, mm, a + 1, b + 1, t );
+      src = base + foff + int64_t( m.face[k] ) * fin + i;
+   }
+   else if ( ( j -= 4 * fin ) < 6 * ein )
+   {
+      const int     k = int( j / ein );
+      const int64_t s = j - k * ein + 1;
+      edgeToCell( m, k, mm, s, t );
+      src = base + eoff + int64_t( m.edge[k] ) * ein + ( s - 1 );
+   }
+   else
+   {
+      const int k = int( j - 6 * ein );
+      t[0] = t[1] = t[2] = t[3] = 0;
+      t[k]                      = mm;
+      src                       = base + m.vert[k];
+   }
+   v[( ( c * sc + tetIndex( w, t[1], t[2], t[3] ) ) << lv ) + vec] = v[( src << lv ) + vec];
 }
 template < class T >
 __global__ void kPushGeneral( BndGeom g, const uint8_t* __restrict__ bndFlag, int64_t nb, int64_t nc, int excludeFlag,
@@ -369,11 +396,29 @@ __global__ void kPushGeneral( BndGeom g, const uint8_t* __restrict__ bndFlag, in
    const int64_t b = tid >> lv, vec = tid & ( ( int64_t( 1 ) << lv ) - 1 );
    if ( b >= nb || ( bndFlag[b] & excludeFlag ) )
       return;
-   T& out = v[( ( nc * g.sc + b ) << lv ) + vec];
-   A  s   = zeroOut ? A( 0 ) : toAcc( out );
-   forEachIncident( g, b, [&]( int64_t c, int64_t x, int64_t y, int64_t z, int ) {
-      s += toAcc( v[( ( c * g.sc + tetIndex( g.w, x, y, z ) ) << lv ) + vec] );
-   } );
+   T&      out = v[( ( nc * g.sc + b ) << lv ) + vec];
+   A       s   = zeroOut ? A( 0 ) : toAcc( out );
+   int32_t e0, e1;
+   incidentRange( g, b, e0, e1 );
+   for ( int32_t e = e0; e < e1; e += 8 )
+   {
+      A buf[8]; // loads in flight
+#pragma unroll
+      for ( int j = 0; j < 8; ++j )
+      {
+         buf[j] = A( 0 );
+         if ( e + j < e1 )
+         {
+            int64_t       x, y, z;
+            const int64_t c = incidentAt( g, b, e + j, x, y, z );
+            buf[j]          = toAcc( v[( ( c * g.sc + tetIndex( g.w, x, y, z ) ) << lv ) + vec] );
+         }
+      }
+#pragma unroll
+      for ( int j = 0; j < 8; ++j )
+         if ( e + j < e1 )
+            s += buf[j];
+   }
    out = fromAcc< T >( s );
 }
 
@@ -386,8 +431,9 @@ void pullHalos( Context* ctx, Storage& st, Lattice& lat, void* data, int dtype, 
    {
       dispatchType( dtype, [&]( auto tag ) {
          using T = decltype( tag );
-         kPullGeneral< T ><<< gridFor( lat.nb << lv ), kBlock, 0, ctx->stream >>>( BndGeom::of( st, lat ), lat.nc, lat.nb,
-                                                                                  lv, (T*) data );
+         kPullGeneral< T ><<< gridFor( per * lat.nc ), kBlock, 0, ctx->stream >>>( st.meta.p, lat.nc, lat.sc, lat.w, lat.mm,
+                                                                                  lat.num.fin, lat.num.ein, lat.num.eoff,
+                                                                                  lat.num.foff, lv, (T*) data );
       } );
       HG_CHECK_HIP( hipGetLastError() );
       return;
@@ -406,7 +452,7 @@ void pushAdditive( Context* ctx, Storage& st, Lattice& lat, void* data, int dtyp
 {
    if ( lat.nb == 0 )
       return;
-   if ( !haloTables( st, lat, lv ) )
+   if ( !st.facesShared2 || !haloTables( st, lat, lv ) )
    {
       dispatchType( dtype, [&]( auto tag ) {
          using T = decltype( tag );

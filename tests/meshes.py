@@ -12,6 +12,12 @@ def octahedron():
     return d["coords"], d["cells"]
 
 
+def three_on_a_face():
+    """three tetrahedra on one triangle (two of them on the same side)"""
+    X = np.array([[0, 0, 0], [1, 0, 0], [0, 1, 0], [0.2, 0.2, 1], [0.3, 0.3, -1], [1, 1, 0.4]], dtype=np.float64)
+    return X, np.array([[0, 1, 2, 3], [0, 1, 2, 4], [0, 1, 2, 5]], dtype=np.int64)
+
+
 def match(coords_a, coords_b, tol=1e-9):
     """permutation perm with coords_b[perm[i]] == coords_a[i]"""
     ka = np.round(np.asarray(coords_a) / tol).astype(np.int64)

@@ -8,6 +8,7 @@ the oracle:
 * the P2 coarse conjugate gradients on element matrices (levels 0 to 2) and the
   launch-by-launch iteration above, against the same iteration in numpy, over more
   iterations than one launch runs;
+* the halo exchange of a mesh with a face of three cells;
 * P2 restriction into levels whose face points fill several wavefronts;
 * the Stokes blocks over an odd number of interior tiles, and by each of the apply's forms.
 """
@@ -19,7 +20,7 @@ import pytest
 import hyteg_amd as hg
 from hyteg_amd import problems
 from hyteg_amd._lib import lib
-from meshes import octahedron, relmax
+from meshes import octahedron, relmax, three_on_a_face
 from oracle import pyoracle as po
 from test_stokes_gpu import _apply_parity
 
@@ -404,3 +405,58 @@ def test_stokes_masks_can_be_captured_after_one_of_them(ctx):
         src.destroy()
         dst.destroy()
         A.destroy()
+
+
+@pytest.mark.parametrize("L", [1, 2, 3, 4, 5])
+def test_a_face_of_three_cells(ctx, L):
+    """applies, sweeps and restriction, whose sums over a face's cells take the general kernel"""
+    X, c = three_on_a_face()
+    st, om = hg.PrimitiveStorage.from_cells(ctx, X, c), po.Mesh.from_arrays(X, c)
+    rng = np.random.default_rng(L)
+    n, n2, fl = om.ndofs(L), om.ndofs(L + 1), om.flags(L)
+    assert n == st.ndofs(L)
+    A, op = hg.P1ConstantLaplaceOperator(st, L, L), po.P1Op(om, L)
+    colour, _ = A.sor_colours(L)
+    csr, x0, b = op.csr(), rng.uniform(-1, 1, n), rng.uniform(-1, 1, n)
+    for nvec in (1, 4):
+        x, y = (hg.P1Function("f", st, L, L, nvec=nvec) for _ in range(2))
+
+        def put(f, v):
+            f.upload(L, v if nvec == 1 else np.repeat(v[:, None], nvec, axis=1))
+
+        def get(f):
+            return f.download(L).reshape(n, nvec)
+
+        print(f"three cells on a face: P1 L{L} nvec {nvec}", flush=True)
+        put(x, x0)
+        A.apply(x, y, L, hg.ALL)
+        ref = np.zeros(n)
+        op.apply(x0, ref, hg.ALL)
+        assert relmax(get(y), ref[:, None]) < 1e-12
+        for backward in (False, True):
+            put(x, x0)
+            put(y, b)
+            (A.smooth_sor_backwards if backward else A.smooth_sor)(x, y, 1.2, L, hg.ALL)
+            ref = po.sor_multicolour(csr, colour, (fl & hg.ALL) != 0, x0.copy(), b, 1.2, backward)
+            assert relmax(get(x), ref[:, None]) < 1e-12, backward
+        x.destroy()
+        y.destroy()
+    k = problems.shell_coefficient(3)
+    A2 = hg.P2DivKGradOperator(st, L, L, *k)
+    f = hg.P2Function("f", st, L - 1, L)
+    g = hg.P2Function("g", st, L, L)
+    v = rng.uniform(-1, 1, n2)
+    f.upload(L, v)
+    print(f"three cells on a face: P2 L{L}", flush=True)
+    A2.apply(f, g, L, hg.ALL)
+    ref = np.zeros(n2)
+    po.P2Op(om, L, po.KCoeff(*k)).apply(v, ref, hg.ALL, False)
+    assert relmax(g.download(L), ref) < 1e-12
+    ref = np.zeros(n)
+    f.upload(L - 1, ref)
+    hg.restrict(f, L, hg.ALL)
+    om.p2_restrict(L, v, ref, hg.ALL)
+    assert relmax(f.download(L - 1), ref) < 1e-12
+    f.destroy()
+    g.destroy()
+    A2.destroy()
