@@ -1610,8 +1610,10 @@ void p1Apply( Context* ctx, P1Operator& op, Function& src, Function& dst, int L,
 }
 
 // A sweep runs in one workgroup (per 2^lg vectors, lg = sweepVectorsLog) while x fits the
-// LDS budget, a boundary colour has at most about two points a thread and the interior
-// at most eight.
+// LDS budget, a boundary colour has at most about two points a thread and the interior at
+// most four: replayed from a graph, one workgroup against launches, 3640 interior points
+// (octahedron level 4) 36 against 42 us; 4495 (one cell, level 5) 30 against 26; four FP16
+// vectors of 36 cells at level 3 (5040) 65 against 43.
 static int    sweepVectorsLog( int lv ) { return std::min( lv, 2 ); }
 static size_t sweepLds( const Lattice& lat, size_t elem, int lv ) { return ( size_t( lat.nstore ) * elem ) << sweepVectorsLog( lv ); }
 static bool   sweepSmall( const Storage& st, const Lattice& lat, const P1OpLevel& o, size_t elem, int lv )
@@ -1621,7 +1623,7 @@ static bool   sweepSmall( const Storage& st, const Lattice& lat, const P1OpLevel
    const int     lg    = sweepVectorsLog( lv );
    const int64_t nc    = int64_t( o.sorColorStart.size() ) - 1;
    const int64_t inner = lat.nc * ( lat.mm >= 4 ? tet( lat.mm - 3 ) : 0 );
-   return ( o.sorColorStart.back() << lg ) <= 2 * kSweepThreads * nc && ( inner << lg ) <= 8 * kSweepThreads &&
+   return ( o.sorColorStart.back() << lg ) <= 2 * kSweepThreads * nc && ( inner << lg ) <= 4 * kSweepThreads &&
           sweepLds( lat, elem, lv ) <= kSweepLds && lat.nrows <= kSweepRows && lat.nc <= kSweepCells;
 }
 template < class T >
