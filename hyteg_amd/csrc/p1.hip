@@ -1721,8 +1721,8 @@ void p1SOR( Context* ctx, P1Operator& op, Function& x, Function& b, double relax
             return;
          if ( lv == 0 )
          {
-            // a lane more than the longest row has pairs, at least four
-            const int rpb = std::min( 4, rowsPerBlockLog( lat.mm / 2 + 1 ) );
+            // a lane more than the longest row (x < mm - 2) has pairs, at least four
+            const int rpb = std::min( 4, rowsPerBlockLog( lat.mm / 2 ) );
             const auto run = rpb == 0 ? kCellSORPairs< T, true > : kCellSORPairs< T, false >;
             run<<< cellGrid( n * lat.nc, rpb ), 64 * kCellWorkers, 0, ctx->stream >>>(
                 lat.rows.p + 2 * lat.rowGroup[grp], n, lat.nc, lat.sc, lat.w, lat.mm, o.stencil.p, cxFirst, relax,
