@@ -724,12 +724,19 @@ struct alignas( sizeof( T ) * V ) ValuePack
 // values a lane of the interleaved sweeps takes: 8 or 16 bytes, at most all vectors
 template < class T >
 constexpr int kPackLog = sizeof( T ) == 2 ? 2 : 1;
+// lanes that the packs of an interior launch leave at least, FP32 and FP16: on lattices
+// that a launch fills with less, the longer chain of a lane costs more than its wider loads
+// give (a sweep of four FP16 vectors, 36 cells at level 4: 45 us without packs, 49 with;
+// 32 vectors: 54 and 51).  FP64 gains at every size (32 vectors of one cell at level 5: 55
+// and 40 us)
+constexpr int64_t kPackLanes = 16384;
+// most: largest pack (log)
 template < class T, class F >
-static void forPack( int lv, F&& f )
+static void forPack( int most, F&& f )
 {
-   if ( lv >= kPackLog< T > )
+   if ( most >= kPackLog< T > )
       f( std::integral_constant< int, kPackLog< T > >{} );
-   else if ( lv == 1 )
+   else if ( most == 1 )
       f( std::integral_constant< int, 1 >{} );
    else
       f( std::integral_constant< int, 0 >{} );
@@ -1730,15 +1737,16 @@ void p1SOR( Context* ctx, P1Operator& op, Function& x, Function& b, double relax
             HG_CHECK_HIP( hipGetLastError() );
             return;
          }
-         forPack< T >( lv, [&]( auto lg ) {
+         int pack = lv;
+         const int64_t lanes = ( n * lat.nc * ( lat.mm / 4 ) ) << lv;
+         while ( sizeof( T ) < 8 && pack > 0 && ( lanes >> std::min( pack, kPackLog< T > ) ) < kPackLanes )
+            --pack;
+         forPack< T >( pack, [&]( auto lg ) {
             constexpr int lgV = decltype( lg )::value;
-            if constexpr ( lgV > 0 ) // single vectors: above
-            {
-               const int rpb = rowsPerBlockLog( ( ( lat.mm - 2 ) / 2 ) << ( lv - lgV ) );
-               kCellSOR< T, lgV ><<< cellGrid( n * lat.nc, rpb ), 64 * kCellWorkers, 0, ctx->stream >>>(
-                   lat.rows.p + 2 * lat.rowGroup[grp], n, lat.nc, lat.sc, lat.w, lat.mm, o.stencil.p, cxFirst, relax,
-                   (const T*) bp, (T*) xp, lv, rpb );
-            }
+            const int     rpb = rowsPerBlockLog( ( ( lat.mm - 2 ) / 2 ) << ( lv - lgV ) );
+            kCellSOR< T, lgV ><<< cellGrid( n * lat.nc, rpb ), 64 * kCellWorkers, 0, ctx->stream >>>(
+                lat.rows.p + 2 * lat.rowGroup[grp], n, lat.nc, lat.sc, lat.w, lat.mm, o.stencil.p, cxFirst, relax,
+                (const T*) bp, (T*) xp, lv, rpb );
          } );
          HG_CHECK_HIP( hipGetLastError() );
       };
