@@ -1088,7 +1088,9 @@ __global__ void __launch_bounds__( kBlock ) kBndApplySell( int64_t nblk, int64_t
 }
 
 // SOR on the boundary rows of one colour (slots of the sliced rows), 2^lgV vectors a lane
-// (64 FP16 vectors, cube level 6, a launch: 5.3 us one vector a lane, 4.5 us four)
+// (64 FP16 vectors, cube level 6, a launch: 5.3 us one vector a lane, 4.5 us four).  Packs
+// where they leave kPackLanes lanes, in every type: a sweep of two FP64 vectors, 240 cells
+// at level 4, 71 us with packs in small launches and 61 without.
 template < class T, int lgV >
 __global__ void __launch_bounds__( kBlock ) kBndSORSell( int64_t nblk, int64_t slot0, int64_t nslot,
                                                         const int32_t* __restrict__ rowOf,
@@ -1705,7 +1707,10 @@ void p1SOR( Context* ctx, P1Operator& op, Function& x, Function& b, double relax
          {
             const SellRows& sr    = o.sorRows;
             const int64_t   slot0 = o.sorColorStart[cc], ns = o.sorColorStart[cc + 1] - slot0;
-            forPack< T >( lv, [&]( auto lg ) {
+            int pack = lv;
+            while ( pack > 0 && ( ( ns << lv ) >> std::min( pack, kPackLog< T > ) ) < kPackLanes )
+               --pack;
+            forPack< T >( pack, [&]( auto lg ) {
                constexpr int lgV  = decltype( lg )::value;
                const int64_t nblk = ( ( ns << ( lv - lgV ) ) + kBlock - 1 ) / kBlock;
                kBndSORSell< T, lgV ><<< xcdGrid( nblk ), kBlock, 0, ctx->stream >>>(
