@@ -1,8 +1,9 @@
 """Kernel variants at the sizes where their rules change, against the general path or
 the oracle:
 
-* P1 Gauss-Seidel of single vectors (small sweeps in one workgroup, point pairs in
-  registers) against the interleaved form, which runs neither;
+* P1 Gauss-Seidel (small sweeps in one workgroup, point pairs in registers, interleaved
+  vectors in packs) against a sweep colour by colour on the oracle's matrix, and the forms
+  of large levels against each other;
 * P2 constant Gauss-Seidel (assembled rows) against a sweep colour by colour with the
   apply kernel;
 * the P2 coarse conjugate gradients on element matrices (levels 0 to 2) and the
@@ -26,6 +27,7 @@ from test_stokes_gpu import _apply_parity
 
 pytestmark = pytest.mark.gpu
 
+NUMPY = {hg.F64: np.float64, hg.F32: np.float32, hg.F16: np.float16}
 EPS = {hg.F64: 2.0**-53, hg.F32: 2.0**-24, hg.F16: 2.0**-11}
 
 
@@ -33,9 +35,53 @@ def _storage(ctx, name):
     return hg.PrimitiveStorage.cuboid(ctx) if name == "cube" else hg.PrimitiveStorage.from_cells(ctx, *octahedron())
 
 
+def _colour_sweep(A, colour, free, x, b, relax, backward, dtype):
+    """a multicolour sweep of all vectors in FP64 with the results of each colour rounded
+    to the storage type"""
+    d = A.diagonal()[:, None]
+    for c in sorted(set(colour[free]), reverse=backward):
+        r = free & (colour == c)
+        new = (1.0 - relax) * x[r] + relax / d[r] * (b[r] - A[r] @ x + d[r] * x[r])
+        x[r] = new.astype(NUMPY[dtype])
+    return x
+
+
 @pytest.mark.parametrize("dtype", [hg.F64, hg.F32, hg.F16])
-@pytest.mark.parametrize("name,levels", [("cube", range(1, 9)), ("octa", range(1, 7))])
-def test_p1_sweep_variants_equal_the_interleaved_sweep(ctx, name, levels, dtype):
+@pytest.mark.parametrize("name", ["cube", "octa"])
+def test_p1_sweeps_equal_the_sweep_by_colours(ctx, name, dtype):
+    """levels on both sides of the one-workgroup sweep's limit (cube 4 and octahedron 4 for
+    one vector, 3 for several), by vectors: one to four in a workgroup and several workgroups"""
+    st = _storage(ctx, name)
+    om = po.Mesh.cuboid() if name == "cube" else po.Mesh.from_arrays(*octahedron())
+    for L in range(1, 6):
+        A, csr = hg.P1ConstantLaplaceOperator(st, L, L), po.P1Op(om, L).csr()
+        colour, _ = A.sor_colours(L)
+        n = st.ndofs(L)
+        for nvec in (1, 2, 4, 8):
+            rng = np.random.default_rng(10 * L + nvec)
+            x0, b = (rng.uniform(-1, 1, (n, nvec)).astype(np.float16).astype(np.float64) for _ in range(2))
+            x, fb = (hg.P1Function("f", st, L, L, dtype, nvec=nvec) for _ in range(2))
+            fb.upload(L, b.reshape(n) if nvec == 1 else b)
+            for flag, relax, backward in ((hg.GMG_FLAG, 1.0, False), (hg.ALL, 1.3, True)):
+                print(f"P1 sweep by colours {name} L{L} nvec {nvec} dtype {dtype} backward {backward}", flush=True)
+                x.upload(L, x0.reshape(n) if nvec == 1 else x0)
+                (A.smooth_sor_backwards if backward else A.smooth_sor)(x, fb, relax, L, flag)
+                ref = _colour_sweep(csr, colour, (om.flags(L) & flag) != 0, x0.copy(), b, relax, backward, dtype)
+                # rows of at most 30 entries, summed in FP64 or FP32 in another order, whose
+                # errors later colours take in with row sums below 2; FP16: roundings that the
+                # FP32 sum's error turns, at most one a colour and value
+                tol = 64 * EPS[dtype] if dtype != hg.F16 else 8 * EPS[dtype]
+                assert relmax(x.download(L).reshape(n, nvec), ref) <= tol, (L, nvec, backward)
+            x.destroy()
+            fb.destroy()
+
+
+@pytest.mark.parametrize("dtype", [hg.F64, hg.F32, hg.F16])
+@pytest.mark.parametrize("name,levels", [("cube", range(5, 9)), ("octa", range(5, 7))])
+def test_p1_sweep_by_pairs_equals_the_interleaved_sweep(ctx, name, levels, dtype):
+    """point pairs in registers (one vector) against the sweep of two interleaved vectors,
+    with rows shorter and longer than a wavefront's pairs (levels above the one-workgroup
+    sweep's)"""
     st = _storage(ctx, name)
     for L in levels:
         A = hg.P1ConstantLaplaceOperator(st, L, L)
@@ -64,10 +110,11 @@ def test_p1_sweep_variants_equal_the_interleaved_sweep(ctx, name, levels, dtype)
 @pytest.mark.parametrize("dtype", [hg.F64, hg.F32, hg.F16])
 @pytest.mark.parametrize("nvec", [2, 4, 8, 64])
 def test_p1_interleaved_sweep_by_vectors_a_lane(ctx, nvec, dtype):
-    """every width of the interleaved sweep's packs (1, 2 or 4 vectors a lane) on levels
-    with more and with fewer points a row than a wavefront takes: each vector as alone"""
+    """every width of the interleaved sweep's packs (1, 2 or 4 vectors a lane, by the number
+    of lanes) on levels above the one-workgroup sweep's limit for several vectors: each
+    vector as alone (in one workgroup at level 4, in point pairs at level 5)"""
     st = hg.PrimitiveStorage.cuboid(ctx)
-    for L in (3, 5):
+    for L in (4, 5):
         A = hg.P1ConstantLaplaceOperator(st, L, L)
         n = st.ndofs(L)
         rng = np.random.default_rng(nvec + L)
