@@ -10,7 +10,8 @@ the oracle:
   launch-by-launch iteration above, against the same iteration in numpy, over more
   iterations than one launch runs;
 * the halo exchange of a mesh with a face of three cells;
-* P2 restriction into levels whose face points fill several wavefronts;
+* P2 restriction into levels whose face points fill several wavefronts, of interleaved
+  vectors, and from a lattice too wide for the point lists;
 * the Stokes blocks over an odd number of interior tiles, and by each of the apply's forms.
 """
 import ctypes as C
@@ -304,6 +305,35 @@ def test_p2_restriction_into_large_levels(ctx, name, L, dtype):
         assert relmax(f.download(L - 1), ref) < (1e-12 if dtype == hg.F64 else 256 * EPS[hg.F32] if dtype == hg.F32
                                                  else 2 * EPS[hg.F16]), flag
     f.destroy()
+
+
+def test_p2_restriction_from_a_wide_lattice(ctx):
+    """level 10 of one cell (2049 points an edge), beyond the lists of cell and face points:
+    the restriction of 1 is a constant on each class of boundary points, so that its sums
+    over the boundary are polynomials of degree 2 in the edge length, exact in FP16"""
+    X, c = octahedron()
+    used = np.unique(c[:1])
+    lut = np.zeros(len(X), dtype=c.dtype)
+    lut[used] = np.arange(len(used))
+    st = hg.PrimitiveStorage.from_cells(ctx, np.ascontiguousarray(X[used]), np.ascontiguousarray(lut[c[:1]]))
+    sums = {}
+    for L in (3, 4, 5, 6, 10):
+        f, one = hg.P2Function("f", st, L - 1, L, hg.F16), hg.P2Function("g", st, L - 1, L - 1, hg.F16)
+        print(f"P2 restriction of 1 on one cell {L}->{L - 1}", flush=True)
+        f.interpolate(1.0, L)
+        f.interpolate(0.0, L - 1)
+        one.interpolate(1.0, L - 1)
+        hg.restrict(f, L, hg.ALL)
+        sums[L] = np.array([f.dot(one, L - 1, hg.DIRICHLET), f.dot(f, L - 1, hg.DIRICHLET)])
+        f.destroy()
+        one.destroy()
+    edge = np.array([2.0**L for L in sums])
+    V = np.vander(edge[:3], 3)
+    for j in range(2):
+        coef = np.linalg.solve(V, np.array([sums[L][j] for L in (3, 4, 5)]))
+        for L in (6, 10):
+            want = np.polyval(coef, 2.0**L)
+            assert abs(sums[L][j] - want) <= 1e-12 * want, (L, j)
 
 
 @pytest.mark.parametrize("dtype", [hg.F64, hg.F32, hg.F16])
