@@ -170,7 +170,8 @@ struct P2Operator : OperatorBase
    std::map< int, DevBuf< P2ActGeomT< float > > >  ageomF; // the same for the FP32 kernels
    DevBuf< KParams >      kpar;
    std::map< int, DevBuf< double > > invDiag; // by P2 level, lattice L+1 storage
-   // k at the quadrature points (tile-major), by (level, value type of the table)
+   // coefficients at the quadrature points (tile-major; p2Coefficients), by (level, value
+   // type of the table)
    std::map< std::pair< int, int >, DevBuf< char > > kq;
    // reduced element form of the FP32 / FP16 applies (the preconditioner of the
    // mixed-precision refinement): on levels >= reducedFrom every micro-cell is
@@ -1344,11 +1345,10 @@ __global__ __launch_bounds__( 64 ) void kP2SmallApply( const P2ActGeomT< typenam
    }
 }
 
-// k at the quadrature points of level L (built on first use when the operator
-// stores coefficients; nullptr when it evaluates k in the apply kernel)
-// k at the quadrature points of level L in value type K (built on first use
-// when the operator stores coefficients; nullptr when it evaluates k in the
-// apply kernel)
+// the coefficient table of level L in value type K -- FP64: foldedCoefficient, k times
+// the factors of the metric that depend on the point only; FP32 and FP16: k itself --
+// built on first use when the operator stores coefficients (nullptr when it evaluates
+// them in the apply kernel)
 template < class K >
 static const K* p2Coefficients( Context* ctx, P2Operator& op, int L, int dtype )
 {
@@ -1586,7 +1586,7 @@ void p2Apply( Context* ctx, P2Operator& op, Function& src, Function& dst, int L,
    void*         d   = dst.ptr( L );
    const int64_t mm  = int64_t( 1 ) << L;
    if ( lat.w > 1024 )
-      throw Error( HG_ERR_UNSUPPORT, "P2 apply supports levels up to 9 (32-bit lattice offsets)" );
+      throw Error( HG_ERR_UNSUPPORT, "P2 apply supports levels up to 8 (32-bit lattice offsets)" );
    if ( op.nslot > 1 )
    {
       p2ApplyBatched( ctx, op, lat, L, src, dst, flag, update, alpha );
@@ -1990,7 +1990,7 @@ __global__ __launch_bounds__( kCgThreads ) void kP2AssembledCG( int32_t n, int32
                y[j] -= f;
             }
             if ( i == 2 )
-               __builtin_amdgcn_sched_barrier( 0 ); // 24 values in flight: all 45 spill
+               __builtin_amdgcn_sched_barrier( 0 ); // 24 values in flight (with the loop around, eight registers spill)
          }
 #pragma unroll
          for ( int i = 0; i < 10; ++i )

@@ -669,7 +669,7 @@ int hg_p2_const_apply( hg_ctx* h, hg_handle opH, hg_handle src, hg_handle dst, i
       Lattice&      lat = st.lattice( ctx, level + 1 );
       const int64_t mm  = int64_t( 1 ) << level;
       if ( lat.w > 1024 )
-         throw Error( HG_ERR_UNSUPPORT, "P2 apply supports levels up to 9 (32-bit lattice offsets)" );
+         throw Error( HG_ERR_UNSUPPORT, "P2 apply supports levels up to 8 (32-bit lattice offsets)" );
       double* sp = (double*) s.ptr( level );
       double* dp = (double*) d.ptr( level );
       pullHalos( ctx, st, lat, sp, 0 );

@@ -106,7 +106,8 @@ __device__ __forceinline__ TileCoord tileOf( int64_t lb, int64_t mm )
 // kernels read their tile from a per-lattice list instead, one scalar load:
 // entry = c | ti << 32 | tj << 40 | tk << 48 (cell, anchor / kTile).  List kTilesAll
 // follows tileOf; kTilesInterior holds the tiles with ti + tj + tk <= T - 2 (T: tile
-// edge count, at most 255: level 9), kTilesLast the last layer, both cell by cell.
+// edge count, at most 64: P2 level 8, where the tile kernels' 32-bit lattice offsets
+// end, BoxOffsets), kTilesLast the last layer, both cell by cell.
 enum TileListKind
 {
    kTilesAll      = 0,
@@ -116,8 +117,8 @@ enum TileListKind
 inline const uint64_t* tileList( Context* ctx, Lattice& l, int64_t mm, int kind )
 {
    const int64_t T = tileEdges( mm );
-   if ( T > 255 )
-      throw Error( -6, "P2 tile kernels support levels up to 9" );
+   if ( l.w > 1024 )
+      throw Error( -6, "P2 tile kernels support levels up to 8 (32-bit lattice offsets)" );
    DevBuf< uint64_t >& buf = l.tileLists[kind];
    if ( !buf.p )
    {

@@ -788,7 +788,8 @@ __global__ __launch_bounds__( 256 ) void kP2RestrictBndFace( BndGeom gc, const u
    }
    coarse[( nc * gc.sc + b ) << lv] = fromAcc< T >( s );
 }
-// the same, a thread per DoF, for fine lattices wider than kMaxSlices
+// the same, a thread per DoF, for fine lattices wider than kMaxSlices (P2 levels of 10
+// and more, which functions have and no operator)
 template < class T >
 __global__ void kP2RestrictBndFaceGeneral( BndGeom gc, int64_t nbc, int64_t nc, const uint8_t* __restrict__ bndFlag,
                                            int flag, const double* __restrict__ clsInvN, int64_t scf, int64_t wf,
@@ -875,8 +876,8 @@ void p2Restrict( Context* ctx, Function& f, int fineL, int flag )
       }
       if ( lc.nb > 0 )
       {
-         // macro-vertex and -edge DoFs (many incident cells): a wavefront each;
-         // face DoFs: a thread each
+         // macro-vertex and -edge DoFs (many incident cells): a workgroup each; face DoFs:
+         // a wavefront for the points of a class
          const BndGeom gc = BndGeom::of( st, lc );
          const int64_t nve = std::min( gc.foff, lc.nb );
          if ( nve > 0 )

@@ -922,7 +922,7 @@ void stokesViscousLowPrecision( Context* ctx, StokesOperator& op, Function* cons
    Lattice&      l0 = st.lattice( ctx, L );
    const int64_t mm = int64_t( 1 ) << L;
    if ( l1.w > 1024 )
-      throw Error( HG_ERR_UNSUPPORT, "Stokes apply supports levels up to 9 (32-bit lattice offsets)" );
+      throw Error( HG_ERR_UNSUPPORT, "Stokes apply supports levels up to 8 (32-bit lattice offsets)" );
    stokesTileLists( ctx, l1, mm );
    dispatchType( dtype, [&]( auto tag ) {
       using T = decltype( tag );
@@ -983,7 +983,7 @@ void stokesApply( Context* ctx, StokesOperator& op, Function* const src[4], Func
    Lattice&      l0 = st.lattice( ctx, L );
    const int64_t mm = int64_t( 1 ) << L;
    if ( l1.w > 1024 )
-      throw Error( HG_ERR_UNSUPPORT, "Stokes apply supports levels up to 9 (32-bit lattice offsets)" );
+      throw Error( HG_ERR_UNSUPPORT, "Stokes apply supports levels up to 8 (32-bit lattice offsets)" );
    double* u[3] = { nullptr, nullptr, nullptr };
    double* y[3] = { nullptr, nullptr, nullptr };
    double* p    = nullptr;
