@@ -57,50 +57,25 @@ void Storage::init( Context* ctx )
          m[c].ecode[k] = codeOf( edgeOrient, std::array< int8_t, 2 >{ m[c].eperm[k][0], m[c].eperm[k][1] } );
    }
    meta.upload( ctx, m );
-   std::vector< int32_t >                  fi( 4 * size_t( t.nf ), -1 ), ei;
-   std::vector< std::vector< int32_t > >   ec( t.ne );
-   std::vector< int >                      nfi( t.nf, 0 );
-   for ( int c = 0; c < t.nc; ++c )
-   {
-      for ( int k = 0; k < 4; ++k )
-      {
-         const int f = t.cf[c][k];
-         if ( nfi[f] > 1 )
-         {
-            facesShared2 = false; // the general sum takes any number
-            continue;
-         }
-         fi[4 * size_t( f ) + 2 * nfi[f]]     = c;
-         fi[4 * size_t( f ) + 2 * nfi[f] + 1] = m[c].fcode[k];
-         ++nfi[f];
-      }
-      for ( int k = 0; k < 6; ++k )
-      {
-         ec[t.ce[c][k]].push_back( c );
-         ec[t.ce[c][k]].push_back( m[c].ecode[k] );
-      }
-   }
-   for ( const auto& l : ec )
-      ei.insert( ei.end(), l.begin(), l.end() );
-   faceInc.upload( ctx, fi );
-   edgeInc.upload( ctx, ei );
-
-   auto csr = [&]( int nprim, auto primOfLocal, int nlocal, DevBuf< int32_t >& ptr, DevBuf< int32_t >& ent ) {
-      std::vector< std::vector< int32_t > > lists( nprim );
+   PackedUpload< int32_t > inc;
+   auto csr = [&]( int nprim, auto primOfLocal, int nlocal, DevView< int32_t >& ptr, DevView< int32_t >& ent ) {
+      std::vector< int32_t > p( nprim + 1, 0 ), e( 2 * size_t( t.nc ) * size_t( nlocal ) );
+      for ( int c = 0; c < t.nc; ++c )
+         for ( int k = 0; k < nlocal; ++k )
+            ++p[primOfLocal( c, k ) + 1];
+      for ( int i = 0; i < nprim; ++i )
+         p[i + 1] += p[i];
+      std::vector< int32_t > next( p.begin(), p.end() - 1 );
       for ( int c = 0; c < t.nc; ++c )
          for ( int k = 0; k < nlocal; ++k )
          {
-            lists[primOfLocal( c, k )].push_back( c );
-            lists[primOfLocal( c, k )].push_back( k );
+            const int32_t at = next[primOfLocal( c, k )]++;
+            e[2 * size_t( at )]     = c;
+            e[2 * size_t( at ) + 1] = k;
          }
-      std::vector< int32_t > p( nprim + 1, 0 ), e;
-      for ( int i = 0; i < nprim; ++i )
-      {
-         p[i + 1] = p[i] + int32_t( lists[i].size() / 2 );
-         e.insert( e.end(), lists[i].begin(), lists[i].end() );
-      }
-      ptr.upload( ctx, p );
-      ent.upload( ctx, e );
+      inc.add( ptr, p );
+      inc.add( ent, e );
+      return std::make_pair( p, e );
    };
    std::vector< double > inv( 14 * size_t( t.nc ) );
    for ( int c = 0; c < t.nc; ++c )
@@ -112,7 +87,6 @@ void Storage::init( Context* ctx )
       for ( int k = 0; k < 4; ++k )
          inv[14 * c + 10 + k] = 1.0 / t.vnc[t.cv[c][k]];
    }
-   clsInvN.upload( ctx, inv );
    std::vector< double > byMask( 16 * size_t( t.nc ), 1.0 );
    for ( int c = 0; c < t.nc; ++c )
    {
@@ -125,10 +99,32 @@ void Storage::init( Context* ctx )
       for ( int k = 0; k < 6; ++k )
          byMask[16 * size_t( c ) + size_t( 15 ^ edgeKeep[k] )] = inv[14 * size_t( c ) + 4 + k];
    }
-   maskInvN.upload( ctx, byMask );
-   csr( t.nf, [&]( int c, int k ) { return t.cf[c][k]; }, 4, faceCellPtr, faceCells );
-   csr( t.ne, [&]( int c, int k ) { return t.ce[c][k]; }, 6, edgeCellPtr, edgeCells );
+   PackedUpload< double > weights;
+   weights.add( clsInvN, inv );
+   weights.add( maskInvN, byMask );
+   weights.upload( ctx, inverses );
+   const auto faces = csr( t.nf, [&]( int c, int k ) { return t.cf[c][k]; }, 4, faceCellPtr, faceCells );
+   const auto edges = csr( t.ne, [&]( int c, int k ) { return t.ce[c][k]; }, 6, edgeCellPtr, edgeCells );
+   // the same with orientations: the first two cells of a face, all of an edge
+   std::vector< int32_t > fi( 4 * size_t( t.nf ), -1 ), ei( edges.second );
+   for ( int f = 0; f < t.nf; ++f )
+      for ( int32_t i = faces.first[f]; i < faces.first[f + 1]; ++i )
+      {
+         const int32_t j = i - faces.first[f], c = faces.second[2 * size_t( i )];
+         if ( j > 1 )
+         {
+            facesShared2 = false; // the general sum takes any number
+            break;
+         }
+         fi[4 * size_t( f ) + 2 * j]     = c;
+         fi[4 * size_t( f ) + 2 * j + 1] = m[c].fcode[faces.second[2 * size_t( i ) + 1]];
+      }
+   for ( size_t i = 0; i < ei.size(); i += 2 )
+      ei[i + 1] = m[ei[i]].ecode[ei[i + 1]];
+   inc.add( faceInc, fi );
+   inc.add( edgeInc, ei );
    csr( t.nv, [&]( int c, int k ) { return t.cv[c][k]; }, 4, vertCellPtr, vertCells );
+   inc.upload( ctx, incidences );
 }
 
 Lattice& Storage::lattice( Context* ctx, int L )
@@ -167,6 +163,7 @@ Lattice& Storage::lattice( Context* ctx, int L )
             }
    l.cellMask.upload( ctx, mask );
 
+   PackedUpload< int32_t > tables;
    if ( l.sc < ( int64_t( 1 ) << 31 ) )
    {
       const int64_t fin = l.num.fin, ein = l.num.ein, mm = l.mm;
@@ -190,8 +187,7 @@ Lattice& Storage::lattice( Context* ctx, int L )
             t[p[1]]      = s;
             o.push_back( int32_t( tetIndex( l.w, t[1], t[2], t[3] ) ) );
          }
-      o.push_back( 0 ); // never empty
-      l.haloOffsets.upload( ctx, o );
+      tables.add( l.haloOffsets, o );
    }
 
    std::vector< int32_t > rows;
@@ -209,7 +205,7 @@ Lattice& Storage::lattice( Context* ctx, int L )
    }
    l.rowGroup[4] = int64_t( rows.size() / 2 );
    l.nrows       = l.rowGroup[4];
-   l.rows.upload( ctx, rows );
+   tables.add( l.rows, rows );
    rows.clear();
    for ( int64_t z = 1; z <= l.mm - 3; ++z )
       for ( int64_t y = 1; y + z <= l.mm - 2; ++y )
@@ -217,7 +213,9 @@ Lattice& Storage::lattice( Context* ctx, int L )
          rows.push_back( int32_t( y ) );
          rows.push_back( int32_t( z ) );
       }
-   l.rowsNat.upload( ctx, rows );
+   rows.push_back( 0 ); // never empty
+   tables.add( l.rowsNat, rows );
+   tables.upload( ctx, l.tables );
 
    lattices[L] = std::move( lp );
    return l;

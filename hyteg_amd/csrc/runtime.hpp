@@ -67,6 +67,33 @@ struct DevBuf
    void release();
 };
 
+// Several host arrays uploaded into one allocation (an upload waits for its copy, some
+// 15 us): add() them, each with the view that upload() points into the allocation, at
+// multiples of 64 values.
+template < class T >
+struct DevView
+{
+   T* p = nullptr;
+};
+template < class T >
+struct PackedUpload
+{
+   std::vector< T >                                h;
+   std::vector< std::pair< DevView< T >*, size_t > > parts;
+   void add( DevView< T >& view, const std::vector< T >& v )
+   {
+      h.resize( ( h.size() + 63 ) / 64 * 64 );
+      parts.push_back( { &view, h.size() } );
+      h.insert( h.end(), v.begin(), v.end() );
+   }
+   void upload( Context* c, DevBuf< T >& buf )
+   {
+      buf.upload( c, h );
+      for ( auto& [view, at] : parts )
+         view->p = buf.p + at;
+   }
+};
+
 // Per-cell topology as seen from the cell: ids of its faces/edges/vertices and
 // which cell-local vertex each of their (sorted) vertices is.  Level-free.
 struct CellMeta
@@ -100,8 +127,8 @@ struct Lattice
 
    // interior rows (y,z) of a cell lattice, y,z >= 1, y+z <= mm-2, grouped by
    // (y%2, z%2); group g = (y%2) + 2*(z%2) occupies [rowGroup[g], rowGroup[g+1])
-   DevBuf< int32_t > rows; // 2 ints per row
-   DevBuf< int32_t > rowsNat; // the same rows in natural order (z-major, then y)
+   DevView< int32_t > rows; // 2 ints per row
+   DevView< int32_t > rowsNat; // the same rows in natural order (z-major, then y)
    int64_t           rowGroup[5] = { 0, 0, 0, 0, 0 };
    int64_t           nrows       = 0;
 
@@ -139,7 +166,8 @@ struct Lattice
    // cell-local offsets of the halo points by orientation: the face interiors of
    // every face orientation of the storage (num.fin each), then the edge interiors of
    // every edge orientation (num.ein each); empty where they do not fit 32 bits.
-   DevBuf< int32_t > haloOffsets;
+   DevView< int32_t > haloOffsets;
+   DevBuf< int32_t >  tables; // holds these, rows and rowsNat
 
    int64_t cellPos( int c, int64_t x, int64_t y, int64_t z ) const { return c * sc + tetIndex( w, x, y, z ); }
    int64_t ownerPos( const Topology& t, int c, int64_t x, int64_t y, int64_t z ) const
@@ -167,15 +195,17 @@ struct Storage
    DevBuf< CellMeta >                           meta;
    // 1 / (number of cells) of each cell's local faces (0..3), edges (4..9) and
    // vertices (10..13): nc*14
-   DevBuf< double >                             clsInvN;
+   DevView< double >                            clsInvN;
    // the same by the zero pattern of a cell point's barycentric weights (bit 0:
    // x + y + z = mm, 1: x = 0, 2: y = 0, 3: z = 0; no bit: 1): nc*16
-   DevBuf< double >                             maskInvN;
+   DevView< double >                            maskInvN;
    // cells incident to each face / edge / vertex: CSR of (cell, local index)
-   DevBuf< int32_t > faceCellPtr, faceCells, edgeCellPtr, edgeCells, vertCellPtr, vertCells;
+   DevView< int32_t > faceCellPtr, faceCells, edgeCellPtr, edgeCells, vertCellPtr, vertCells;
    // the same incidences as (cell, orientation): two entries a face (cell -1: none),
    // the edges' in the order of edgeCellPtr
-   DevBuf< int32_t >                       faceInc, edgeInc;
+   DevView< int32_t >                      faceInc, edgeInc;
+   DevBuf< int32_t >                       incidences; // holds these and the six above
+   DevBuf< double >                        inverses;   // holds clsInvN and maskInvN
    bool                                    facesShared2 = true; // every face has at most two cells
    std::vector< std::array< int8_t, 3 > > faceOrient; // CellMeta::fperm by fcode
    std::vector< std::array< int8_t, 2 > > edgeOrient; // CellMeta::eperm by ecode
