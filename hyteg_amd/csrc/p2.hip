@@ -364,30 +364,39 @@ __device__ __forceinline__ double foldedCoefficient( const P2CellGeom& g, const 
 // for threads outside the macro-cell).  FP64 tables hold foldedCoefficient, so
 // that the apply reads one value per point and forms no reciprocal square root;
 // FP32 and FP16 tables hold k itself, whose range those types can represent.
-template < class K >
-__global__ __launch_bounds__( kTileThreads ) void kP2TileCoefficients( const P2CellGeom* __restrict__ geom,
-                                                                      const KParams* __restrict__ kp, int64_t mm,
-                                                                      int64_t ntiles, K* __restrict__ table )
+// Entries outside the macro-cell keep the zeros of the table's allocation.  LAST: the
+// last-layer tiles, a wavefront each over the 64 micro-cells inside the macro-cell
+// (cDiagPairs), where the 16 sines and the exponential of a point would otherwise be
+// evaluated for six wavefronts of 4 to 20 active lanes (shell level 3, three tiles in four
+// in the last layer: 1.20 ms with them, 0.55 this way; level 6 216 and 204).
+template < class K, bool LAST >
+__global__ __launch_bounds__( LAST ? 64 : kTileThreads ) void kP2TileCoefficients( const P2CellGeom* __restrict__ geom,
+                                                                                   const KParams* __restrict__ kp,
+                                                                                   int64_t mm, int64_t ntiles,
+                                                                                   const uint64_t* __restrict__ tiles,
+                                                                                   K* __restrict__ table )
 {
-   const int64_t lb = blockIdx.x;
-   if ( lb >= ntiles )
+   const int64_t li = blockIdx.x;
+   if ( li >= ntiles )
       return;
-   const TileCoord            tc = tileOf( lb, mm );
+   int64_t         lb = li;
+   const TileCoord tc = tiles ? tileFromList( tiles, li, mm, lb ) : tileOf( li, mm );
+   const int       pair = LAST ? cDiagPairs[threadIdx.x] : 0;
+   const int       t = LAST ? pair & 7 : int( threadIdx.x ) >> 6, a = LAST ? pair >> 3 : int( threadIdx.x ) & 63;
    const P2CellGeom&          g  = geom[tc.c];
-   const TileThread< double > th = tileThread( g, tc, mm );
+   const TileThread< double > th = tileThreadAt( g, tc, mm, t, a );
+   if ( !th.valid )
+      return;
    for ( int q = 0; q < 11; ++q )
    {
-      const double* xq   = g.XQ[th.t][q];
+      const double* xq   = g.XQ[t][q];
       const double  x[3] = { th.p0[0] + xq[0], th.p0[1] + xq[1], th.p0[2] + xq[2] };
-      double        v    = 0.0;
+      double        v;
       if constexpr ( std::is_same< K, double >::value )
-      {
-         if ( th.valid )
-            v = foldedCoefficient( g, *kp, th.t, q, x, th.ls0 + xq[3] );
-      }
-      else if ( th.valid )
+         v = foldedCoefficient( g, *kp, t, q, x, th.ls0 + xq[3] );
+      else
          v = kAt( g, *kp, x, th.ls0 + xq[3] );
-      table[( lb * 11 + q ) * kTileThreads + threadIdx.x] = fromAcc< K >( typename Acc< K >::type( v ) );
+      table[( lb * 11 + q ) * kTileThreads + 64 * t + a] = fromAcc< K >( typename Acc< K >::type( v ) );
    }
 }
 
@@ -1345,6 +1354,25 @@ __global__ __launch_bounds__( 64 ) void kP2SmallApply( const P2ActGeomT< typenam
    }
 }
 
+template < class K >
+static void p2FillCoefficients( Context* ctx, P2Operator& op, int L, const KParams* kp, K* table )
+{
+   Lattice&          lat  = op.st->lattice( ctx, L + 1 );
+   const int64_t     mm   = int64_t( 1 ) << L, T = tileEdges( mm );
+   const P2CellGeom* geom = op.tgeom.at( L ).p;
+   auto fill = [&]( auto last, const uint64_t* tiles, int64_t n ) {
+      constexpr bool LAST = decltype( last )::value;
+      if ( n > 0 )
+         kP2TileCoefficients< K, LAST ><<< gridFor( n, 1 ), LAST ? 64 : kTileThreads, 0, ctx->stream >>>( geom, kp, mm, n,
+                                                                                                     tiles, table );
+      HG_CHECK_HIP( hipGetLastError() );
+   };
+   if ( mm <= kSmallMaxMM )
+      return fill( std::false_type{}, nullptr, lat.nc );
+   fill( std::false_type{}, tileList( ctx, lat, mm, kTilesInterior ), tet( T - 1 ) * lat.nc );
+   fill( std::true_type{}, tileList( ctx, lat, mm, kTilesLast ), tri( T ) * lat.nc );
+}
+
 // the coefficient table of level L in value type K -- FP64: foldedCoefficient, k times
 // the factors of the metric that depend on the point only; FP32 and FP16: k itself --
 // built on first use when the operator stores coefficients (nullptr when it evaluates
@@ -1364,9 +1392,7 @@ static const K* p2Coefficients( Context* ctx, P2Operator& op, int L, int dtype )
    buf.alloc( ctx, size_t( per * op.nslot ) * sizeof( K ) );
    op.tableStride[L] = per;
    for ( int sl = 0; sl < op.nslot; ++sl )
-      kP2TileCoefficients< K ><<< gridFor( ntiles, 1 ), kTileThreads, 0, ctx->stream >>>(
-          op.tgeom.at( L ).p, op.kpar.p + sl, mm, ntiles, (K*) buf.p + sl * per );
-   HG_CHECK_HIP( hipGetLastError() );
+      p2FillCoefficients( ctx, op, L, op.kpar.p + sl, (K*) buf.p + sl * per );
    return (const K*) buf.p;
 }
 
@@ -1744,12 +1770,8 @@ static void p2SetSlot( Context* ctx, P2Operator& op, int sl, const KParams& kp )
    {
       if ( key.second != 0 )
          continue; // batched operators build FP64 tables only
-      const int     L      = key.first;
-      const int64_t mm     = int64_t( 1 ) << L;
-      const int64_t ntiles = tilesPerCell( mm ) * int64_t( op.st->topo.nc );
-      kP2TileCoefficients< double ><<< gridFor( ntiles, 1 ), kTileThreads, 0, ctx->stream >>>(
-          op.tgeom.at( L ).p, op.kpar.p + sl, mm, ntiles, (double*) buf.p + sl * op.tableStride.at( L ) );
-      HG_CHECK_HIP( hipGetLastError() );
+      const int L = key.first;
+      p2FillCoefficients( ctx, op, L, op.kpar.p + sl, (double*) buf.p + sl * op.tableStride.at( L ) );
    }
    for ( auto& [L, buf] : op.invDiag )
       p2RefreshSlotDiagonal( ctx, op, L, sl );
