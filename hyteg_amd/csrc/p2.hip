@@ -1367,8 +1367,11 @@ static void p2FillCoefficients( Context* ctx, P2Operator& op, int L, const KPara
                                                                                                      tiles, table );
       HG_CHECK_HIP( hipGetLastError() );
    };
-   if ( mm <= kSmallMaxMM )
-      return fill( std::false_type{}, nullptr, lat.nc );
+   // few tiles: one launch, whose latency counts (cube level 3, 24 tiles, a first apply: 146 us,
+   // 183 with two)
+   const int64_t n = tilesPerCell( mm ) * lat.nc;
+   if ( mm <= kSmallMaxMM || n < 1024 )
+      return fill( std::false_type{}, nullptr, n );
    fill( std::false_type{}, tileList( ctx, lat, mm, kTilesInterior ), tet( T - 1 ) * lat.nc );
    fill( std::true_type{}, tileList( ctx, lat, mm, kTilesLast ), tri( T ) * lat.nc );
 }
