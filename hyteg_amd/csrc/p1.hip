@@ -750,8 +750,9 @@ static void forPack( int most, F&& f )
 // workgroup-scope fence between the two passes makes the first pass's stores
 // visible to the second (the result is that of two colour sweeps in turn).
 // Interleaved functions; a lane takes 2^lgV vectors.  Bound by the rounds of loads of a
-// row: 64 FP16 vectors, cube level 6, a launch: 19.8 us with a lane a vector, 15.0 us with four
-// (31 rounds of 16 two-byte loads a row, now 8 of eight-byte loads).
+// row: 64 FP16 vectors, the launches of cube levels 4 to 6 in V-cycles: 19.8 us on average
+// with a lane a vector, 15.0 us with four (at level 6 31 rounds of 16 two-byte loads a row
+// against 8 of eight-byte loads).
 template < class T, int lgV >
 __global__ __launch_bounds__( 64 * kCellWorkers ) void kCellSOR( const int32_t* __restrict__ rows, int64_t nrows,
                                                                  int64_t nc, int64_t sc, int64_t w, int64_t mm,
@@ -1088,7 +1089,8 @@ __global__ void __launch_bounds__( kBlock ) kBndApplySell( int64_t nblk, int64_t
 }
 
 // SOR on the boundary rows of one colour (slots of the sliced rows), 2^lgV vectors a lane
-// (64 FP16 vectors, cube level 6, a launch: 5.3 us one vector a lane, 4.5 us four).  Packs
+// (64 FP16 vectors, cube levels 4 to 6 in V-cycles, a launch on average: 5.3 us one vector a
+// lane, 4.5 us four).  Packs
 // where they leave kPackLanes lanes, in every type: a sweep of two FP64 vectors, 240 cells
 // at level 4, 71 us with packs in small launches and 61 without.
 template < class T, int lgV >
